@@ -139,9 +139,10 @@ def draw(rng):
 # ---- what a program has in hand before the call ----
 
 class _Shared:
-    """A device buffer of the library as an array that torch can take without a copy."""
+    """A device buffer of the library as an array that torch can take without a copy; keeps the batch it belongs to."""
 
-    def __init__(self, pointer, count):
+    def __init__(self, owner, pointer, count):
+        self.owner = owner
         self.__cuda_array_interface__ = dict(shape=(count,), typestr="<i4", data=(pointer, False), version=3)
 
 
@@ -200,8 +201,8 @@ def _prepare_step(case, seed):
     s["batch"].select(s["params"])
     if case["evaluator"] == "gpu":
         d = s["batch"].device()
-        s["leaf"] = torch.as_tensor(_Shared(d.d_leaf, n), device="cuda")
-        s["path_len"] = torch.as_tensor(_Shared(d.d_path_len, n), device="cuda")
+        s["leaf"] = torch.as_tensor(_Shared(s["batch"], d.d_leaf, n), device="cuda")
+        s["path_len"] = torch.as_tensor(_Shared(s["batch"], d.d_path_len, n), device="cuda")
     s["forest"].sync()
     return s
 
