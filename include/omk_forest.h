@@ -309,8 +309,7 @@ int omk_batch_set_stats(omk_batch *b, int32_t enabled);
  * word 4 = time of its boundaries | time of its batches << 32 (100 MHz clock) and word 5 = entries its
  * boundaries put in its batch (-1: it searched for the batch itself) | visitors it settled << 32; the other
  * words are 0.
- * h_trace has room for max_entries records; the records live in the staging memory of
- * omk_batch_read until the next call of it. */
+ * h_trace has room for max_entries records (a select records 16384 at most). */
 int omk_debug_trace(omk_batch *b, long long *h_trace, int32_t max_entries, int32_t *h_n);
 /* Switches the recording of that timeline on or off for the selects that follow (off by default: a
  * record costs one atomic and twelve stores per work item). */

@@ -67,6 +67,14 @@ struct omk_forest {
     int32_t *alias = nullptr;
     bool redirected = false;
     size_t key_stage_bytes = 0;
+    // The way between the host and the kernels: one block of pinned memory that both sides address (see link_*).
+    char *link = nullptr;
+    size_t link_bytes = 0;
+    size_t link_used = 0;         // staging handed out since the stream was last known to be idle
+    int32_t link_seq = 0;         // number of the last call that waited
+    int32_t *link_count = nullptr;  // HostSignal::count
+    // counts the calls that change N or child ranges: what was read of them before is stale after
+    int64_t changes = 0;
     int children = 0;       // live batches and tables created on this forest
     bool released = false;  // omk_forest_destroy was called while children were alive
 
@@ -108,6 +116,7 @@ constexpr int kSchedStep = 1024;  // int32 words between two scheduler words: 4 
 // Simulations cut by max_depth: two counters, used in turn (select calls of even / odd number).  Every
 // select clears the counter of the next one, so that a select of lone traversals needs no reset launch.
 constexpr int kTruncatedWord = 40;
+constexpr int kTraceCap = 16384;  // records of the timeline of one select
 
 struct omk_batch {
     omk_forest *f = nullptr;
@@ -143,8 +152,9 @@ struct omk_batch {
     int32_t spin_limit = 1 << 18;  // polls of about a microsecond: a quarter of a second, a selection takes a millisecond
     int32_t n_cus = 0;
     int32_t n_items0 = 0;
-    int32_t *out_paths = nullptr, *out_actions = nullptr;  // row-major staging for the host
-    int64_t out_ints = 0;  // int32 words of out_paths
+    int32_t *out = nullptr;  // the leaf gather of the last read, in pinned memory (see omk_batch_read)
+    size_t out_bytes = 0;
+    long long *trace = nullptr;  // records of the timeline, kTraceCap of them
     void *exp_buf = nullptr;  // staging of an expansion: jobs, moves, priors, status
     size_t exp_bytes = 0;
 };
@@ -190,6 +200,66 @@ static int tt_work(omk_tt *tt, size_t bytes) {
 template <typename T>
 static hipError_t dalloc(T **p, int64_t count) {
     return hipMalloc((void **)p, (size_t)std::max<int64_t>(count, 1) * sizeof(T));
+}
+
+// ---- the host's side of the pinned block ----
+//
+// A copy of a few hundred bytes between pageable memory and the card costs 12 us (to the card) to 20 us (back)
+// on an MI355X, and hipStreamSynchronize 5 us more than a kernel's store into pinned memory that the host polls.
+// So a call's inputs are copied into the staging part of this block, which the kernels read through the host
+// link, and its results come back into pinned memory, followed by the call's number in the flag word.
+// Staging is handed out front to back; once a call has seen its flag everything enqueued before has run, and
+// the next one starts at the front again.
+constexpr size_t kLinkHead = 4096;         // flag word, and behind it (64 bytes on) the results of small calls
+constexpr size_t kLinkStaging = 256 << 10; // staging a forest starts with
+static hipError_t link_alloc(omk_forest *f, size_t staging) {
+    char *p = nullptr;
+    hipError_t e = hipHostMalloc((void **)&p, kLinkHead + staging, hipHostMallocDefault);
+    if (e != hipSuccess) return e;
+    if (f->link) (void)hipHostFree(f->link);
+    f->link = p;
+    f->link_bytes = kLinkHead + staging;
+    f->link_used = 0;
+    *(int32_t *)p = f->link_seq;
+    return hipSuccess;
+}
+
+// `bytes` of staging, aligned to a cache line; valid until the next call that waits for the stream.
+static int link_stage(omk_forest *f, size_t bytes, void **out) {
+    bytes = (bytes + 127) & ~(size_t)127;
+    if (kLinkHead + f->link_used + bytes > f->link_bytes) {
+        HIP_TRY(hipStreamSynchronize(f->stream));
+        f->link_used = 0;
+        if (kLinkHead + bytes > f->link_bytes) HIP_TRY(link_alloc(f, bytes + bytes / 2));
+    }
+    *out = f->link + kLinkHead + f->link_used;
+    f->link_used += bytes;
+    return OMK_OK;
+}
+
+static HostSignal link_signal(omk_forest *f) {
+    f->link_seq = (int32_t)((uint32_t)f->link_seq + 1u);
+    return HostSignal{f->link_count, (int32_t *)f->link, f->link_seq};
+}
+
+// Waits for the kernel that carries the last link_signal.  A wait of more than about a millisecond goes to the
+// runtime, which does not burn the core and reports an error of the stream.
+static int link_wait(omk_forest *f) {
+    const int32_t *flag = (const int32_t *)f->link;
+    for (int i = 0; i < 20000; i++) {
+        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == f->link_seq) {
+            f->link_used = 0;
+            return OMK_OK;
+        }
+#if defined(__x86_64__)
+        __builtin_ia32_pause();
+#endif
+    }
+    HIP_TRY(hipStreamSynchronize(f->stream));
+    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != f->link_seq)
+        return fail(OMK_ERR_HIP, "the kernel that was waited for did not report");
+    f->link_used = 0;
+    return OMK_OK;
 }
 
 static int use_device(const omk_forest *f) {
@@ -246,6 +316,9 @@ int omk_forest_create(const omk_forest_desc *desc, omk_forest **out) {
     if (e == hipSuccess && f->has_rave) e = dalloc(&f->rN, n);
     if (e == hipSuccess && f->has_rave) e = dalloc(&f->rW, n);
     if (e == hipSuccess && f->has_rave) e = dalloc(&f->Q2, n);
+    if (e == hipSuccess) e = dalloc(&f->link_count, 64);
+    if (e == hipSuccess) e = launch_fill_words(f->link_count, 0u, 64, f->own_stream);
+    if (e == hipSuccess) e = link_alloc(f, kLinkStaging);
     if (e != hipSuccess) {
         int rc = fail(OMK_ERR_HIP, "omk_forest_create: %s", hipGetErrorString(e));
         omk_forest_destroy(f);
@@ -259,9 +332,10 @@ int omk_forest_create(const omk_forest_desc *desc, omk_forest **out) {
 static void forest_free(omk_forest *f) {
     (void)hipSetDevice(f->device);
     if (f->own_stream) (void)hipStreamSynchronize(f->own_stream);
-    void *ptrs[] = {f->span, f->N, f->W, f->P, f->VL, f->rN, f->rW, f->Q2, f->action, f->legal, f->hash, f->key_stage, f->alias};
+    void *ptrs[] = {f->span, f->N, f->W, f->P, f->VL, f->rN, f->rW, f->Q2, f->action, f->legal, f->hash, f->key_stage, f->alias, f->link_count};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    if (f->link) (void)hipHostFree(f->link);
     if (f->own_stream) (void)hipStreamDestroy(f->own_stream);
     (void)hipGetLastError();
     delete f;
@@ -964,10 +1038,6 @@ int omk_batch_create(omk_forest *f, int32_t max_traversals, int32_t max_depth, o
     if (e == hipSuccess) e = dalloc(&b->single_ready, max_traversals);
     if (e == hipSuccess) e = hipMemset(b->single_ready, 0, (size_t)std::max(max_traversals, 1) * 4);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&b->n_cus, hipDeviceAttributeMultiprocessorCount, f->device);
-    // (also the staging of the timeline records, omk_debug_trace: room for 16384 of them at least)
-    b->out_ints = std::max<int64_t>(B * (max_depth + 1), 24 * 16384);
-    if (e == hipSuccess) e = dalloc(&b->out_paths, b->out_ints);
-    if (e == hipSuccess) e = dalloc(&b->out_actions, B * max_depth);
     if (e == hipSuccess) e = hipMemset(b->values, 0, (size_t)B * 4);
     if (e != hipSuccess) {
         int rc = fail(OMK_ERR_HIP, "omk_batch_create: %s", hipGetErrorString(e));
@@ -983,10 +1053,11 @@ int omk_batch_destroy(omk_batch *b) {
     (void)hipSetDevice(b->f->device);
     (void)hipStreamSynchronize(b->f->stream);
     void *ptrs[] = {b->paths,  b->path_len, b->leaf,     b->values, b->items0,   b->items_q,  b->seg0,
-                    b->seg[0], b->seg[1],   b->sc_child, b->sc_occ, b->counters, b->out_paths, b->out_actions,
+                    b->seg[0], b->seg[1],   b->sc_child, b->sc_occ, b->counters, b->trace,
                     b->singles0, b->singles_q, b->q_ready, b->hctx, b->hbound, b->exp_buf, b->list_flag, b->single_ready};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    if (b->out) (void)hipHostFree(b->out);
     (void)hipGetLastError();
     forest_child_gone(b->f);
     delete b;
@@ -1071,8 +1142,10 @@ int omk_batch_set_values(omk_batch *b, const float *h_values, int32_t n) {
     if (!b || !h_values) return fail(OMK_ERR_INVALID, "omk_batch_set_values: null argument");
     if (n <= 0 || n > b->max_traversals) return fail(OMK_ERR_CAPACITY, "omk_batch_set_values: %d values", n);
     if (int rc = use_device(b->f)) return rc;
-    HIP_TRY(hipMemcpyAsync(b->values, h_values, (size_t)n * 4, hipMemcpyHostToDevice, b->f->stream));
-    HIP_TRY(hipStreamSynchronize(b->f->stream));
+    void *staged = nullptr;
+    if (int rc = link_stage(b->f, (size_t)n * 4, &staged)) return rc;
+    memcpy(staged, h_values, (size_t)n * 4);
+    HIP_TRY(launch_copy_words(b->values, staged, n, b->f->stream));
     return OMK_OK;
 }
 
@@ -1159,9 +1232,9 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
     a.list_flag = b->list_flag;
     static_assert(kHeavyCtxInts >= 16 + OMK_MAX_FANOUT, "context too small");
     a.times = b->counters + 26;
-    a.trace = b->trace_on ? (long long *)b->out_paths : nullptr;  // staging that only omk_batch_read uses
+    a.trace = b->trace_on ? b->trace : nullptr;
     a.trace_n = b->counters + 24;
-    a.trace_cap = (int32_t)(b->out_ints / 24);
+    a.trace_cap = kTraceCap;
     a.singles0 = b->singles0;
     a.singles_q = b->singles_q;
     a.sc_child = b->sc_child;
@@ -1448,18 +1521,38 @@ int omk_batch_read(omk_batch *b, int32_t *h_paths, int32_t *h_path_len, int32_t 
     if (int rc = fresh_batch("omk_batch_read", b)) return rc;
     omk_forest *f = b->f;
     if (int rc = use_device(f)) return rc;
-    hipStream_t s = f->stream;
-    const int n = b->n, D = b->max_depth;
-    if (h_paths || h_actions)
-        HIP_TRY(launch_export(f->dev(), b->paths, b->path_len, n, b->stride, D, h_paths ? b->out_paths : nullptr,
-                              h_actions ? b->out_actions : nullptr, s));
-    if (h_paths) HIP_TRY(hipMemcpyAsync(h_paths, b->out_paths, (size_t)n * (D + 1) * 4, hipMemcpyDeviceToHost, s));
-    if (h_actions) HIP_TRY(hipMemcpyAsync(h_actions, b->out_actions, (size_t)n * D * 4, hipMemcpyDeviceToHost, s));
-    if (h_path_len) HIP_TRY(hipMemcpyAsync(h_path_len, b->path_len, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-    if (h_leaf) HIP_TRY(hipMemcpyAsync(h_leaf, b->leaf, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-    int32_t ab[4] = {0, 0, 0, 0};  // abort flag and what the wavefront that raised it was waiting for
-    HIP_TRY(hipMemcpyAsync(ab, b->counters + 3 * kSchedStep + 1, sizeof(ab), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    const size_t n = (size_t)b->n, D = (size_t)b->max_depth;
+    // pinned: lengths | leaves | their child counts | their visit counts | abort words | paths | actions
+    const size_t ints = n * (2 * D + 5) + 4;
+    if (ints * 4 > b->out_bytes) {
+        if (b->out) {
+            HIP_TRY(hipStreamSynchronize(f->stream));
+            HIP_TRY(hipHostFree(b->out));
+        }
+        b->out = nullptr;
+        b->out_bytes = 0;
+        const size_t room = (size_t)b->stride * (2 * D + 5) * 4 + 64;
+        HIP_TRY(hipHostMalloc((void **)&b->out, room, hipHostMallocDefault));
+        b->out_bytes = room;
+    }
+    ExportOut o;
+    int32_t *at = b->out;
+    o.len = at;
+    o.leaf = at += n;
+    o.children = at += n;
+    o.visits = at += n;
+    o.abort = at += n;
+    int32_t *rows = at + 4;
+    o.paths = h_paths ? rows : nullptr;
+    o.actions = h_actions ? rows + n * (D + 1) : nullptr;
+    HIP_TRY(launch_export(f->dev(), b->paths, b->path_len, b->leaf, b->counters + 3 * kSchedStep + 1, b->n, b->stride,
+                          b->max_depth, o, link_signal(f), f->stream));
+    if (int rc = link_wait(f)) return rc;
+    if (h_paths) memcpy(h_paths, o.paths, n * (D + 1) * 4);
+    if (h_actions) memcpy(h_actions, o.actions, n * D * 4);
+    if (h_path_len) memcpy(h_path_len, o.len, n * 4);
+    if (h_leaf) memcpy(h_leaf, o.leaf, n * 4);
+    const int32_t *ab = o.abort;  // abort flag and what the wavefront that raised it was waiting for
     if (ab[0] == 1)
         return fail(OMK_ERR_STATE,
                     "omk_batch_read: the selection gave up (a wavefront waited longer than the spin limit for item %d "
@@ -1547,14 +1640,18 @@ int omk_debug_trace(omk_batch *b, long long *h_trace, int32_t max_entries, int32
     if (int rc = use_device(b->f)) return rc;
     HIP_TRY(hipStreamSynchronize(b->f->stream));
     HIP_TRY(hipMemcpy(h_n, b->counters + 24, 4, hipMemcpyDeviceToHost));
-    int32_t n = std::min(std::min(*h_n, max_entries), (int32_t)(b->out_ints / 24));
-    if (n > 0) HIP_TRY(hipMemcpy(h_trace, b->out_paths, (size_t)n * 96, hipMemcpyDeviceToHost));
+    int32_t n = std::min(std::min(*h_n, max_entries), kTraceCap);
+    if (n > 0) HIP_TRY(hipMemcpy(h_trace, b->trace, (size_t)n * 96, hipMemcpyDeviceToHost));
     *h_n = n;
     return OMK_OK;
 }
 
 int omk_batch_set_trace(omk_batch *b, int32_t enabled) {
     if (!b) return fail(OMK_ERR_INVALID, "omk_batch_set_trace: null batch");
+    if (enabled && !b->trace) {
+        if (int rc = use_device(b->f)) return rc;
+        HIP_TRY(dalloc(&b->trace, 12ll * kTraceCap));
+    }
     b->trace_on = enabled != 0;
     return OMK_OK;
 }

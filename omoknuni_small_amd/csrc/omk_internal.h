@@ -128,9 +128,25 @@ hipError_t launch_backup(const ForestDev &f, const int32_t *paths, const int32_t
 hipError_t launch_blend_all(const ForestDev &f, float rave_k, hipStream_t s);
 hipError_t launch_blend_paths(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                               int max_len, float rave_k, hipStream_t s);
-// row-major copies for the host: paths [n][max_depth+1], actions [n][max_depth], -1 padded
-hipError_t launch_export(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
-                         int max_depth, int32_t *out_paths, int32_t *out_actions, hipStream_t s);
+
+// How a kernel tells the waiting host that its results lie in pinned memory: the last block to finish stores
+// `seq` to the host's flag word.  `count` is a device word that is zero between two such kernels.
+struct HostSignal {
+    int32_t *count;
+    int32_t *flag;
+    int32_t seq;
+};
+// Where the leaf gather of a batch goes (pinned host memory that the kernel writes itself; any of the first two
+// may be null): row-major paths [n][max_depth+1] and actions [n][max_depth], -1 padded; per traversal the path
+// length, the leaf, and the leaf's child and visit count; the four abort words of the selection.
+struct ExportOut {
+    int32_t *paths, *actions;
+    int32_t *len, *leaf, *children, *visits;
+    int32_t *abort;
+};
+hipError_t launch_export(const ForestDev &f, const int32_t *paths, const int32_t *path_len, const int32_t *leaf,
+                         const int32_t *abort_words, int n, int stride, int max_depth, const ExportOut &out,
+                         const HostSignal &sig, hipStream_t s);
 
 hipError_t launch_leaf_keys(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                             const uint64_t *piece, int cells, const uint64_t *player, const uint64_t *root_key,

@@ -1,0 +1,34 @@
+"""What crosses between the host and the card through pinned memory: leaf gather, roots, values, offers, keys.
+At the sizes where the kernels that carry it can go wrong (edges of their tiles), against the CPU checker."""
+import numpy as np
+import pytest
+
+from oracle import ref_cpu as R
+from tests.helpers import random_tree
+
+pytestmark = pytest.mark.gpu
+
+
+# the gather takes 64 traversals x 32 depths at a time (a path has one node more than the depth bound)
+@pytest.mark.parametrize("depth", [1, 30, 31, 32, 33, 70])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 300])
+def test_leaf_gather_at_the_edges_of_its_tiles(n, depth):
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(5 + n, n_expand=300, fanout=(1, 5), max_depth=60, n_roots=3)
+    ref = R.RefTree.from_soa(soa)
+    troots = roots[np.arange(n) % 3]
+    f = omk.Forest.from_soa(soa)
+    b = omk.Batch(f, n, depth)
+    rng = np.random.default_rng(n)
+    b.set_roots(troots)
+    for _ in range(3):
+        rpaths, rlen, rleaf, _ = ref.select_batch(troots, R.make_params(c_puct=1.4, virtual_loss=3, max_depth=depth))
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+        paths, plen, leaf, actions = b.read()
+        assert (paths == rpaths).all() and (plen == rlen).all() and (leaf == rleaf).all()
+        assert (actions == ref.gather_actions(rpaths, rlen)).all()
+        values = (rng.integers(-64, 65, n) / 64.0).astype(np.float32)
+        ref.backup_batch(rpaths, rlen, values, 3)
+        b.set_values(values)
+        b.backup(3)
+        ref.W[:] = f.download()["W"]
