@@ -155,6 +155,8 @@ struct omk_batch {
     int32_t *out = nullptr;  // the leaf gather of the last read, in pinned memory (see omk_batch_read)
     size_t out_bytes = 0;
     long long *trace = nullptr;  // records of the timeline, kTraceCap of them
+    std::vector<int32_t> order, order_tmp;  // work space of omk_batch_set_roots
+    std::vector<Item> items_h, singles_h;
     void *exp_buf = nullptr;  // staging of an expansion: jobs, moves, priors, status
     size_t exp_bytes = 0;
 };
@@ -1064,6 +1066,34 @@ int omk_batch_destroy(omk_batch *b) {
     return OMK_OK;
 }
 
+}  // extern "C"
+
+// The traversals in ascending order of their roots, those of one root in ascending order: what a stable sort
+// gives.  One root for all, and roots that ascend already (one traversal per tree), are in order as they are; else
+// a radix sort, eleven bits a pass, as many passes as the largest root has digits.
+static void order_by_root(const int32_t *roots, int32_t n, std::vector<int32_t> &order, std::vector<int32_t> &tmp) {
+    order.resize((size_t)n);
+    bool ascending = true;
+    int32_t top = 0;
+    for (int32_t t = 0; t < n; t++) {
+        order[(size_t)t] = t;
+        ascending &= t == 0 || roots[t - 1] <= roots[t];
+        top = std::max(top, roots[t]);
+    }
+    if (ascending) return;
+    tmp.resize((size_t)n);
+    for (int shift = 0; shift == 0 || (top >> shift) > 0; shift += 11) {
+        int32_t start[2049] = {0};
+        for (int32_t t = 0; t < n; t++) start[((roots[t] >> shift) & 2047) + 1]++;
+        for (int i = 0; i < 2048; i++) start[i + 1] += start[i];
+        for (int32_t i = 0; i < n; i++) tmp[(size_t)start[(roots[order[(size_t)i]] >> shift) & 2047]++] = order[(size_t)i];
+        order.swap(tmp);
+        if (shift == 22) break;
+    }
+}
+
+extern "C" {
+
 int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) {
     if (!b || !h_roots) return fail(OMK_ERR_INVALID, "omk_batch_set_roots: null argument");
     if (n <= 0 || n > b->max_traversals)
@@ -1075,16 +1105,18 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) {
             return fail(OMK_ERR_INVALID, "omk_batch_set_roots: root %d of traversal %d outside [0, %lld)", h_roots[t],
                         t, (long long)f->n_nodes);
     // level-0 work items: traversals grouped by root, ascending traversal index inside a group
-    std::vector<int32_t> order((size_t)n);
-    for (int32_t t = 0; t < n; t++) order[(size_t)t] = t;
-    std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t c) { return h_roots[a] < h_roots[c]; });
-    std::vector<Item> items, singles;
+    std::vector<int32_t> &order = b->order;
+    order_by_root(h_roots, n, order, b->order_tmp);
+    std::vector<Item> &items = b->items_h, &singles = b->singles_h;
+    items.clear();
+    singles.clear();
     for (int32_t i = 0; i < n;) {
-        int32_t j = i;
-        while (j < n && h_roots[order[(size_t)j]] == h_roots[order[(size_t)i]]) j++;
+        const int32_t root = h_roots[order[(size_t)i]];
+        int32_t j = i + 1;
+        while (j < n && h_roots[order[(size_t)j]] == root) j++;
         Item it;
         memset(&it, 0, sizeof(it));
-        it.node = h_roots[order[(size_t)i]];
+        it.node = root;
         if (j - i > 1) {
             it.off = i;
             it.m = j - i;
@@ -1120,15 +1152,20 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) {
         }
     }
     if (int rc = use_device(f)) return rc;
-    HIP_TRY(hipStreamSynchronize(f->stream));
-    HIP_TRY(hipMemcpy(b->seg0, order.data(), (size_t)n * 4, hipMemcpyHostToDevice));
-    // every path starts at its root: written here once, not by every selection (the wavefront that takes a
+    // one trip: visitor lists | roots | items | lone traversals, staged side by side and spread by one kernel.
+    // Every path starts at its root: written here once, not by every selection (the wavefront that takes a
     // crowded root would spend its first microseconds on thousands of path entries)
-    HIP_TRY(hipMemcpy(b->paths, h_roots, (size_t)n * 4, hipMemcpyHostToDevice));
-    if (!items.empty())
-        HIP_TRY(hipMemcpy(b->items0, items.data(), items.size() * sizeof(Item), hipMemcpyHostToDevice));
+    const size_t words = (size_t)n * 2 + (items.size() + singles.size()) * (sizeof(Item) / 4);
+    void *staged = nullptr;
+    if (int rc = link_stage(f, words * 4, &staged)) return rc;
+    int32_t *at = (int32_t *)staged;
+    memcpy(at, order.data(), (size_t)n * 4);
+    memcpy(at + n, h_roots, (size_t)n * 4);
+    if (!items.empty()) memcpy(at + 2 * (size_t)n, items.data(), items.size() * sizeof(Item));
     if (!singles.empty())
-        HIP_TRY(hipMemcpy(b->singles0, singles.data(), singles.size() * sizeof(Item), hipMemcpyHostToDevice));
+        memcpy(at + 2 * (size_t)n + items.size() * (sizeof(Item) / 4), singles.data(), singles.size() * sizeof(Item));
+    HIP_TRY(launch_set_roots(b->seg0, b->paths, b->items0, b->singles0, at, n, (int)items.size(), (int)singles.size(),
+                             f->stream));
     b->n_items0 = (int32_t)items.size();
     b->n_hctx0 = n_hctx0;
     b->n_singles0 = (int32_t)singles.size();

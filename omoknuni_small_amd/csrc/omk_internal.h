@@ -117,6 +117,10 @@ struct SelectArgs {
 hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, int n_singles0, int n_traversals,
                          int max_fanout, bool rave, int n_cus, int n_hctx0, hipStream_t s);
 
+// What omk_batch_set_roots has staged (n visitors | n roots | items | lone traversals) to the batch's arrays.
+hipError_t launch_set_roots(int32_t *seg0, int32_t *paths, Item *items0, Item *singles0, const int32_t *staged, int n,
+                            int n_items, int n_singles, hipStream_t s);
+
 hipError_t launch_apply_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                            int max_len, int vl, hipStream_t s);
 hipError_t launch_revert_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,

@@ -32,3 +32,22 @@ def test_leaf_gather_at_the_edges_of_its_tiles(n, depth):
         b.set_values(values)
         b.backup(3)
         ref.W[:] = f.download()["W"]
+
+
+# roots in any order, with and without crowds: the grouping is a radix sort of eleven bits a pass
+@pytest.mark.parametrize("n,n_roots,shuffled", [(2, 1, False), (5, 5, True), (64, 64, False), (500, 7, True), (3000, 2100, True)])
+def test_roots_in_any_order(n, n_roots, shuffled):
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(n, n_expand=2 * n_roots, fanout=(1, 6), max_depth=5, n_roots=n_roots)
+    troots = roots[np.arange(n) % n_roots]
+    if shuffled:
+        troots = np.random.default_rng(n).permutation(troots)
+    ref = R.RefTree.from_soa(soa)
+    f = omk.Forest.from_soa(soa)
+    b = omk.Batch(f, n + 10, 6)
+    for use in (troots, troots[::-1][:max(1, n // 2)]):
+        rpaths, rlen, rleaf, _ = ref.select_batch(use, R.make_params(c_puct=1.4, virtual_loss=3, max_depth=6))
+        b.set_roots(use)
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+        paths, plen, leaf, _ = b.read()
+        assert (paths == rpaths).all() and (plen == rlen).all() and (leaf == rleaf).all()
