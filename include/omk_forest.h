@@ -239,7 +239,9 @@ int omk_forest_compact_static(omk_forest *f, int32_t new_root, int64_t *h_nodes_
  * clamp(policy[move], 0, 1), or 0.01 for a move outside the action space.  New node ids are
  * handed out from the current node count on, in simulation order; OMK_ERR_CAPACITY (and no
  * change) when the forest's capacity would be exceeded.  h_first_child (NULL or [n]): first
- * new id for the simulation whose list was used, else -1.  Waits for the stream. */
+ * new id for the simulation whose list was used, else -1.  The caller's arrays are free again on
+ * return; the children are written in stream order.  Waits for the selection unless
+ * omk_batch_read already has. */
 int omk_expand_batch(omk_batch *b, const int32_t *h_move_begin, const int32_t *h_moves, const float *h_policy,
                      int32_t action_space, int32_t *h_first_child);
 

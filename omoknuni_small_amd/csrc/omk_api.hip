@@ -152,13 +152,17 @@ struct omk_batch {
     int32_t spin_limit = 1 << 18;  // polls of about a microsecond: a quarter of a second, a selection takes a millisecond
     int32_t n_cus = 0;
     int32_t n_items0 = 0;
-    int32_t *out = nullptr;  // the leaf gather of the last read, in pinned memory (see omk_batch_read)
+    int32_t *out = nullptr;  // the leaf gather in pinned memory (see gather)
     size_t out_bytes = 0;
+    ExportOut gathered = {};      // its parts
+    // which selection it is of (the forest's and the batch's counts when it was made): an expansion takes leaves,
+    // child counts and visit counts from it while nothing has changed them
+    int64_t select_calls = 0, gathered_call = -1, gathered_changes = -1;
+    std::vector<int32_t> leaf_table;  // work space of an expansion
+    std::vector<int32_t> winners;
     long long *trace = nullptr;  // records of the timeline, kTraceCap of them
     std::vector<int32_t> order, order_tmp;  // work space of omk_batch_set_roots
     std::vector<Item> items_h, singles_h;
-    void *exp_buf = nullptr;  // staging of an expansion: jobs, moves, priors, status
-    size_t exp_bytes = 0;
 };
 
 struct omk_tt {
@@ -462,6 +466,7 @@ int omk_forest_upload(omk_forest *f, const omk_soa_view *v) {
         if (!f->hash) HIP_TRY(dalloc(&f->hash, f->capacity));
         HIP_TRY(hipMemcpy(f->hash, v->hash, (size_t)n * 8, hipMemcpyHostToDevice));
     }
+    f->changes++;
     // the same structure again (statistics put back): node ids keep their meaning
     if (!f->uploaded || f->structure_changed || n != f->n_nodes || ssum != f->structure_sum) f->generation++;
     f->structure_sum = ssum;
@@ -871,6 +876,7 @@ static int compact_in(omk_forest *f, int32_t new_root, int64_t *h_nodes_after, i
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return fail(OMK_ERR_HIP, "omk_forest_compact: %s", hipGetErrorString(e));
     f->n_nodes = k;
+    f->changes++;
     f->generation++;
     f->structure_changed = true;
     if (h_nodes_after) *h_nodes_after = k;
@@ -1056,7 +1062,7 @@ int omk_batch_destroy(omk_batch *b) {
     (void)hipStreamSynchronize(b->f->stream);
     void *ptrs[] = {b->paths,  b->path_len, b->leaf,     b->values, b->items0,   b->items_q,  b->seg0,
                     b->seg[0], b->seg[1],   b->sc_child, b->sc_occ, b->counters, b->trace,
-                    b->singles0, b->singles_q, b->q_ready, b->hctx, b->hbound, b->exp_buf, b->list_flag, b->single_ready};
+                    b->singles0, b->singles_q, b->q_ready, b->hctx, b->hbound, b->list_flag, b->single_ready};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (b->out) (void)hipHostFree(b->out);
@@ -1288,6 +1294,7 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
     HIP_TRY(launch_select(f->dev(), a, b->n_items0, b->n_singles0, b->n, f->max_fanout, p->use_rave != 0, b->n_cus,
                           b->n_hctx0, f->stream));
     b->selected = true;
+    b->select_calls++;
     return OMK_OK;
 }
 
@@ -1296,6 +1303,7 @@ int omk_backup_batch(omk_batch *b, int32_t virtual_loss) {
     if (!b->selected) return fail(OMK_ERR_STATE, "omk_backup_batch: no selected paths");
     if (int rc = fresh_batch("omk_backup_batch", b)) return rc;
     if (int rc = use_device(b->f)) return rc;
+    b->f->changes++;
     HIP_TRY(launch_backup(b->f->dev(), b->paths, b->path_len, b->values, b->n, b->stride, b->max_depth + 1,
                           virtual_loss, b->f->stream));
     // N and W of the nodes on the paths have changed: their RAVE blend with them
@@ -1355,11 +1363,50 @@ int omk_backup_paths(omk_forest *f, const int32_t *d_paths, const int32_t *d_pat
                      int32_t n, int32_t stride, int32_t max_len, int32_t virtual_loss) {
     if (int rc = check_paths_args("omk_backup_paths", f, d_paths, d_path_len, n, stride, max_len)) return rc;
     if (!d_values) return fail(OMK_ERR_INVALID, "omk_backup_paths: null values");
+    f->changes++;
     HIP_TRY(launch_backup(f->dev(), d_paths, d_path_len, d_values, n, stride, max_len, virtual_loss, f->stream));
     if (f->has_rave && f->blend_valid)
         HIP_TRY(launch_blend_paths(f->dev(), d_paths, d_path_len, n, stride, max_len, f->blend_k, f->stream));
     return OMK_OK;
 }
+
+}  // extern "C"
+
+// The leaf gather of the last selection into the batch's pinned buffer; waits for it.
+static int gather(omk_batch *b, bool paths, bool actions) {
+    omk_forest *f = b->f;
+    const size_t n = (size_t)b->n, D = (size_t)b->max_depth;
+    // lengths | leaves | their child counts | their visit counts | abort words | paths | actions
+    const size_t need = (n * (2 * D + 5) + 4) * 4;
+    if (need > b->out_bytes) {
+        if (b->out) {
+            HIP_TRY(hipStreamSynchronize(f->stream));
+            HIP_TRY(hipHostFree(b->out));
+        }
+        b->out = nullptr;
+        b->out_bytes = 0;
+        const size_t room = ((size_t)b->stride * (2 * D + 5) + 4) * 4;
+        HIP_TRY(hipHostMalloc((void **)&b->out, room, hipHostMallocDefault));
+        b->out_bytes = room;
+    }
+    ExportOut &o = b->gathered;
+    o.len = b->out;
+    o.leaf = o.len + n;
+    o.children = o.leaf + n;
+    o.visits = o.children + n;
+    o.abort = o.visits + n;
+    o.paths = paths ? o.abort + 4 : nullptr;
+    o.actions = actions ? o.abort + 4 + n * (D + 1) : nullptr;
+    b->gathered_call = -1;
+    HIP_TRY(launch_export(f->dev(), b->paths, b->path_len, b->leaf, b->counters + 3 * kSchedStep + 1, b->n, b->stride,
+                          b->max_depth, o, link_signal(f), f->stream));
+    if (int rc = link_wait(f)) return rc;
+    b->gathered_call = b->select_calls;
+    b->gathered_changes = f->changes;
+    return OMK_OK;
+}
+
+extern "C" {
 
 // How many children MCTSNode::expand creates for a node of `visits` visits that is offered `legal`
 // moves (src/mcts/mcts_node.cpp:296-341): without progressive widening all of them; with it
@@ -1391,146 +1438,89 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
         return fail(OMK_ERR_INVALID, "omk_expand_batch_ex: a policy needs action_space > 0 (got %d)", action_space);
     omk_forest *f = b->f;
     if (int rc = use_device(f)) return rc;
-    hipStream_t s = f->stream;
     const int n = b->n;
-    std::vector<int32_t> leaf((size_t)n);
-    HIP_TRY(hipMemcpyAsync(leaf.data(), b->leaf, (size_t)n * 4, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    // one job per distinct leaf: the first traversal (in index order) that offers moves wins
-    std::vector<ExpandJob> jobs;
-    std::vector<int32_t> job_of((size_t)n, -1), moves;
-    std::vector<float> priors;
-    {
-        std::vector<std::pair<int32_t, int32_t>> order;  // (leaf, traversal) of every offer
-        for (int t = 0; t < n; t++) {
-            if (h_move_begin[t + 1] < h_move_begin[t])
-                return fail(OMK_ERR_INVALID, "omk_expand_batch_ex: move_begin decreases at traversal %d", t);
-            if (h_policy_begin && h_policy_begin[t + 1] < h_policy_begin[t])
-                return fail(OMK_ERR_INVALID, "omk_expand_batch_ex: policy_begin decreases at traversal %d", t);
-            if (h_move_begin[t + 1] > h_move_begin[t] && leaf[(size_t)t] >= 0) order.emplace_back(leaf[(size_t)t], t);
-        }
-        std::sort(order.begin(), order.end());
-        std::vector<int32_t> winners;
-        for (size_t i = 0; i < order.size(); i++)
-            if (i == 0 || order[i].first != order[i - 1].first) winners.push_back(order[i].second);
-        std::sort(winners.begin(), winners.end());  // ids are handed out in traversal order
-        // A leaf that has children already (the selection stopped at it because of the depth bound) is left alone
-        // and takes no ids: its child range is read first.  Progressive widening reads the visit count of every
-        // leaf that is about to be expanded: it comes in the same trip.
-        std::vector<int32_t> visits(winners.size(), 0);
-        if (!winners.empty()) {
-            const size_t nw = winners.size();
-            if (nw * 16 > b->exp_bytes) {
-                if (b->exp_buf) HIP_TRY(hipFree(b->exp_buf));
-                b->exp_buf = nullptr;
-                b->exp_bytes = 0;
-                HIP_TRY(hipMalloc(&b->exp_buf, nw * 32));
-                b->exp_bytes = nw * 32;
-            }
-            std::vector<int32_t> ids(nw);
-            std::vector<int2> spans(nw);
-            for (size_t i = 0; i < nw; i++) ids[i] = leaf[(size_t)winners[i]];
-            int32_t *d_ids = (int32_t *)b->exp_buf, *d_n = d_ids + nw;
-            uint64_t *d_span = (uint64_t *)(d_ids + 2 * nw);
-            HIP_TRY(hipMemcpyAsync(d_ids, ids.data(), nw * 4, hipMemcpyHostToDevice, s));
-            HIP_TRY(launch_gather_words((uint32_t *)d_n, (const uint32_t *)f->N, d_ids, (int64_t)nw, s));
-            HIP_TRY(launch_gather_dwords(d_span, (const uint64_t *)f->span, d_ids, (int64_t)nw, s));
-            HIP_TRY(hipMemcpyAsync(visits.data(), d_n, nw * 4, hipMemcpyDeviceToHost, s));
-            HIP_TRY(hipMemcpyAsync(spans.data(), d_span, nw * 8, hipMemcpyDeviceToHost, s));
-            HIP_TRY(hipStreamSynchronize(s));
-            size_t kept = 0;
-            for (size_t i = 0; i < nw; i++) {
-                if (spans[i].y != 0) continue;
-                winners[kept] = winners[i];
-                visits[kept] = visits[i];
-                kept++;
-            }
-            winners.resize(kept);
-            visits.resize(kept);
-        }
-        int64_t cursor = f->n_nodes;
-        bool sorted = true;
-        int mf = f->max_fanout;
-        for (size_t wi = 0; wi < winners.size(); wi++) {
-            const int32_t t = winners[wi];
-            int32_t cnt = h_move_begin[t + 1] - h_move_begin[t];
-            if (cnt > 1000) cnt = 1000;  // MCTSNode::expand: max_reasonable_moves
-            cnt = widened_children(cnt, visits[wi], params);
-            // MCTSNode::setPriorProbabilities (:512-593) is only called with a policy that is not empty
-            // (mcts_engine_batch_tree_simple.cpp:256-258); otherwise expand's uniform prior stays
-            const int32_t psize = h_policy_begin ? h_policy_begin[t + 1] - h_policy_begin[t] : 0;
-            const float *pol = psize > 0 ? h_policy + h_policy_begin[t] : nullptr;
-            ExpandJob j;
-            j.leaf = leaf[(size_t)t];
-            j.begin = (int32_t)cursor;
-            j.count = cnt;
-            j.off = (int32_t)moves.size();
-            float prev = 2.0f;
-            for (int32_t i = 0; i < cnt; i++) {
-                const int32_t mv = h_moves[h_move_begin[t] + i];
-                float prior;
-                if (!pol) {
-                    prior = 1.0f / (float)cnt;  // expand(): uniform prior
-                } else if (psize == action_space) {  // a policy over the action space (:537-560)
-                    if (mv >= 0 && mv < action_space) {
-                        prior = pol[mv];
-                        prior = std::min(1.0f, std::max(0.0f, prior));  // clamp to [0, 1]
-                    } else {
-                        prior = 0.01f;  // move outside the action space
-                    }
-                } else if (psize == cnt) {  // one value per child, by child index (:561-575)
-                    prior = pol[i];
-                    prior = std::min(1.0f, std::max(0.0f, prior));
-                } else {  // neither size: uniform (:576-584)
-                    prior = 1.0f / (float)cnt;
-                }
-                if (prior > prev) sorted = false;
-                prev = prior;
-                moves.push_back(mv);
-                priors.push_back(prior);
-            }
-            job_of[(size_t)t] = (int32_t)jobs.size();
-            jobs.push_back(j);
-            cursor += cnt;
-            mf = std::max(mf, (int)cnt);
-        }
-        if (cursor > f->capacity)
-            return fail(OMK_ERR_CAPACITY, "omk_expand_batch_ex: %lld nodes needed, capacity %lld", (long long)cursor,
-                        (long long)f->capacity);
-        if (cursor > INT32_MAX) return fail(OMK_ERR_CAPACITY, "omk_expand_batch_ex: node ids exceed 32 bits");
-        if (h_first_child)
-            for (int t = 0; t < n; t++) h_first_child[t] = -1;
-        if (jobs.empty()) return OMK_OK;
-        // staging: jobs | moves | priors | status
-        const size_t nj = jobs.size(), nm = moves.size();
-        const size_t bytes = nj * sizeof(ExpandJob) + nm * 8 + nj * 4;
-        if (bytes > b->exp_bytes) {
-            if (b->exp_buf) HIP_TRY(hipFree(b->exp_buf));
-            b->exp_buf = nullptr;
-            b->exp_bytes = 0;
-            HIP_TRY(hipMalloc(&b->exp_buf, bytes * 2));
-            b->exp_bytes = bytes * 2;
-        }
-        char *base = (char *)b->exp_buf;
-        ExpandJob *d_jobs = (ExpandJob *)base;
-        int32_t *d_moves = (int32_t *)(base + nj * sizeof(ExpandJob));
-        float *d_priors = (float *)(d_moves + nm);
-        int32_t *d_status = (int32_t *)(d_priors + nm);
-        HIP_TRY(hipMemcpyAsync(d_jobs, jobs.data(), nj * sizeof(ExpandJob), hipMemcpyHostToDevice, s));
-        HIP_TRY(hipMemcpyAsync(d_moves, moves.data(), nm * 4, hipMemcpyHostToDevice, s));
-        HIP_TRY(hipMemcpyAsync(d_priors, priors.data(), nm * 4, hipMemcpyHostToDevice, s));
-        HIP_TRY(launch_expand(f->mut(), d_jobs, (int)nj, d_moves, d_priors, d_status, f->n_nodes, cursor, s));
-        std::vector<int32_t> status(nj);
-        HIP_TRY(hipMemcpyAsync(status.data(), d_status, nj * 4, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
-        f->n_nodes = cursor;
-        f->structure_changed = true;  // ids keep their meaning, but an upload of the old arrays would not
-        f->max_fanout = mf;
-        if (!sorted) f->prior_sorted = false;
-        if (h_first_child)
-            for (int t = 0; t < n; t++)
-                if (job_of[(size_t)t] >= 0) h_first_child[t] = status[(size_t)job_of[(size_t)t]];
+    for (int t = 0; t < n; t++) {
+        if (h_move_begin[t + 1] < h_move_begin[t])
+            return fail(OMK_ERR_INVALID, "omk_expand_batch_ex: move_begin decreases at traversal %d", t);
+        if (h_policy_begin && h_policy_begin[t + 1] < h_policy_begin[t])
+            return fail(OMK_ERR_INVALID, "omk_expand_batch_ex: policy_begin decreases at traversal %d", t);
     }
+    // The leaves with their child and visit counts: a search has just read them (omk_batch_read brings all
+    // three), and one that has not gathers them now.
+    if (b->gathered_call != b->select_calls || b->gathered_changes != f->changes)
+        if (int rc = gather(b, false, false)) return rc;
+    const int32_t *leaf = b->gathered.leaf, *children = b->gathered.children, *visits = b->gathered.visits;
+    // One job per distinct leaf: the first traversal (in index order) that offers moves wins.  A leaf that has
+    // children already (the selection stopped at it because of the depth bound) is left alone and takes no ids.
+    // The leaves met so far: open addressing, at most half full.
+    int bits = 4;
+    while ((1 << bits) < 2 * n) bits++;
+    std::vector<int32_t> &table = b->leaf_table, &winners = b->winners;
+    table.assign((size_t)1 << bits, -1);
+    winners.clear();
+    int64_t cursor = f->n_nodes;
+    for (int t = 0; t < n; t++) {
+        const int32_t offered = h_move_begin[t + 1] - h_move_begin[t];
+        if (offered <= 0 || leaf[t] < 0) continue;
+        uint32_t h = ((uint32_t)leaf[t] * 2654435761u) >> (32 - bits);
+        while (table[h] >= 0 && table[h] != leaf[t]) h = (h + 1) & ((1u << bits) - 1u);
+        if (table[h] >= 0) continue;
+        table[h] = leaf[t];
+        if (children[t] != 0) continue;
+        winners.push_back(t);
+        // MCTSNode::expand: max_reasonable_moves
+        cursor += widened_children(std::min(offered, 1000), visits[t], params);
+    }
+    if (cursor > f->capacity)
+        return fail(OMK_ERR_CAPACITY, "omk_expand_batch_ex: %lld nodes needed, capacity %lld", (long long)cursor,
+                    (long long)f->capacity);
+    if (cursor > INT32_MAX) return fail(OMK_ERR_CAPACITY, "omk_expand_batch_ex: node ids exceed 32 bits");
+    if (h_first_child)
+        for (int t = 0; t < n; t++) h_first_child[t] = -1;
+    if (winners.empty()) return OMK_OK;
+    // staged for the kernel: jobs | moves | priors
+    const size_t nj = winners.size(), nm = (size_t)(cursor - f->n_nodes);
+    void *staged = nullptr;
+    if (int rc = link_stage(f, nj * sizeof(ExpandJob) + nm * 8, &staged)) return rc;
+    ExpandJob *jobs = (ExpandJob *)staged;
+    int32_t *moves = (int32_t *)(jobs + nj);
+    float *priors = (float *)(moves + nm);
+    bool sorted = true;
+    int mf = f->max_fanout;
+    cursor = f->n_nodes;
+    size_t off = 0;
+    for (size_t wi = 0; wi < nj; wi++) {
+        const int32_t t = winners[wi];
+        const int32_t cnt = widened_children(std::min(h_move_begin[t + 1] - h_move_begin[t], 1000), visits[t], params);
+        // MCTSNode::setPriorProbabilities (:512-593) is only called with a policy that is not empty
+        // (mcts_engine_batch_tree_simple.cpp:256-258); otherwise expand's uniform prior stays
+        const int32_t psize = h_policy_begin ? h_policy_begin[t + 1] - h_policy_begin[t] : 0;
+        const float *pol = psize > 0 ? h_policy + h_policy_begin[t] : nullptr;
+        jobs[wi] = ExpandJob{leaf[t], (int32_t)cursor, cnt, (int32_t)off};
+        const int32_t *mv = h_moves + h_move_begin[t];
+        float *pr = priors + off;
+        memcpy(moves + off, mv, (size_t)cnt * 4);
+        if (pol && psize == action_space) {  // a policy over the action space (:537-560)
+            for (int32_t i = 0; i < cnt; i++)
+                pr[i] = mv[i] >= 0 && mv[i] < action_space ? std::min(1.0f, std::max(0.0f, pol[mv[i]]))  // clamp to [0, 1]
+                                                           : 0.01f;  // move outside the action space
+        } else if (pol && psize == cnt) {  // one value per child, by child index (:561-575)
+            for (int32_t i = 0; i < cnt; i++) pr[i] = std::min(1.0f, std::max(0.0f, pol[i]));
+        } else {  // expand(): uniform prior; a policy of neither size likewise (:576-584)
+            for (int32_t i = 0; i < cnt; i++) pr[i] = 1.0f / (float)cnt;
+        }
+        for (int32_t i = 1; i < cnt && sorted; i++) sorted = !(pr[i] > pr[i - 1]);
+        if (h_first_child) h_first_child[t] = (int32_t)cursor;
+        off += (size_t)cnt;
+        cursor += cnt;
+        mf = std::max(mf, (int)cnt);
+    }
+    HIP_TRY(launch_expand(f->mut(), jobs, (int)nj, moves, priors, f->n_nodes, cursor, f->stream));
+    f->n_nodes = cursor;
+    f->changes++;
+    f->structure_changed = true;  // ids keep their meaning, but an upload of the old arrays would not
+    f->max_fanout = mf;
+    if (!sorted) f->prior_sorted = false;
     return OMK_OK;
 }
 
@@ -1559,32 +1549,8 @@ int omk_batch_read(omk_batch *b, int32_t *h_paths, int32_t *h_path_len, int32_t 
     omk_forest *f = b->f;
     if (int rc = use_device(f)) return rc;
     const size_t n = (size_t)b->n, D = (size_t)b->max_depth;
-    // pinned: lengths | leaves | their child counts | their visit counts | abort words | paths | actions
-    const size_t ints = n * (2 * D + 5) + 4;
-    if (ints * 4 > b->out_bytes) {
-        if (b->out) {
-            HIP_TRY(hipStreamSynchronize(f->stream));
-            HIP_TRY(hipHostFree(b->out));
-        }
-        b->out = nullptr;
-        b->out_bytes = 0;
-        const size_t room = (size_t)b->stride * (2 * D + 5) * 4 + 64;
-        HIP_TRY(hipHostMalloc((void **)&b->out, room, hipHostMallocDefault));
-        b->out_bytes = room;
-    }
-    ExportOut o;
-    int32_t *at = b->out;
-    o.len = at;
-    o.leaf = at += n;
-    o.children = at += n;
-    o.visits = at += n;
-    o.abort = at += n;
-    int32_t *rows = at + 4;
-    o.paths = h_paths ? rows : nullptr;
-    o.actions = h_actions ? rows + n * (D + 1) : nullptr;
-    HIP_TRY(launch_export(f->dev(), b->paths, b->path_len, b->leaf, b->counters + 3 * kSchedStep + 1, b->n, b->stride,
-                          b->max_depth, o, link_signal(f), f->stream));
-    if (int rc = link_wait(f)) return rc;
+    if (int rc = gather(b, h_paths != nullptr, h_actions != nullptr)) return rc;
+    const ExportOut &o = b->gathered;
     if (h_paths) memcpy(h_paths, o.paths, n * (D + 1) * 4);
     if (h_actions) memcpy(h_actions, o.actions, n * D * 4);
     if (h_path_len) memcpy(h_path_len, o.len, n * 4);
@@ -1912,6 +1878,7 @@ int omk_tt_select_redirect(omk_tt *tt, omk_batch *b, const omk_select_params *p,
     a.abort_word = b->counters + 3 * kSchedStep + 1;
     HIP_TRY(launch_select_redirect(f->dev(), a, p->use_rave != 0, s));
     b->selected = true;
+    b->select_calls++;
     HIP_TRY(hipMemcpyAsync(status, tt->d_status, sizeof(status), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     tt->clock += (uint32_t)status[6];  // the ticks of the access counter

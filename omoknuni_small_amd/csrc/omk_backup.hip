@@ -239,18 +239,19 @@ __global__ void k_expand_mask(uint32_t *legal, int64_t old_nodes, int64_t new_no
     }
 }
 
-// One wavefront per leaf.  The children are written first, the leaf's child range last: a
-// node is a leaf exactly while its child count is 0.  The host offers no job for a leaf that
-// already has children (the selection stopped at it because of the depth bound: it reads the
-// child ranges first, so that such a leaf takes no ids); should one come all the same it is left
+// One block per leaf, a child per thread (a Go board is two rounds): jobs, moves and priors are read from pinned
+// host memory, and what bounds the kernel is that trip, twice in a row (the job, then its moves and priors): 225
+// children of 64 leaves were four rounds of one wavefront before.  The children are written first, the leaf's child
+// range last: a node is a leaf exactly while its child count is 0.  The host offers no job for a leaf that already
+// has children (the selection stopped at it because of the depth bound); should one come all the same it is left
 // alone.
-__global__ __launch_bounds__(64) void k_expand(ForestMut f, const ExpandJob *jobs, int n_jobs, const int32_t *moves,
-                                               const float *priors, int32_t *status) {
+__global__ __launch_bounds__(256) void k_expand(ForestMut f, const ExpandJob *jobs, int n_jobs, const int32_t *moves,
+                                                const float *priors) {
     const int j = blockIdx.x;
     if (j >= n_jobs) return;
     const ExpandJob job = jobs[j];
     const bool fresh = f.span[job.leaf].y == 0;
-    for (int i = threadIdx.x; i < job.count; i += 64) {
+    for (int i = threadIdx.x; i < job.count; i += 256) {
         const int id = job.begin + i;
         f.N[id] = 0;
         f.W[id] = 0.0f;
@@ -265,17 +266,14 @@ __global__ __launch_bounds__(64) void k_expand(ForestMut f, const ExpandJob *job
         if (f.legal && fresh) atomicOr(f.legal + ((uint32_t)id >> 5), 1u << ((uint32_t)id & 31u));
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        if (fresh) f.span[job.leaf] = int2{job.begin, job.count};
-        status[j] = fresh ? job.begin : -1;
-    }
+    if (threadIdx.x == 0 && fresh) f.span[job.leaf] = int2{job.begin, job.count};
 }
 
 hipError_t launch_expand(const ForestMut &f, const ExpandJob *jobs, int n_jobs, const int32_t *moves,
-                         const float *priors, int32_t *status, int64_t old_nodes, int64_t new_nodes, hipStream_t s) {
+                         const float *priors, int64_t old_nodes, int64_t new_nodes, hipStream_t s) {
     if (n_jobs <= 0) return hipSuccess;
     if (f.legal) hipLaunchKernelGGL(k_expand_mask, dim3(64), dim3(256), 0, s, f.legal, old_nodes, new_nodes);
-    hipLaunchKernelGGL(k_expand, dim3(n_jobs), dim3(64), 0, s, f, jobs, n_jobs, moves, priors, status);
+    hipLaunchKernelGGL(k_expand, dim3(n_jobs), dim3(256), 0, s, f, jobs, n_jobs, moves, priors);
     return hipGetLastError();
 }
 

@@ -51,3 +51,44 @@ def test_roots_in_any_order(n, n_roots, shuffled):
         b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
         paths, plen, leaf, _ = b.read()
         assert (paths == rpaths).all() and (plen == rlen).all() and (leaf == rleaf).all()
+
+
+# one thread per child, 256 a round; leaves known from a read, from none, and from one that a backup has overtaken
+@pytest.mark.parametrize("moves", [1, 255, 256, 257, 1000])
+def test_expansion_after_a_read_and_without(moves):
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(11, n_expand=30, fanout=(2, 6), max_depth=4, n_roots=2, vl_frac=0.0)
+    ref = R.RefTree.from_soa(soa)
+    n, A = 24, 1003
+    troots = roots[np.arange(n) % 2]
+    f = omk.Forest.from_soa(soa, capacity=ref.n + 3 * n * moves)
+    b = omk.Batch(f, n, 8)
+    b.set_roots(troots)
+    rng = np.random.default_rng(moves)
+    for step in range(3):
+        rpaths, rlen, rleaf, _ = ref.select_batch(troots, R.make_params(c_puct=1.4, virtual_loss=3, max_depth=8))
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+        if step != 1:
+            assert (b.read()[2] == rleaf).all()
+        counts = np.where(rng.random(n) < 0.3, 0, moves)
+        begin = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+        mv = np.concatenate([rng.permutation(A + 2)[:c] for c in counts] + [[]]).astype(np.int32)  # two outside
+        policy = rng.uniform(-0.2, 1.2, (n, A)).astype(np.float32)
+        values = (rng.integers(-64, 65, n) / 64.0).astype(np.float32)
+        widening = (2.0, 0.5) if step == 2 else None
+        if step == 2:  # the widening then has to see the visits of this backup
+            ref.backup_batch(rpaths, rlen, values, 3)
+            b.set_values(values)
+            b.backup(3)
+        want = ref.expand_batch(rleaf, begin, mv, policy=policy, action_space=A, widening=widening)
+        got = b.expand_ex(begin, mv, (np.arange(n + 1) * A).astype(np.int32), policy, A, widening=widening)
+        assert (got == want).all()
+        if step != 2:
+            ref.backup_batch(rpaths, rlen, values, 3)
+            b.set_values(values)
+            b.backup(3)
+        st, sx = f.download(), f.download_structure()
+        ref.W[:] = st["W"]
+        assert (st["N"] == ref.N).all() and st["P"].tobytes() == ref.P.tobytes() and (st["VL"] == ref.VL).all()
+        assert (sx["child_begin"] == ref.child_begin).all() and (sx["child_count"] == ref.child_count).all()
+        assert (sx["action"] == ref.action).all()
