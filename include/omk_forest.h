@@ -180,7 +180,7 @@ int omk_backup_paths(omk_forest *f, const int32_t *d_paths, const int32_t *d_pat
  * uniform 1/children when it is not positive) and sets
  * prior = (1 - epsilon) * prior + epsilon * noise, child by child in the reference's
  * order.  n_gamma must be the number of children (legal slots).  A root without children
- * is left alone.  Waits for the stream; the arithmetic is done on the host. */
+ * is left alone.  Waits for the stream. */
 int omk_forest_add_root_noise(omk_forest *f, int32_t root, const float *h_gamma, int32_t n_gamma, float epsilon);
 
 /* The search result's move probabilities (MCTSEngine::getActionProbabilities,
@@ -361,8 +361,8 @@ int omk_batch_leaf_keys(omk_batch *b, const uint64_t *d_piece_keys, int32_t cell
  * every leaf it evaluates (the clone with the moves replayed, mcts_engine_batch_tree_simple.cpp:170-178)
  * and passes state->getHash() (include/core/igamestate.h) for the leaf's node.  A forest uploaded without
  * keys gets the array on the first call; a node that has no key yet (all of them then, and every node that
- * omk_expand_batch* adds) carries the key ~0, which the table neither stores nor finds.  Waits for the
- * stream. */
+ * omk_expand_batch* adds) carries the key ~0, which the table neither stores nor finds.  The caller's
+ * arrays are free again on return; the keys are written in stream order. */
 int omk_forest_set_keys(omk_forest *f, const int32_t *h_nodes, const uint64_t *h_keys, int64_t n);
 
 int omk_tt_create(omk_forest *f, int32_t log2_slots, omk_tt **out);

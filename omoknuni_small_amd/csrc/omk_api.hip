@@ -60,13 +60,11 @@ struct omk_forest {
     uint32_t *legal = nullptr;
     uint64_t *hash = nullptr;
     bool has_legal = false, has_action = false, has_hash = false;
-    void *key_stage = nullptr;  // staging of omk_forest_set_keys: keys, node ids, one status word
     // Child slots re-pointed at transpositions (omk_tt_select_redirect): alias[s] >= 0 = the node slot s holds
     // instead of node s.  Allocated by the first such call; `redirected` once a slot has been re-pointed: the
     // forest is then a graph, and what assumes a tree refuses it until the next upload.
     int32_t *alias = nullptr;
     bool redirected = false;
-    size_t key_stage_bytes = 0;
     // The way between the host and the kernels: one block of pinned memory that both sides address (see link_*).
     char *link = nullptr;
     size_t link_bytes = 0;
@@ -170,7 +168,7 @@ struct omk_tt {
     int log2_slots = 0;
     TTSlot *slots = nullptr;
     TTMeta *meta = nullptr;
-    int *d_status = nullptr;       // 8 counters of the last call
+    int *d_status = nullptr;       // 8 counters: zero between calls, read and cleared at the end of one (tt_counts)
     uint32_t clock = 0;            // access_counter_ of the reference: entry i of a call has the time clock + i
     float threshold = 0.1f;        // Config::replacement_threshold
     void *work = nullptr;          // staging of store / traverse calls
@@ -268,6 +266,17 @@ static int link_wait(omk_forest *f) {
     return OMK_OK;
 }
 
+// `words` 32-bit words of device memory to the host; waits for the stream.  Up to kLinkStaging bytes through the
+// pinned block (8 us), more by the runtime's copy into pageable memory.
+static int link_fetch(omk_forest *f, void *h_dst, const void *d_src, size_t words) {
+    void *staged = nullptr;
+    if (int rc = link_stage(f, words * 4, &staged)) return rc;
+    HIP_TRY(launch_fetch((uint32_t *)staged, (const uint32_t *)d_src, (int64_t)words, link_signal(f), f->stream));
+    if (int rc = link_wait(f)) return rc;
+    memcpy(h_dst, staged, words * 4);
+    return OMK_OK;
+}
+
 static int use_device(const omk_forest *f) {
     if (f->released) return fail(OMK_ERR_STATE, "the forest of this handle has been destroyed");
     HIP_TRY(hipSetDevice(f->device));
@@ -338,7 +347,7 @@ int omk_forest_create(const omk_forest_desc *desc, omk_forest **out) {
 static void forest_free(omk_forest *f) {
     (void)hipSetDevice(f->device);
     if (f->own_stream) (void)hipStreamSynchronize(f->own_stream);
-    void *ptrs[] = {f->span, f->N, f->W, f->P, f->VL, f->rN, f->rW, f->Q2, f->action, f->legal, f->hash, f->key_stage, f->alias, f->link_count};
+    void *ptrs[] = {f->span, f->N, f->W, f->P, f->VL, f->rN, f->rW, f->Q2, f->action, f->legal, f->hash, f->alias, f->link_count};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (f->link) (void)hipHostFree(f->link);
@@ -612,31 +621,45 @@ int omk_forest_set_keys(omk_forest *f, const int32_t *h_nodes, const uint64_t *h
         f->has_hash = true;
     }
     if (n == 0) return OMK_OK;
-    // staging kept with the forest (a search calls this every batch): keys | node ids | status word
-    const size_t need = (size_t)n * 12 + 8;
-    if (need > f->key_stage_bytes) {
-        HIP_TRY(hipStreamSynchronize(s));
-        if (f->key_stage) HIP_TRY(hipFree(f->key_stage));
-        f->key_stage = nullptr;
-        f->key_stage_bytes = 0;
-        const size_t room = need + need / 2;
-        HIP_TRY(hipMalloc(&f->key_stage, room));
-        f->key_stage_bytes = room;
-    }
-    uint64_t *d_keys = (uint64_t *)f->key_stage;
-    int32_t *d_nodes = (int32_t *)(d_keys + n);
-    int *d_bad = (int *)(d_nodes + n + (n & 1));
-    int bad = 0;
-    hipError_t e = hipMemcpyAsync(d_nodes, h_nodes, (size_t)n * 4, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(d_keys, h_keys, (size_t)n * 8, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(d_bad, &bad, 4, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = launch_set_keys(f->hash, d_nodes, d_keys, n, f->n_nodes, d_bad, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(&bad, d_bad, 4, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return fail(OMK_ERR_HIP, "omk_forest_set_keys: %s", hipGetErrorString(e));
-    if (bad) return fail(OMK_ERR_INVALID, "omk_forest_set_keys: %d node ids outside the forest (skipped)", bad);
+    int64_t bad = 0;
+    for (int64_t i = 0; i < n; i++) bad += h_nodes[i] < 0 || h_nodes[i] >= f->n_nodes;
+    void *staged = nullptr;
+    if (int rc = link_stage(f, (size_t)n * 12, &staged)) return rc;
+    uint64_t *keys = (uint64_t *)staged;
+    int32_t *nodes = (int32_t *)(keys + n);
+    memcpy(keys, h_keys, (size_t)n * 8);
+    memcpy(nodes, h_nodes, (size_t)n * 4);
+    HIP_TRY(launch_set_keys(f->hash, nodes, keys, n, f->n_nodes, s));
+    if (bad) return fail(OMK_ERR_INVALID, "omk_forest_set_keys: %lld node ids outside the forest (skipped)", (long long)bad);
     return OMK_OK;
 }
+
+}  // extern "C"
+
+// What the host asks about a node's children, in pinned memory until the next call that stages something: one
+// kernel and one wait (8 us) where every array was a synchronous copy of its own (42 us a call, and a self-play
+// program asks for every game).
+struct RootChildren {
+    int32_t begin, count;
+    const int32_t *visits, *action, *legal;  // visits: of the node the slot holds
+};
+
+static int root_children(omk_forest *f, int32_t root, RootChildren *out) {
+    void *staged = nullptr;
+    if (int rc = link_stage(f, 128 + 12ull * OMK_MAX_FANOUT, &staged)) return rc;
+    int32_t *r = (int32_t *)staged;
+    HIP_TRY(launch_root_children(f->dev(), f->redirected ? f->alias : nullptr, root, r, r + 32, OMK_MAX_FANOUT,
+                                 link_signal(f), f->stream));
+    if (int rc = link_wait(f)) return rc;
+    out->begin = r[0];
+    out->count = r[1];
+    out->visits = r + 32;
+    out->action = r + 32 + OMK_MAX_FANOUT;
+    out->legal = r + 32 + 2 * OMK_MAX_FANOUT;
+    return OMK_OK;
+}
+
+extern "C" {
 
 int omk_forest_add_root_noise(omk_forest *f, int32_t root, const float *h_gamma, int32_t n_gamma, float epsilon) {
     if (!f || !h_gamma) return fail(OMK_ERR_INVALID, "omk_forest_add_root_noise: null argument");
@@ -644,47 +667,22 @@ int omk_forest_add_root_noise(omk_forest *f, int32_t root, const float *h_gamma,
     if (root < 0 || root >= f->n_nodes) return fail(OMK_ERR_INVALID, "omk_forest_add_root_noise: root %d", root);
     if (int rc = tree_only("omk_forest_add_root_noise", f)) return rc;
     if (int rc = use_device(f)) return rc;
-    HIP_TRY(hipStreamSynchronize(f->stream));
-    int2 sp;
-    HIP_TRY(hipMemcpy(&sp, f->span + root, sizeof(sp), hipMemcpyDeviceToHost));
-    const int32_t cb = sp.x, cc = sp.y;
-    if (cc <= 0) return OMK_OK;  // no children to add noise to (mcts_engine_eval.cpp:78-80)
-    std::vector<float> prior((size_t)cc);
-    HIP_TRY(hipMemcpy(prior.data(), f->P + cb, (size_t)cc * 4, hipMemcpyDeviceToHost));
-    std::vector<uint32_t> legal;
-    const int64_t w0 = (int64_t)cb >> 5, w1 = ((int64_t)cb + cc + 31) >> 5;
-    if (f->has_legal) {
-        legal.resize((size_t)(w1 - w0));
-        HIP_TRY(hipMemcpy(legal.data(), f->legal + w0, legal.size() * 4, hipMemcpyDeviceToHost));
-    }
-    auto is_child = [&](int32_t i) {
-        if (!f->has_legal) return true;
-        const int64_t id = (int64_t)cb + i;
-        return ((legal[(size_t)((id >> 5) - w0)] >> (id & 31)) & 1u) != 0u;
-    };
-    int32_t children = 0;
-    for (int32_t i = 0; i < cc; i++) children += is_child(i) ? 1 : 0;
-    if (children == 0) return OMK_OK;
-    if (n_gamma != children)
-        return fail(OMK_ERR_INVALID, "omk_forest_add_root_noise: %d samples for %d children", n_gamma, children);
-    // MCTSEngine::addDirichletNoise from the normalisation on, statement by statement
+    // MCTSEngine::addDirichletNoise from the normalisation on, statement by statement; the mix is the kernel's,
+    // child by child in the same arithmetic, and happens only if the samples are as many as the children
+    const int32_t given = std::max(0, std::min(n_gamma, (int32_t)OMK_MAX_FANOUT));
+    void *staged = nullptr;
+    if (int rc = link_stage(f, 128 + (size_t)given * 4, &staged)) return rc;
+    int32_t *result = (int32_t *)staged;
+    float *noise = (float *)staged + 32;
     float sum = 0.0f;
-    for (int32_t j = 0; j < children; j++) sum = sum + h_gamma[j];
-    std::vector<float> noise(h_gamma, h_gamma + children);
-    if (sum > 0.0f) {
-        for (auto &x : noise) x /= sum;
-    } else {
-        const float uniform_noise = 1.0f / (float)children;
-        for (auto &x : noise) x = uniform_noise;
-    }
-    int32_t j = 0;
-    for (int32_t i = 0; i < cc; i++) {
-        if (!is_child(i)) continue;
-        const float keep = (1.0f - epsilon) * prior[(size_t)i];
-        const float add = epsilon * noise[(size_t)j++];
-        prior[(size_t)i] = keep + add;
-    }
-    HIP_TRY(hipMemcpy(f->P + cb, prior.data(), (size_t)cc * 4, hipMemcpyHostToDevice));
+    for (int32_t j = 0; j < given; j++) sum = sum + h_gamma[j];
+    const float uniform_noise = 1.0f / (float)std::max(given, 1);
+    for (int32_t j = 0; j < given; j++) noise[j] = sum > 0.0f ? h_gamma[j] / sum : uniform_noise;
+    HIP_TRY(launch_root_noise(f->mut(), root, noise, n_gamma, epsilon, result, link_signal(f), f->stream));
+    if (int rc = link_wait(f)) return rc;
+    const int32_t children = result[0];
+    if (children > 0 && n_gamma != children)
+        return fail(OMK_ERR_INVALID, "omk_forest_add_root_noise: %d samples for %d children", n_gamma, children);
     return OMK_OK;
 }
 
@@ -695,46 +693,21 @@ int omk_forest_action_probabilities(omk_forest *f, int32_t root, float temperatu
     if (root < 0 || root >= f->n_nodes || action_space <= 0)
         return fail(OMK_ERR_INVALID, "omk_forest_action_probabilities: root %d, action space %d", root, action_space);
     if (int rc = use_device(f)) return rc;
-    HIP_TRY(hipStreamSynchronize(f->stream));
-    int2 sp;
-    HIP_TRY(hipMemcpy(&sp, f->span + root, sizeof(sp), hipMemcpyDeviceToHost));
+    RootChildren kids;
+    if (int rc = root_children(f, root, &kids)) return rc;
     for (int32_t a = 0; a < action_space; a++) h_probabilities[a] = 0.0f;
     if (h_children) *h_children = 0;
-    const int32_t cb = sp.x, cc = sp.y;
-    if (cc <= 0) return OMK_OK;
-    std::vector<int32_t> n((size_t)cc), act((size_t)cc);
-    HIP_TRY(hipMemcpy(n.data(), f->N + cb, (size_t)cc * 4, hipMemcpyDeviceToHost));
-    if (f->redirected) {
-        // the counts are those of the nodes the children vector holds (child->getVisitCount(),
-        // mcts_engine_tree.cpp:401-403), the actions those of the slots (root->getActions(), :395)
-        std::vector<int32_t> al((size_t)cc);
-        HIP_TRY(hipMemcpy(al.data(), f->alias + cb, (size_t)cc * 4, hipMemcpyDeviceToHost));
-        for (int32_t i = 0; i < cc; i++)
-            if (al[(size_t)i] >= 0) HIP_TRY(hipMemcpy(&n[(size_t)i], f->N + al[(size_t)i], 4, hipMemcpyDeviceToHost));
-    }
-    if (f->has_action) {
-        HIP_TRY(hipMemcpy(act.data(), f->action + cb, (size_t)cc * 4, hipMemcpyDeviceToHost));
-    } else {
-        for (int32_t i = 0; i < cc; i++) act[(size_t)i] = cb + i;
-    }
-    std::vector<uint32_t> legal;
-    const int64_t w0 = (int64_t)cb >> 5, w1 = ((int64_t)cb + cc + 31) >> 5;
-    if (f->has_legal) {
-        legal.resize((size_t)(w1 - w0));
-        HIP_TRY(hipMemcpy(legal.data(), f->legal + w0, legal.size() * 4, hipMemcpyDeviceToHost));
-    }
-    auto is_child = [&](int32_t i) {
-        if (!f->has_legal) return true;
-        const int64_t id = (int64_t)cb + i;
-        return ((legal[(size_t)((id >> 5) - w0)] >> (id & 31)) & 1u) != 0u;
-    };
+    // the counts are those of the nodes the children vector holds (child->getVisitCount(),
+    // mcts_engine_tree.cpp:401-403), the actions those of the slots (root->getActions(), :395)
+    const int32_t cc = kids.count, *n = kids.visits, *act = kids.action;
+    auto is_child = [&](int32_t i) { return kids.legal[i] != 0; };
     // MCTSEngine::getActionProbabilities, statement by statement
     int32_t children = 0, max_idx = -1;
     float max_count = 0.0f;
     for (int32_t i = 0; i < cc; i++) {
         if (!is_child(i)) continue;
         children++;
-        const float c = (float)n[(size_t)i];
+        const float c = (float)n[i];
         if (max_idx < 0 || c > max_count) {  // std::max_element: the first of the largest
             max_count = c;
             max_idx = i;
@@ -743,14 +716,14 @@ int omk_forest_action_probabilities(omk_forest *f, int32_t root, float temperatu
     if (h_children) *h_children = children;
     if (children == 0) return OMK_OK;
     const bool near_zero = temperature < 0.01f;
-    float sum = 0.0f;
+    float sum = 0.0f, scaled[OMK_MAX_FANOUT];
     if (!near_zero && max_count > 0.0f)
         for (int32_t i = 0; i < cc; i++) {
             if (!is_child(i)) continue;
-            const float c = (float)n[(size_t)i];
-            float scaled = 0.0f;
-            if (c > 0.0f) scaled = powf(c / max_count, 1.0f / temperature);
-            sum += scaled;
+            const float c = (float)n[i];
+            scaled[i] = 0.0f;
+            if (c > 0.0f) scaled[i] = powf(c / max_count, 1.0f / temperature);
+            sum += scaled[i];
         }
     for (int32_t i = 0; i < cc; i++) {
         if (!is_child(i)) continue;
@@ -760,12 +733,9 @@ int omk_forest_action_probabilities(omk_forest *f, int32_t root, float temperatu
         } else if (max_count <= 0.0f || !(sum > 0.0f)) {
             prob = 1.0f / (float)children;
         } else {
-            const float c = (float)n[(size_t)i];
-            float scaled = 0.0f;
-            if (c > 0.0f) scaled = powf(c / max_count, 1.0f / temperature);
-            prob = scaled / sum;
+            prob = scaled[i] / sum;
         }
-        const int32_t a = act[(size_t)i];
+        const int32_t a = act[i];
         if (a >= 0 && a < action_space) h_probabilities[a] = prob;
     }
     return OMK_OK;
@@ -778,30 +748,13 @@ int omk_forest_reroot_child(omk_forest *f, int32_t root, int32_t last_action, in
     *h_child = -1;
     if (last_action < 0) return OMK_OK;
     if (int rc = use_device(f)) return rc;
-    HIP_TRY(hipStreamSynchronize(f->stream));
-    int2 sp;
-    HIP_TRY(hipMemcpy(&sp, f->span + root, sizeof(sp), hipMemcpyDeviceToHost));
-    if (sp.y <= 0) return OMK_OK;
-    std::vector<int32_t> act((size_t)sp.y);
-    if (f->has_action) {
-        HIP_TRY(hipMemcpy(act.data(), f->action + sp.x, (size_t)sp.y * 4, hipMemcpyDeviceToHost));
-    } else {
-        for (int32_t i = 0; i < sp.y; i++) act[(size_t)i] = sp.x + i;
-    }
-    std::vector<uint32_t> legal;
-    const int64_t w0 = (int64_t)sp.x >> 5, w1 = ((int64_t)sp.x + sp.y + 31) >> 5;
-    if (f->has_legal) {
-        legal.resize((size_t)(w1 - w0));
-        HIP_TRY(hipMemcpy(legal.data(), f->legal + w0, legal.size() * 4, hipMemcpyDeviceToHost));
-    }
-    for (int32_t i = 0; i < sp.y; i++) {
-        const int64_t id = (int64_t)sp.x + i;
-        if (f->has_legal && !((legal[(size_t)((id >> 5) - w0)] >> (id & 31)) & 1u)) continue;
-        if (act[(size_t)i] == last_action) {
-            *h_child = (int32_t)id;
+    RootChildren kids;
+    if (int rc = root_children(f, root, &kids)) return rc;
+    for (int32_t i = 0; i < kids.count; i++)
+        if (kids.legal[i] && kids.action[i] == last_action) {
+            *h_child = kids.begin + i;
             break;
         }
-    }
     return OMK_OK;
 }
 
@@ -1585,10 +1538,7 @@ int omk_batch_truncated(omk_batch *b, int32_t *h_count) {
     if (!b || !h_count) return fail(OMK_ERR_INVALID, "omk_batch_truncated: null argument");
     if (!b->selected) return fail(OMK_ERR_STATE, "omk_batch_truncated: no selected paths");
     if (int rc = use_device(b->f)) return rc;
-    HIP_TRY(hipMemcpyAsync(h_count, b->counters + kTruncatedWord + (b->epoch & 1), 4, hipMemcpyDeviceToHost,
-                           b->f->stream));
-    HIP_TRY(hipStreamSynchronize(b->f->stream));
-    return OMK_OK;
+    return link_fetch(b->f, h_count, b->counters + kTruncatedWord + (b->epoch & 1), 1);
 }
 
 int omk_batch_set_stats(omk_batch *b, int32_t enabled) {
@@ -1678,6 +1628,11 @@ int omk_tt_create(omk_forest *f, int32_t log2_slots, omk_tt **out) {
         omk_tt_destroy(tt);
         return rc;
     }
+    if (hipError_t z = launch_fill_words(tt->d_status, 0u, 8, f->stream); z != hipSuccess) {
+        int rc = fail(OMK_ERR_HIP, "omk_tt_create: %s", hipGetErrorString(z));
+        omk_tt_destroy(tt);
+        return rc;
+    }
     *out = tt;
     return omk_tt_clear(tt);
 }
@@ -1705,17 +1660,29 @@ int omk_tt_clear(omk_tt *tt) {
     return OMK_OK;
 }
 
+}  // extern "C"
+
+// The counters of the call just enqueued, which are left at zero; waits for it.
+static int tt_counts(omk_tt *tt, int32_t status[8]) {
+    omk_forest *f = tt->f;
+    void *staged = nullptr;
+    if (int rc = link_stage(f, 32, &staged)) return rc;
+    HIP_TRY(launch_report(tt->d_status, 8, (int32_t *)staged, link_signal(f), f->stream));
+    if (int rc = link_wait(f)) return rc;
+    memcpy(status, staged, 32);
+    return OMK_OK;
+}
+
+extern "C" {
+
 int omk_tt_insert(omk_tt *tt, const uint64_t *d_keys, const int32_t *d_nodes, const int32_t *d_depths, int64_t n) {
     if (!tt || !d_keys || !d_nodes) return fail(OMK_ERR_INVALID, "omk_tt_insert: null argument");
     if (n < 0) return fail(OMK_ERR_INVALID, "omk_tt_insert: n %lld", (long long)n);
     if (int rc = use_device(tt->f)) return rc;
     if (int rc = tt_same_tree(tt)) return rc;
-    hipStream_t s = tt->f->stream;
-    int status[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    HIP_TRY(hipMemcpyAsync(tt->d_status, status, sizeof(status), hipMemcpyHostToDevice, s));
-    HIP_TRY(launch_tt_insert(tt->slots, tt->log2_slots, d_keys, d_nodes, d_depths, n, tt->d_status, s));
-    HIP_TRY(hipMemcpyAsync(status, tt->d_status, sizeof(status), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    int32_t status[8];
+    HIP_TRY(launch_tt_insert(tt->slots, tt->log2_slots, d_keys, d_nodes, d_depths, n, tt->d_status, tt->f->stream));
+    if (int rc = tt_counts(tt, status)) return rc;
     if (status[1]) return fail(OMK_ERR_INVALID, "omk_tt_insert: %d keys equal the empty marker ~0", status[1]);
     if (status[0]) return fail(OMK_ERR_CAPACITY, "omk_tt_insert: table full, %d entries dropped", status[0]);
     return OMK_OK;
@@ -1772,14 +1739,11 @@ int omk_tt_store(omk_tt *tt, const uint64_t *d_keys, const int32_t *d_nodes, con
     if (int rc = use_device(tt->f)) return rc;
     if (int rc = tt_same_tree(tt)) return rc;
     if (int rc = tt_work(tt, (size_t)std::max<int64_t>(n, 1) * 8)) return rc;
-    hipStream_t s = tt->f->stream;
-    int status[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    HIP_TRY(hipMemcpyAsync(tt->d_status, status, sizeof(status), hipMemcpyHostToDevice, s));
+    int32_t status[8];
     HIP_TRY(launch_tt_store(tt->f->dev(), tt->slots, tt->meta, tt->log2_slots, d_keys, d_nodes, d_depths, n,
-                            (int64_t *)tt->work, tt->clock, tt->threshold, tt->d_status, s));
+                            (int64_t *)tt->work, tt->clock, tt->threshold, tt->d_status, tt->f->stream));
     tt->clock += (uint32_t)n;
-    HIP_TRY(hipMemcpyAsync(status, tt->d_status, sizeof(status), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    if (int rc = tt_counts(tt, status)) return rc;
     return tt_report("omk_tt_store", status, h_counts);
 }
 
@@ -1801,32 +1765,29 @@ int omk_tt_traverse(omk_tt *tt, omk_batch *b, const uint64_t *d_piece_keys, int3
     if (int rc = tt_same_tree(tt)) return rc;
     hipStream_t s = f->stream;
     const int64_t n = (int64_t)b->n * b->max_depth;
-    // staging: slot_of [n] i64 | keys [n] u64 | step_nodes, store_nodes, depths, found [n] i32 each
-    if (int rc = tt_work(tt, (size_t)n * 32)) return rc;
+    // work space: slot_of [n] i64 | keys [n] u64 | step_nodes, store_nodes [n] i32 each
+    if (int rc = tt_work(tt, (size_t)n * 24)) return rc;
     int64_t *slot_of = (int64_t *)tt->work;
     uint64_t *keys = (uint64_t *)(slot_of + n);
-    int32_t *step_nodes = (int32_t *)(keys + n), *store_nodes = step_nodes + n, *depths = store_nodes + n;
-    int32_t *found = depths + n;
-    int status[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    HIP_TRY(hipMemcpyAsync(tt->d_status, status, sizeof(status), hipMemcpyHostToDevice, s));
-    HIP_TRY(launch_step_keys(f->dev(), b->paths, b->path_len, b->n, b->stride, b->max_depth, d_piece_keys, cells,
-                             d_player_keys, d_root_keys, d_root_players, keys, step_nodes, store_nodes, depths,
-                             tt->d_status, s));
+    int32_t *step_nodes = (int32_t *)(keys + n), *store_nodes = step_nodes + n;
+    void *staged = nullptr;
+    if (int rc = link_stage(f, 32, &staged)) return rc;
+    const int32_t *status = (const int32_t *)staged;
     // all stores first, then all lookups: a lookup that the serial loop makes before a later step's
     // store can only miss a node without visits, and such a node is no transposition (:142)
-    HIP_TRY(launch_tt_store(f->dev(), tt->slots, tt->meta, tt->log2_slots, keys, store_nodes, depths, n, slot_of,
-                            tt->clock, tt->threshold, tt->d_status, s));
-    tt->clock += (uint32_t)n;
-    HIP_TRY(launch_tt_probe(tt->slots, tt->log2_slots, keys, nullptr, nullptr, 0, n, 0, found, tt->meta, tt->clock, s));
-    tt->clock += (uint32_t)n;
-    HIP_TRY(launch_tt_hits(f->dev(), step_nodes, found, n, d_hits, tt->d_status, s));
-    HIP_TRY(hipMemcpyAsync(status, tt->d_status, sizeof(status), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HIP_TRY(launch_tt_traverse(f->dev(), tt->slots, tt->meta, tt->log2_slots, b->paths, b->path_len, b->n, b->stride,
+                               b->max_depth, d_piece_keys, cells, d_player_keys, d_root_keys, d_root_players, keys,
+                               step_nodes, store_nodes, slot_of, tt->clock, tt->threshold, d_hits, tt->d_status,
+                               (int32_t *)staged, link_signal(f), s));
+    tt->clock += 2u * (uint32_t)n;  // a time for every store, then one for every lookup
+    if (int rc = link_wait(f)) return rc;
     if (status[5])
         return fail(OMK_ERR_INVALID, "omk_tt_traverse: %d paths hold a node outside the forest or a move outside [0, %d)",
                     status[5], cells);
-    status[1] = 0;  // steps that do not exist carry the empty marker on purpose
-    return tt_report("omk_tt_traverse", status, h_counts);
+    int32_t st[8];
+    memcpy(st, status, 32);
+    st[1] = 0;  // steps that do not exist carry the empty marker on purpose
+    return tt_report("omk_tt_traverse", st, h_counts);
 }
 
 int omk_tt_select_redirect(omk_tt *tt, omk_batch *b, const omk_select_params *p, int32_t *d_moves, int32_t *h_counts) {
@@ -1852,8 +1813,6 @@ int omk_tt_select_redirect(omk_tt *tt, omk_batch *b, const omk_select_params *p,
         HIP_TRY(launch_fill_words(f->alias, 0xFFFFFFFFu, f->capacity, s));
     }
     if (int rc = next_epoch(b)) return rc;
-    int status[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    HIP_TRY(hipMemcpyAsync(tt->d_status, status, sizeof(status), hipMemcpyHostToDevice, s));
     RedirectArgs a;
     memset(&a, 0, sizeof(a));
     a.alias = f->alias;
@@ -1879,8 +1838,8 @@ int omk_tt_select_redirect(omk_tt *tt, omk_batch *b, const omk_select_params *p,
     HIP_TRY(launch_select_redirect(f->dev(), a, p->use_rave != 0, s));
     b->selected = true;
     b->select_calls++;
-    HIP_TRY(hipMemcpyAsync(status, tt->d_status, sizeof(status), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    int32_t status[8];
+    if (int rc = tt_counts(tt, status)) return rc;
     tt->clock += (uint32_t)status[6];  // the ticks of the access counter
     if (status[3] > 0) f->redirected = true;
     if (h_counts)
@@ -1925,13 +1884,14 @@ int omk_batch_leaf_keys(omk_batch *b, const uint64_t *d_piece_keys, int32_t cell
     omk_forest *f = b->f;
     if (int rc = use_device(f)) return rc;
     hipStream_t s = f->stream;
-    int32_t *d_status = b->counters + 32;  // a word of the batch's counter block that nothing else uses
-    int bad = 0;
-    HIP_TRY(hipMemcpyAsync(d_status, &bad, sizeof(bad), hipMemcpyHostToDevice, s));
+    int32_t *d_status = b->counters + 32;  // a word of the batch's counter block that nothing else uses: zero between calls
+    void *staged = nullptr;
+    if (int rc = link_stage(f, 4, &staged)) return rc;
     HIP_TRY(launch_leaf_keys(f->dev(), b->paths, b->path_len, b->n, b->stride, d_piece_keys, cells, d_player_keys,
                              d_root_keys, d_root_players, d_out, d_status, s));
-    HIP_TRY(hipMemcpyAsync(&bad, d_status, sizeof(bad), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HIP_TRY(launch_report(d_status, 1, (int32_t *)staged, link_signal(f), s));
+    if (int rc = link_wait(f)) return rc;
+    const int bad = *(const int32_t *)staged;
     if (bad)
         return fail(OMK_ERR_INVALID, "omk_batch_leaf_keys: %d paths hold a move outside [0, %d) or no node at all "
                     "(their keys are ~0)", bad, cells);
@@ -1982,6 +1942,14 @@ int omk_dev_copy(omk_forest *f, void *d_dst, const void *d_src, int64_t bytes) {
 int omk_dev_h2d(omk_forest *f, void *d_dst, const void *h_src, int64_t bytes) {
     if (!f || !d_dst || !h_src || bytes < 0) return fail(OMK_ERR_INVALID, "omk_dev_h2d: bad argument");
     if (int rc = use_device(f)) return rc;
+    if (bytes == 0) return OMK_OK;
+    if (((uintptr_t)d_dst & 3) == 0 && (bytes & 3) == 0 && (size_t)bytes <= kLinkStaging) {
+        void *staged = nullptr;
+        if (int rc = link_stage(f, (size_t)bytes, &staged)) return rc;
+        memcpy(staged, h_src, (size_t)bytes);
+        HIP_TRY(launch_fetch((uint32_t *)d_dst, (const uint32_t *)staged, bytes / 4, link_signal(f), f->stream));
+        return link_wait(f);  // the copy is done on return, whatever stream reads it
+    }
     HIP_TRY(hipMemcpyAsync(d_dst, h_src, (size_t)bytes, hipMemcpyHostToDevice, f->stream));
     HIP_TRY(hipStreamSynchronize(f->stream));
     return OMK_OK;
@@ -1990,6 +1958,9 @@ int omk_dev_h2d(omk_forest *f, void *d_dst, const void *h_src, int64_t bytes) {
 int omk_dev_d2h(omk_forest *f, void *h_dst, const void *d_src, int64_t bytes) {
     if (!f || !h_dst || !d_src || bytes < 0) return fail(OMK_ERR_INVALID, "omk_dev_d2h: bad argument");
     if (int rc = use_device(f)) return rc;
+    if (bytes == 0) return OMK_OK;
+    if (((uintptr_t)d_src & 3) == 0 && (bytes & 3) == 0 && (size_t)bytes <= kLinkStaging)
+        return link_fetch(f, h_dst, d_src, (size_t)bytes / 4);
     HIP_TRY(hipMemcpyAsync(h_dst, d_src, (size_t)bytes, hipMemcpyDeviceToHost, f->stream));
     HIP_TRY(hipStreamSynchronize(f->stream));
     return OMK_OK;

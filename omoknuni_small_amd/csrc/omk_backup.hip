@@ -277,6 +277,62 @@ hipError_t launch_expand(const ForestMut &f, const ExpandJob *jobs, int n_jobs, 
     return hipGetLastError();
 }
 
+// ---- a root's children for the host, and the noise on their priors ----
+
+__global__ __launch_bounds__(256) void k_root_children(ForestDev f, const int32_t *alias, int32_t root, int32_t *head,
+                                                       int32_t *rows, int room, HostSignal sig) {
+    const int2 sp = f.span[root];
+    if (threadIdx.x == 0) {
+        host_store(head, sp.x);
+        host_store(head + 1, sp.y);
+    }
+    for (int i = threadIdx.x; i < sp.y && i < room; i += 256) {
+        const int id = sp.x + i;
+        const int al = alias ? alias[id] : -1;
+        host_store(rows + i, f.N[al >= 0 ? al : id]);
+        host_store(rows + room + i, f.action ? f.action[id] : id);
+        host_store(rows + 2 * room + i, f.legal ? (int)((f.legal[(uint32_t)id >> 5] >> ((uint32_t)id & 31u)) & 1u) : 1);
+    }
+    host_signal(sig.count, sig.flag, sig.seq, 1);
+}
+
+hipError_t launch_root_children(const ForestDev &f, const int32_t *alias, int32_t root, int32_t *head, int32_t *rows,
+                                int room, const HostSignal &sig, hipStream_t s) {
+    hipLaunchKernelGGL(k_root_children, dim3(1), dim3(256), 0, s, f, alias, root, head, rows, room, sig);
+    return hipGetLastError();
+}
+
+// MCTSEngine::addDirichletNoise's mix (src/mcts/mcts_engine_eval.cpp:100-109).  Noise j belongs to the j-th legal
+// slot; one block, 1024 threads: a slot per thread (OMK_MAX_FANOUT), its rank from the ballots of the wavefronts.
+__global__ __launch_bounds__(1024) void k_root_noise(ForestMut f, int32_t root, const float *noise, int n_noise,
+                                                     float epsilon, int32_t *head, HostSignal sig) {
+    __shared__ int s_count[16];
+    const int2 sp = f.span[root];
+    const int i = threadIdx.x, id = sp.x + i;
+    const bool child = i < sp.y && (!f.legal || ((f.legal[(uint32_t)id >> 5] >> ((uint32_t)id & 31u)) & 1u));
+    const uint64_t mask = __ballot(child);
+    if ((i & 63) == 0) s_count[i >> 6] = __popcll(mask);
+    __syncthreads();
+    int rank = __popcll(mask & ((1ull << (i & 63)) - 1ull)), children = 0;
+    for (int w = 0; w < 16; w++) {
+        if (w < (i >> 6)) rank += s_count[w];
+        children += s_count[w];
+    }
+    if (child && children == n_noise) {
+        const float keep = (1.0f - epsilon) * f.P[id];
+        const float add = epsilon * noise[rank];
+        f.P[id] = keep + add;
+    }
+    if (i == 0) host_store(head, children);
+    host_signal(sig.count, sig.flag, sig.seq, 1);
+}
+
+hipError_t launch_root_noise(const ForestMut &f, int32_t root, const float *noise, int n_noise, float epsilon,
+                             int32_t *head, const HostSignal &sig, hipStream_t s) {
+    hipLaunchKernelGGL(k_root_noise, dim3(1), dim3(1024), 0, s, f, root, noise, n_noise, epsilon, head, sig);
+    return hipGetLastError();
+}
+
 // ---- RAVE statistics of MCTSEngine::backPropagate (src/mcts/mcts_engine_tree.cpp:288-331,
 // MCTSNode::updateRAVE src/mcts/mcts_node.cpp:631-643): every child of a path node whose
 // action occurs among the path's actions gets rN += 1, rW += the node's signed value ----
@@ -373,6 +429,31 @@ hipError_t launch_copy_words(void *dst, const void *src, int64_t n_words, hipStr
     if (blocks > 65536) blocks = 65536;
     hipLaunchKernelGGL(k_copy_words, dim3((unsigned)blocks), dim3(256), 0, s, (uint32_t *)dst, (const uint32_t *)src,
                        n_words);
+    return hipGetLastError();
+}
+
+__global__ __launch_bounds__(256) void k_fetch(uint32_t *h_dst, const uint32_t *src, int64_t n, HostSignal sig) {
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) host_store(h_dst + i, src[i]);
+    host_signal(sig.count, sig.flag, sig.seq, gridDim.x);
+}
+
+hipError_t launch_fetch(uint32_t *h_dst, const uint32_t *src, int64_t n, const HostSignal &sig, hipStream_t s) {
+    const int64_t blocks = n > 0 ? (n + 255) / 256 : 1;
+    hipLaunchKernelGGL(k_fetch, dim3((unsigned)blocks), dim3(256), 0, s, h_dst, src, n, sig);
+    return hipGetLastError();
+}
+
+__global__ __launch_bounds__(64) void k_report(int *words, int n, int32_t *h_dst, HostSignal sig) {
+    if ((int)threadIdx.x < n) {
+        host_store(h_dst + threadIdx.x, words[threadIdx.x]);
+        words[threadIdx.x] = 0;
+    }
+    host_signal(sig.count, sig.flag, sig.seq, 1);
+}
+
+hipError_t launch_report(int *words, int n, int32_t *h_dst, const HostSignal &sig, hipStream_t s) {
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, s, words, n, h_dst, sig);
     return hipGetLastError();
 }
 
@@ -487,17 +568,13 @@ __global__ __launch_bounds__(256) void k_tt_clear(TTSlot *slots, TTMeta *meta, i
 // score 0, and never replaces; the leaves expanded in one step are distinct).
 
 // Pass 1: every entry finds the slot of its key, or claims an empty one, and bids for it with its index.
-__global__ __launch_bounds__(256) void k_tt_store_claim(TTSlot *slots, TTMeta *meta, int log2_slots,
-                                                        const uint64_t *keys, const int32_t *nodes, int64_t n,
-                                                        int64_t *slot_of, int *d_status) {
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    slot_of[i] = -1;
-    if (nodes[i] < 0) return;  // nothing to store for this entry (store(): if (!node) return)
-    unsigned long long key = keys[i];
+// Returns that slot, or -1 when there is nothing to store.
+__device__ __forceinline__ int64_t tt_claim(TTSlot *slots, TTMeta *meta, int log2_slots, unsigned long long key, int node,
+                                            int i, int *d_status) {
+    if (node < 0) return -1;  // nothing to store for this entry (store(): if (!node) return)
     if (key == kTTEmpty) {
         atomicAdd(d_status + 1, 1);
-        return;
+        return -1;
     }
     uint64_t mask = (1ull << log2_slots) - 1ull;
     uint64_t s = tt_home(key, log2_slots);
@@ -505,12 +582,19 @@ __global__ __launch_bounds__(256) void k_tt_store_claim(TTSlot *slots, TTMeta *m
         unsigned long long prev = atomicCAS(&slots[s].key, kTTEmpty, key);
         if (prev == kTTEmpty) slots[s].depth = INT32_MIN;  // claimed just now: no entry behind the key yet
         if (prev == kTTEmpty || prev == key) {
-            atomicMin(&meta[s].claim, (int)i);
-            slot_of[i] = (int64_t)s;
-            return;
+            atomicMin(&meta[s].claim, i);
+            return (int64_t)s;
         }
     }
     atomicAdd(d_status, 1);
+    return -1;
+}
+
+__global__ __launch_bounds__(256) void k_tt_store_claim(TTSlot *slots, TTMeta *meta, int log2_slots,
+                                                        const uint64_t *keys, const int32_t *nodes, int64_t n,
+                                                        int64_t *slot_of, int *d_status) {
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) slot_of[i] = tt_claim(slots, meta, log2_slots, keys[i], nodes[i], (int)i, d_status);
 }
 
 __device__ __forceinline__ float tt_replacement_score(uint32_t visits, float value, int depth, uint32_t now,
@@ -525,8 +609,8 @@ __device__ __forceinline__ float tt_replacement_score(uint32_t visits, float val
 // node as they are now) or replaces the one that is there when its score is better by the threshold.
 // d_status[2] duplicates dropped, [3] new entries, [4] replacements.
 __global__ __launch_bounds__(256) void k_tt_store_apply(ForestDev f, TTSlot *slots, TTMeta *meta,
-                                                        const int32_t *nodes, const int32_t *depths, int64_t n,
-                                                        const int64_t *slot_of, uint32_t t0, float threshold,
+                                                        const int32_t *nodes, const int32_t *depths, int path_steps,
+                                                        int64_t n, const int64_t *slot_of, uint32_t t0, float threshold,
                                                         int *d_status) {
     int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
@@ -537,7 +621,9 @@ __global__ __launch_bounds__(256) void k_tt_store_apply(ForestDev f, TTSlot *slo
         return;
     }
     const int node = nodes[i];
-    const int depth = (int)(uint16_t)(depths ? depths[i] : 0);  // Entry::depth is a uint16_t
+    // (entries laid out by path: entry i is step i % path_steps + 1 of its path)
+    const int given = depths ? depths[i] : path_steps > 0 ? (int)(i % path_steps) + 1 : 0;
+    const int depth = (int)(uint16_t)given;  // Entry::depth is a uint16_t
     uint32_t visits = 0u;
     float value = 0.0f;
     if (node < f.n_nodes) {
@@ -581,7 +667,7 @@ hipError_t launch_tt_store(const ForestDev &f, TTSlot *slots, TTMeta *meta, int 
     if (n <= 0) return hipSuccess;
     const dim3 grid((unsigned)((n + 255) / 256)), block(256);
     hipLaunchKernelGGL(k_tt_store_claim, grid, block, 0, s, slots, meta, log2_slots, keys, nodes, n, slot_of, d_status);
-    hipLaunchKernelGGL(k_tt_store_apply, grid, block, 0, s, f, slots, meta, nodes, depths, n, slot_of, t0, threshold,
+    hipLaunchKernelGGL(k_tt_store_apply, grid, block, 0, s, f, slots, meta, nodes, depths, 0, n, slot_of, t0, threshold,
                        d_status);
     hipLaunchKernelGGL(k_tt_store_reset, grid, block, 0, s, meta, slot_of, n);
     return hipGetLastError();
@@ -592,20 +678,20 @@ hipError_t launch_tt_store(const ForestDev &f, TTSlot *slots, TTMeta *meta, int 
 
 // The key of the state after every step of every path, the node selected there and its depth, laid
 // out in the order the serial loop visits them (traversal-major: entry t * max_depth + d - 1 for step
-// d >= 1 of traversal t); node -1 where the path has no such step.  Keys: the forest's per-node
-// position keys, or (piece != nullptr) the root state's key with the piece keys of the path's moves
-// folded in, as in k_leaf_keys.  store_nodes receives the node where the reference stores it
-// (its visit count is 0, :116) and -1 elsewhere.
+// d >= 1 of traversal t); node -1 where the path has no such step.  Keys: the root state's key with
+// the piece keys of the path's moves folded in, as in k_leaf_keys, one thread along a path.
+// store_nodes receives the node where the reference stores it (its visit count is 0, :116) and -1
+// elsewhere.
 __global__ __launch_bounds__(256) void k_step_keys(ForestDev f, const int32_t *paths, const int32_t *path_len, int n,
                                                    int stride, int max_depth, const uint64_t *piece, int cells,
                                                    const uint64_t *player, const uint64_t *root_key,
                                                    const int32_t *root_player, uint64_t *keys, int32_t *step_nodes,
-                                                   int32_t *store_nodes, int32_t *depths, int *d_status) {
+                                                   int32_t *store_nodes, int *d_status) {
     const int t = blockIdx.x * 256 + threadIdx.x;
     if (t >= n) return;
     const int len = path_len[t];
-    const int p0 = piece ? (root_player[t] & 1) : 0;
-    uint64_t h = piece ? root_key[t] : 0ull;
+    const int p0 = root_player[t] & 1;
+    uint64_t h = root_key[t];
     bool bad = false;
     for (int d = 1; d <= max_depth; d++) {
         const size_t e = (size_t)t * max_depth + (d - 1);
@@ -616,7 +702,7 @@ __global__ __launch_bounds__(256) void k_step_keys(ForestDev f, const int32_t *p
             if (node < 0 || node >= f.n_nodes) {
                 bad = true;
                 node = -1;
-            } else if (piece) {
+            } else {
                 const int act = f.action ? f.action[node] : node;
                 if (act < 0 || act >= cells) {
                     bad = true;
@@ -625,89 +711,50 @@ __global__ __launch_bounds__(256) void k_step_keys(ForestDev f, const int32_t *p
                     h ^= piece[(size_t)((p0 + d - 1) & 1) * cells + act];
                     key = (d & 1) ? h ^ player[p0] ^ player[p0 ^ 1] : h;
                 }
-            } else {
-                key = f.hash[node];
             }
         }
         keys[e] = key;
         step_nodes[e] = node;
         store_nodes[e] = node >= 0 && f.N[node] == 0 ? node : -1;
-        depths[e] = d;
     }
     if (bad) atomicAdd(d_status + 5, 1);
 }
 
-// What the loop does with a lookup (:141-156): a node other than the selected one, with visits, is a
-// transposition.  It is reported (hit[e] = that node, else -1), never followed.
-__global__ __launch_bounds__(256) void k_tt_hits(ForestDev f, const int32_t *step_nodes, const int32_t *found, int64_t n,
-                                                 int32_t *hit, int *d_status) {
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int fn = found[i], node = step_nodes[i];
-    int out = -1;
-    if (node >= 0 && fn >= 0 && fn != node && fn < f.n_nodes && f.N[fn] > 0) out = fn;
-    if (hit) hit[i] = out;  // a caller that only wants the count passes no array
-    if (out >= 0) atomicAdd(d_status + 6, 1);
-}
-
-hipError_t launch_step_keys(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
-                            int max_depth, const uint64_t *piece, int cells, const uint64_t *player,
-                            const uint64_t *root_key, const int32_t *root_player, uint64_t *keys, int32_t *step_nodes,
-                            int32_t *store_nodes, int32_t *depths, int *d_status, hipStream_t s) {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_step_keys, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, f, paths, path_len, n, stride,
-                       max_depth, piece, cells, player, root_key, root_player, keys, step_nodes, store_nodes, depths,
-                       d_status);
-    return hipGetLastError();
-}
-
-hipError_t launch_tt_hits(const ForestDev &f, const int32_t *step_nodes, const int32_t *found, int64_t n, int32_t *hit,
-                          int *d_status, hipStream_t s) {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_tt_hits, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, f, step_nodes, found, n, hit,
-                       d_status);
-    return hipGetLastError();
-}
-
-// d_status[0] counts entries that found no slot, d_status[1] keys equal to the empty marker
-__global__ __launch_bounds__(256) void k_tt_insert(TTSlot *slots, int log2_slots, const uint64_t *keys,
-                                                   const int32_t *nodes, const int32_t *depths, int64_t n,
-                                                   int *d_status) {
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    unsigned long long key = keys[i];
-    if (key == kTTEmpty) {
-        atomicAdd(d_status + 1, 1);
-        return;
-    }
-    uint64_t mask = (1ull << log2_slots) - 1ull;
-    uint64_t s = tt_home(key, log2_slots);
-    for (uint64_t probe = 0; probe <= mask; probe++, s = (s + 1) & mask) {
-        unsigned long long prev = atomicCAS(&slots[s].key, kTTEmpty, key);
-        if (prev == kTTEmpty) {
-            slots[s].node = nodes[i];
-            slots[s].depth = depths ? depths[i] : 0;
-            return;
+// The same for per-node keys, which need no walk along the path: a thread per step, all trips in flight at once,
+// and pass 1 of the store at once (one thread per path took a trip to memory per level one after the other).
+__global__ __launch_bounds__(256) void k_step_claim(ForestDev f, TTSlot *slots, TTMeta *meta, int log2_slots,
+                                                    const int32_t *paths, const int32_t *path_len, int n, int stride,
+                                                    int max_depth, uint64_t *keys, int32_t *step_nodes,
+                                                    int32_t *store_nodes, int64_t *slot_of, int *d_status) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= (int64_t)n * max_depth) return;
+    const int t = (int)(e / max_depth), d = (int)(e - (int64_t)t * max_depth) + 1;
+    int node = -1;
+    if (d < path_len[t]) {
+        node = paths[(size_t)d * stride + t];
+        if (node < 0 || node >= f.n_nodes) {  // a path counts once, and ends there
+            bool first = true;
+            for (int q = 1; q < d && first; q++) {
+                const int above = paths[(size_t)q * stride + t];
+                first = above >= 0 && above < f.n_nodes;
+            }
+            if (first) atomicAdd(d_status + 5, 1);
+            node = -1;
         }
-        if (prev == key) return;  // already present: the first entry stays
     }
-    atomicAdd(d_status, 1);
+    const uint64_t key = node >= 0 ? f.hash[node] : kTTEmpty;
+    const int store = node >= 0 && f.N[node] == 0 ? node : -1;
+    keys[e] = key;
+    step_nodes[e] = node;
+    store_nodes[e] = store;
+    slot_of[e] = tt_claim(slots, meta, log2_slots, key, store, (int)e, d_status);
 }
 
-// meta / t0: a successful lookup stamps the entry with its time (PHMapTranspositionTable::lookup,
-// phmap_transposition_table.cpp:107: last_access = access_counter++); lookup i of a call has the time
-// t0 + i, the latest wins.
-__global__ __launch_bounds__(256) void k_tt_probe(const TTSlot *slots, int log2_slots, const uint64_t *keys,
-                                                  const int32_t *leaf, const uint64_t *node_hash, int64_t n_nodes,
-                                                  int64_t n, int min_depth, int32_t *out, TTMeta *meta, uint32_t t0) {
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const bool valid = i < n;
-    unsigned long long key = kTTEmpty;
-    if (valid) {
-        if (keys) key = keys[i];
-        // a traversal without a leaf finds nothing; never index the forest with an id it does not have
-        else if (leaf[i] >= 0 && leaf[i] < n_nodes) key = node_hash[leaf[i]];
-    }
+// One lookup per lane (key kTTEmpty: none): the node found or -1.  meta / t0: a successful lookup stamps the entry
+// with its time (PHMapTranspositionTable::lookup, phmap_transposition_table.cpp:107: last_access =
+// access_counter++); lookup i of a call has the time t0 + i, the latest wins.  All 64 lanes take part.
+__device__ __forceinline__ int tt_lookup(const TTSlot *slots, int log2_slots, unsigned long long key, int min_depth,
+                                         TTMeta *meta, uint32_t time) {
     int found = -1;
     unsigned long long hit_slot = ~0ull;
     if (key != kTTEmpty) {
@@ -738,31 +785,123 @@ __global__ __launch_bounds__(256) void k_tt_probe(const TTSlot *slots, int log2_
             const int lead = __ffsll((long long)todo) - 1;
             const unsigned long long s0 = __shfl(hit_slot, lead);
             const unsigned long long same = __ballot(hit_slot == s0);
-            if (lane == 63u - (unsigned)__clzll((long long)same)) atomicMax(&meta[s0].last_access, t0 + (uint32_t)i);
+            if (lane == 63u - (unsigned)__clzll((long long)same)) atomicMax(&meta[s0].last_access, time);
             todo &= ~same;
         }
     }
+    return found;
+}
+
+// What the loop does with a lookup (:141-156): a node other than the selected one, with visits, is a
+// transposition.  It is reported (hit[e] = that node, else -1), never followed.  The bids of the stores before are
+// withdrawn on the way (pass 3), and the counters go to the host with the last block.
+__global__ __launch_bounds__(256) void k_tt_hits(ForestDev f, const TTSlot *slots, TTMeta *meta, int log2_slots,
+                                                 const uint64_t *keys, const int32_t *step_nodes, const int64_t *slot_of,
+                                                 int64_t n, uint32_t t0, int32_t *hit, int *d_status, int32_t *h_status,
+                                                 HostSignal sig) {
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const bool valid = i < n;
+    const int node = valid ? step_nodes[i] : -1;
+    const int fn = tt_lookup(slots, log2_slots, valid ? keys[i] : kTTEmpty, 0, meta, t0 + (uint32_t)i);
+    int out = -1;
+    if (node >= 0 && fn >= 0 && fn != node && fn < f.n_nodes && f.N[fn] > 0) out = fn;
+    if (valid) {
+        if (hit) hit[i] = out;  // a caller that only wants the count passes no array
+        const int64_t s = slot_of[i];
+        if (s >= 0) meta[s].claim = 0x7FFFFFFF;
+    }
+    const uint64_t any = __ballot(out >= 0);
+    if (any && (threadIdx.x & 63) == 0) atomicAdd(d_status + 6, __popcll(any));
+    // host_signal with the counters before the flag
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    if (__hip_atomic_fetch_add(sig.count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (int)gridDim.x - 1) return;
+    __hip_atomic_store(sig.count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int q = 0; q < 8; q++)
+        host_store(h_status + q, __hip_atomic_exchange(d_status + q, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    host_store(sig.flag, sig.seq);
+}
+
+hipError_t launch_tt_traverse(const ForestDev &f, TTSlot *slots, TTMeta *meta, int log2_slots, const int32_t *paths,
+                              const int32_t *path_len, int n, int stride, int max_depth, const uint64_t *piece, int cells,
+                              const uint64_t *player, const uint64_t *root_key, const int32_t *root_player,
+                              uint64_t *keys, int32_t *step_nodes, int32_t *store_nodes, int64_t *slot_of, uint32_t t0,
+                              float threshold, int32_t *hit, int *d_status, int32_t *h_status, const HostSignal &sig,
+                              hipStream_t s) {
+    const int64_t steps = (int64_t)n * max_depth;
+    const dim3 grid((unsigned)((steps + 255) / 256)), block(256);
+    if (piece) {
+        hipLaunchKernelGGL(k_step_keys, dim3((unsigned)((n + 255) / 256)), block, 0, s, f, paths, path_len, n, stride,
+                           max_depth, piece, cells, player, root_key, root_player, keys, step_nodes, store_nodes, d_status);
+        hipLaunchKernelGGL(k_tt_store_claim, grid, block, 0, s, slots, meta, log2_slots, keys, store_nodes, steps, slot_of,
+                           d_status);
+    } else {
+        hipLaunchKernelGGL(k_step_claim, grid, block, 0, s, f, slots, meta, log2_slots, paths, path_len, n, stride,
+                           max_depth, keys, step_nodes, store_nodes, slot_of, d_status);
+    }
+    hipLaunchKernelGGL(k_tt_store_apply, grid, block, 0, s, f, slots, meta, store_nodes, (const int32_t *)nullptr,
+                       max_depth, steps, slot_of, t0, threshold, d_status);
+    hipLaunchKernelGGL(k_tt_hits, grid, block, 0, s, f, slots, meta, log2_slots, keys, step_nodes, slot_of, steps,
+                       t0 + (uint32_t)steps, hit, d_status, h_status, sig);
+    return hipGetLastError();
+}
+
+// d_status[0] counts entries that found no slot, d_status[1] keys equal to the empty marker
+__global__ __launch_bounds__(256) void k_tt_insert(TTSlot *slots, int log2_slots, const uint64_t *keys,
+                                                   const int32_t *nodes, const int32_t *depths, int64_t n,
+                                                   int *d_status) {
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    unsigned long long key = keys[i];
+    if (key == kTTEmpty) {
+        atomicAdd(d_status + 1, 1);
+        return;
+    }
+    uint64_t mask = (1ull << log2_slots) - 1ull;
+    uint64_t s = tt_home(key, log2_slots);
+    for (uint64_t probe = 0; probe <= mask; probe++, s = (s + 1) & mask) {
+        unsigned long long prev = atomicCAS(&slots[s].key, kTTEmpty, key);
+        if (prev == kTTEmpty) {
+            slots[s].node = nodes[i];
+            slots[s].depth = depths ? depths[i] : 0;
+            return;
+        }
+        if (prev == key) return;  // already present: the first entry stays
+    }
+    atomicAdd(d_status, 1);
+}
+
+__global__ __launch_bounds__(256) void k_tt_probe(const TTSlot *slots, int log2_slots, const uint64_t *keys,
+                                                  const int32_t *leaf, const uint64_t *node_hash, int64_t n_nodes,
+                                                  int64_t n, int min_depth, int32_t *out, TTMeta *meta, uint32_t t0) {
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const bool valid = i < n;
+    unsigned long long key = kTTEmpty;
+    if (valid) {
+        if (keys) key = keys[i];
+        // a traversal without a leaf finds nothing; never index the forest with an id it does not have
+        else if (leaf[i] >= 0 && leaf[i] < n_nodes) key = node_hash[leaf[i]];
+    }
+    const int found = tt_lookup(slots, log2_slots, key, min_depth, meta, t0 + (uint32_t)i);
     if (valid) out[i] = found;
 }
 
 // Position keys of single nodes, from the host's game states (IGameState::getHash of the state a
-// node stands for).  An id outside the forest is counted, not written.
+// node stands for).  An id outside the forest is not written (the host counts them).
 __global__ __launch_bounds__(256) void k_set_keys(uint64_t *hash, const int32_t *nodes, const uint64_t *keys, int64_t n,
-                                                  int64_t n_nodes, int *d_bad) {
+                                                  int64_t n_nodes) {
     int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     const int node = nodes[i];
-    if (node < 0 || node >= n_nodes) {
-        atomicAdd(d_bad, 1);
-        return;
-    }
-    hash[node] = keys[i];
+    if (node >= 0 && node < n_nodes) hash[node] = keys[i];
 }
 
 hipError_t launch_set_keys(uint64_t *hash, const int32_t *nodes, const uint64_t *keys, int64_t n, int64_t n_nodes,
-                           int *d_bad, hipStream_t s) {
+                           hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_set_keys, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, hash, nodes, keys, n, n_nodes, d_bad);
+    hipLaunchKernelGGL(k_set_keys, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, hash, nodes, keys, n, n_nodes);
     return hipGetLastError();
 }
 

@@ -155,10 +155,17 @@ hipError_t launch_export(const ForestDev &f, const int32_t *paths, const int32_t
 hipError_t launch_leaf_keys(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                             const uint64_t *piece, int cells, const uint64_t *player, const uint64_t *root_key,
                             const int32_t *root_player, uint64_t *out, int *d_status, hipStream_t s);
+// `n` device words to pinned memory; launch_report takes at most 64 and leaves zeros behind.
+hipError_t launch_fetch(uint32_t *h_dst, const uint32_t *src, int64_t n, const HostSignal &sig, hipStream_t s);
+hipError_t launch_report(int *words, int n, int32_t *h_dst, const HostSignal &sig, hipStream_t s);
 hipError_t launch_copy_words(void *dst, const void *src, int64_t n_words, hipStream_t s);
 hipError_t launch_fill_words(void *dst, uint32_t value, int64_t n_words, hipStream_t s);
 hipError_t launch_set_keys(uint64_t *hash, const int32_t *nodes, const uint64_t *keys, int64_t n, int64_t n_nodes,
-                           int *d_bad, hipStream_t s);
+                           hipStream_t s);
+// head[0..1] = child range of `root`; rows[i], rows[room + i], rows[2 * room + i] = visits of the node its slot i
+// holds, action and legality of the slot, i < room.  head and rows are pinned host memory.
+hipError_t launch_root_children(const ForestDev &f, const int32_t *alias, int32_t root, int32_t *head, int32_t *rows,
+                                int room, const HostSignal &sig, hipStream_t s);
 
 // The same arrays for the one operation that writes the structure (leaf expansion).
 struct ForestMut {
@@ -174,6 +181,10 @@ struct ForestMut {
     int32_t *action;
     uint64_t *hash;
 };
+
+// head[0] = children of `root`; if they are n_noise, prior = (1 - epsilon) * prior + epsilon * noise for each.
+hipError_t launch_root_noise(const ForestMut &f, int32_t root, const float *noise, int n_noise, float epsilon,
+                             int32_t *head, const HostSignal &sig, hipStream_t s);
 
 // One leaf to expand: its children get the ids [begin, begin + count) and the moves / priors
 // moves[off .. off + count), priors[off .. off + count).
@@ -223,12 +234,14 @@ hipError_t launch_tt_clear(TTSlot *slots, TTMeta *meta, int log2_slots, hipStrea
 hipError_t launch_tt_store(const ForestDev &f, TTSlot *slots, TTMeta *meta, int log2_slots, const uint64_t *keys,
                            const int32_t *nodes, const int32_t *depths, int64_t n, int64_t *slot_of, uint32_t t0,
                            float threshold, int *d_status, hipStream_t s);
-hipError_t launch_step_keys(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
-                            int max_depth, const uint64_t *piece, int cells, const uint64_t *player,
-                            const uint64_t *root_key, const int32_t *root_player, uint64_t *keys, int32_t *step_nodes,
-                            int32_t *store_nodes, int32_t *depths, int *d_status, hipStream_t s);
-hipError_t launch_tt_hits(const ForestDev &f, const int32_t *step_nodes, const int32_t *found, int64_t n, int32_t *hit,
-                          int *d_status, hipStream_t s);
+// The table's part of the traversal over selected paths: all stores, then all lookups.  The eight counters end up in
+// `h_status` (pinned) and are zero again; hits as in omk_tt_traverse.
+hipError_t launch_tt_traverse(const ForestDev &f, TTSlot *slots, TTMeta *meta, int log2_slots, const int32_t *paths,
+                              const int32_t *path_len, int n, int stride, int max_depth, const uint64_t *piece, int cells,
+                              const uint64_t *player, const uint64_t *root_key, const int32_t *root_player,
+                              uint64_t *keys, int32_t *step_nodes, int32_t *store_nodes, int64_t *slot_of, uint32_t t0,
+                              float threshold, int32_t *hit, int *d_status, int32_t *h_status, const HostSignal &sig,
+                              hipStream_t s);
 // The traversal loop with the table on, redirects included, one traversal after the other (omk_backup.hip).
 struct RedirectArgs {
     int32_t *alias;

@@ -155,6 +155,7 @@ class Forest:
         self._h = C.c_void_p()
         self.has_rave = bool(has_rave)
         self.n_nodes = 0
+        self._kept = set()  # device buffers that tables keep between calls: freed with the table, or with the forest
         desc = _ForestDesc(int(capacity_nodes), int(device), int(self.has_rave))
         _check(self._lib.omk_forest_create(C.byref(desc), C.byref(self._h)))
 
@@ -167,6 +168,9 @@ class Forest:
 
     def close(self):
         if self._h:
+            for p in self._kept:
+                self.dev_free(p)
+            self._kept = set()
             self._lib.omk_forest_destroy(self._h)
             self._h = C.c_void_p()
 
@@ -489,10 +493,12 @@ class TranspositionTable:
         self.forest = forest
         self.log2 = int(log2_slots)
         self._h = C.c_void_p()
+        self._hits, self._hits_bytes = 0, 0  # device buffer of traverse()
         _check(self._lib.omk_tt_create(forest._h, self.log2, C.byref(self._h)))
 
     def close(self):
         if self._h:
+            self._drop_hits()
             self._lib.omk_tt_destroy(self._h)
             self._h = C.c_void_p()
 
@@ -501,6 +507,12 @@ class TranspositionTable:
             self.close()
         except Exception:
             pass
+
+    def _drop_hits(self):
+        if self._hits in self.forest._kept:
+            self.forest._kept.remove(self._hits)
+            self.forest.dev_free(self._hits)
+        self._hits, self._hits_bytes = 0, 0
 
     def clear(self):
         _check(self._lib.omk_tt_clear(self._h))
@@ -595,7 +607,11 @@ class TranspositionTable:
         n, D = batch.n, batch.max_depth
         hits = np.empty((n, D), np.int32)
         counts = np.zeros(4, np.int32)
-        bufs = [f.dev_alloc(hits.nbytes)]
+        if hits.nbytes > self._hits_bytes:  # kept for the next batch of the search
+            self._drop_hits()
+            self._hits, self._hits_bytes = f.dev_alloc(hits.nbytes), hits.nbytes
+            f._kept.add(self._hits)
+        bufs = []
         args = [0, 0, 0, 0, 0]
         try:
             if zobrist is not None:
@@ -605,11 +621,11 @@ class TranspositionTable:
                 for x in arrs:
                     bufs.append(f.dev_alloc(x.nbytes))
                     f.h2d(bufs[-1], x)
-                args = [bufs[1], pk.shape[1], bufs[2], bufs[3], bufs[4]]
+                args = [bufs[0], pk.shape[1], bufs[1], bufs[2], bufs[3]]
             _check(self._lib.omk_tt_traverse(self._h, batch._h, C.c_void_p(args[0]), C.c_int32(int(args[1])),
                                              C.c_void_p(args[2]), C.c_void_p(args[3]), C.c_void_p(args[4]),
-                                             C.c_void_p(bufs[0]), _ptr(counts, i32p)))
-            f.d2h(hits, bufs[0])
+                                             C.c_void_p(self._hits), _ptr(counts, i32p)))
+            f.d2h(hits, self._hits)
         finally:
             for d in bufs:
                 f.dev_free(d)

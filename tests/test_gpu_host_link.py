@@ -92,3 +92,28 @@ def test_expansion_after_a_read_and_without(moves):
         assert (st["N"] == ref.N).all() and st["P"].tobytes() == ref.P.tobytes() and (st["VL"] == ref.VL).all()
         assert (sx["child_begin"] == ref.child_begin).all() and (sx["child_count"] == ref.child_count).all()
         assert (sx["action"] == ref.action).all()
+
+
+# one block serves a root: up to 1024 slots, ranks from the ballots of 16 wavefronts
+@pytest.mark.parametrize("slots,mask_frac", [(1, 0.0), (64, 0.0), (65, 0.4), (1024, 0.0), (1024, 0.5)])
+def test_root_queries_at_every_width(slots, mask_frac):
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(slots, n_expand=1, fanout=(slots, slots), max_depth=1, mask_frac=mask_frac, n_max=90)
+    ids = np.arange(1, slots + 1)
+    legal = ids if not mask_frac else ids[((soa["legal"][ids >> 5] >> (ids & 31).astype(np.uint32)) & 1) == 1]
+    f = omk.Forest.from_soa(soa)
+    gamma = np.random.default_rng(slots).gamma(0.3, 1.0, len(legal)).astype(np.float32)
+    with pytest.raises(omk.OmkError):
+        f.add_root_noise(0, np.append(gamma, gamma[:1]), 0.25)
+    assert f.download()["P"].tobytes() == soa["P"].tobytes()
+    f.add_root_noise(0, gamma, 0.25)
+    total = np.float32(0.0)
+    for g in gamma:
+        total = np.float32(total + g)
+    want = soa["P"].copy()
+    want[legal] = np.float32(0.75) * want[legal] + np.float32(0.25) * (gamma / total)
+    assert f.download()["P"].tobytes() == want.tobytes()
+    probs, n = f.action_probabilities(0, 0.0, slots)
+    best = legal[np.argmax(soa["N"][legal])]
+    assert n == len(legal) and np.flatnonzero(probs).tolist() == [soa["action"][best]]
+    assert f.reroot_child(0, int(soa["action"][legal[-1]])) == legal[-1] and f.reroot_child(0, slots) == -1
