@@ -215,7 +215,7 @@ static hipError_t dalloc(T **p, int64_t count) {
 // Staging is handed out front to back; once a call has seen its flag everything enqueued before has run, and
 // the next one starts at the front again.
 constexpr size_t kLinkHead = 4096;         // flag word, and behind it (64 bytes on) the results of small calls
-constexpr size_t kLinkStaging = 256 << 10; // staging a forest starts with
+constexpr size_t kLinkStaging = 4 << 20;   // staging a forest starts with (30 us to allocate, like 4 KiB)
 static hipError_t link_alloc(omk_forest *f, size_t staging) {
     char *p = nullptr;
     hipError_t e = hipHostMalloc((void **)&p, kLinkHead + staging, hipHostMallocDefault);
@@ -246,22 +246,105 @@ static HostSignal link_signal(omk_forest *f) {
     return HostSignal{f->link_count, (int32_t *)f->link, f->link_seq};
 }
 
-// Waits for the kernel that carries the last link_signal.  A wait of more than about a millisecond goes to the
-// runtime, which does not burn the core and reports an error of the stream.
-static int link_wait(omk_forest *f) {
+// Waits for the kernel that carries the link_signal of number `seq`.  A wait of more than about a millisecond goes
+// to the runtime, which does not burn the core and reports an error of the stream.
+static int link_wait_for(omk_forest *f, int32_t seq) {
     const int32_t *flag = (const int32_t *)f->link;
+    auto reached = [&] { return (int32_t)((uint32_t)__atomic_load_n(flag, __ATOMIC_ACQUIRE) - (uint32_t)seq) >= 0; };
     for (int i = 0; i < 20000; i++) {
-        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == f->link_seq) {
-            f->link_used = 0;
-            return OMK_OK;
-        }
+        if (reached()) return OMK_OK;
 #if defined(__x86_64__)
         __builtin_ia32_pause();
 #endif
     }
     HIP_TRY(hipStreamSynchronize(f->stream));
-    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != f->link_seq)
-        return fail(OMK_ERR_HIP, "the kernel that was waited for did not report");
+    if (!reached()) return fail(OMK_ERR_HIP, "the kernel that was waited for did not report");
+    return OMK_OK;
+}
+
+// Waits for the last one: everything enqueued has run, and staging starts at the front again.
+static int link_wait(omk_forest *f) {
+    if (int rc = link_wait_for(f, f->link_seq)) return rc;
+    f->link_used = 0;
+    return OMK_OK;
+}
+
+// Bulk transfers (omk_link.hip): arrays of the host, one per segment, to or from the device.  What fits in the
+// staging goes in one piece; more is cut into pieces of kBulkWords, kBulkSlots of them on their way at a time, so
+// that the host's copy of one piece runs beside the link's transfer of the next.
+struct Bulk {
+    Segments g = {};
+    char *host[kMaxSegments] = {};
+    Bulk() { g.start[0] = 0; }
+    void add(void *dev, int step, const void *h, int64_t words) {
+        if (!h || words <= 0) return;
+        g.dev[g.n] = (uint32_t *)dev;
+        g.step[g.n] = step;
+        host[g.n] = (char *)const_cast<void *>(h);
+        g.n++;
+        g.start[g.n] = g.start[g.n - 1] + words;
+    }
+    int64_t words() const { return g.start[g.n]; }
+    // the host's side of words [first, first + count)
+    template <class F>
+    void each(int64_t first, int64_t count, F &&f) const {
+        for (int q = 0; q < g.n; q++) {
+            const int64_t lo = std::max(first, g.start[q]), hi = std::min(first + count, g.start[q + 1]);
+            if (lo < hi) f(host[q] + (lo - g.start[q]) * 4, (lo - first) * 4, (size_t)(hi - lo) * 4);
+        }
+    }
+};
+constexpr int64_t kBulkWords = 1 << 18;
+constexpr int kBulkSlots = 4;
+static_assert(kBulkWords * kBulkSlots * 4 <= (int64_t)kLinkStaging, "the slots are the staging");
+
+static int bulk_put(omk_forest *f, const Bulk &b) {
+    const int64_t words = b.words();
+    const bool whole = words <= kBulkWords * kBulkSlots;
+    void *staged = nullptr;
+    if (int rc = link_stage(f, (size_t)(whole ? words : kBulkWords * kBulkSlots) * 4, &staged)) return rc;
+    char *at = (char *)staged;
+    if (whole) {
+        b.each(0, words, [&](char *h, int64_t off, size_t n) { memcpy(at + off, h, n); });
+        HIP_TRY(launch_put(b.g, (const uint32_t *)at, 0, words, HostSignal{nullptr, nullptr, 0}, f->stream));
+        return OMK_OK;
+    }
+    int32_t seq[kBulkSlots] = {};
+    for (int64_t c = 0; c * kBulkWords < words; c++) {
+        const int slot = (int)(c % kBulkSlots);
+        char *p = at + (size_t)slot * kBulkWords * 4;
+        const int64_t first = c * kBulkWords, n = std::min(kBulkWords, words - first);
+        if (c >= kBulkSlots)
+            if (int rc = link_wait_for(f, seq[slot])) return rc;
+        b.each(first, n, [&](char *h, int64_t off, size_t bytes) { memcpy(p + off, h, bytes); });
+        const HostSignal sig = link_signal(f);
+        seq[slot] = sig.seq;
+        HIP_TRY(launch_put(b.g, (const uint32_t *)p, first, n, sig, f->stream));
+    }
+    return link_wait(f);
+}
+
+static int bulk_get(omk_forest *f, const Bulk &b) {
+    const int64_t words = b.words(), pieces = (words + kBulkWords - 1) / kBulkWords;
+    if (pieces == 0) return OMK_OK;
+    void *staged = nullptr;
+    if (int rc = link_stage(f, (size_t)std::min<int64_t>(words, kBulkWords * kBulkSlots) * 4, &staged)) return rc;
+    char *at = (char *)staged;
+    int32_t seq[kBulkSlots] = {};
+    auto ask = [&](int64_t c) {
+        const HostSignal sig = link_signal(f);
+        seq[c % kBulkSlots] = sig.seq;
+        return launch_get(b.g, (uint32_t *)(at + (size_t)(c % kBulkSlots) * kBulkWords * 4), c * kBulkWords,
+                          std::min(kBulkWords, words - c * kBulkWords), sig, f->stream);
+    };
+    for (int64_t c = 0; c < std::min<int64_t>(pieces, kBulkSlots); c++) HIP_TRY(ask(c));
+    for (int64_t c = 0; c < pieces; c++) {
+        if (int rc = link_wait_for(f, seq[c % kBulkSlots])) return rc;
+        const char *p = at + (size_t)(c % kBulkSlots) * kBulkWords * 4;
+        b.each(c * kBulkWords, std::min(kBulkWords, words - c * kBulkWords),
+               [&](char *h, int64_t off, size_t bytes) { memcpy(h, p + off, bytes); });
+        if (c + kBulkSlots < pieces) HIP_TRY(ask(c + kBulkSlots));
+    }
     f->link_used = 0;
     return OMK_OK;
 }
@@ -397,11 +480,8 @@ int omk_sync(omk_forest *f) {
 // correct when every node is the child of at most one parent, so it is checked here, on
 // the host, before anything reaches the device (it also keeps every child range in
 // bounds, which is what protects the kernels from wild reads).
-static int validate(const omk_soa_view *v, int64_t n, int *max_fanout, bool *prior_sorted, uint64_t *structure_sum) {
+static int find_fault(const omk_soa_view *v, int64_t n) {
     std::vector<uint8_t> is_child((size_t)n, 0);
-    int mf = 0;
-    bool sorted = true;
-    uint64_t h = 0xCBF29CE484222325ull ^ (uint64_t)n;  // checksum of (node, child range) of every expanded node
     for (int64_t i = 0; i < n; i++) {
         int32_t cc = v->child_count[i];
         if (cc == 0) continue;
@@ -417,13 +497,51 @@ static int validate(const omk_soa_view *v, int64_t n, int *max_fanout, bool *pri
             if (c == i) return fail(OMK_ERR_STRUCTURE, "node %lld is its own child", (long long)i);
             if (is_child[(size_t)c]) return fail(OMK_ERR_STRUCTURE, "node %d has two parents", c);
             is_child[(size_t)c] = 1;
-            if (sorted && c > cb && !(v->P[c - 1] >= v->P[c])) sorted = false;
         }
+    }
+    return OMK_OK;
+}
+
+// Marks the bits [at, at + count) of `bits`; false when one was marked before.
+static bool mark_range(uint64_t *bits, int64_t at, int32_t count) {
+    uint64_t met = 0;
+    for (int64_t w = at >> 6, end = (at + count + 63) >> 6; w < end; w++) {
+        uint64_t m = ~0ull;
+        if (w == at >> 6) m &= ~0ull << (at & 63);
+        if (w == (at + count - 1) >> 6) m &= ~0ull >> (63 - ((at + count - 1) & 63));
+        met |= bits[w] & m;
+        bits[w] |= m;
+    }
+    return met == 0;
+}
+
+// The same test in one pass over the child counts, eight at a time (most nodes are leaves), and a bit per node for
+// "is somebody's child"; a structure that fails it goes through find_fault for the message.  On the way: the widest
+// fan-out, whether every node's children are stored by descending prior, and a checksum of the structure.
+static int validate(const omk_soa_view *v, int64_t n, int *max_fanout, bool *prior_sorted, uint64_t *structure_sum) {
+    std::vector<uint64_t> is_child((size_t)(n + 63) / 64, 0);
+    int mf = 0;
+    bool sorted = v->legal == nullptr;
+    uint64_t h = 0xCBF29CE484222325ull ^ (uint64_t)n;  // of (node, child range) of every expanded node
+    const int32_t *count = v->child_count;
+    for (int64_t i = 0; i < n; i++) {
+        while (i + 8 <= n && !(count[i] | count[i + 1] | count[i + 2] | count[i + 3] | count[i + 4] | count[i + 5] |
+                               count[i + 6] | count[i + 7]))
+            i += 8;
+        if (i >= n) break;
+        const int32_t cc = count[i];
+        if (cc == 0) continue;
+        const int32_t cb = v->child_begin[i];
+        if (cc < 0 || cc > OMK_MAX_FANOUT || cb < 0 || (int64_t)cb + cc > n || (i >= cb && i < (int64_t)cb + cc) ||
+            !mark_range(is_child.data(), cb, cc))
+            return find_fault(v, n);
+        if (sorted)
+            for (int32_t c = cb + 1; c < cb + cc && sorted; c++) sorted = v->P[c - 1] >= v->P[c];
         mf = std::max(mf, (int)cc);
         h = (h ^ ((uint64_t)i * 0x9E3779B97F4A7C15ull + ((uint64_t)(uint32_t)cb << 32) + (uint32_t)cc)) * 0x100000001B3ull;
     }
     *max_fanout = mf;
-    *prior_sorted = sorted && v->legal == nullptr;
+    *prior_sorted = sorted;
     *structure_sum = h;
     return OMK_OK;
 }
@@ -444,36 +562,31 @@ int omk_forest_upload(omk_forest *f, const omk_soa_view *v) {
     if (int rc = validate(v, n, &mf, &sorted, &ssum)) return rc;
     if (int rc = use_device(f)) return rc;
 
-    std::vector<int2> span((size_t)n);
-    for (int64_t i = 0; i < n; i++) {
-        span[(size_t)i].x = v->child_begin[i];
-        span[(size_t)i].y = v->child_count[i];
-    }
     hipStream_t s = f->stream;
-    HIP_TRY(hipStreamSynchronize(s));
-    HIP_TRY(hipMemcpy(f->span, span.data(), (size_t)n * sizeof(int2), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(f->N, v->N, (size_t)n * 4, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(f->W, v->W, (size_t)n * 4, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(f->P, v->P, (size_t)n * 4, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(f->VL, v->VL, (size_t)n * 4, hipMemcpyHostToDevice));
-    if (f->has_rave) {
-        HIP_TRY(hipMemcpy(f->rN, v->rN, (size_t)n * 4, hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(f->rW, v->rW, (size_t)n * 4, hipMemcpyHostToDevice));
-    }
     f->has_action = v->action != nullptr;
-    if (f->has_action) {
-        if (!f->action) HIP_TRY(dalloc(&f->action, f->capacity));
-        HIP_TRY(hipMemcpy(f->action, v->action, (size_t)n * 4, hipMemcpyHostToDevice));
-    }
+    if (f->has_action && !f->action) HIP_TRY(dalloc(&f->action, f->capacity));
     f->has_legal = v->legal != nullptr;
-    if (f->has_legal) {
-        if (!f->legal) HIP_TRY(dalloc(&f->legal, (f->capacity + 31) / 32));
-        HIP_TRY(hipMemcpy(f->legal, v->legal, (size_t)((n + 31) / 32) * 4, hipMemcpyHostToDevice));
-    }
+    if (f->has_legal && !f->legal) HIP_TRY(dalloc(&f->legal, (f->capacity + 31) / 32));
     f->has_hash = v->hash != nullptr;
-    if (f->has_hash) {
-        if (!f->hash) HIP_TRY(dalloc(&f->hash, f->capacity));
-        HIP_TRY(hipMemcpy(f->hash, v->hash, (size_t)n * 8, hipMemcpyHostToDevice));
+    if (f->has_hash && !f->hash) HIP_TRY(dalloc(&f->hash, f->capacity));
+    Bulk up;
+    up.add(f->span, 2, v->child_begin, n);
+    up.add((int32_t *)f->span + 1, 2, v->child_count, n);
+    up.add(f->N, 1, v->N, n);
+    up.add(f->W, 1, v->W, n);
+    up.add(f->P, 1, v->P, n);
+    up.add(f->VL, 1, v->VL, n);
+    if (f->has_rave) {
+        up.add(f->rN, 1, v->rN, n);
+        up.add(f->rW, 1, v->rW, n);
+    }
+    if (f->has_action) up.add(f->action, 1, v->action, n);
+    if (int rc = bulk_put(f, up)) return rc;
+    if (f->has_legal || f->has_hash) {
+        Bulk more;
+        if (f->has_legal) more.add(f->legal, 1, v->legal, (n + 31) / 32);
+        if (f->has_hash) more.add(f->hash, 1, v->hash, 2 * n);
+        if (int rc = bulk_put(f, more)) return rc;
     }
     f->changes++;
     // the same structure again (statistics put back): node ids keep their meaning
@@ -505,15 +618,17 @@ int omk_forest_download(omk_forest *f, omk_soa_view *v) {
         return fail(OMK_ERR_INVALID, "omk_forest_download: view has %lld nodes, forest %lld", (long long)v->n_nodes,
                     (long long)f->n_nodes);
     if (int rc = use_device(f)) return rc;
-    HIP_TRY(hipStreamSynchronize(f->stream));
-    const size_t b = (size_t)f->n_nodes * 4;
-    if (v->N) HIP_TRY(hipMemcpy(v->N, f->N, b, hipMemcpyDeviceToHost));
-    if (v->W) HIP_TRY(hipMemcpy(v->W, f->W, b, hipMemcpyDeviceToHost));
-    if (v->P) HIP_TRY(hipMemcpy(v->P, f->P, b, hipMemcpyDeviceToHost));
-    if (v->VL) HIP_TRY(hipMemcpy(v->VL, f->VL, b, hipMemcpyDeviceToHost));
-    if (f->has_rave && v->rN) HIP_TRY(hipMemcpy(v->rN, f->rN, b, hipMemcpyDeviceToHost));
-    if (f->has_rave && v->rW) HIP_TRY(hipMemcpy(v->rW, f->rW, b, hipMemcpyDeviceToHost));
-    return OMK_OK;
+    const int64_t n = f->n_nodes;
+    Bulk down;
+    down.add(f->N, 1, v->N, n);
+    down.add(f->W, 1, v->W, n);
+    down.add(f->P, 1, v->P, n);
+    down.add(f->VL, 1, v->VL, n);
+    if (f->has_rave) {
+        down.add(f->rN, 1, v->rN, n);
+        down.add(f->rW, 1, v->rW, n);
+    }
+    return bulk_get(f, down);
 }
 
 static inline bool view_legal(const omk_soa_view *v, int64_t i) {
@@ -589,22 +704,13 @@ int omk_forest_download_structure(omk_forest *f, int64_t n_nodes, int32_t *h_chi
         return fail(OMK_ERR_INVALID, "omk_forest_download_structure: room for %lld nodes, forest has %lld",
                     (long long)n_nodes, (long long)f->n_nodes);
     if (int rc = use_device(f)) return rc;
-    HIP_TRY(hipStreamSynchronize(f->stream));
-    if (h_action) {
-        if (f->has_action) {
-            HIP_TRY(hipMemcpy(h_action, f->action, (size_t)n_nodes * 4, hipMemcpyDeviceToHost));
-        } else {
-            for (int64_t i = 0; i < n_nodes; i++) h_action[i] = (int32_t)i;
-        }
-    }
-    if (h_child_begin || h_child_count) {
-        std::vector<int2> sp((size_t)n_nodes);
-        HIP_TRY(hipMemcpy(sp.data(), f->span, (size_t)n_nodes * sizeof(int2), hipMemcpyDeviceToHost));
-        for (int64_t i = 0; i < n_nodes; i++) {
-            if (h_child_begin) h_child_begin[i] = sp[(size_t)i].x;
-            if (h_child_count) h_child_count[i] = sp[(size_t)i].y;
-        }
-    }
+    Bulk down;
+    down.add(f->span, 2, h_child_begin, n_nodes);
+    down.add((int32_t *)f->span + 1, 2, h_child_count, n_nodes);
+    if (f->has_action) down.add(f->action, 1, h_action, n_nodes);
+    if (int rc = bulk_get(f, down)) return rc;
+    if (h_action && !f->has_action)
+        for (int64_t i = 0; i < n_nodes; i++) h_action[i] = (int32_t)i;
     return OMK_OK;
 }
 

@@ -140,6 +140,21 @@ struct HostSignal {
     int32_t *flag;
     int32_t seq;
 };
+// Arrays of 32-bit words on the device, read as one stream (omk_link.hip): word start[q] + i of the stream is word
+// i * step[q] of dev[q].
+constexpr int kMaxSegments = 10;
+struct Segments {
+    int n;
+    int step[kMaxSegments];
+    uint32_t *dev[kMaxSegments];
+    int64_t start[kMaxSegments + 1];
+};
+// Words [first, first + count) of the stream from / to pinned memory.  (put: sig.flag may be null.)
+hipError_t launch_put(const Segments &g, const uint32_t *staged, int64_t first, int64_t count, const HostSignal &sig,
+                      hipStream_t s);
+hipError_t launch_get(const Segments &g, uint32_t *staged, int64_t first, int64_t count, const HostSignal &sig,
+                      hipStream_t s);
+
 // Where the leaf gather of a batch goes (pinned host memory that the kernel writes itself; any of the first two
 // may be null): row-major paths [n][max_depth+1] and actions [n][max_depth], -1 padded; per traversal the path
 // length, the leaf, and the leaf's child and visit count; the four abort words of the selection.

@@ -92,6 +92,8 @@ def load_library():
     for name in EXPORTS:
         if name != "omk_last_error":
             getattr(L, name).restype = C.c_int
+    for name, types in _EVERY_BATCH.items():
+        getattr(L, name).argtypes = types
     L.omk_soa_count_legal.restype = C.c_int64
     _LIB = L
     return L
@@ -104,6 +106,31 @@ def _check(rc):
 
 def _ptr(a, ty):
     return a.ctypes.data_as(ty) if a is not None else ty()
+
+
+def _at(a):
+    """Address of an array for an argument declared c_void_p: a tenth of what a typed pointer object costs, which
+    is what the calls of every batch use."""
+    return a.__array_interface__["data"][0]
+
+
+# The entry points a search calls every batch, with their argument types declared once.
+_VP, _I32, _I64, _F32 = C.c_void_p, C.c_int32, C.c_int64, C.c_float
+_EVERY_BATCH = {
+    "omk_batch_set_roots": (_VP, _VP, _I32), "omk_batch_set_values": (_VP, _VP, _I32), "omk_select_batch": (_VP, _VP),
+    "omk_backup_batch": (_VP, _I32), "omk_revert_vl": (_VP, _I32), "omk_backup_rave_batch": (_VP,),
+    "omk_batch_read": (_VP, _VP, _VP, _VP, _VP), "omk_expand_batch_ex": (_VP, _VP, _VP, _VP, _VP, _VP, _VP),
+    "omk_forest_set_keys": (_VP, _VP, _VP, _I64), "omk_forest_action_probabilities": (_VP, _I32, _F32, _I32, _VP, _VP),
+    "omk_forest_add_root_noise": (_VP, _I32, _VP, _I32, _F32), "omk_forest_node_count": (_VP, _VP, _VP),
+    "omk_tt_probe_leaves": (_VP, _VP, _I32, _VP),
+}
+
+
+def _together(n, **dtypes):
+    """Arrays of n 32-bit elements each, side by side in one block: one allocation that the C library keeps at hand
+    when it is freed, where several of a few megabytes each are given back and faulted in again every time."""
+    block = np.empty((len(dtypes), n), np.int32)
+    return {k: row.view(t) for (k, t), row in zip(dtypes.items(), block)}
 
 
 def _arr(x, dtype):
@@ -214,8 +241,8 @@ class Forest:
         """(nodes now, capacity): the forest grows with Batch.expand()."""
         n, cap = C.c_int64(), C.c_int64()
         _check(self._lib.omk_forest_node_count(self._h, C.byref(n), C.byref(cap)))
-        self.n_nodes = int(n.value)
-        return int(n.value), int(cap.value)
+        self.n_nodes = n.value
+        return n.value, cap.value
 
     def reroot_child(self, root, last_action):
         """searchWithTreeReuse: the first child of root reached by last_action, or -1."""
@@ -239,23 +266,21 @@ class Forest:
         """MCTSEngine::getActionProbabilities from the root's children; (probabilities, children)."""
         out = np.empty(int(action_space), np.float32)
         n = C.c_int32()
-        _check(self._lib.omk_forest_action_probabilities(self._h, C.c_int32(int(root)), C.c_float(temperature),
-                                                         C.c_int32(int(action_space)), _ptr(out, f32p), C.byref(n)))
-        return out, int(n.value)
+        _check(self._lib.omk_forest_action_probabilities(self._h, int(root), temperature, int(action_space), _at(out),
+                                                         C.byref(n)))
+        return out, n.value
 
     def add_root_noise(self, root, gamma, epsilon):
         """MCTSEngine::addDirichletNoise: one caller-drawn gamma(alpha, 1) sample per child of `root`."""
         gamma = np.ascontiguousarray(gamma, dtype=np.float32)
-        _check(self._lib.omk_forest_add_root_noise(self._h, C.c_int32(int(root)), _ptr(gamma, f32p),
-                                                   C.c_int32(len(gamma)), C.c_float(epsilon)))
+        _check(self._lib.omk_forest_add_root_noise(self._h, int(root), _at(gamma), len(gamma), epsilon))
 
     def set_keys(self, nodes, keys):
         """Position keys of single nodes (the game's own getHash() of the states they stand for)."""
         nodes = np.ascontiguousarray(nodes, dtype=np.int32)
         keys = np.ascontiguousarray(keys, dtype=np.uint64)
         assert len(nodes) == len(keys)
-        _check(self._lib.omk_forest_set_keys(self._h, _ptr(nodes, i32p), _ptr(keys, C.POINTER(C.c_uint64)),
-                                             C.c_int64(len(nodes))))
+        _check(self._lib.omk_forest_set_keys(self._h, _at(nodes), _at(keys), len(nodes)))
 
     def download_redirects(self):
         """Per child slot the node it holds instead of its own, or -1 (slots re-pointed by
@@ -268,7 +293,7 @@ class Forest:
     def download_structure(self):
         """Returns dict(child_begin, child_count, action) of the current nodes."""
         n, _ = self.node_count()
-        out = dict(child_begin=np.empty(n, np.int32), child_count=np.empty(n, np.int32), action=np.empty(n, np.int32))
+        out = _together(n, child_begin=np.int32, child_count=np.int32, action=np.int32)
         _check(self._lib.omk_forest_download_structure(self._h, C.c_int64(n), _ptr(out["child_begin"], i32p),
                                                        _ptr(out["child_count"], i32p), _ptr(out["action"], i32p)))
         return out
@@ -276,11 +301,8 @@ class Forest:
     def download(self):
         """Returns dict(N, W, P, VL[, rN, rW]) as numpy arrays."""
         n, _ = self.node_count()
-        out = dict(N=np.empty(n, np.int32), W=np.empty(n, np.float32), P=np.empty(n, np.float32),
-                   VL=np.empty(n, np.int32))
-        if self.has_rave:
-            out["rN"] = np.empty(n, np.int32)
-            out["rW"] = np.empty(n, np.float32)
+        rave = dict(rN=np.int32, rW=np.float32) if self.has_rave else {}
+        out = _together(n, N=np.int32, W=np.float32, P=np.float32, VL=np.int32, **rave)
         v = _SoaView(n, _ptr(out["N"], i32p), _ptr(out["W"], f32p), _ptr(out["P"], f32p), _ptr(out["VL"], i32p),
                      _ptr(out.get("rN"), i32p), _ptr(out.get("rW"), f32p), i32p(), i32p(), i32p(), u32p(), u64p())
         _check(self._lib.omk_forest_download(self._h, C.byref(v)))
@@ -345,12 +367,12 @@ class Batch:
 
     def set_roots(self, roots):
         roots = np.ascontiguousarray(roots, dtype=np.int32)
-        _check(self._lib.omk_batch_set_roots(self._h, _ptr(roots, i32p), len(roots)))
+        _check(self._lib.omk_batch_set_roots(self._h, _at(roots), len(roots)))
         self.n = len(roots)
 
     def set_values(self, values):
         values = np.ascontiguousarray(values, dtype=np.float32)
-        _check(self._lib.omk_batch_set_values(self._h, _ptr(values, f32p), len(values)))
+        _check(self._lib.omk_batch_set_values(self._h, _at(values), len(values)))
 
     def select(self, params):
         _check(self._lib.omk_select_batch(self._h, C.byref(params)))
@@ -372,8 +394,7 @@ class Batch:
         plen = np.empty(n, np.int32)
         leaf = np.empty(n, np.int32)
         actions = np.empty((n, D), np.int32)
-        _check(self._lib.omk_batch_read(self._h, _ptr(paths, i32p), _ptr(plen, i32p), _ptr(leaf, i32p),
-                                        _ptr(actions, i32p)))
+        _check(self._lib.omk_batch_read(self._h, _at(paths), _at(plen), _at(leaf), _at(actions)))
         return paths, plen, leaf, actions
 
     def leaf_keys_dev(self, d_piece_keys, cells, d_player_keys, d_root_keys, d_root_players, d_out):
@@ -433,8 +454,8 @@ class Batch:
         par = _ExpandParams(int(action_space), 0 if widening is None else 1,
                             0.0 if widening is None else float(widening[0]), 0.0 if widening is None else float(widening[1]))
         first = np.empty(len(mb) - 1, np.int32)
-        _check(self._lib.omk_expand_batch_ex(self._h, _ptr(mb, i32p), _ptr(mv, i32p), _ptr(pb, i32p), _ptr(pol, f32p),
-                                             C.byref(par), _ptr(first, i32p)))
+        _check(self._lib.omk_expand_batch_ex(self._h, _at(mb), _at(mv), None if pb is None else _at(pb),
+                                             None if pol is None else _at(pol), C.byref(par), _at(first)))
         self.forest.node_count()
         return first
 
@@ -525,7 +546,7 @@ class TranspositionTable:
         _check(self._lib.omk_tt_probe(self._h, C.c_void_p(d_keys), int(n), int(min_depth), C.c_void_p(d_out)))
 
     def probe_leaves_dev(self, batch, d_out, min_depth=0):
-        _check(self._lib.omk_tt_probe_leaves(self._h, batch._h, int(min_depth), C.c_void_p(d_out)))
+        _check(self._lib.omk_tt_probe_leaves(self._h, batch._h, int(min_depth), d_out))
 
     def insert(self, keys, nodes, depths=None):
         f = self.forest

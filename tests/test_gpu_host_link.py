@@ -117,3 +117,49 @@ def test_root_queries_at_every_width(slots, mask_frac):
     best = legal[np.argmax(soa["N"][legal])]
     assert n == len(legal) and np.flatnonzero(probs).tolist() == [soa["action"][best]]
     assert f.reroot_child(0, int(soa["action"][legal[-1]])) == legal[-1] and f.reroot_child(0, slots) == -1
+
+
+# arrays cross as one stream of words, in pieces of 2^18, four on their way at a time
+@pytest.mark.parametrize("n", [1, 37, 43690, 43691, 200_001])
+@pytest.mark.parametrize("rave", [False, True])
+def test_arrays_cross_in_pieces(n, rave):
+    import omoknuni_small_amd as omk
+    rng = np.random.default_rng(n)
+    fan = rng.integers(1, 9, n)
+    soa = dict(N=rng.integers(0, 999, n).astype(np.int32), W=rng.random(n).astype(np.float32),
+               P=rng.random(n).astype(np.float32), VL=rng.integers(0, 9, n).astype(np.int32),
+               child_begin=np.zeros(n, np.int32), child_count=np.zeros(n, np.int32),
+               action=rng.integers(0, 400, n).astype(np.int32), hash=rng.integers(0, 1 << 63, n).astype(np.uint64))
+    at, node = 1, 0
+    while at < n and node < at:
+        k = int(min(fan[node], n - at))
+        soa["child_begin"][node], soa["child_count"][node] = at, k
+        at, node = at + k, node + int(rng.integers(1, 3))
+    if rave:
+        soa.update(rN=rng.integers(0, 99, n).astype(np.int32), rW=rng.random(n).astype(np.float32))
+    f = omk.Forest.from_soa(soa, capacity=n + 5)
+    for scale in (1, 2):
+        soa["W"] = soa["W"] * np.float32(scale)
+        f.upload(soa)
+        got = dict(f.download(), **f.download_structure())
+        for k in got:
+            assert got[k].tobytes() == soa[k].tobytes(), k
+
+
+@pytest.mark.parametrize("fault,message", [("two parents", "two parents"), ("own child", "own child"), ("outside", "outside"),
+                                           ("negative", "< 0"), ("wide", "exceeds")])
+def test_structures_that_are_no_forest_are_refused(fault, message):
+    import omoknuni_small_amd as omk
+    n = 5000
+    soa = dict(N=np.ones(n, np.int32), W=np.zeros(n, np.float32), P=np.zeros(n, np.float32), VL=np.zeros(n, np.int32),
+               child_begin=np.zeros(n, np.int32), child_count=np.zeros(n, np.int32))
+    soa["child_begin"][[0, 70, 133]], soa["child_count"][[0, 70, 133]] = [1, 100, 1003], [64, 903, 1]
+    f = omk.Forest.from_soa(soa)
+    before = f.download_structure()
+    bad = dict(soa, child_begin=soa["child_begin"].copy(), child_count=soa["child_count"].copy())
+    bad["child_begin"][199], bad["child_count"][199] = {"two parents": (1002, 3), "own child": (199, 1), "outside": (n - 1, 2),
+                                                        "negative": (3, -1), "wide": (1100, 1025)}[fault]
+    with pytest.raises(omk.OmkError, match=message):
+        f.upload(bad)
+    after = f.download_structure()
+    assert all((before[k] == after[k]).all() for k in before)
