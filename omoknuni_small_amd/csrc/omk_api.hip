@@ -71,6 +71,8 @@ struct omk_forest {
     size_t link_used = 0;         // staging handed out since the stream was last known to be idle
     int32_t link_seq = 0;         // number of the last call that waited
     int32_t *link_count = nullptr;  // HostSignal::count
+    char *scratch = nullptr;  // work space of a compaction, kept for the next (kKeepScratch)
+    size_t scratch_bytes = 0;
     // counts the calls that change N or child ranges: what was read of them before is stale after
     int64_t changes = 0;
     int children = 0;       // live batches and tables created on this forest
@@ -430,7 +432,7 @@ int omk_forest_create(const omk_forest_desc *desc, omk_forest **out) {
 static void forest_free(omk_forest *f) {
     (void)hipSetDevice(f->device);
     if (f->own_stream) (void)hipStreamSynchronize(f->own_stream);
-    void *ptrs[] = {f->span, f->N, f->W, f->P, f->VL, f->rN, f->rW, f->Q2, f->action, f->legal, f->hash, f->alias, f->link_count};
+    void *ptrs[] = {f->span, f->N, f->W, f->P, f->VL, f->rN, f->rW, f->Q2, f->action, f->legal, f->hash, f->alias, f->link_count, f->scratch};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (f->link) (void)hipHostFree(f->link);
@@ -864,76 +866,76 @@ int omk_forest_reroot_child(omk_forest *f, int32_t root, int32_t last_action, in
     return OMK_OK;
 }
 
+}  // extern "C"
+
 // Device memory a compaction works in, beyond the forest's own arrays.
 struct CompactScratch {
-    int32_t *map = nullptr;    // [n] old id of every new node
-    int32_t *begin = nullptr;  // [n] new id of every new node's first child
-    int32_t *cc = nullptr;     // [n] child counts of the level at hand
-    int32_t *scan = nullptr;   // [n] their exclusive prefix
-    void *scan_tmp = nullptr;  // work space of the scan
-    size_t scan_bytes = 0;
-    uint64_t *tmp = nullptr;   // [n] the array every field passes through
-    uint32_t *legal = nullptr; // [(n + 31) / 32] the new legal mask
+    int32_t *map = nullptr;       // [n] old id of every new node
+    int32_t *begin = nullptr;     // [n] new id of every new node's first child
+    uint32_t *tmp = nullptr;      // the arrays pass through here, as many at a time as fit
+    int64_t tmp_words = 0;
+    int32_t *sums = nullptr;      // [kBfsSums]
+    BfsLevel *levels = nullptr;   // [kCompactLevels + 1]
 };
+constexpr int kBfsLevels = 12;        // levels enqueued before the host looks
+constexpr int kCompactLevels = 4104;  // more levels than a path has nodes are walked in turns of this many
+constexpr size_t kCompactFixed = 1024 + ((kCompactLevels + 1) * sizeof(BfsLevel) + 255) / 256 * 256;
 
 // The compaction itself, in scratch memory the caller provides (room for the forest's node count).
 static int compact_in(omk_forest *f, int32_t new_root, int64_t *h_nodes_after, int32_t *h_old_of_new,
                       const CompactScratch &sc) {
     hipStream_t s = f->stream;
     const int64_t n = f->n_nodes;
-    // breadth-first order of the subtree, on the device: map[new id] = old id, begin[new id]
-    // = new id of its first child.  One level per round; the levels' sizes come back to the
-    // host (a handful of bytes per level).
-    hipError_t e = hipMemcpyAsync(sc.map, &new_root, 4, hipMemcpyHostToDevice, s);
-    int64_t lo = 0, hi = 1;
-    bool not_a_tree = false;
-    while (e == hipSuccess && hi > lo) {
-        int64_t total = 0;
-        e = launch_bfs_level(f->span, sc.map, sc.begin, lo, hi - lo, n - hi, sc.cc, sc.scan, sc.scan_tmp,
-                             sc.scan_bytes, &total, s);
-        if (e == hipSuccess && total > n - hi) {
-            not_a_tree = true;
-            break;
+    HIP_TRY(launch_bfs_start(sc.map, sc.levels, new_root, s));
+    int64_t k = 1;
+    for (int level = 0;;) {
+        HIP_TRY(launch_bfs(f->span, sc.map, sc.begin, sc.levels, level, kBfsLevels, sc.sums, n, s));
+        level += kBfsLevels;
+        BfsLevel reached;
+        if (int rc = link_fetch(f, &reached, sc.levels + level, sizeof(BfsLevel) / 4)) return rc;
+        if (reached.cnt < 0)
+            return fail(OMK_ERR_STRUCTURE, "omk_forest_compact: the child ranges do not form a tree");
+        k = reached.lo;
+        if (reached.cnt == 0) break;
+        if (level + kBfsLevels > kCompactLevels) {  // go on from the front of the table
+            HIP_TRY(launch_copy_words(sc.levels, sc.levels + level, sizeof(BfsLevel) / 4, s));
+            level = 0;
         }
-        lo = hi;
-        hi += total;
     }
-    if (e != hipSuccess || not_a_tree) {
-        (void)hipStreamSynchronize(s);
-        if (not_a_tree) return fail(OMK_ERR_STRUCTURE, "omk_forest_compact: the child ranges do not form a tree");
-        return fail(OMK_ERR_HIP, "omk_forest_compact: %s", hipGetErrorString(e));
-    }
-    const int64_t k = hi;
-    auto move_words = [&](void *arr) {
-        if (e != hipSuccess || !arr) return;
-        e = launch_gather_words((uint32_t *)sc.tmp, (const uint32_t *)arr, sc.map, k, s);
-        if (e == hipSuccess) e = launch_copy_words(arr, sc.tmp, k, s);
+    struct {
+        void *array;
+        int kind;
+    } fields[] = {{f->N, 1}, {f->W, 1}, {f->P, 1}, {f->VL, 1}, {f->has_rave ? f->rN : nullptr, 1},
+                  {f->has_rave ? f->rW : nullptr, 1},
+                  {f->has_rave ? f->Q2 : nullptr, 1},  // the nodes keep their statistics, hence their RAVE blend
+                  {f->has_action ? f->action : nullptr, 1}, {f->has_hash ? f->hash : nullptr, 2}, {f->span, 3}};
+    CompactFields g = {};
+    int64_t used = 0;
+    // (a 64-bit array starts at an even word of tmp: after an odd number of arrays of an odd count, in a pass of its own)
+    auto move = [&]() -> int {
+        if (g.n) HIP_TRY(launch_compact(g, sc.tmp, sc.map, sc.begin, k, s));
+        g.n = 0;
+        used = 0;
+        return OMK_OK;
     };
-    move_words(f->N);
-    move_words(f->W);
-    move_words(f->P);
-    move_words(f->VL);
-    if (f->has_rave) {
-        move_words(f->rN);
-        move_words(f->rW);
-        move_words(f->Q2);  // the nodes keep their statistics, hence their RAVE blend
+    for (const auto &fd : fields) {
+        if (!fd.array) continue;
+        if (used + compact_words(fd.kind, k) > sc.tmp_words || (fd.kind != 1 && (used & 1)))
+            if (int rc = move()) return rc;
+        g.array[g.n] = (uint32_t *)fd.array;
+        g.kind[g.n++] = fd.kind;
+        used += compact_words(fd.kind, k);
     }
-    if (f->has_action) move_words(f->action);
-    if (e == hipSuccess && f->has_hash) {
-        e = launch_gather_dwords(sc.tmp, f->hash, sc.map, k, s);
-        if (e == hipSuccess) e = launch_copy_words(f->hash, sc.tmp, k * 2, s);
+    if (int rc = move()) return rc;
+    if (f->has_legal) {
+        HIP_TRY(launch_gather_legal(sc.tmp, f->legal, sc.map, k, s));
+        HIP_TRY(launch_copy_words(f->legal, sc.tmp, (k + 31) / 32, s));
     }
-    if (e == hipSuccess) {
-        e = launch_gather_span((int2 *)sc.tmp, f->span, sc.map, sc.begin, k, s);
-        if (e == hipSuccess) e = launch_copy_words(f->span, sc.tmp, k * 2, s);
+    if (h_old_of_new) {
+        Bulk down;
+        down.add(sc.map, 1, h_old_of_new, k);
+        if (int rc = bulk_get(f, down)) return rc;
     }
-    if (e == hipSuccess && f->has_legal) {
-        e = launch_gather_legal(sc.legal, f->legal, sc.map, k, s);
-        if (e == hipSuccess) e = launch_copy_words(f->legal, sc.legal, (k + 31) / 32, s);
-    }
-    if (e == hipSuccess && h_old_of_new) e = hipMemcpyAsync(h_old_of_new, sc.map, (size_t)k * 4, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return fail(OMK_ERR_HIP, "omk_forest_compact: %s", hipGetErrorString(e));
     f->n_nodes = k;
     f->changes++;
     f->generation++;
@@ -942,29 +944,46 @@ static int compact_in(omk_forest *f, int32_t new_root, int64_t *h_nodes_after, i
     return OMK_OK;
 }
 
+// Scratch of up to this much stays with the forest from one move to the next (a tree of a million nodes); more is
+// given back after the call.
+constexpr size_t kKeepScratch = 64 << 20;
+
+extern "C" {
+
 int omk_forest_compact(omk_forest *f, int32_t new_root, int64_t *h_nodes_after, int32_t *h_old_of_new) {
     if (!f) return fail(OMK_ERR_INVALID, "omk_forest_compact: null forest");
     if (!f->uploaded) return fail(OMK_ERR_STATE, "omk_forest_compact: nothing uploaded");
     if (new_root < 0 || new_root >= f->n_nodes) return fail(OMK_ERR_INVALID, "omk_forest_compact: root %d", new_root);
     if (int rc = tree_only("omk_forest_compact", f)) return rc;
     if (int rc = use_device(f)) return rc;
-    HIP_TRY(hipStreamSynchronize(f->stream));
     const int64_t n = f->n_nodes;
+    // every array at once: eight of 32-bit words and two of 64-bit ones
     CompactScratch sc;
-    hipError_t e = bfs_scan_bytes(n, &sc.scan_bytes);
-    if (e == hipSuccess) e = hipMalloc((void **)&sc.map, (size_t)n * 4);
-    if (e == hipSuccess) e = hipMalloc((void **)&sc.begin, (size_t)n * 4);
-    if (e == hipSuccess) e = hipMalloc((void **)&sc.cc, (size_t)n * 4);
-    if (e == hipSuccess) e = hipMalloc((void **)&sc.scan, (size_t)n * 4);
-    if (e == hipSuccess) e = hipMalloc(&sc.scan_tmp, sc.scan_bytes > 0 ? sc.scan_bytes : 4);
-    if (e == hipSuccess) e = hipMalloc((void **)&sc.tmp, (size_t)n * 8);
-    if (e == hipSuccess && f->has_legal) e = hipMalloc((void **)&sc.legal, (size_t)((n + 31) / 32) * 4);
-    int rc = e == hipSuccess ? compact_in(f, new_root, h_nodes_after, h_old_of_new, sc)
-                             : fail(OMK_ERR_HIP, "omk_forest_compact: %s", hipGetErrorString(e));
-    (void)hipStreamSynchronize(f->stream);
-    for (void *p : {(void *)sc.map, (void *)sc.begin, (void *)sc.cc, (void *)sc.scan, (void *)sc.legal, (void *)sc.tmp,
-                    sc.scan_tmp})
-        if (p) (void)hipFree(p);
+    sc.tmp_words = 12 * n;
+    const size_t words = ((size_t)n + 63) / 64 * 64;
+    const size_t bytes = kCompactFixed + words * 8 + (size_t)sc.tmp_words * 4;
+    if (bytes > f->scratch_bytes) {
+        if (f->scratch) {
+            HIP_TRY(hipStreamSynchronize(f->stream));
+            HIP_TRY(hipFree(f->scratch));
+        }
+        f->scratch = nullptr;
+        f->scratch_bytes = 0;
+        HIP_TRY(hipMalloc((void **)&f->scratch, bytes));
+        f->scratch_bytes = bytes;
+    }
+    sc.sums = (int32_t *)f->scratch;
+    sc.levels = (BfsLevel *)(f->scratch + 1024);
+    sc.map = (int32_t *)(f->scratch + kCompactFixed);
+    sc.begin = sc.map + words;
+    sc.tmp = (uint32_t *)(sc.begin + words);
+    const int rc = compact_in(f, new_root, h_nodes_after, h_old_of_new, sc);
+    if (rc != OMK_OK || f->scratch_bytes > kKeepScratch) {
+        (void)hipStreamSynchronize(f->stream);
+        (void)hipFree(f->scratch);
+        f->scratch = nullptr;
+        f->scratch_bytes = 0;
+    }
     return rc;
 }
 
@@ -975,17 +994,13 @@ int omk_forest_compact(omk_forest *f, int32_t new_root, int64_t *h_nodes_after, 
 // process.  In host code the array's name is only a handle for hipGetSymbolAddress; the address the
 // kernels get is looked up once per device (static_scratch) and kept.
 constexpr int64_t kStaticCompactNodes = 1ll << 20;
-constexpr size_t kStaticScanBytes = 1u << 20;  // work space of the level scan (a few KiB are used)
 constexpr size_t kStaticWords = (size_t)kStaticCompactNodes * 4;
-constexpr size_t kStaticOffMap = 0;
+constexpr size_t kStaticOffMap = kCompactFixed;
 constexpr size_t kStaticOffBegin = kStaticOffMap + kStaticWords;
-constexpr size_t kStaticOffCc = kStaticOffBegin + kStaticWords;
-constexpr size_t kStaticOffScan = kStaticOffCc + kStaticWords;
-constexpr size_t kStaticOffTmp = kStaticOffScan + kStaticWords;
-constexpr size_t kStaticOffLegal = kStaticOffTmp + 2 * kStaticWords;
-constexpr size_t kStaticOffScanTmp = kStaticOffLegal + kStaticWords / 32;
-constexpr size_t kStaticScratchBytes = kStaticOffScanTmp + kStaticScanBytes;
-static_assert(kStaticOffScanTmp % 256 == 0 && kStaticOffLegal % 256 == 0, "parts of the scratch keep its alignment");
+constexpr size_t kStaticOffTmp = kStaticOffBegin + kStaticWords;
+constexpr size_t kStaticTmpWords = 4 * (size_t)kStaticCompactNodes;  // four arrays of 32-bit words at a time
+constexpr size_t kStaticScratchBytes = kStaticOffTmp + kStaticTmpWords * 4;
+static_assert(kStaticOffMap % 256 == 0, "parts of the scratch keep its alignment");
 
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
@@ -1022,24 +1037,19 @@ int omk_forest_compact_static(omk_forest *f, int32_t new_root, int64_t *h_nodes_
     if (int rc = use_device(f)) return rc;
     unsigned char *base = nullptr;
     if (int rc = static_scratch(f->device, &base)) return rc;
-    HIP_TRY(hipStreamSynchronize(f->stream));
     CompactScratch sc;
-    size_t need = 0;
-    HIP_TRY(bfs_scan_bytes(f->n_nodes, &need));
-    if (need > kStaticScanBytes)
-        return fail(OMK_ERR_CAPACITY, "omk_forest_compact_static: the level scan wants %zu bytes of work space, %zu are reserved",
-                    need, kStaticScanBytes);
-    // every part is written by this call before it is read (the order map from the root on, the
-    // counts and their scan per level, the staging array per field): nothing has to start at zero
+    // every part is written by this call before it is read (the order map and the levels from the root on, the sums
+    // per level, the staging array per pass): nothing has to start at zero
+    sc.sums = (int32_t *)base;
+    sc.levels = (BfsLevel *)(base + 1024);
     sc.map = (int32_t *)(base + kStaticOffMap);
     sc.begin = (int32_t *)(base + kStaticOffBegin);
-    sc.cc = (int32_t *)(base + kStaticOffCc);
-    sc.scan = (int32_t *)(base + kStaticOffScan);
-    sc.tmp = (uint64_t *)(base + kStaticOffTmp);
-    sc.legal = (uint32_t *)(base + kStaticOffLegal);
-    sc.scan_tmp = base + kStaticOffScanTmp;
-    sc.scan_bytes = kStaticScanBytes;
-    return compact_in(f, new_root, h_nodes_after, h_old_of_new, sc);
+    sc.tmp = (uint32_t *)(base + kStaticOffTmp);
+    sc.tmp_words = (int64_t)kStaticTmpWords;
+    const int rc = compact_in(f, new_root, h_nodes_after, h_old_of_new, sc);
+    // (the array is the next call's, perhaps of another forest on another stream: this one's kernels have to be done)
+    HIP_TRY(hipStreamSynchronize(f->stream));
+    return rc;
 }
 
 int omk_forest_node_count(omk_forest *f, int64_t *h_nodes, int64_t *h_capacity) {

@@ -216,18 +216,27 @@ hipError_t launch_expand(const ForestMut &f, const ExpandJob *jobs, int n_jobs, 
 hipError_t launch_rave_backup(const ForestMut &f, const int32_t *paths, const int32_t *path_len, const float *values,
                               int n, int stride, int max_len, hipStream_t s);
 
-// Compaction: new node i takes the statistics of old node map[i]; its child range keeps its
-// length and starts at new_begin[i].
-// Breadth-first renumbering of a subtree, level by level (omk_compact.hip).
-hipError_t bfs_scan_bytes(int64_t max_items, size_t *bytes);
-hipError_t launch_bfs_level(const int2 *span, int32_t *order, int32_t *new_begin, int64_t lo, int64_t cnt,
-                            int64_t room, int32_t *cc, int32_t *scan, void *temp, size_t temp_bytes,
-                            int64_t *h_total, hipStream_t s);
+// Breadth-first renumbering of a subtree (omk_compact.hip).  A level: nodes order[lo .. lo + cnt); cnt -1: the child
+// ranges do not form a tree.  launch_bfs runs levels [from, from + n_levels), each leaving where the next one lies;
+// levels beyond the last are empty.  sums: kBfsSums ints of work space; room: ids `order` holds.
+struct BfsLevel {
+    int64_t lo, cnt;
+};
+constexpr int kBfsSums = 256;
+hipError_t launch_bfs_start(int32_t *order, BfsLevel *levels, int32_t root, hipStream_t s);
+hipError_t launch_bfs(const int2 *span, int32_t *order, int32_t *new_begin, BfsLevel *levels, int from, int n_levels,
+                      int *sums, int64_t room, hipStream_t s);
+// Arrays that a compaction moves through the map: kind 1 = 32-bit words, 2 = 64-bit words, 3 = the child ranges.
+struct CompactFields {
+    int n;
+    int kind[10];
+    uint32_t *array[10];
+};
+// words of `tmp` that an array of k nodes takes
+inline int64_t compact_words(int kind, int64_t k) { return kind == 1 ? k : 2 * k; }
+hipError_t launch_compact(const CompactFields &g, uint32_t *tmp, const int32_t *map, const int32_t *new_begin, int64_t k,
+                          hipStream_t s);
 hipError_t launch_gather_legal(uint32_t *dst, const uint32_t *src, const int32_t *order, int64_t k, hipStream_t s);
-hipError_t launch_gather_words(uint32_t *dst, const uint32_t *src, const int32_t *map, int64_t k, hipStream_t s);
-hipError_t launch_gather_dwords(uint64_t *dst, const uint64_t *src, const int32_t *map, int64_t k, hipStream_t s);
-hipError_t launch_gather_span(int2 *dst, const int2 *src, const int32_t *map, const int32_t *new_begin, int64_t k,
-                              hipStream_t s);
 
 struct TTSlot {
     unsigned long long key;

@@ -163,3 +163,34 @@ def test_structures_that_are_no_forest_are_refused(fault, message):
         f.upload(bad)
     after = f.download_structure()
     assert all((before[k] == after[k]).all() for k in before)
+
+
+# 256 blocks share a level and write 64 nodes' children at a time; twelve levels are enqueued before the host looks
+@pytest.mark.parametrize("shape", ["chain of 40", "one level of 1000", "wide levels", "a leaf"])
+@pytest.mark.parametrize("static", [False, True])
+def test_compaction_of_every_shape(shape, static):
+    import omoknuni_small_amd as omk
+    rng = np.random.default_rng(len(shape))
+    counts = {"chain of 40": [1] * 40, "one level of 1000": [1000], "a leaf": [3],
+              "wide levels": [200] + [int(x) for x in rng.integers(0, 60, 200)] + [int(x) for x in rng.integers(0, 9, 3000)]}[shape]
+    n = 1 + sum(counts) + 17
+    begin, count = np.zeros(n, np.int32), np.zeros(n, np.int32)
+    at = 1
+    for node, c in enumerate(counts):
+        if node < at and c:
+            begin[node], count[node] = at, c
+            at += c
+    soa = dict(N=rng.integers(0, 99, n).astype(np.int32), W=rng.random(n).astype(np.float32), P=rng.random(n).astype(np.float32),
+               VL=rng.integers(0, 5, n).astype(np.int32), child_begin=begin, child_count=count,
+               action=rng.integers(0, 99, n).astype(np.int32), legal=rng.integers(0, 1 << 32, (n + 31) // 32).astype(np.uint32),
+               hash=rng.integers(0, 1 << 63, n).astype(np.uint64), rN=rng.integers(0, 9, n).astype(np.int32),
+               rW=rng.random(n).astype(np.float32))
+    root = 2 if shape == "a leaf" else 0
+    f = omk.Forest.from_soa(soa)
+    order = f.compact(root, static=static)
+    ref, want = R.RefTree.from_soa(soa).compacted(root)
+    assert (order == want).all()
+    got = dict(f.download(), **f.download_structure())
+    for k in ("N", "W", "P", "VL", "rN", "rW", "action"):
+        assert got[k].tobytes() == soa[k][order].tobytes(), k
+    assert (got["child_begin"] == ref.child_begin).all() and (got["child_count"] == ref.child_count).all()
