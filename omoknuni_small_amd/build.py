@@ -5,7 +5,7 @@ import subprocess
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 
-def build_library(force=True, jobs=4):
+def build_library(force=True, jobs=8):
     """Runs make in csrc/.  With force the objects are rebuilt even when up to date."""
     cmd = ["make", "-C", os.path.join(HERE, "csrc"), "-j%d" % jobs]
     if force:

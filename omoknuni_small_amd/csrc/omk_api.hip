@@ -1207,7 +1207,7 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) {
     std::stable_sort(items.begin(), items.end(), [](const Item &x, const Item &y) { return x.m > y.m; });
     // A root that will be cut into slices (kHeavyMin visitors or more): its boundaries depend on its statistics
     // only, so they are queued right behind the roots (items of kind 4, see prefetch_boundaries in
-    // omk_select.hip) and worked out by other wavefronts while the root's own wavefront still loads its children.
+    // omk_select_kernels.h) and worked out by other wavefronts while the root's own wavefront still loads its children.
     int32_t n_hctx0 = 0;
     {
         const size_t n_roots = items.size();

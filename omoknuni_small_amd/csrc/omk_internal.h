@@ -121,6 +121,11 @@ hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, 
 hipError_t launch_set_roots(int32_t *seg0, int32_t *paths, Item *items0, Item *singles0, const int32_t *staged, int n,
                             int n_items, int n_singles, hipStream_t s);
 
+// The kernels of one fan-out class (rounds of 64 children: 1, 4, 6 or 16), behind the reset launch.
+template <int RMAX, bool RAVE>
+hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a, int n_items0, int n_traversals, int n_cus,
+                               hipStream_t s);
+
 hipError_t launch_apply_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                            int max_len, int vl, hipStream_t s);
 hipError_t launch_revert_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,

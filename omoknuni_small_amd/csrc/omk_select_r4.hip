@@ -1,0 +1,7 @@
+// The selection kernels of forests whose nodes have at most 256 children.
+#include "omk_select_kernels.h"
+
+namespace omk {
+template hipError_t launch_select_class<4, false>(const ForestDev &, const SelectArgs &, int, int, int, hipStream_t);
+template hipError_t launch_select_class<4, true>(const ForestDev &, const SelectArgs &, int, int, int, hipStream_t);
+}  // namespace omk

@@ -1,0 +1,7 @@
+// The selection kernels of forests whose nodes have at most 384 children.
+#include "omk_select_kernels.h"
+
+namespace omk {
+template hipError_t launch_select_class<6, false>(const ForestDev &, const SelectArgs &, int, int, int, hipStream_t);
+template hipError_t launch_select_class<6, true>(const ForestDev &, const SelectArgs &, int, int, int, hipStream_t);
+}  // namespace omk
