@@ -4452,10 +4452,12 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_i
         // on the 4 M-node chess-like tree: 0.247 ms a selection with two blocks per unit, 0.222 with one.
         int capacity = n_cus;
         if (capacity < 2) capacity = 2;
-        int walkers = n_traversals / 64;
+        int walkers = n_traversals / 4;
         if (walkers > capacity / 4) walkers = capacity / 4;
         if (walkers > kMaxWalkerBlocks) walkers = kMaxWalkerBlocks;  // idle walkers poll: more of them slow the teams
-        if (walkers < 4) walkers = 4;  // (a small batch ends with a handful of lone walks: enough walkers to take them at once)
+        // (a wavefront per visitor while that is at most kMaxWalkerBlocks: the root of a young tree leaves nearly
+        // every visitor of a small batch alone, and 64 of them on 16 walkers took four rounds, 26 us of 54)
+        if (walkers < 4) walkers = 4;
         int teams = capacity - walkers;
         const int most = n_traversals / 2;
         if (teams > most) teams = most;
