@@ -130,6 +130,7 @@ struct omk_batch {
     float *values = nullptr;
     Item *items0 = nullptr, *items_q = nullptr, *singles0 = nullptr, *singles_q = nullptr;
     int32_t n_singles0 = 0;
+    int32_t most_visitors = 1;  // of one root
     int32_t n_hctx0 = 0;  // contexts of heavy roots, handed out when the roots are set
     int32_t *seg0 = nullptr, *seg[2] = {nullptr, nullptr};
     int32_t *sc_child = nullptr, *sc_occ = nullptr;
@@ -1241,6 +1242,7 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) {
         memcpy(at + 2 * (size_t)n + items.size() * (sizeof(Item) / 4), singles.data(), singles.size() * sizeof(Item));
     HIP_TRY(launch_set_roots(b->seg0, b->paths, b->items0, b->singles0, at, n, (int)items.size(), (int)singles.size(),
                              f->stream));
+    b->most_visitors = items.empty() ? 1 : items[0].m;
     b->n_items0 = (int32_t)items.size();
     b->n_hctx0 = n_hctx0;
     b->n_singles0 = (int32_t)singles.size();
@@ -1360,7 +1362,7 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
     a.pw = p->pw;
     a.c_puct = p->c_puct;
     a.rave_k = p->rave_k;
-    HIP_TRY(launch_select(f->dev(), a, b->n_items0, b->n_singles0, b->n, f->max_fanout, p->use_rave != 0, b->n_cus,
+    HIP_TRY(launch_select(f->dev(), a, b->n_items0, b->n_singles0, b->n, b->most_visitors, f->max_fanout, p->use_rave != 0, b->n_cus,
                           b->n_hctx0, f->stream));
     b->selected = true;
     b->select_calls++;

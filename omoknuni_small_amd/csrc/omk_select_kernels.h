@@ -2988,7 +2988,12 @@ struct Continuation {
 // wavefront that finishes last (a counter in the node's context) partitions the visitors
 // and walks on, every other returns kStepParked.  Any failed check sends the whole node
 // back to the one-wavefront path.
-template <int R, bool RAVE, int RMAX>
+//
+// HEAVY: the kernel for batches in which a node of kHeavyMin visitors can occur.  Without it (every root has fewer) the
+// slices, their boundaries and their joins are left out, and with them registers that the rest of the code then has
+// (narrow class 160 -> 145, four rounds 224 -> 216, six 276 -> 245): 64 visitors of a Gomoku tree 104.3 -> 98.9 us a
+// pass, 16 on each of 64 Go trees 124 -> 119, 8 on a tree 70 -> 68.
+template <int R, bool RAVE, int RMAX, bool HEAVY>
 __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs &a, const NodeCtx &c, int lane,
                                             const Item &item, const int32_t *seg_in, int32_t *seg_out,
                                             WaveLds<R> &lds, PartLds<RMAX> &pl, bool &pending, Continuation &next,
@@ -2997,6 +3002,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
     // one-winner nodes stopped at this node and left its children, scored, in the LDS scratch, with the verdict
     bool ahead = preload == 1;
     const int off = item.off, m = item.m, depth = item.depth;
+    const bool heavy = HEAVY && m >= kHeavyMin;
     // a heavy node is settled and shared out by several wavefronts, which read its visitor
     // list: it must be complete before any of them is called in
     // where this node's winner order goes in sc_child / sc_occ when it does not fit LDS: the
@@ -3005,12 +3011,12 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
     const int soff = off + (depth & 1) * a.stride;
     // the visitor list of an item of kind 3, and of the slices of one, may not be there yet:
     // whoever shares out the visitors waits for it (below), settling them does not need it
-    bool list_ok = !(item.pad[0] == 3 || (item.pad[0] == 1 && ((item.pad[2] >> 30) & 1)));
-    if (m >= kHeavyMin) close_pending(pending);
+    bool list_ok = !HEAVY || !(item.pad[0] == 3 || (item.pad[0] == 1 && ((item.pad[2] >> 30) & 1)));
+    if (heavy) close_pending(pending);
     Kids<R, RAVE> k;
     int cnt[R];
     uint32_t bk = 0u, bpos = 0xFFFFFFFFu;
-    if (item.pad[0] == 2) {
+    if (HEAVY && item.pad[0] == 2) {
         // a part of a heavy node's partition: of the children only the visit counts are needed
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -3118,10 +3124,10 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
     // run_child, or the winner order is still in LDS buffer lds_cur, or (both -1) it is in the
     // sc_child / sc_occ arrays in device memory
     int run_child = -1, lds_cur = -1;
-    bool as_slice = item.pad[0] == 1;
-    const bool as_scatter = item.pad[0] == 2;
+    bool as_slice = HEAVY && item.pad[0] == 1;
+    const bool as_scatter = HEAVY && item.pad[0] == 2;
     // one boundary of this node, to be worked out ahead of time (prefetch_boundaries): into the table, nothing else
-    const bool just_boundary = item.pad[0] == 4;
+    const bool just_boundary = HEAVY && item.pad[0] == 4;
     int hid = as_slice || as_scatter || just_boundary ? item.pad[1] : -1, slice = item.pad[2] & 0xFFFF,
         n_slices = (item.pad[2] >> 16) & 0x3FFF;
     if (as_scatter) {
@@ -3143,7 +3149,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
     } else if (!as_slice && !just_boundary && !settled && m >= kRunMin && a.vl > 0 && !odd)
         settled = single_run<R, RAVE>(a, c, lane, k, bk, bpos, soff, m, m >= kRunShareMin, cnt, run_child, contested, best0,
                                       lk0, lp0);
-    if (!settled && contested && m >= kSparseMin && m < kHeavyMin && !odd) {
+    if (!settled && contested && m >= kSparseMin && !heavy && !odd) {
         settled = sparse_merge<R, RAVE>(a, c, lane, k, best0, lk0, lp0, m, lds, pl.order, cnt, pending);
         if (settled) {
             lds_cur = 0;
@@ -3153,8 +3159,8 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
             for (int r = 0; r < R; r++) cnt[r] = 0;
         }
     }
-    if (R * kWave <= kHeavyFanout) {
-        if (!as_slice && !just_boundary && !settled && m >= kHeavyMin && m <= kWaterLevelMaxJ && a.vl > 0 && !odd) {
+    if (HEAVY && R * kWave <= kHeavyFanout) {
+        if (!as_slice && !just_boundary && !settled && heavy && m <= kWaterLevelMaxJ && a.vl > 0 && !odd) {
             // cut the node into slices: the others go to the queue, this wavefront takes the first
             const int K = (m + slice_size(m) - 1) / slice_size(m);  // at most kMaxSlices
             // (a node whose boundaries are being worked out ahead of time has its context already)
@@ -3324,7 +3330,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
     // (with RAVE, where every probe of the water level scores two scans per child; without it the path's code
     // costs the kernel more than its shorter probes save)
     if constexpr (R > 1 && RAVE) {
-        if (!settled && contested && m >= kWaterLevelMin && m < kHeavyMin && a.vl > 0 && !odd && !as_slice &&
+        if (!settled && contested && m >= kWaterLevelMin && !heavy && a.vl > 0 && !odd && !as_slice &&
             !as_scatter) {
             settled = narrow_water_level<R, RAVE>(a, c, lane, k, soff, best0, lk0, lp0, m, lds, cnt, lds_cur, pl.order,
                                                   pending);
@@ -3340,7 +3346,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
         int zero[R];
 #pragma unroll
         for (int r = 0; r < R; r++) zero[r] = 0;
-        settled = water_level<R, RAVE>(a, c, lane, k, soff, 0, m, zero, lds, cnt, m < kHeavyMin, lds_cur, false, zero,
+        settled = water_level<R, RAVE>(a, c, lane, k, soff, 0, m, zero, lds, cnt, !heavy, lds_cur, false, zero,
                                        pl.order, pending);
         if (!settled) st_replay = 1;
     }
@@ -3348,7 +3354,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
         // one visitor after the other
         run_child = -1;
         lds_cur = -1;
-        const bool seq_lds = m < kHeavyMin;  // few enough visitors to keep their order in LDS
+        const bool seq_lds = !heavy;  // few enough visitors to keep their order in LDS
         if (seq_lds) close_pending(pending);  // the previous node's partition may still read that buffer
         for (int done = 0; done < m; done++) {
             int i = wave_pick<R, RAVE>(k, lane, bk, bpos);
@@ -3407,7 +3413,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
         if (!wait_list(a, off, depth, lane)) return kStepParked;
         list_ok = true;
     }
-    if (run_child >= 0 && !as_scatter && !as_slice && m < kHeavyMin && a.vl > 0) {
+    if (run_child >= 0 && !as_scatter && !as_slice && !heavy && a.vl > 0) {
         // Every visitor follows one child: nothing to share out.  The helpers walk down from that child for as
         // long as the visitors stay together, and write the path entries of all those levels, this node's
         // included (chain_walk, chain_finish); the owner takes the walk's barriers with them (owner_loop).
@@ -3461,7 +3467,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
     // shares out the visitors and publishes the other children (partition_async), this one
     // walks on into the kept child at once.  What the kept child needs of that work, its
     // visitor list, it needs last (close_pending).
-    if (!as_scatter && !as_slice && ((m < kHeavyMin && lds_cur >= 0) || (run_child >= 0 && m < kRunShareMin))) {
+    if (!as_scatter && !as_slice && ((!heavy && lds_cur >= 0) || (run_child >= 0 && m < kRunShareMin))) {
         int carry = 0, ex_keep = 0, np_keep = 0;
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -3526,7 +3532,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
     }
     int lone0 = 0, slot0 = -1;
     bool have_slots = false;
-    if (!as_scatter && (m < kHeavyMin || R * kWave > kHeavyFanout)) {
+    if (!as_scatter && (!heavy || R * kWave > kHeavyFanout)) {
         // not a node whose scatter is shared out: the answers arrive during the next steps
         if (lane == 0) {
             if (n_lone > 0) lone0 = atomicAdd(a.n_singles, n_lone);
@@ -3554,7 +3560,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
     // through the queue, and the wavefront that finishes last goes on
     int r0 = 0, r1 = m;
     bool shared = false;
-    if (R * kWave <= kHeavyFanout) {
+    if (HEAVY && R * kWave <= kHeavyFanout) {
         int part = 0, n_parts = 1;
         if (as_scatter) {
             part = slice;
@@ -3562,7 +3568,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
             shared = true;
             lone0 = a.hctx[(size_t)hid * kHeavyCtxInts + 3];
             have_slots = true;  // the wavefront that finishes the scatter asks for the work queue's
-        } else if (m >= kHeavyMin) {
+        } else if (heavy) {
             if (hid < 0) {
                 int id = a.hctx_cap;
                 if (lane == 0) id = atomicAdd(a.hctx_n, 1);
@@ -3795,7 +3801,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
 //
 // A block is a team: its first wavefront (the owner) runs this loop, the other wavefronts
 // wait at a block barrier until the owner shares out the batch work of a node (team_help).
-template <int RMAX, bool RAVE>
+template <int RMAX, bool RAVE, bool HEAVY>
 __device__ __forceinline__ void owner_loop(const ForestDev &f, const SelectArgs &a, WaveLds<RMAX> &s_lds,
                                            PartLds<RMAX> &s_part, bool &pending, int lane) {
     for (;;) {
@@ -3836,7 +3842,7 @@ __device__ __forceinline__ void owner_loop(const ForestDev &f, const SelectArgs 
         // compute unit every time); one acquire once the item is there
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         Item it = a.items_q[ticket];
-        if (it.depth == 0 && (it.pad[0] == 0 || it.pad[0] == 4)) {  // (items the host wrote: a root, a boundary of one)
+        if (it.depth == 0 && (!HEAVY || it.pad[0] == 0 || it.pad[0] == 4)) {  // (items the host wrote: a root, a boundary of one)
             it.np = f.N[it.node];  // (the paths' first entries, the roots, are written when the roots are set)
         }
         bool have_span = false, chain_open = false;
@@ -3873,7 +3879,7 @@ __device__ __forceinline__ void owner_loop(const ForestDev &f, const SelectArgs 
             const int preload_now = preload;
             preload = 0;
             // a boundary to work out ahead of time, of a node that turns out to have no children to choose from
-            if (it.pad[0] == 4 && !(c.cc > 0 && depth < a.max_depth)) break;
+            if (HEAVY && it.pad[0] == 4 && !(c.cc > 0 && depth < a.max_depth)) break;
             int status = kStepLeaf;
             Continuation next;
             next.node = -1;
@@ -3881,11 +3887,11 @@ __device__ __forceinline__ void owner_loop(const ForestDev &f, const SelectArgs 
             next.chain_open = false;
             if (c.cc > 0 && depth < a.max_depth) {
                 if (c.cc <= kWave)
-                    status = select_group<1, RAVE, RMAX>(f, a, c, lane, it, seg_in, seg_out,
+                    status = select_group<1, RAVE, RMAX, HEAVY>(f, a, c, lane, it, seg_in, seg_out,
                                                          reinterpret_cast<WaveLds<1> &>(s_lds), s_part, pending,
                                                          next, preload_now == 2 ? 2 : 0);
                 else
-                    status = select_group<RMAX, RAVE, RMAX>(f, a, c, lane, it, seg_in, seg_out, s_lds, s_part, pending,
+                    status = select_group<RMAX, RAVE, RMAX, HEAVY>(f, a, c, lane, it, seg_in, seg_out, s_lds, s_part, pending,
                                                             next, preload_now);
             }
             if (a.trace && lane == 0) {
@@ -3897,16 +3903,16 @@ __device__ __forceinline__ void owner_loop(const ForestDev &f, const SelectArgs 
                     // a slice or a part of a heavy node: its number and their number in the upper half
                     a.trace[12 * ti + 3] = (long long)it.node | ((long long)(uint32_t)it.pad[2] << 32);
                     for (int q = 0; q < 8; q++) a.trace[12 * ti + 4 + q] = 0;
-                    if (it.pad[0] == 1 || it.m >= kHeavyMin) {
+                    if (HEAVY && (it.pad[0] == 1 || it.m >= kHeavyMin)) {
                         a.trace[12 * ti + 4] = (long long)(uint32_t)g_slice_note[0] | ((long long)(uint32_t)g_slice_note[1] << 32);
                         a.trace[12 * ti + 5] = (long long)(uint32_t)g_slice_note[2] | ((long long)(uint32_t)g_slice_note[3] << 32);
                     }
                 }
             }
-            if (status == kStepParked) break;  // a slice of a heavy node: another wavefront goes on with it
+            if (HEAVY && status == kStepParked) break;  // a slice of a heavy node: another wavefront goes on with it
             if (status == kStepLeaf) {
                 close_pending(pending);  // the visitor list comes from the previous node's partition
-                if (it.pad[0] == 3 && !wait_list(a, it.off, depth, lane)) break;
+                if (HEAVY && it.pad[0] == 3 && !wait_list(a, it.off, depth, lane)) break;
                 for (int j = lane; j < it.m; j += kWave) {
                     int t = seg_in[it.off + j];
                     a.leaf[t] = it.node;
@@ -4068,7 +4074,7 @@ __device__ __forceinline__ void team_help(const ForestDev &f, const SelectArgs &
 template <int RMAX, bool RAVE>
 __device__ void walkers_loop(ForestDev f, SelectArgs a, int lane);
 
-template <int RMAX, bool RAVE>
+template <int RMAX, bool RAVE, bool HEAVY>
 __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs a) {
     __shared__ WaveLds<RMAX> s_lds;
     __shared__ PartLds<RMAX> s_part;
@@ -4084,7 +4090,7 @@ __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs
     if (tid < kWave) {
         // every path out of the owner's loop comes back here: the helpers are always released
         bool pending = false;
-        owner_loop<RMAX, RAVE>(f, a, s_lds, s_part, pending, tid);
+        owner_loop<RMAX, RAVE, HEAVY>(f, a, s_lds, s_part, pending, tid);
         close_pending(pending);
         if (tid == 0) atomicMax(a.times + 1, (int)(wall_clock64() & 0x7FFFFFFF));
         if (tid == 0) s_lds.cmd.op = kOpExit;
@@ -4435,8 +4441,8 @@ __device__ __noinline__ void walkers_loop(ForestDev f, SelectArgs a, int lane) {
 }
 
 template <int RMAX, bool RAVE>
-hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_items0, int n_traversals,
-                                 int n_cus, hipStream_t s) {
+hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_items0, int most_visitors,
+                                 int n_traversals, int n_cus, hipStream_t s) {
     // Few walkers cannot keep the memory system busy: then the variant that spends bytes to save
     // dependent trips (select_single, FAST).  The number of lone visitors is only known on the
     // device; the number of traversals bounds it.  Measured: it pays on a board layout (legal
@@ -4465,7 +4471,10 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_i
         SelectArgs a = a0;
         a.n_team_blocks = teams;
         a.fast_singles = fast ? 1 : 0;
-        hipLaunchKernelGGL((k_select_groups<RMAX, RAVE>), dim3(teams + walkers), dim3(kTeam), 0, s, f, a);
+        if (most_visitors >= kHeavyMin)
+            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, true>), dim3(teams + walkers), dim3(kTeam), 0, s, f, a);
+        else
+            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, false>), dim3(teams + walkers), dim3(kTeam), 0, s, f, a);
         return hipGetLastError();
     }
     // every traversal is alone at its root: the walkers are the host's list
