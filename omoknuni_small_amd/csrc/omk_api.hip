@@ -40,6 +40,7 @@ struct omk_forest {
     bool has_rave = false;
     bool uploaded = false;
     bool prior_sorted = false;
+    bool grown = false;  // expanded since the last upload: most children have no visits
     int max_fanout = 0;
     // Counts the changes that give node ids a new meaning (a compaction, an upload of a different
     // structure): paths, roots and work items of a batch made before such a change are stale.
@@ -602,6 +603,7 @@ int omk_forest_upload(omk_forest *f, const omk_soa_view *v) {
     }
     f->n_nodes = n;
     f->max_fanout = mf;
+    f->grown = false;
     f->prior_sorted = sorted;
     f->uploaded = true;
     // the RAVE blend of every node from the new statistics, for the constant the selections have been using
@@ -1362,7 +1364,7 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
     a.pw = p->pw;
     a.c_puct = p->c_puct;
     a.rave_k = p->rave_k;
-    HIP_TRY(launch_select(f->dev(), a, b->n_items0, b->n_singles0, b->n, b->most_visitors, f->max_fanout, p->use_rave != 0, b->n_cus,
+    HIP_TRY(launch_select(f->dev(), a, b->n_items0, b->n_singles0, b->n, b->most_visitors, f->max_fanout, p->use_rave != 0, f->grown, b->n_cus,
                           b->n_hctx0, f->stream));
     b->selected = true;
     b->select_calls++;
@@ -1589,6 +1591,7 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
     HIP_TRY(launch_expand(f->mut(), jobs, (int)nj, moves, priors, f->n_nodes, cursor, f->stream));
     f->n_nodes = cursor;
     f->changes++;
+    f->grown = true;
     f->structure_changed = true;  // ids keep their meaning, but an upload of the old arrays would not
     f->max_fanout = mf;
     if (!sorted) f->prior_sorted = false;

@@ -114,9 +114,10 @@ struct SelectArgs {
     float rave_k;
 };
 
-// most_visitors: traversals of the most crowded root
+// most_visitors: traversals of the most crowded root; grown: the forest has been expanded since it was uploaded
 hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, int n_singles0, int n_traversals,
-                         int most_visitors, int max_fanout, bool rave, int n_cus, int n_hctx0, hipStream_t s);
+                         int most_visitors, int max_fanout, bool rave, bool grown, int n_cus, int n_hctx0,
+                         hipStream_t s);
 
 // What omk_batch_set_roots has staged (n visitors | n roots | items | lone traversals) to the batch's arrays.
 hipError_t launch_set_roots(int32_t *seg0, int32_t *paths, Item *items0, Item *singles0, const int32_t *staged, int n,
@@ -125,7 +126,7 @@ hipError_t launch_set_roots(int32_t *seg0, int32_t *paths, Item *items0, Item *s
 // The kernels of one fan-out class (rounds of 64 children: 1, 4, 6 or 16), behind the reset launch.
 template <int RMAX, bool RAVE>
 hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a, int n_items0, int most_visitors, int n_traversals,
-                               int n_cus, hipStream_t s);
+                               int n_cus, bool grown, hipStream_t s);
 
 hipError_t launch_apply_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                            int max_len, int vl, hipStream_t s);

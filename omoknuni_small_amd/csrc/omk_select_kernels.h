@@ -2132,8 +2132,39 @@ __device__ __forceinline__ int count_before(int n, float w, float p, int vl, flo
 
 constexpr int kSparseMax = 64;  // entries of other children a nearly-one-winner node may hold (one per lane)
 constexpr int kSparseMin = 8;    // visitors from which that direct merge is tried
+enum { kMergeNo = 0, kMergeDone = 1, kMergeMany = 2 };
 static_assert(2 * kHeavyMin <= kBatchCap, "the (key, position) list of the dominant child fits one sort buffer");
 
+
+// A lower end of the key range with at least `least` and at most 64 of the keys that `count` counts at or above it,
+// found by halving; `top`: no key lies above it; 0: there is none (keys tied).
+template <typename Count>
+__device__ __forceinline__ uint32_t halve_to_lanes(const Count &count, uint32_t top, int least) {
+    uint32_t lo = 1u, hi = top + 1u;  // count(lo) > 64, count(hi) < least
+    while (hi - lo > 1u) {
+        const uint32_t mid = lo + ((hi - lo) >> 1);
+        const int n = count(mid);
+        if (n < least) hi = mid;
+        else if (n > kWave) lo = mid;
+        else return mid;
+    }
+    return 0u;
+}
+
+// Of a node's children only those can be chosen by its m visitors whose next entries are among the m first of all:
+// as long as fewer than m visitors have chosen, at least one of m better heads is still there.  For m <= 64 and more
+// children than lanes: a key with at least m and at most 64 heads at or above it.
+template <int R, bool RAVE>
+__device__ __forceinline__ uint32_t first_heads(const Kids<R, RAVE> &k, uint32_t best_key, int m) {
+    auto heads = [&](uint32_t T) {
+        int n = 0;
+#pragma unroll
+        for (int r = 0; r < R; r++) n += __popcll(__ballot(umax32(k.k1[r], k.k2[r]) >= T));
+        return n;
+    };
+    if (heads(1u) <= kWave) return 1u;
+    return halve_to_lanes(heads, wave_max_u32(best_key), m);
+}
 
 // A node where one child wins ALMOST every time: the winner order is that child's list with
 // a few entries of other children merged in.  The child, A, is the one that holds out longest,
@@ -2150,10 +2181,10 @@ static_assert(2 * kHeavyMin <= kBatchCap, "the (key, position) list of the domin
 // (lk, lp) (count_before brackets the count by two exact evaluations) or looked at and placed
 // behind the m-th winner (checked).  Then the best head at any step is never one of the heads
 // left out, and merging the lists by (key, position) is the serial order.
-// On success: order[q] = (child << 21) | visit number for the m visitors, cnt[] the visits
-// per child.  On failure nothing the caller relies on has changed (order[] is scratch).
+// On success (kMergeDone): order[q] = (child << 21) | visit number for the m visitors, cnt[] the visits
+// per child.  kMergeMany: the entries of the others are too many for one per lane.  On failure nothing the caller relies on has changed (order[] is scratch).
 template <int R, bool RAVE>
-__device__ __forceinline__ bool sparse_merge(const SelectArgs &a, const NodeCtx &c, int lane, const Kids<R, RAVE> &k,
+__device__ __forceinline__ int sparse_merge(const SelectArgs &a, const NodeCtx &c, int lane, const Kids<R, RAVE> &k,
                                              int best0, uint32_t lk0, uint32_t lp0, int m, WaveLds<R> &lds,
                                              uint32_t *order, int (&cnt)[R], bool &pending) {
     constexpr int F = R * kWave;
@@ -2184,7 +2215,8 @@ __device__ __forceinline__ bool sparse_merge(const SelectArgs &a, const NodeCtx 
         }
         n0 += __popcll(cm);
     }
-    if (n0 < 2 || n0 > kSparseMax) return false;
+    if (n0 < 2) return kMergeNo;
+    if (n0 > kSparseMax) return kMergeMany;
     wave_sync_memory();
     int ci = -1, cn = 0, cvl = 0;
     float cw = 0.0f, cp = 0.0f, cq2 = 0.0f;
@@ -2202,9 +2234,9 @@ __device__ __forceinline__ bool sparse_merge(const SelectArgs &a, const NodeCtx 
     // ---- A: the child that holds out longest ----
     uint32_t lk, lp;
     wave_best(zk, zp, lk, lp);
-    if (lk == 0u) return false;
+    if (lk == 0u) return kMergeNo;
     const uint64_t am = __ballot(lane < n0 && zk == lk && zp == lp);
-    if (am == 0ull) return false;
+    if (am == 0ull) return kMergeNo;
     const int a_lane = __ffsll((long long)am) - 1;
     const int a_child = __builtin_amdgcn_readlane(ci, a_lane);
     const int a_n = __builtin_amdgcn_readlane(cn, a_lane);
@@ -2214,7 +2246,7 @@ __device__ __forceinline__ bool sparse_merge(const SelectArgs &a, const NodeCtx 
     const float a_q2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cq2), a_lane));
     // ---- the others that can get an entry in: next entry before (lk, lp) ----
     const bool is_cand = lane < n0 && lane != a_lane && hk != 0u && comes_before(hk, hp, lk, lp);
-    if (__ballot(is_cand) == 0ull) return false;
+    if (__ballot(is_cand) == 0ull) return kMergeNo;
     {
         // Far too many entries by the estimates: leave before anything exact is paid for.  An entry
         // of a child gets in only if fewer than m entries come before it; the child's next entry has
@@ -2231,7 +2263,7 @@ __device__ __forceinline__ bool sparse_merge(const SelectArgs &a, const NodeCtx 
         }
         // (a little below the capacity: the exact counts tend to come out above the estimates, and
         // a refusal after them costs three times what one here does)
-        if (wave_sum_i32(est) > kSparseMax - 4) return false;
+        if (wave_sum_i32(est) > kSparseMax - 4) return kMergeMany;
     }
     // ---- A's entries, all m of them, evaluated once into LDS and checked: none may come before its
     // predecessor (its head then stays at or before (lk, lp) throughout) ----
@@ -2257,7 +2289,7 @@ __device__ __forceinline__ bool sparse_merge(const SelectArgs &a, const NodeCtx 
             carry_k = (uint32_t)__builtin_amdgcn_readlane((int)kk, 63);
             carry_p = (uint32_t)__builtin_amdgcn_readlane((int)pp, 63);
         }
-        if (__ballot(bad_a) != 0ull) return false;
+        if (__ballot(bad_a) != 0ull) return kMergeNo;
     }
     wave_sync_memory();
     // how many of A's entries come before the entry (tk, tp): the list is in order, so a bisection
@@ -2282,7 +2314,7 @@ __device__ __forceinline__ bool sparse_merge(const SelectArgs &a, const NodeCtx 
     }
     const int inc = wave_inclusive_sum(cc, lane);
     const int total = __builtin_amdgcn_readlane(inc, 63);
-    if (total > kSparseMax) return false;
+    if (total > kSparseMax) return kMergeMany;
     const int start = inc - cc;
     // ---- one lane per entry: (lane of its child, visit number) ----
     for (int t = 0; t < cc; t++) lds.hist[start + t] = lane | (t << 8);  // start + cc <= total <= 64
@@ -2341,7 +2373,7 @@ __device__ __forceinline__ bool sparse_merge(const SelectArgs &a, const NodeCtx 
     }
     {
         const int why = (int)wave_max_u32((uint32_t)bad);
-        if (why != 0) return false;
+        if (why != 0) return kMergeNo;
     }
     // ---- the winner order: the others' entries at their places, A's in between ----
     close_pending(pending);  // the previous node's partition may still read the order buffer
@@ -2359,7 +2391,7 @@ __device__ __forceinline__ bool sparse_merge(const SelectArgs &a, const NodeCtx 
         if (q < m) order[q] = other ? (v & 0x7FFFFFFFu) : (((uint32_t)a_child << 21) | (uint32_t)(q - below));
         seen += __popcll(om);
     }
-    if (seen != nfv) return false;  // two entries at one place: cannot happen when the checks hold
+    if (seen != nfv) return kMergeNo;  // two entries at one place: cannot happen when the checks hold
     // ---- visits per child, back to the lanes that hold the children ----
     if (lane < n0) lds.hist[kSparseMax + lane] = lane == a_lane ? m - nfv : mine_in;
     wave_sync_memory();
@@ -2370,9 +2402,171 @@ __device__ __forceinline__ bool sparse_merge(const SelectArgs &a, const NodeCtx 
         cnt[r] = listed[r] ? lds.hist[kSparseMax + cl_run + __popcll(cm & ((1ull << lane) - 1ull))] : 0;
         cl_run += __popcll(cm);
     }
+    return kMergeDone;
+}
+
+
+constexpr int kFewMax = 64;  // visitors of a node that few_visitors settles, at most
+constexpr int kFewEntries = 4;  // entries of every child it evaluates
+
+// A contested node of at most 64 visitors that spread out (more entries of other children than the merge above has
+// lanes for), settled at once.  Only the children with the m first heads matter (first_heads), one per lane.  Every
+// lane evaluates its child's next kFewEntries entries, independently of each other where the serial loop waits for a
+// division chain per visitor; a threshold with at least m and at most 64 of all these entries above it is found by
+// halving the key range, and the entries above it, one per lane, find their places by counting the ones before them.
+// Exact because: every child's entries used are in order (checked), so the merge of the lists in the order (key,
+// position, visit) is the serial order; and no child has all its evaluated entries above the threshold (declined),
+// so an entry not evaluated comes after one that is never reached.
+// A function of its own, and only in the kernel for trees that have grown on the device (SPREAD), whose nodes have
+// many children without visits: anywhere else its mere presence cost the other nodes 2 to 4 %.
+// Measured on an MI355X: a search of 64 visitors a batch from the bare root 1.51 -> 1.32 ms, of 48 with RAVE on a Go
+// board 1.74 -> 1.64.
+struct FewLds {
+    int child[kWave];  // the children that matter, one per lane, in child order: index in the node ...
+    int n[kWave];      // ... and statistics
+    float w[kWave], p[kWave], q2[kWave];
+    int vl[kWave];
+    unsigned long long entry[kWave];  // the entries above the threshold: smaller = played earlier, all different
+    int who[kWave];                   // lane of the child | number of the visit << 8
+    uint32_t order[kWave];            // (child << 21) | number of the visit, per visitor
+    int count[kWave];                 // visits per child
+};
+__shared__ FewLds g_few;
+
+template <bool RAVE>
+__device__ __noinline__ bool few_order(int n0, int m, float ep, uint32_t uvl, uint32_t top, int lane) {
+    constexpr int K = kFewEntries;
+    uint32_t ek[K];
+    bool second[K];
+#pragma unroll
+    for (int j = 0; j < K; j++) {
+        ek[j] = 0u;
+        second[j] = false;
+    }
+    if (lane < n0) {
+        const int cn = g_few.n[lane], cvl = g_few.vl[lane];
+        const float cw = g_few.w[lane], cp = g_few.p[lane], cq2 = RAVE ? g_few.q2[lane] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            uint32_t pos;
+            entry_key<1, RAVE>(cn, cw, cp, cvl, cq2, ep, uvl, j, lane, ek[j], pos);
+            second[j] = pos >= (uint32_t)kWave;
+        }
+    }
+    auto entries = [&](uint32_t T) {
+        int n = 0;
+#pragma unroll
+        for (int j = 0; j < K; j++) n += __popcll(__ballot(ek[j] >= T));
+        return n;
+    };
+    const int all = entries(1u);
+    if (all < m) return false;
+    const uint32_t T = all <= kWave ? 1u : halve_to_lanes(entries, top, m);
+    if (T == 0u) return false;
+    int mine = 0;
+    bool bad = ek[K - 1] >= T;
+#pragma unroll
+    for (int j = 0; j < K; j++) {
+        const bool in = ek[j] >= T;
+        mine += in ? 1 : 0;
+        // (an entry of the second scan at the key of the one of the first scan before it is in order)
+        if (j > 0 && in && (ek[j] > ek[j - 1] || (ek[j] == ek[j - 1] && second[j - 1] && !second[j]))) bad = true;
+    }
+    if (__ballot(bad) != 0ull) return false;
+    const int inc = wave_inclusive_sum(mine, lane);
+    const int start = inc - mine, total = __builtin_amdgcn_readlane(inc, 63);
+    g_few.entry[lane] = ~0ull;
+    wave_sync_memory();
+#pragma unroll
+    for (int j = 0; j < K; j++) {
+        if (j < mine) {
+            const uint32_t pos = (uint32_t)((second[j] ? kWave : 0) + lane);
+            g_few.entry[start + j] = ((unsigned long long)~ek[j] << 32) | (pos << 8) | (unsigned)(start + j);
+            g_few.who[start + j] = lane | (j << 8);
+        }
+    }
+    wave_sync_memory();
+    const unsigned long long e64 = g_few.entry[lane];
+    int rank = 0;
+    for (int e0 = 0; e0 < total; e0 += 8) {
+        unsigned long long o[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) o[u] = g_few.entry[e0 + u];
+#pragma unroll
+        for (int u = 0; u < 8; u++) rank += o[u] < e64 ? 1 : 0;
+    }
+    const bool valid = lane < total && rank < m;
+    const uint64_t vmask = __ballot(valid);
+    if (valid) {
+        const int who = g_few.who[lane];
+        g_few.order[rank] = ((uint32_t)g_few.child[who & 255] << 21) | (uint32_t)(who >> 8);
+    }
+    g_few.count[lane] = __popcll((vmask >> (start & 63)) & ((1ull << mine) - 1ull));  // (mine < 64; none: 0)
+    wave_sync_memory();
     return true;
 }
 
+// Returns false with nothing the caller relies on changed.
+template <int R, bool RAVE>
+__device__ __forceinline__ bool few_visitors(const SelectArgs &a, const NodeCtx &c, int lane, const Kids<R, RAVE> &k,
+                                             uint32_t best_key, int best, int m, uint32_t *order, int (&cnt)[R],
+                                             bool &pending) {
+    // Only where the visitors are sure to spread: m children's next entries come before the second entry of the best
+    // one.  (Where they do not, finding that out below costs 5 us; this test a twentieth of a node.)
+    {
+        int bn = 0, bvl = 0;
+        float bw = 0.0f, bp = 0.0f, bq2 = 0.0f;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (r == (best >> 6)) {
+                bn = k.n[r];
+                bw = k.w[r];
+                bp = k.p[r];
+                bvl = k.vl[r];
+                bq2 = k.q2[r];
+            }
+        }
+        uint32_t key, pos;
+        entry_key<1, RAVE>(bn, bw, bp, bvl, bq2, c.ep, (uint32_t)a.vl, 1, 0, key, pos);
+        key = (uint32_t)__builtin_amdgcn_readlane((int)key, best & 63);
+        int before = 0;
+#pragma unroll
+        for (int r = 0; r < R; r++) before += __popcll(__ballot(umax32(k.k1[r], k.k2[r]) > key));
+        if (before < m) return false;
+    }
+    const uint32_t T0 = first_heads<R, RAVE>(k, best_key, m);
+    if (T0 == 0u) return false;
+    int n0 = 0;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const bool in = umax32(k.k1[r], k.k2[r]) >= T0;
+        const uint64_t cm = __ballot(in);
+        if (in) {
+            const int cl = n0 + __popcll(cm & ((1ull << lane) - 1ull));
+            g_few.child[cl] = r * kWave + lane;
+            g_few.n[cl] = k.n[r];
+            g_few.w[cl] = k.w[r];
+            g_few.p[cl] = k.p[r];
+            g_few.vl[cl] = k.vl[r];
+            if (RAVE) g_few.q2[cl] = k.q2[r];
+        }
+        n0 += __popcll(cm);
+    }
+    wave_sync_memory();
+    if (!few_order<RAVE>(n0, m, c.ep, (uint32_t)a.vl, wave_max_u32(best_key), lane)) return false;
+    close_pending(pending);  // the previous node's partition may still read the order buffer
+    if (lane < m) order[lane] = g_few.order[lane];
+    int base = 0;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const bool in = umax32(k.k1[r], k.k2[r]) >= T0;
+        const uint64_t cm = __ballot(in);
+        cnt[r] = in ? g_few.count[base + __popcll(cm & ((1ull << lane) - 1ull))] : 0;
+        base += __popcll(cm);
+    }
+    wave_sync_memory();
+    return true;
+}
 
 // A wide node (more than 64 child slots) whose visitors split, settled as a narrow one.  Of all its
 // children only those can be chosen whose next entry comes before the entry (lk0, lp0) that the child
@@ -2993,7 +3187,8 @@ struct Continuation {
 // slices, their boundaries and their joins are left out, and with them registers that the rest of the code then has
 // (narrow class 160 -> 145, four rounds 224 -> 216, six 276 -> 245): 64 visitors of a Gomoku tree 104.3 -> 98.9 us a
 // pass, 16 on each of 64 Go trees 124 -> 119, 8 on a tree 70 -> 68.
-template <int R, bool RAVE, int RMAX, bool HEAVY>
+// SPREAD: the kernel for trees that grow on the device, whose nodes have many children without visits (few_visitors).
+template <int R, bool RAVE, int RMAX, bool HEAVY, bool SPREAD>
 __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs &a, const NodeCtx &c, int lane,
                                             const Item &item, const int32_t *seg_in, int32_t *seg_out,
                                             WaveLds<R> &lds, PartLds<RMAX> &pl, bool &pending, Continuation &next,
@@ -3150,10 +3345,19 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
         settled = single_run<R, RAVE>(a, c, lane, k, bk, bpos, soff, m, m >= kRunShareMin, cnt, run_child, contested, best0,
                                       lk0, lp0);
     if (!settled && contested && m >= kSparseMin && !heavy && !odd) {
-        settled = sparse_merge<R, RAVE>(a, c, lane, k, best0, lk0, lp0, m, lds, pl.order, cnt, pending);
+        const int merged =
+            sparse_merge<R, RAVE>(a, c, lane, k, best0, lk0, lp0, m, lds, pl.order, cnt, pending);
+        settled = merged == kMergeDone;
+        if (settled) {
+            if (a.stats && lane == 0) atomicAdd(a.stats + 7, 1);
+        } else if constexpr (SPREAD && R > 1) {
+            if (merged == kMergeMany && m <= kFewMax) {
+                settled = few_visitors<R, RAVE>(a, c, lane, k, bk, best0, m, pl.order, cnt, pending);
+                if (settled && a.stats && lane == 0) atomicAdd(a.stats + 13, 1);
+            }
+        }
         if (settled) {
             lds_cur = 0;
-            if (a.stats && lane == 0) atomicAdd(a.stats + 7, 1);
         } else {
 #pragma unroll
             for (int r = 0; r < R; r++) cnt[r] = 0;
@@ -3801,7 +4005,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
 //
 // A block is a team: its first wavefront (the owner) runs this loop, the other wavefronts
 // wait at a block barrier until the owner shares out the batch work of a node (team_help).
-template <int RMAX, bool RAVE, bool HEAVY>
+template <int RMAX, bool RAVE, bool HEAVY, bool SPREAD>
 __device__ __forceinline__ void owner_loop(const ForestDev &f, const SelectArgs &a, WaveLds<RMAX> &s_lds,
                                            PartLds<RMAX> &s_part, bool &pending, int lane) {
     for (;;) {
@@ -3887,11 +4091,11 @@ __device__ __forceinline__ void owner_loop(const ForestDev &f, const SelectArgs 
             next.chain_open = false;
             if (c.cc > 0 && depth < a.max_depth) {
                 if (c.cc <= kWave)
-                    status = select_group<1, RAVE, RMAX, HEAVY>(f, a, c, lane, it, seg_in, seg_out,
+                    status = select_group<1, RAVE, RMAX, HEAVY, SPREAD>(f, a, c, lane, it, seg_in, seg_out,
                                                          reinterpret_cast<WaveLds<1> &>(s_lds), s_part, pending,
                                                          next, preload_now == 2 ? 2 : 0);
                 else
-                    status = select_group<RMAX, RAVE, RMAX, HEAVY>(f, a, c, lane, it, seg_in, seg_out, s_lds, s_part, pending,
+                    status = select_group<RMAX, RAVE, RMAX, HEAVY, SPREAD>(f, a, c, lane, it, seg_in, seg_out, s_lds, s_part, pending,
                                                             next, preload_now);
             }
             if (a.trace && lane == 0) {
@@ -4074,7 +4278,7 @@ __device__ __forceinline__ void team_help(const ForestDev &f, const SelectArgs &
 template <int RMAX, bool RAVE>
 __device__ void walkers_loop(ForestDev f, SelectArgs a, int lane);
 
-template <int RMAX, bool RAVE, bool HEAVY>
+template <int RMAX, bool RAVE, bool HEAVY, bool SPREAD>
 __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs a) {
     __shared__ WaveLds<RMAX> s_lds;
     __shared__ PartLds<RMAX> s_part;
@@ -4090,7 +4294,7 @@ __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs
     if (tid < kWave) {
         // every path out of the owner's loop comes back here: the helpers are always released
         bool pending = false;
-        owner_loop<RMAX, RAVE, HEAVY>(f, a, s_lds, s_part, pending, tid);
+        owner_loop<RMAX, RAVE, HEAVY, SPREAD>(f, a, s_lds, s_part, pending, tid);
         close_pending(pending);
         if (tid == 0) atomicMax(a.times + 1, (int)(wall_clock64() & 0x7FFFFFFF));
         if (tid == 0) s_lds.cmd.op = kOpExit;
@@ -4442,7 +4646,7 @@ __device__ __noinline__ void walkers_loop(ForestDev f, SelectArgs a, int lane) {
 
 template <int RMAX, bool RAVE>
 hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_items0, int most_visitors,
-                                 int n_traversals, int n_cus, hipStream_t s) {
+                                 int n_traversals, int n_cus, bool grown, hipStream_t s) {
     // Few walkers cannot keep the memory system busy: then the variant that spends bytes to save
     // dependent trips (select_single, FAST).  The number of lone visitors is only known on the
     // device; the number of traversals bounds it.  Measured: it pays on a board layout (legal
@@ -4471,10 +4675,13 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_i
         SelectArgs a = a0;
         a.n_team_blocks = teams;
         a.fast_singles = fast ? 1 : 0;
+        const dim3 grid(teams + walkers), block(kTeam);
         if (most_visitors >= kHeavyMin)
-            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, true>), dim3(teams + walkers), dim3(kTeam), 0, s, f, a);
+            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, true, false>), grid, block, 0, s, f, a);
+        else if (RMAX > 1 && grown)
+            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, false, (RMAX > 1)>), grid, block, 0, s, f, a);
         else
-            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, false>), dim3(teams + walkers), dim3(kTeam), 0, s, f, a);
+            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, false, false>), grid, block, 0, s, f, a);
         return hipGetLastError();
     }
     // every traversal is alone at its root: the walkers are the host's list

@@ -2,6 +2,8 @@
 #include "omk_select_kernels.h"
 
 namespace omk {
-template hipError_t launch_select_class<1, false>(const ForestDev &, const SelectArgs &, int, int, int, int, hipStream_t);
-template hipError_t launch_select_class<1, true>(const ForestDev &, const SelectArgs &, int, int, int, int, hipStream_t);
+template hipError_t launch_select_class<1, false>(const ForestDev &, const SelectArgs &, int, int, int, int, bool,
+                                                      hipStream_t);
+template hipError_t launch_select_class<1, true>(const ForestDev &, const SelectArgs &, int, int, int, int, bool,
+                                                      hipStream_t);
 }  // namespace omk

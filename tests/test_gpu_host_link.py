@@ -194,3 +194,44 @@ def test_compaction_of_every_shape(shape, static):
     for k in ("N", "W", "P", "VL", "rN", "rW", "action"):
         assert got[k].tobytes() == soa[k][order].tobytes(), k
     assert (got["child_begin"] == ref.child_begin).all() and (got["child_count"] == ref.child_count).all()
+
+
+# a young tree: the visitors spread over children without visits (up to 64 of them, one entry per lane)
+@pytest.mark.parametrize("children", [65, 130, 225, 362, 700])
+@pytest.mark.parametrize("n", [8, 23, 63, 64, 65])
+@pytest.mark.parametrize("rave", [False, True])
+def test_visitors_spread_over_a_fresh_node(children, n, rave):
+    import omoknuni_small_amd as omk
+    soa = dict(N=np.zeros(1, np.int32), W=np.zeros(1, np.float32), P=np.ones(1, np.float32), VL=np.zeros(1, np.int32),
+               child_begin=np.zeros(1, np.int32), child_count=np.zeros(1, np.int32), action=np.full(1, -1, np.int32))
+    if rave:
+        soa.update(rN=np.zeros(1, np.int32), rW=np.zeros(1, np.float32))
+    ref = R.RefTree.from_soa(soa)
+    f = omk.Forest.from_soa(soa, capacity=1 + children * (1 + 3 * n))
+    b = omk.Batch(f, n, 6)
+    b.enable_stats()
+    rng = np.random.default_rng(children + n)
+    spread = 0
+    for step in range(4):
+        k = 1 if step == 0 else n
+        roots = np.zeros(k, np.int32)
+        rpaths, rlen, rleaf, _ = ref.select_batch(roots, R.make_params(c_puct=1.4, virtual_loss=3, use_rave=rave, rave_k=1000.0,
+                                                                       max_depth=6))
+        b.set_roots(roots)
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3, use_rave=rave, rave_k=1000.0))
+        paths, plen, leaf, _ = b.read()
+        assert (paths == rpaths).all() and (plen == rlen).all() and (leaf == rleaf).all(), step
+        spread += b.stats()["spread_nodes"]
+        begin = (np.arange(k + 1) * children).astype(np.int32)
+        moves = np.tile(np.arange(children, dtype=np.int32), k)
+        policy = rng.random((k, children)).astype(np.float32)
+        policy = np.round(policy * 50) / 50 if step == 2 else policy  # ties
+        ref.expand_batch(rleaf, begin, moves, policy=policy, action_space=children)
+        b.expand(begin, moves, policy=policy.astype(np.float32), action_space=children)
+        values = (rng.integers(-64, 65, k) / 64.0).astype(np.float32)
+        ref.backup_batch(rpaths, rlen, values, 3)
+        b.set_values(values)
+        b.backup(3)
+    assert (f.download()["N"] == ref.N).all()
+    if not rave and n in (23, 63, 64):
+        assert spread > 0
