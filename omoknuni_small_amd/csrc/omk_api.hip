@@ -1371,6 +1371,9 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
     return OMK_OK;
 }
 
+// Every traversal has a root of its own, and the trees are disjoint (a redirected forest's are not).
+static bool alone(const omk_batch *b) { return b->n_items0 == 0 && !b->f->redirected; }
+
 int omk_backup_batch(omk_batch *b, int32_t virtual_loss) {
     if (!b) return fail(OMK_ERR_INVALID, "omk_backup_batch: null batch");
     if (!b->selected) return fail(OMK_ERR_STATE, "omk_backup_batch: no selected paths");
@@ -1378,7 +1381,7 @@ int omk_backup_batch(omk_batch *b, int32_t virtual_loss) {
     if (int rc = use_device(b->f)) return rc;
     b->f->changes++;
     HIP_TRY(launch_backup(b->f->dev(), b->paths, b->path_len, b->values, b->n, b->stride, b->max_depth + 1,
-                          virtual_loss, b->f->stream));
+                          virtual_loss, alone(b), b->f->stream));
     // N and W of the nodes on the paths have changed: their RAVE blend with them
     if (b->f->has_rave && b->f->blend_valid)
         HIP_TRY(launch_blend_paths(b->f->dev(), b->paths, b->path_len, b->n, b->stride, b->max_depth + 1, b->f->blend_k,
@@ -1405,7 +1408,7 @@ int omk_revert_vl(omk_batch *b, int32_t virtual_loss) {
     if (int rc = fresh_batch("omk_revert_vl", b)) return rc;
     if (int rc = use_device(b->f)) return rc;
     HIP_TRY(launch_revert_vl(b->f->dev(), b->paths, b->path_len, b->n, b->stride, b->max_depth + 1, virtual_loss,
-                             b->f->stream));
+                             alone(b), b->f->stream));
     return OMK_OK;
 }
 
@@ -1428,7 +1431,7 @@ int omk_apply_vl_paths(omk_forest *f, const int32_t *d_paths, const int32_t *d_p
 int omk_revert_vl_paths(omk_forest *f, const int32_t *d_paths, const int32_t *d_path_len, int32_t n, int32_t stride,
                         int32_t max_len, int32_t virtual_loss) {
     if (int rc = check_paths_args("omk_revert_vl_paths", f, d_paths, d_path_len, n, stride, max_len)) return rc;
-    HIP_TRY(launch_revert_vl(f->dev(), d_paths, d_path_len, n, stride, max_len, virtual_loss, f->stream));
+    HIP_TRY(launch_revert_vl(f->dev(), d_paths, d_path_len, n, stride, max_len, virtual_loss, false, f->stream));
     return OMK_OK;
 }
 
@@ -1437,7 +1440,7 @@ int omk_backup_paths(omk_forest *f, const int32_t *d_paths, const int32_t *d_pat
     if (int rc = check_paths_args("omk_backup_paths", f, d_paths, d_path_len, n, stride, max_len)) return rc;
     if (!d_values) return fail(OMK_ERR_INVALID, "omk_backup_paths: null values");
     f->changes++;
-    HIP_TRY(launch_backup(f->dev(), d_paths, d_path_len, d_values, n, stride, max_len, virtual_loss, f->stream));
+    HIP_TRY(launch_backup(f->dev(), d_paths, d_path_len, d_values, n, stride, max_len, virtual_loss, false, f->stream));
     if (f->has_rave && f->blend_valid)
         HIP_TRY(launch_blend_paths(f->dev(), d_paths, d_path_len, n, stride, max_len, f->blend_k, f->stream));
     return OMK_OK;

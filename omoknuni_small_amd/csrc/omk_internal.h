@@ -130,10 +130,11 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a, int n_it
 
 hipError_t launch_apply_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                            int max_len, int vl, hipStream_t s);
+// alone: no two of the paths share a node (every traversal has a root of its own)
 hipError_t launch_revert_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
-                            int max_len, int vl, hipStream_t s);
+                            int max_len, int vl, bool alone, hipStream_t s);
 hipError_t launch_backup(const ForestDev &f, const int32_t *paths, const int32_t *path_len, const float *values,
-                         int n, int stride, int max_len, int vl, hipStream_t s);
+                         int n, int stride, int max_len, int vl, bool alone, hipStream_t s);
 // The per-node RAVE blend f.q2 from the node's statistics as they are: of every node, or of the nodes on the
 // paths given (after a backup has changed their N and W).
 hipError_t launch_blend_all(const ForestDev &f, float rave_k, hipStream_t s);

@@ -235,3 +235,33 @@ def test_visitors_spread_over_a_fresh_node(children, n, rave):
     assert (f.download()["N"] == ref.N).all()
     if not rave and n in (23, 63, 64):
         assert spread > 0
+
+
+# settling a batch: 256 traversals share a table of their nodes; with a root each nothing is atomic
+@pytest.mark.parametrize("n,n_roots", [(1, 1), (255, 1), (257, 3), (40, 40), (300, 300)])
+@pytest.mark.parametrize("vl", [3, 0])
+@pytest.mark.parametrize("how", ["backup", "revert"])
+def test_settling_a_batch(n, n_roots, vl, how):
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(n, n_expand=3 * n_roots + 20, fanout=(1, 6), max_depth=6, n_roots=n_roots, vl_frac=0.4)
+    troots = roots[np.arange(n) % n_roots]
+    ref = R.RefTree.from_soa(soa)
+    f = omk.Forest.from_soa(soa)
+    b = omk.Batch(f, n, 7)
+    b.set_roots(troots)
+    values = (np.random.default_rng(n).integers(-64, 65, n) / 64.0).astype(np.float32)
+    b.set_values(values)
+    for _ in range(2):
+        rpaths, rlen, _, _ = ref.select_batch(troots, R.make_params(c_puct=1.4, virtual_loss=vl, max_depth=7))
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=vl))
+        if how == "backup":
+            ref.backup_batch(rpaths, rlen, values, vl)
+            b.backup(vl)
+        else:
+            ref.revert_vl_paths(rpaths, rlen, vl)
+            b.revert_vl(vl)
+        got = f.download()
+        assert (got["N"] == ref.N).all() and (got["VL"] == ref.VL).all()
+        err = np.abs(got["W"].astype(np.float64) - ref.W) / np.maximum(np.abs(ref.W), 1.0)
+        assert err.max() <= 1e-5
+        ref.W[:] = got["W"]
