@@ -154,6 +154,7 @@ struct omk_batch {
     int32_t spin_limit = 1 << 18;  // polls of about a microsecond: a quarter of a second, a selection takes a millisecond
     int32_t n_cus = 0;
     int32_t n_items0 = 0;
+    int32_t prepared = 0;        // number of the call that omk_batch_set_roots has made the reset for (0: none)
     int32_t *out = nullptr;  // the leaf gather in pinned memory (see gather)
     size_t out_bytes = 0;
     ExportOut gathered = {};      // its parts
@@ -1165,6 +1166,58 @@ static void order_by_root(const int32_t *roots, int32_t n, std::vector<int32_t> 
         for (int32_t t = 0; t < n; t++) start[((roots[t] >> shift) & 2047) + 1]++;
         for (int i = 0; i < 2048; i++) start[i + 1] += start[i];
         for (int32_t i = 0; i < n; i++) tmp[(size_t)start[(roots[order[(size_t)i]] >> shift) & 2047]++] = order[(size_t)i];
+// What a selection of the batch with call number `epoch` is told, the caller's parameters apart.
+static SelectArgs select_args(omk_batch *b, int32_t epoch) {
+    SelectArgs a;
+    memset(&a, 0, sizeof(a));
+    a.items0 = b->items0;
+    a.seg0 = b->seg0;
+    a.items_q = b->items_q;
+    a.seg[0] = b->seg[0];
+    a.seg[1] = b->seg[1];
+    a.q_ready = b->q_ready;
+    a.q_cap = b->q_cap;
+    a.epoch = epoch;
+    a.spin_limit = b->spin_limit;
+    a.truncated = b->counters + kTruncatedWord + (epoch & 1);
+    a.truncated_next = b->counters + kTruncatedWord + ((epoch + 1) & 1);
+    a.stats = b->stats_on ? b->counters + 1 : nullptr;
+    a.n_singles = b->counters + 17;
+    a.sched_head = b->counters + 1 * kSchedStep;
+    a.sched_tail = b->counters + 2 * kSchedStep;
+    a.sched_wait = b->counters + 3 * kSchedStep;
+    a.singles_head = b->counters + 4 * kSchedStep;
+    a.single_ready = b->single_ready;
+    a.n_trav = b->n;
+    a.n_team_blocks = 0;
+    a.fast_singles = 0;
+    // A waiting wavefront sleeps about a microsecond between two polls, so that hundreds of them leave the memory
+    // system to those that work.  A small batch has few wavefronts waiting and a short chain of crowded nodes, every
+    // hand-over of which pays that sleep: they poll without it (measured on 64 traversals: 0.095 -> 0.092 ms; on
+    // 4096, with the sleep off: 0.216 -> 0.221).
+    a.poll_sleep = b->n <= 256 ? 0 : b->poll_sleep;
+    a.hctx = b->hctx;
+    a.hbound = b->hbound;
+    a.hctx_n = b->counters + 2 * kSchedStep + 64;
+    a.hctx_cap = b->hctx_cap;
+    a.list_flag = b->list_flag;
+    static_assert(kHeavyCtxInts >= 16 + OMK_MAX_FANOUT, "context too small");
+    a.times = b->counters + 26;
+    a.trace = b->trace_on ? b->trace : nullptr;
+    a.trace_n = b->counters + 24;
+    a.trace_cap = kTraceCap;
+    a.singles0 = b->singles0;
+    a.singles_q = b->singles_q;
+    a.sc_child = b->sc_child;
+    a.sc_occ = b->sc_occ;
+    a.paths = b->paths;
+    a.path_len = b->path_len;
+    a.leaf = b->leaf;
+    a.stride = b->stride;
+    a.max_depth = b->max_depth;
+    return a;
+}
+
         order.swap(tmp);
         if (shift == 22) break;
     }
@@ -1242,8 +1295,12 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) {
     if (!items.empty()) memcpy(at + 2 * (size_t)n, items.data(), items.size() * sizeof(Item));
     if (!singles.empty())
         memcpy(at + 2 * (size_t)n + items.size() * (sizeof(Item) / 4), singles.data(), singles.size() * sizeof(Item));
-    HIP_TRY(launch_set_roots(b->seg0, b->paths, b->items0, b->singles0, at, n, (int)items.size(), (int)singles.size(),
-                             f->stream));
+    // The next selection's reset comes along (k_set_roots), unless its call number starts over or, with every
+    // traversal alone at its root, it needs none (launch_select).
+    const int32_t next = !items.empty() && b->epoch < (1 << 30) - 2 ? b->epoch + 1 : 0;
+    HIP_TRY(launch_set_roots(select_args(b, next), b->seg0, b->items0, b->singles0, at, n, (int)items.size(),
+                             (int)singles.size(), n_hctx0, next > 0, f->stream));
+    b->prepared = next;
     b->most_visitors = items.empty() ? 1 : items[0].m;
     b->n_items0 = (int32_t)items.size();
     b->n_hctx0 = n_hctx0;
@@ -1312,60 +1369,14 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
         f->blend_valid = f->blend_k_known = true;
         f->blend_k = p->rave_k;
     }
-    SelectArgs a;
-    memset(&a, 0, sizeof(a));
-    a.items0 = b->items0;
-    a.seg0 = b->seg0;
-    a.items_q = b->items_q;
-    a.seg[0] = b->seg[0];
-    a.seg[1] = b->seg[1];
     if (int rc = next_epoch(b)) return rc;
-    a.q_ready = b->q_ready;
-    a.q_cap = b->q_cap;
-    a.epoch = b->epoch;
-    a.spin_limit = b->spin_limit;
-    a.truncated = b->counters + kTruncatedWord + (b->epoch & 1);
-    a.truncated_next = b->counters + kTruncatedWord + ((b->epoch + 1) & 1);
-    a.stats = b->stats_on ? b->counters + 1 : nullptr;
-    a.n_singles = b->counters + 17;
-    a.sched_head = b->counters + 1 * kSchedStep;
-    a.sched_tail = b->counters + 2 * kSchedStep;
-    a.sched_wait = b->counters + 3 * kSchedStep;
-    a.singles_head = b->counters + 4 * kSchedStep;
-    a.single_ready = b->single_ready;
-    a.n_trav = b->n;
-    a.n_team_blocks = 0;
-    a.fast_singles = 0;
-    // A waiting wavefront sleeps about a microsecond between two polls, so that hundreds of them leave the memory
-    // system to those that work.  A small batch has few wavefronts waiting and a short chain of crowded nodes, every
-    // hand-over of which pays that sleep: they poll without it (measured on 64 traversals: 0.095 -> 0.092 ms; on
-    // 4096, with the sleep off: 0.216 -> 0.221).
-    a.poll_sleep = b->n <= 256 ? 0 : b->poll_sleep;
-    a.hctx = b->hctx;
-    a.hbound = b->hbound;
-    a.hctx_n = b->counters + 2 * kSchedStep + 64;
-    a.hctx_cap = b->hctx_cap;
-    a.list_flag = b->list_flag;
-    static_assert(kHeavyCtxInts >= 16 + OMK_MAX_FANOUT, "context too small");
-    a.times = b->counters + 26;
-    a.trace = b->trace_on ? b->trace : nullptr;
-    a.trace_n = b->counters + 24;
-    a.trace_cap = kTraceCap;
-    a.singles0 = b->singles0;
-    a.singles_q = b->singles_q;
-    a.sc_child = b->sc_child;
-    a.sc_occ = b->sc_occ;
-    a.paths = b->paths;
-    a.path_len = b->path_len;
-    a.leaf = b->leaf;
-    a.stride = b->stride;
-    a.max_depth = b->max_depth;
+    SelectArgs a = select_args(b, b->epoch);
     a.vl = p->virtual_loss;
     a.pw = p->pw;
     a.c_puct = p->c_puct;
     a.rave_k = p->rave_k;
-    HIP_TRY(launch_select(f->dev(), a, b->n_items0, b->n_singles0, b->n, b->most_visitors, f->max_fanout, p->use_rave != 0, f->grown, b->n_cus,
-                          b->n_hctx0, f->stream));
+    HIP_TRY(launch_select(f->dev(), a, b->n_items0, b->n_singles0, b->n, b->most_visitors, f->max_fanout, p->use_rave != 0,
+                          f->grown, b->n_cus, b->n_hctx0, b->prepared == b->epoch, f->stream));
     b->selected = true;
     b->select_calls++;
     return OMK_OK;

@@ -187,28 +187,6 @@ __global__ __launch_bounds__(256) void k_export(ForestDev f, const int32_t *path
     host_signal(sig.count, sig.flag, sig.seq, gridDim.x * gridDim.y);
 }
 
-// Four arrays from one staging block in pinned memory: a word per thread, so that every read of the host link is in
-// flight at once (three synchronous copies and the wait before them took 51 us, this launch 3 us of the host).
-__global__ __launch_bounds__(256) void k_set_roots(int32_t *seg0, int32_t *paths, int32_t *items0, int32_t *singles0,
-                                                   const int32_t *staged, int n, int item_words, int single_words) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= 2 * n + item_words + single_words) return;
-    const int32_t v = staged[i];
-    if (i < n) seg0[i] = v;
-    else if (i < 2 * n) paths[i - n] = v;
-    else if (i < 2 * n + item_words) items0[i - 2 * n] = v;
-    else singles0[i - 2 * n - item_words] = v;
-}
-
-hipError_t launch_set_roots(int32_t *seg0, int32_t *paths, Item *items0, Item *singles0, const int32_t *staged, int n,
-                            int n_items, int n_singles, hipStream_t s) {
-    const int iw = n_items * (int)(sizeof(Item) / 4), sw = n_singles * (int)(sizeof(Item) / 4);
-    const int64_t words = 2ll * n + iw + sw;
-    hipLaunchKernelGGL(k_set_roots, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, seg0, paths, (int32_t *)items0,
-                       (int32_t *)singles0, staged, n, iw, sw);
-    return hipGetLastError();
-}
-
 // ---- position keys of the selected leaves: GomokuState::compute_hash_signature_internal
 // (src/games/gomoku/gomoku_state.cpp:947-957) over the tables of utils::ZobristHash
 // (src/utils/zobrist_hash.cpp:9-36), for the state the traversal loop rebuilds by replaying its

@@ -114,14 +114,16 @@ struct SelectArgs {
     float rave_k;
 };
 
-// most_visitors: traversals of the most crowded root; grown: the forest has been expanded since it was uploaded
+// most_visitors: traversals of the most crowded root; grown: the forest has been expanded since it was uploaded;
+// prepared: launch_set_roots has made the reset
 hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, int n_singles0, int n_traversals,
                          int most_visitors, int max_fanout, bool rave, bool grown, int n_cus, int n_hctx0,
-                         hipStream_t s);
+                         bool prepared, hipStream_t s);
 
 // What omk_batch_set_roots has staged (n visitors | n roots | items | lone traversals) to the batch's arrays.
-hipError_t launch_set_roots(int32_t *seg0, int32_t *paths, Item *items0, Item *singles0, const int32_t *staged, int n,
-                            int n_items, int n_singles, hipStream_t s);
+// prepare: and what launch_select's reset does for the selection that `a` belongs to.
+hipError_t launch_set_roots(const SelectArgs &a, int32_t *seg0, Item *items0, Item *singles0, const int32_t *staged,
+                            int n, int n_items, int n_singles, int n_hctx0, bool prepare, hipStream_t s);
 
 // The kernels of one fan-out class (rounds of 64 children: 1, 4, 6 or 16), behind the reset launch.
 template <int RMAX, bool RAVE>

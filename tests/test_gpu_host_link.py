@@ -265,3 +265,29 @@ def test_settling_a_batch(n, n_roots, vl, how):
         err = np.abs(got["W"].astype(np.float64) - ref.W) / np.maximum(np.abs(ref.W), 1.0)
         assert err.max() <= 1e-5
         ref.W[:] = got["W"]
+
+
+# set_roots makes the next selection's reset; one without new roots, one whose number has been changed since and one
+# with statistics make their own
+@pytest.mark.parametrize("n,n_roots", [(2, 1), (256, 3), (257, 250), (1500, 1)])
+def test_selections_after_set_roots_and_without(n, n_roots):
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(n, n_expand=2 * n_roots + 60, fanout=(1, 6), max_depth=6, n_roots=n_roots)
+    troots = roots[np.arange(n) % n_roots]
+    ref = R.RefTree.from_soa(soa)
+    f = omk.Forest.from_soa(soa)
+    b = omk.Batch(f, n, 7)
+    for step in range(7):
+        rpaths, rlen, _, _ = ref.select_batch(troots, R.make_params(c_puct=1.4, virtual_loss=3, max_depth=7))
+        if step not in (1, 4):
+            b.set_roots(troots)
+        if step == 2:
+            b.debug_set_select_count(1000)
+        if step == 3:
+            b.debug_set_select_count((1 << 30) - 3)
+        b.enable_stats(step == 5)
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+        paths, plen, _, _ = b.read()
+        assert (paths == rpaths).all() and (plen == rlen).all()
+        ref.revert_vl_paths(rpaths, rlen, 3)
+        b.revert_vl(3)
