@@ -180,7 +180,7 @@ int omk_backup_paths(omk_forest *f, const int32_t *d_paths, const int32_t *d_pat
  * uniform 1/children when it is not positive) and sets
  * prior = (1 - epsilon) * prior + epsilon * noise, child by child in the reference's
  * order.  n_gamma must be the number of children (legal slots).  A root without children
- * is left alone.  Waits for the stream. */
+ * is left alone.  Waits for the stream unless the omk_expand_batch before gave the root its children. */
 int omk_forest_add_root_noise(omk_forest *f, int32_t root, const float *h_gamma, int32_t n_gamma, float epsilon);
 
 /* The search result's move probabilities (MCTSEngine::getActionProbabilities,

@@ -42,6 +42,8 @@ struct omk_forest {
     bool prior_sorted = false;
     bool grown = false;  // expanded since the last upload: most children have no visits
     int max_fanout = 0;
+    // What the last call changed the structure by, if it was an expansion: node made_node[i] has made_count[i] children
+    std::vector<int32_t> made_node, made_count;
     // Counts the changes that give node ids a new meaning (a compaction, an upload of a different
     // structure): paths, roots and work items of a batch made before such a change are stale.
     int64_t generation = 0;
@@ -606,6 +608,8 @@ int omk_forest_upload(omk_forest *f, const omk_soa_view *v) {
     f->max_fanout = mf;
     f->grown = false;
     f->prior_sorted = sorted;
+    f->made_node.clear();
+    f->made_count.clear();
     f->uploaded = true;
     // the RAVE blend of every node from the new statistics, for the constant the selections have been using
     // (a first selection, or one with another constant, computes it itself)
@@ -780,6 +784,15 @@ int omk_forest_add_root_noise(omk_forest *f, int32_t root, const float *h_gamma,
     if (int rc = tree_only("omk_forest_add_root_noise", f)) return rc;
     if (int rc = use_device(f)) return rc;
     // MCTSEngine::addDirichletNoise from the normalisation on, statement by statement; the mix is the kernel's,
+    // A root that the expansion before this call gave its children (a self-play program expands its roots and then
+    // adds the noise, game by game): their number is known here, and nothing has to be waited for (11 -> 4 us a
+    // root).  The list is short for a program's roots; of a long one only the head is searched.
+    int32_t known = -1;
+    const size_t made = std::min<size_t>(f->made_node.size(), 4096);
+    for (size_t i = 0; i < made && known < 0; i++)
+        if (f->made_node[i] == root) known = f->made_count[i];
+    if (known > 0 && n_gamma != known)
+        return fail(OMK_ERR_INVALID, "omk_forest_add_root_noise: %d samples for %d children", n_gamma, known);
     // child by child in the same arithmetic, and happens only if the samples are as many as the children
     const int32_t given = std::max(0, std::min(n_gamma, (int32_t)OMK_MAX_FANOUT));
     void *staged = nullptr;
@@ -790,7 +803,10 @@ int omk_forest_add_root_noise(omk_forest *f, int32_t root, const float *h_gamma,
     for (int32_t j = 0; j < given; j++) sum = sum + h_gamma[j];
     const float uniform_noise = 1.0f / (float)std::max(given, 1);
     for (int32_t j = 0; j < given; j++) noise[j] = sum > 0.0f ? h_gamma[j] / sum : uniform_noise;
-    HIP_TRY(launch_root_noise(f->mut(), root, noise, n_gamma, epsilon, result, link_signal(f), f->stream));
+    HostSignal sig = {nullptr, nullptr, 0};
+    if (known < 0) sig = link_signal(f);
+    HIP_TRY(launch_root_noise(f->mut(), root, noise, n_gamma, epsilon, result, sig, f->stream));
+    if (known >= 0) return OMK_OK;
     if (int rc = link_wait(f)) return rc;
     const int32_t children = result[0];
     if (children > 0 && n_gamma != children)
@@ -942,6 +958,8 @@ static int compact_in(omk_forest *f, int32_t new_root, int64_t *h_nodes_after, i
     }
     f->n_nodes = k;
     f->changes++;
+    f->made_node.clear();
+    f->made_count.clear();
     f->generation++;
     f->structure_changed = true;
     if (h_nodes_after) *h_nodes_after = k;
@@ -1576,6 +1594,8 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
     int mf = f->max_fanout;
     cursor = f->n_nodes;
     size_t off = 0;
+    f->made_node.clear();
+    f->made_count.clear();
     for (size_t wi = 0; wi < nj; wi++) {
         const int32_t t = winners[wi];
         const int32_t cnt = widened_children(std::min(h_move_begin[t + 1] - h_move_begin[t], 1000), visits[t], params);
@@ -1598,6 +1618,8 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
         }
         for (int32_t i = 1; i < cnt && sorted; i++) sorted = !(pr[i] > pr[i - 1]);
         if (h_first_child) h_first_child[t] = (int32_t)cursor;
+        f->made_node.push_back(leaf[t]);
+        f->made_count.push_back(cnt);
         off += (size_t)cnt;
         cursor += cnt;
         mf = std::max(mf, (int)cnt);

@@ -323,6 +323,7 @@ __global__ __launch_bounds__(1024) void k_root_noise(ForestMut f, int32_t root, 
         const float add = epsilon * noise[rank];
         f.P[id] = keep + add;
     }
+    if (!sig.flag) return;  // the host knows the number of children and does not wait
     if (i == 0) host_store(head, children);
     host_signal(sig.count, sig.flag, sig.seq, 1);
 }

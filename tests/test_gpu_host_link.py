@@ -291,3 +291,38 @@ def test_selections_after_set_roots_and_without(n, n_roots):
         assert (paths == rpaths).all() and (plen == rlen).all()
         ref.revert_vl_paths(rpaths, rlen, 3)
         b.revert_vl(3)
+
+
+# the noise of a root that the expansion before has given its children, of another node, and after an upload
+@pytest.mark.parametrize("moves", [1, 63, 64, 257])
+def test_root_noise_after_an_expansion(moves):
+    import omoknuni_small_amd as omk
+    n = 5
+    zeros = np.zeros(n, np.int32)
+    soa = dict(N=zeros, W=np.zeros(n, np.float32), P=np.ones(n, np.float32), VL=zeros, child_begin=zeros,
+               child_count=zeros, action=zeros - 1)
+    f = omk.Forest.from_soa(soa, capacity=n * (2 * moves + 1))
+    b = omk.Batch(f, n, 4)
+    rng = np.random.default_rng(moves)
+    gamma = rng.gamma(0.3, 1.0, moves).astype(np.float32)
+    total = np.float32(0)
+    for g in gamma:
+        total = total + g
+    noise = gamma / total if total > 0 else np.full(moves, np.float32(1) / np.float32(moves))
+    begin = (np.arange(n + 1) * moves).astype(np.int32)
+    b.set_roots(np.arange(n, dtype=np.int32))
+    for step in range(2):  # the second expansion is that of a child of each root
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+        first = b.expand(begin, np.tile(np.arange(moves, dtype=np.int32), n))
+        b.revert_vl(3)
+        for root in (1, 3):
+            with pytest.raises(omk.OmkError, match="samples"):
+                f.add_root_noise(root, np.append(gamma, gamma[:1]), 0.25)
+            before = f.download()["P"]
+            f.add_root_noise(root, gamma, 0.25)
+            begins = f.download_structure()["child_begin"][root]
+            want = before.copy()
+            mine = slice(begins, begins + moves)
+            want[mine] = (np.float32(1) - np.float32(0.25)) * before[mine] + np.float32(0.25) * noise
+            assert (f.download()["P"] == want).all()
+    assert len(first) == n
