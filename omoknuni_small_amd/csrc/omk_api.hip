@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "omk_internal.h"
+#include "omk_priors.h"
 
 using namespace omk;
 
@@ -41,9 +42,9 @@ struct omk_forest {
     bool uploaded = false;
     bool prior_sorted = false;
     bool grown = false;  // expanded since the last upload: most children have no visits
-    int max_fanout = 0;
     // What the last call changed the structure by, if it was an expansion: node made_node[i] has made_count[i] children
     std::vector<int32_t> made_node, made_count;
+    int max_fanout = 0;
     // Counts the changes that give node ids a new meaning (a compaction, an upload of a different
     // structure): paths, roots and work items of a batch made before such a change are stale.
     int64_t generation = 0;
@@ -153,10 +154,10 @@ struct omk_batch {
     int32_t hctx_cap = 0;
     int32_t q_cap = 0;
     int32_t epoch = 0;           // select calls so far
+    int32_t prepared = 0;        // number of the call that omk_batch_set_roots has made the reset for (0: none)
     int32_t spin_limit = 1 << 18;  // polls of about a microsecond: a quarter of a second, a selection takes a millisecond
     int32_t n_cus = 0;
     int32_t n_items0 = 0;
-    int32_t prepared = 0;        // number of the call that omk_batch_set_roots has made the reset for (0: none)
     int32_t *out = nullptr;  // the leaf gather in pinned memory (see gather)
     size_t out_bytes = 0;
     ExportOut gathered = {};      // its parts
@@ -607,9 +608,9 @@ int omk_forest_upload(omk_forest *f, const omk_soa_view *v) {
     f->n_nodes = n;
     f->max_fanout = mf;
     f->grown = false;
-    f->prior_sorted = sorted;
     f->made_node.clear();
     f->made_count.clear();
+    f->prior_sorted = sorted;
     f->uploaded = true;
     // the RAVE blend of every node from the new statistics, for the constant the selections have been using
     // (a first selection, or one with another constant, computes it itself)
@@ -783,7 +784,6 @@ int omk_forest_add_root_noise(omk_forest *f, int32_t root, const float *h_gamma,
     if (root < 0 || root >= f->n_nodes) return fail(OMK_ERR_INVALID, "omk_forest_add_root_noise: root %d", root);
     if (int rc = tree_only("omk_forest_add_root_noise", f)) return rc;
     if (int rc = use_device(f)) return rc;
-    // MCTSEngine::addDirichletNoise from the normalisation on, statement by statement; the mix is the kernel's,
     // A root that the expansion before this call gave its children (a self-play program expands its roots and then
     // adds the noise, game by game): their number is known here, and nothing has to be waited for (11 -> 4 us a
     // root).  The list is short for a program's roots; of a long one only the head is searched.
@@ -793,6 +793,7 @@ int omk_forest_add_root_noise(omk_forest *f, int32_t root, const float *h_gamma,
         if (f->made_node[i] == root) known = f->made_count[i];
     if (known > 0 && n_gamma != known)
         return fail(OMK_ERR_INVALID, "omk_forest_add_root_noise: %d samples for %d children", n_gamma, known);
+    // MCTSEngine::addDirichletNoise from the normalisation on, statement by statement; the mix is the kernel's,
     // child by child in the same arithmetic, and happens only if the samples are as many as the children
     const int32_t given = std::max(0, std::min(n_gamma, (int32_t)OMK_MAX_FANOUT));
     void *staged = nullptr;
@@ -957,9 +958,9 @@ static int compact_in(omk_forest *f, int32_t new_root, int64_t *h_nodes_after, i
         if (int rc = bulk_get(f, down)) return rc;
     }
     f->n_nodes = k;
-    f->changes++;
     f->made_node.clear();
     f->made_count.clear();
+    f->changes++;
     f->generation++;
     f->structure_changed = true;
     if (h_nodes_after) *h_nodes_after = k;
@@ -1165,25 +1166,6 @@ int omk_batch_destroy(omk_batch *b) {
 
 }  // extern "C"
 
-// The traversals in ascending order of their roots, those of one root in ascending order: what a stable sort
-// gives.  One root for all, and roots that ascend already (one traversal per tree), are in order as they are; else
-// a radix sort, eleven bits a pass, as many passes as the largest root has digits.
-static void order_by_root(const int32_t *roots, int32_t n, std::vector<int32_t> &order, std::vector<int32_t> &tmp) {
-    order.resize((size_t)n);
-    bool ascending = true;
-    int32_t top = 0;
-    for (int32_t t = 0; t < n; t++) {
-        order[(size_t)t] = t;
-        ascending &= t == 0 || roots[t - 1] <= roots[t];
-        top = std::max(top, roots[t]);
-    }
-    if (ascending) return;
-    tmp.resize((size_t)n);
-    for (int shift = 0; shift == 0 || (top >> shift) > 0; shift += 11) {
-        int32_t start[2049] = {0};
-        for (int32_t t = 0; t < n; t++) start[((roots[t] >> shift) & 2047) + 1]++;
-        for (int i = 0; i < 2048; i++) start[i + 1] += start[i];
-        for (int32_t i = 0; i < n; i++) tmp[(size_t)start[(roots[order[(size_t)i]] >> shift) & 2047]++] = order[(size_t)i];
 // What a selection of the batch with call number `epoch` is told, the caller's parameters apart.
 static SelectArgs select_args(omk_batch *b, int32_t epoch) {
     SelectArgs a;
@@ -1236,6 +1218,25 @@ static SelectArgs select_args(omk_batch *b, int32_t epoch) {
     return a;
 }
 
+// The traversals in ascending order of their roots, those of one root in ascending order: what a stable sort
+// gives.  One root for all, and roots that ascend already (one traversal per tree), are in order as they are; else
+// a radix sort, eleven bits a pass, as many passes as the largest root has digits.
+static void order_by_root(const int32_t *roots, int32_t n, std::vector<int32_t> &order, std::vector<int32_t> &tmp) {
+    order.resize((size_t)n);
+    bool ascending = true;
+    int32_t top = 0;
+    for (int32_t t = 0; t < n; t++) {
+        order[(size_t)t] = t;
+        ascending &= t == 0 || roots[t - 1] <= roots[t];
+        top = std::max(top, roots[t]);
+    }
+    if (ascending) return;
+    tmp.resize((size_t)n);
+    for (int shift = 0; shift == 0 || (top >> shift) > 0; shift += 11) {
+        int32_t start[2049] = {0};
+        for (int32_t t = 0; t < n; t++) start[((roots[t] >> shift) & 2047) + 1]++;
+        for (int i = 0; i < 2048; i++) start[i + 1] += start[i];
+        for (int32_t i = 0; i < n; i++) tmp[(size_t)start[(roots[order[(size_t)i]] >> shift) & 2047]++] = order[(size_t)i];
         order.swap(tmp);
         if (shift == 22) break;
     }
@@ -1590,12 +1591,12 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
     ExpandJob *jobs = (ExpandJob *)staged;
     int32_t *moves = (int32_t *)(jobs + nj);
     float *priors = (float *)(moves + nm);
-    bool sorted = true;
+    bool sorted = f->prior_sorted;  // (once they are not, no later child makes it so)
     int mf = f->max_fanout;
     cursor = f->n_nodes;
-    size_t off = 0;
     f->made_node.clear();
     f->made_count.clear();
+    size_t off = 0;
     for (size_t wi = 0; wi < nj; wi++) {
         const int32_t t = winners[wi];
         const int32_t cnt = widened_children(std::min(h_move_begin[t + 1] - h_move_begin[t], 1000), visits[t], params);
@@ -1606,14 +1607,13 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
         jobs[wi] = ExpandJob{leaf[t], (int32_t)cursor, cnt, (int32_t)off};
         const int32_t *mv = h_moves + h_move_begin[t];
         float *pr = priors + off;
-        memcpy(moves + off, mv, (size_t)cnt * 4);
-        if (pol && psize == action_space) {  // a policy over the action space (:537-560)
-            for (int32_t i = 0; i < cnt; i++)
-                pr[i] = mv[i] >= 0 && mv[i] < action_space ? std::min(1.0f, std::max(0.0f, pol[mv[i]]))  // clamp to [0, 1]
-                                                           : 0.01f;  // move outside the action space
+        if (pol && psize == action_space) {  // a policy over the action space (:537-560); the moves along with it
+            gather_priors(mv, cnt, pol, action_space, moves + off, pr);
         } else if (pol && psize == cnt) {  // one value per child, by child index (:561-575)
+            memcpy(moves + off, mv, (size_t)cnt * 4);
             for (int32_t i = 0; i < cnt; i++) pr[i] = std::min(1.0f, std::max(0.0f, pol[i]));
         } else {  // expand(): uniform prior; a policy of neither size likewise (:576-584)
+            memcpy(moves + off, mv, (size_t)cnt * 4);
             for (int32_t i = 0; i < cnt; i++) pr[i] = 1.0f / (float)cnt;
         }
         for (int32_t i = 1; i < cnt && sorted; i++) sorted = !(pr[i] > pr[i - 1]);
@@ -1630,7 +1630,7 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
     f->grown = true;
     f->structure_changed = true;  // ids keep their meaning, but an upload of the old arrays would not
     f->max_fanout = mf;
-    if (!sorted) f->prior_sorted = false;
+    f->prior_sorted = sorted;
     return OMK_OK;
 }
 

@@ -326,3 +326,29 @@ def test_root_noise_after_an_expansion(moves):
             want[mine] = (np.float32(1) - np.float32(0.25)) * before[mine] + np.float32(0.25) * noise
             assert (f.download()["P"] == want).all()
     assert len(first) == n
+
+
+# eight moves at a time and the rest one by one; values that the clamp changes, moves outside the action space
+@pytest.mark.parametrize("moves", list(range(1, 18)) + [225])
+def test_priors_from_a_policy(moves):
+    import omoknuni_small_amd as omk
+    zeros = np.zeros(1, np.int32)
+    soa = dict(N=zeros, W=np.zeros(1, np.float32), P=np.ones(1, np.float32), VL=zeros, child_begin=zeros,
+               child_count=zeros, action=zeros - 1)
+    f = omk.Forest.from_soa(soa, capacity=1 + moves)
+    b = omk.Batch(f, 1, 4)
+    b.set_roots([0])
+    b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+    A = 300
+    rng = np.random.default_rng(moves)
+    policy = (rng.standard_normal(A) * 2).astype(np.float32)
+    policy[rng.integers(0, A, 90)] = np.repeat(np.float32([np.nan, np.inf, -np.inf, -0.0, 1.0, 0.0]), 15)
+    mv = rng.integers(-3, A + 3, moves).astype(np.int32)
+    b.expand_ex([0, moves], mv, [0, A], policy, A)
+    value = policy[np.clip(mv, 0, A - 1)]
+    with np.errstate(invalid="ignore"):
+        want = np.where(value > 0, np.where(value < 1, value, np.float32(1)), np.float32(0))
+    want = np.where((mv >= 0) & (mv < A), want, np.float32(0.01)).astype(np.float32)
+    got = f.download()["P"][1:]
+    assert (got.view(np.int32) == want.view(np.int32)).all()
+    assert (f.download_structure()["action"][1:] == mv).all()
