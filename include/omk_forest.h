@@ -406,6 +406,9 @@ int omk_tt_set_replacement_threshold(omk_tt *tt, float threshold);
  * call, transpositions reported.  Waits for the stream. */
 int omk_tt_traverse(omk_tt *tt, omk_batch *b, const uint64_t *d_piece_keys, int32_t cells, const uint64_t *d_player_keys,
                     const uint64_t *d_root_keys, const int32_t *d_root_players, int32_t *d_hits, int32_t *h_counts);
+/* As omk_tt_traverse, with the hits in host memory (not NULL): they cross with the counts. */
+int omk_tt_traverse_read(omk_tt *tt, omk_batch *b, const uint64_t *d_piece_keys, int32_t cells, const uint64_t *d_player_keys,
+                    const uint64_t *d_root_keys, const int32_t *d_root_players, int32_t *h_hits, int32_t *h_counts);
 /* The whole traversal loop with the table on, redirects INCLUDED (mcts_engine_batch_tree_simple.cpp:88-165;
  * the redirect is :142-156 with MCTSNode::updateChildReference, mcts_node.cpp:617-630): a select for the
  * batch's roots that, at every step, stores the selected child when it has no visits, looks the position

@@ -1904,47 +1904,74 @@ int omk_tt_store(omk_tt *tt, const uint64_t *d_keys, const int32_t *d_nodes, con
     return tt_report("omk_tt_store", status, h_counts);
 }
 
-int omk_tt_traverse(omk_tt *tt, omk_batch *b, const uint64_t *d_piece_keys, int32_t cells, const uint64_t *d_player_keys,
-                    const uint64_t *d_root_keys, const int32_t *d_root_players, int32_t *d_hits, int32_t *h_counts) {
-    if (!tt || !b) return fail(OMK_ERR_INVALID, "omk_tt_traverse: null argument");
-    if (tt->f != b->f) return fail(OMK_ERR_INVALID, "omk_tt_traverse: table and batch belong to different forests");
-    if (!b->selected) return fail(OMK_ERR_STATE, "omk_tt_traverse: no selected paths");
-    if (int rc = fresh_batch("omk_tt_traverse", b)) return rc;
+}  // extern "C"
+
+// The hits to device memory, to the host's, or to neither.  Up to a megabyte crosses with the counters, as one wait
+// (42.5 -> 28.3 us a batch of 500 x 24); more is kept on the device first, where the link's rate counts and not the wait.
+static int tt_traverse_to(const char *who, omk_tt *tt, omk_batch *b, const uint64_t *d_piece_keys, int32_t cells,
+                          const uint64_t *d_player_keys, const uint64_t *d_root_keys, const int32_t *d_root_players,
+                          int32_t *d_hits, int32_t *h_hits, int32_t *h_counts) {
+    if (!tt || !b) return fail(OMK_ERR_INVALID, "%s: null argument", who);
+    if (tt->f != b->f) return fail(OMK_ERR_INVALID, "%s: table and batch belong to different forests", who);
+    if (!b->selected) return fail(OMK_ERR_STATE, "%s: no selected paths", who);
+    if (int rc = fresh_batch(who, b)) return rc;
     omk_forest *f = b->f;
     if (d_piece_keys) {
         if (!d_player_keys || !d_root_keys || !d_root_players || cells <= 0)
-            return fail(OMK_ERR_INVALID, "omk_tt_traverse: the game's key tables need player keys, root keys, root players "
-                        "and cells > 0");
+            return fail(OMK_ERR_INVALID, "%s: the game's key tables need player keys, root keys, root players "
+                        "and cells > 0", who);
     } else if (!f->has_hash) {
-        return fail(OMK_ERR_STATE, "omk_tt_traverse: no key tables given and the forest was uploaded without position keys");
+        return fail(OMK_ERR_STATE, "%s: no key tables given and the forest was uploaded without position keys", who);
     }
     if (int rc = use_device(f)) return rc;
     if (int rc = tt_same_tree(tt)) return rc;
     hipStream_t s = f->stream;
     const int64_t n = (int64_t)b->n * b->max_depth;
-    // work space: slot_of [n] i64 | keys [n] u64 | step_nodes, store_nodes [n] i32 each
-    if (int rc = tt_work(tt, (size_t)n * 24)) return rc;
+    const bool beside = h_hits && n * 4 <= (1 << 20), after = h_hits && !beside;
+    // work space: slot_of [n] i64 | keys [n] u64 | step_nodes, store_nodes, hits (if they cross later) [n] i32 each
+    if (int rc = tt_work(tt, (size_t)n * (after ? 28 : 24))) return rc;
     int64_t *slot_of = (int64_t *)tt->work;
     uint64_t *keys = (uint64_t *)(slot_of + n);
     int32_t *step_nodes = (int32_t *)(keys + n), *store_nodes = step_nodes + n;
+    if (after) d_hits = store_nodes + n;
     void *staged = nullptr;
-    if (int rc = link_stage(f, 32, &staged)) return rc;
+    if (int rc = link_stage(f, 128 + (beside ? (size_t)n * 4 : 0), &staged)) return rc;
+    int32_t *crossing = beside ? (int32_t *)staged + 32 : nullptr;
     const int32_t *status = (const int32_t *)staged;
     // all stores first, then all lookups: a lookup that the serial loop makes before a later step's
     // store can only miss a node without visits, and such a node is no transposition (:142)
     HIP_TRY(launch_tt_traverse(f->dev(), tt->slots, tt->meta, tt->log2_slots, b->paths, b->path_len, b->n, b->stride,
                                b->max_depth, d_piece_keys, cells, d_player_keys, d_root_keys, d_root_players, keys,
-                               step_nodes, store_nodes, slot_of, tt->clock, tt->threshold, d_hits, tt->d_status,
-                               (int32_t *)staged, link_signal(f), s));
+                               step_nodes, store_nodes, slot_of, tt->clock, tt->threshold, d_hits, crossing,
+                               tt->d_status, (int32_t *)staged, link_signal(f), s));
     tt->clock += 2u * (uint32_t)n;  // a time for every store, then one for every lookup
     if (int rc = link_wait(f)) return rc;
     if (status[5])
-        return fail(OMK_ERR_INVALID, "omk_tt_traverse: %d paths hold a node outside the forest or a move outside [0, %d)",
-                    status[5], cells);
+        return fail(OMK_ERR_INVALID, "%s: %d paths hold a node outside the forest or a move outside [0, %d)",
+                    who, status[5], cells);
     int32_t st[8];
     memcpy(st, status, 32);
+    if (beside) memcpy(h_hits, crossing, (size_t)n * 4);
+    if (after)
+        if (int rc = omk_dev_d2h(f, h_hits, d_hits, n * 4)) return rc;
     st[1] = 0;  // steps that do not exist carry the empty marker on purpose
-    return tt_report("omk_tt_traverse", st, h_counts);
+    return tt_report(who, st, h_counts);
+}
+
+extern "C" {
+
+int omk_tt_traverse(omk_tt *tt, omk_batch *b, const uint64_t *d_piece_keys, int32_t cells, const uint64_t *d_player_keys,
+                    const uint64_t *d_root_keys, const int32_t *d_root_players, int32_t *d_hits, int32_t *h_counts) {
+    return tt_traverse_to("omk_tt_traverse", tt, b, d_piece_keys, cells, d_player_keys, d_root_keys, d_root_players,
+                          d_hits, nullptr, h_counts);
+}
+
+int omk_tt_traverse_read(omk_tt *tt, omk_batch *b, const uint64_t *d_piece_keys, int32_t cells,
+                         const uint64_t *d_player_keys, const uint64_t *d_root_keys, const int32_t *d_root_players,
+                         int32_t *h_hits, int32_t *h_counts) {
+    if (!h_hits) return fail(OMK_ERR_INVALID, "omk_tt_traverse_read: null argument");
+    return tt_traverse_to("omk_tt_traverse_read", tt, b, d_piece_keys, cells, d_player_keys, d_root_keys, d_root_players,
+                          nullptr, h_hits, h_counts);
 }
 
 int omk_tt_select_redirect(omk_tt *tt, omk_batch *b, const omk_select_params *p, int32_t *d_moves, int32_t *h_counts) {

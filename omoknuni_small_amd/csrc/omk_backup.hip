@@ -751,7 +751,7 @@ __device__ __forceinline__ int tt_lookup(const TTSlot *slots, int log2_slots, un
         unsigned long long todo = __ballot(hit_slot != ~0ull);
         while (todo) {
             const int lead = __ffsll((long long)todo) - 1;
-            const unsigned long long s0 = __shfl(hit_slot, lead);
+            const unsigned long long s0 = (uint32_t)__builtin_amdgcn_readlane((int)hit_slot, lead);  // (below 2^31)
             const unsigned long long same = __ballot(hit_slot == s0);
             if (lane == 63u - (unsigned)__clzll((long long)same)) atomicMax(&meta[s0].last_access, time);
             todo &= ~same;
@@ -765,8 +765,8 @@ __device__ __forceinline__ int tt_lookup(const TTSlot *slots, int log2_slots, un
 // withdrawn on the way (pass 3), and the counters go to the host with the last block.
 __global__ __launch_bounds__(256) void k_tt_hits(ForestDev f, const TTSlot *slots, TTMeta *meta, int log2_slots,
                                                  const uint64_t *keys, const int32_t *step_nodes, const int64_t *slot_of,
-                                                 int64_t n, uint32_t t0, int32_t *hit, int *d_status, int32_t *h_status,
-                                                 HostSignal sig) {
+                                                 int64_t n, uint32_t t0, int32_t *hit, int32_t *h_hit, int *d_status,
+                                                 int32_t *h_status, HostSignal sig) {
     int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool valid = i < n;
     const int node = valid ? step_nodes[i] : -1;
@@ -775,29 +775,33 @@ __global__ __launch_bounds__(256) void k_tt_hits(ForestDev f, const TTSlot *slot
     if (node >= 0 && fn >= 0 && fn != node && fn < f.n_nodes && f.N[fn] > 0) out = fn;
     if (valid) {
         if (hit) hit[i] = out;  // a caller that only wants the count passes no array
+        if (h_hit) host_store(h_hit + i, out);
         const int64_t s = slot_of[i];
         if (s >= 0) meta[s].claim = 0x7FFFFFFF;
     }
     const uint64_t any = __ballot(out >= 0);
     if (any && (threadIdx.x & 63) == 0) atomicAdd(d_status + 6, __popcll(any));
-    // host_signal with the counters before the flag
+    // host_signal with the counters before the flag: eight lanes take them, one round trip instead of eight
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x != 0) return;
-    if (__hip_atomic_fetch_add(sig.count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (int)gridDim.x - 1) return;
-    __hip_atomic_store(sig.count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int q = 0; q < 8; q++)
-        host_store(h_status + q, __hip_atomic_exchange(d_status + q, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (threadIdx.x >= 64) return;
+    int before = 0;
+    if (threadIdx.x == 0) before = __hip_atomic_fetch_add(sig.count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(before) != (int)gridDim.x - 1) return;
+    if (threadIdx.x == 0) __hip_atomic_store(sig.count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x < 8)
+        host_store(h_status + threadIdx.x,
+                   __hip_atomic_exchange(d_status + threadIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    host_store(sig.flag, sig.seq);
+    if (threadIdx.x == 0) host_store(sig.flag, sig.seq);
 }
 
 hipError_t launch_tt_traverse(const ForestDev &f, TTSlot *slots, TTMeta *meta, int log2_slots, const int32_t *paths,
                               const int32_t *path_len, int n, int stride, int max_depth, const uint64_t *piece, int cells,
                               const uint64_t *player, const uint64_t *root_key, const int32_t *root_player,
                               uint64_t *keys, int32_t *step_nodes, int32_t *store_nodes, int64_t *slot_of, uint32_t t0,
-                              float threshold, int32_t *hit, int *d_status, int32_t *h_status, const HostSignal &sig,
-                              hipStream_t s) {
+                              float threshold, int32_t *hit, int32_t *h_hit, int *d_status, int32_t *h_status,
+                              const HostSignal &sig, hipStream_t s) {
     const int64_t steps = (int64_t)n * max_depth;
     const dim3 grid((unsigned)((steps + 255) / 256)), block(256);
     if (piece) {
@@ -812,7 +816,7 @@ hipError_t launch_tt_traverse(const ForestDev &f, TTSlot *slots, TTMeta *meta, i
     hipLaunchKernelGGL(k_tt_store_apply, grid, block, 0, s, f, slots, meta, store_nodes, (const int32_t *)nullptr,
                        max_depth, steps, slot_of, t0, threshold, d_status);
     hipLaunchKernelGGL(k_tt_hits, grid, block, 0, s, f, slots, meta, log2_slots, keys, step_nodes, slot_of, steps,
-                       t0 + (uint32_t)steps, hit, d_status, h_status, sig);
+                       t0 + (uint32_t)steps, hit, h_hit, d_status, h_status, sig);
     return hipGetLastError();
 }
 

@@ -269,13 +269,13 @@ hipError_t launch_tt_store(const ForestDev &f, TTSlot *slots, TTMeta *meta, int 
                            const int32_t *nodes, const int32_t *depths, int64_t n, int64_t *slot_of, uint32_t t0,
                            float threshold, int *d_status, hipStream_t s);
 // The table's part of the traversal over selected paths: all stores, then all lookups.  The eight counters end up in
-// `h_status` (pinned) and are zero again; hits as in omk_tt_traverse.
+// `h_status` (pinned) and are zero again; hits as in omk_tt_traverse, h_hit (pinned) likewise, either may be NULL.
 hipError_t launch_tt_traverse(const ForestDev &f, TTSlot *slots, TTMeta *meta, int log2_slots, const int32_t *paths,
                               const int32_t *path_len, int n, int stride, int max_depth, const uint64_t *piece, int cells,
                               const uint64_t *player, const uint64_t *root_key, const int32_t *root_player,
                               uint64_t *keys, int32_t *step_nodes, int32_t *store_nodes, int64_t *slot_of, uint32_t t0,
-                              float threshold, int32_t *hit, int *d_status, int32_t *h_status, const HostSignal &sig,
-                              hipStream_t s);
+                              float threshold, int32_t *hit, int32_t *h_hit, int *d_status, int32_t *h_status,
+                              const HostSignal &sig, hipStream_t s);
 // The traversal loop with the table on, redirects included, one traversal after the other (omk_backup.hip).
 struct RedirectArgs {
     int32_t *alias;

@@ -28,7 +28,7 @@ EXPORTS = [
     "omk_batch_set_roots", "omk_batch_set_values", "omk_batch_device", "omk_select_batch", "omk_backup_batch",
     "omk_revert_vl", "omk_backup_rave_batch", "omk_apply_vl_paths", "omk_revert_vl_paths", "omk_backup_paths", "omk_batch_read",
     "omk_batch_leaf_keys", "omk_debug_trace", "omk_batch_set_trace", "omk_batch_truncated", "omk_batch_stats", "omk_batch_set_stats", "omk_batch_set_spin_limit", "omk_debug_set_select_count", "omk_tt_create", "omk_tt_destroy", "omk_tt_clear", "omk_tt_insert", "omk_tt_probe",
-    "omk_tt_probe_leaves", "omk_tt_store", "omk_tt_set_replacement_threshold", "omk_tt_traverse", "omk_tt_select_redirect", "omk_forest_download_redirects", "omk_tt_download_meta", "omk_tt_upload", "omk_tt_download", "omk_dev_alloc", "omk_dev_free", "omk_dev_h2d",
+    "omk_tt_probe_leaves", "omk_tt_store", "omk_tt_set_replacement_threshold", "omk_tt_traverse", "omk_tt_traverse_read", "omk_tt_select_redirect", "omk_forest_download_redirects", "omk_tt_download_meta", "omk_tt_upload", "omk_tt_download", "omk_dev_alloc", "omk_dev_free", "omk_dev_h2d",
     "omk_dev_d2h", "omk_dev_copy", "omk_soa_count_legal", "omk_soa_compact_legal",
 ]
 
@@ -122,7 +122,7 @@ _EVERY_BATCH = {
     "omk_batch_read": (_VP, _VP, _VP, _VP, _VP), "omk_expand_batch_ex": (_VP, _VP, _VP, _VP, _VP, _VP, _VP),
     "omk_forest_set_keys": (_VP, _VP, _VP, _I64), "omk_forest_action_probabilities": (_VP, _I32, _F32, _I32, _VP, _VP),
     "omk_forest_add_root_noise": (_VP, _I32, _VP, _I32, _F32), "omk_forest_node_count": (_VP, _VP, _VP),
-    "omk_tt_probe_leaves": (_VP, _VP, _I32, _VP),
+    "omk_tt_probe_leaves": (_VP, _VP, _I32, _VP), "omk_tt_traverse_read": (_VP, _VP, _VP, _I32, _VP, _VP, _VP, _VP, _VP),
 }
 
 
@@ -182,7 +182,6 @@ class Forest:
         self._h = C.c_void_p()
         self.has_rave = bool(has_rave)
         self.n_nodes = 0
-        self._kept = set()  # device buffers that tables keep between calls: freed with the table, or with the forest
         desc = _ForestDesc(int(capacity_nodes), int(device), int(self.has_rave))
         _check(self._lib.omk_forest_create(C.byref(desc), C.byref(self._h)))
 
@@ -195,9 +194,6 @@ class Forest:
 
     def close(self):
         if self._h:
-            for p in self._kept:
-                self.dev_free(p)
-            self._kept = set()
             self._lib.omk_forest_destroy(self._h)
             self._h = C.c_void_p()
 
@@ -514,12 +510,10 @@ class TranspositionTable:
         self.forest = forest
         self.log2 = int(log2_slots)
         self._h = C.c_void_p()
-        self._hits, self._hits_bytes = 0, 0  # device buffer of traverse()
         _check(self._lib.omk_tt_create(forest._h, self.log2, C.byref(self._h)))
 
     def close(self):
         if self._h:
-            self._drop_hits()
             self._lib.omk_tt_destroy(self._h)
             self._h = C.c_void_p()
 
@@ -528,12 +522,6 @@ class TranspositionTable:
             self.close()
         except Exception:
             pass
-
-    def _drop_hits(self):
-        if self._hits in self.forest._kept:
-            self.forest._kept.remove(self._hits)
-            self.forest.dev_free(self._hits)
-        self._hits, self._hits_bytes = 0, 0
 
     def clear(self):
         _check(self._lib.omk_tt_clear(self._h))
@@ -627,11 +615,7 @@ class TranspositionTable:
         f = self.forest
         n, D = batch.n, batch.max_depth
         hits = np.empty((n, D), np.int32)
-        counts = np.zeros(4, np.int32)
-        if hits.nbytes > self._hits_bytes:  # kept for the next batch of the search
-            self._drop_hits()
-            self._hits, self._hits_bytes = f.dev_alloc(hits.nbytes), hits.nbytes
-            f._kept.add(self._hits)
+        counts = np.empty(4, np.int32)
         bufs = []
         args = [0, 0, 0, 0, 0]
         try:
@@ -643,14 +627,11 @@ class TranspositionTable:
                     bufs.append(f.dev_alloc(x.nbytes))
                     f.h2d(bufs[-1], x)
                 args = [bufs[0], pk.shape[1], bufs[1], bufs[2], bufs[3]]
-            _check(self._lib.omk_tt_traverse(self._h, batch._h, C.c_void_p(args[0]), C.c_int32(int(args[1])),
-                                             C.c_void_p(args[2]), C.c_void_p(args[3]), C.c_void_p(args[4]),
-                                             C.c_void_p(self._hits), _ptr(counts, i32p)))
-            f.d2h(hits, self._hits)
+            _check(self._lib.omk_tt_traverse_read(self._h, batch._h, *args, _at(hits), _at(counts)))
         finally:
             for d in bufs:
                 f.dev_free(d)
-        return hits, tuple(int(x) for x in counts)
+        return hits, tuple(counts.tolist())
 
     def select_redirect(self, batch, params, want_moves=True):
         """The traversal loop with the table on, redirects included (omk_tt_select_redirect): a select for

@@ -352,3 +352,35 @@ def test_priors_from_a_policy(moves):
     got = f.download()["P"][1:]
     assert (got.view(np.int32) == want.view(np.int32)).all()
     assert (f.download_structure()["action"][1:] == mv).all()
+
+
+# hits straight to the host, with the counts up to a megabyte and after them beyond: the same as on the device
+@pytest.mark.parametrize("n,depth", [(1, 1), (51, 5), (64, 4), (513, 7), (262144 // 8, 8), (262144 // 8 + 1, 8)])
+def test_table_hits_on_the_host_and_on_the_device(n, depth):
+    import ctypes as C
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(n, n_expand=400, fanout=(2, 6), max_depth=9, n_roots=3)
+    soa = dict(soa, hash=np.random.default_rng(n).integers(1, 60, len(soa["N"])).astype(np.uint64))
+    got = []
+    for direct in (True, False):
+        f = omk.Forest.from_soa(soa)
+        b = omk.Batch(f, n, depth)
+        table = omk.TranspositionTable(f, 12)
+        b.set_roots(roots[np.arange(n) % 3])
+        for _ in range(2):
+            b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+            if direct:
+                hits, counts = table.traverse(b)
+            else:
+                hits, words = np.empty((n, depth), np.int32), np.zeros(4, np.int32)
+                buf = f.dev_alloc(hits.nbytes)
+                assert f._lib.omk_tt_traverse(table._h, b._h, None, 0, None, None, None, C.c_void_p(buf),
+                                              words.ctypes.data_as(C.c_void_p)) == 0
+                f.d2h(hits, buf)
+                f.dev_free(buf)
+                counts = tuple(words.tolist())
+            got.append((hits, counts))
+            b.backup(3)
+    for a, b in zip(got[:2], got[2:]):
+        assert (a[0] == b[0]).all() and a[1] == b[1]
+    assert n == 1 or (got[1][0] >= 0).any()
