@@ -278,7 +278,7 @@ static int link_wait(omk_forest *f) {
 }
 
 // Bulk transfers (omk_link.hip): arrays of the host, one per segment, to or from the device.  What fits in the
-// staging goes in one piece; more is cut into pieces of kBulkWords, kBulkSlots of them on their way at a time, so
+// staging goes in one piece; more is cut into pieces, kBulkSlots or kBackSlots of them on their way at a time, so
 // that the host's copy of one piece runs beside the link's transfer of the next.
 struct Bulk {
     Segments g = {};
@@ -302,14 +302,18 @@ struct Bulk {
         }
     }
 };
-constexpr int64_t kBulkWords = 1 << 18;
-constexpr int kBulkSlots = 4;
+// Pieces to the card: of 1 MB, what counts is the kernels' reading of the link, which smaller ones slow down (8.4 MB:
+// 285 us, in pieces of 512 KB 300).  Pieces back: of 512 KB, what counts is the host's copy out of them, which works
+// best on what its cache holds (11.5 MB: 372 us, in pieces of 1 MB 411, of 256 KB 435, without the copy 262).
+constexpr int64_t kBulkWords = 1 << 18, kBackWords = 1 << 17;
+constexpr int kBulkSlots = 4, kBackSlots = 8;
 static_assert(kBulkWords * kBulkSlots * 4 <= (int64_t)kLinkStaging, "the slots are the staging");
 
 static int bulk_put(omk_forest *f, const Bulk &b) {
     const int64_t words = b.words();
     const bool whole = words <= kBulkWords * kBulkSlots;
     void *staged = nullptr;
+static_assert(kBackWords * kBackSlots * 4 <= (int64_t)kLinkStaging, "the slots are the staging");
     if (int rc = link_stage(f, (size_t)(whole ? words : kBulkWords * kBulkSlots) * 4, &staged)) return rc;
     char *at = (char *)staged;
     if (whole) {
@@ -333,25 +337,25 @@ static int bulk_put(omk_forest *f, const Bulk &b) {
 }
 
 static int bulk_get(omk_forest *f, const Bulk &b) {
-    const int64_t words = b.words(), pieces = (words + kBulkWords - 1) / kBulkWords;
+    const int64_t words = b.words(), pieces = (words + kBackWords - 1) / kBackWords;
     if (pieces == 0) return OMK_OK;
     void *staged = nullptr;
-    if (int rc = link_stage(f, (size_t)std::min<int64_t>(words, kBulkWords * kBulkSlots) * 4, &staged)) return rc;
+    if (int rc = link_stage(f, (size_t)std::min<int64_t>(words, kBackWords * kBackSlots) * 4, &staged)) return rc;
     char *at = (char *)staged;
-    int32_t seq[kBulkSlots] = {};
+    int32_t seq[kBackSlots] = {};
     auto ask = [&](int64_t c) {
         const HostSignal sig = link_signal(f);
-        seq[c % kBulkSlots] = sig.seq;
-        return launch_get(b.g, (uint32_t *)(at + (size_t)(c % kBulkSlots) * kBulkWords * 4), c * kBulkWords,
-                          std::min(kBulkWords, words - c * kBulkWords), sig, f->stream);
+        seq[c % kBackSlots] = sig.seq;
+        return launch_get(b.g, (uint32_t *)(at + (size_t)(c % kBackSlots) * kBackWords * 4), c * kBackWords,
+                          std::min(kBackWords, words - c * kBackWords), sig, f->stream);
     };
-    for (int64_t c = 0; c < std::min<int64_t>(pieces, kBulkSlots); c++) HIP_TRY(ask(c));
+    for (int64_t c = 0; c < std::min<int64_t>(pieces, kBackSlots); c++) HIP_TRY(ask(c));
     for (int64_t c = 0; c < pieces; c++) {
-        if (int rc = link_wait_for(f, seq[c % kBulkSlots])) return rc;
-        const char *p = at + (size_t)(c % kBulkSlots) * kBulkWords * 4;
-        b.each(c * kBulkWords, std::min(kBulkWords, words - c * kBulkWords),
+        if (int rc = link_wait_for(f, seq[c % kBackSlots])) return rc;
+        const char *p = at + (size_t)(c % kBackSlots) * kBackWords * 4;
+        b.each(c * kBackWords, std::min(kBackWords, words - c * kBackWords),
                [&](char *h, int64_t off, size_t bytes) { memcpy(h, p + off, bytes); });
-        if (c + kBulkSlots < pieces) HIP_TRY(ask(c + kBulkSlots));
+        if (c + kBackSlots < pieces) HIP_TRY(ask(c + kBackSlots));
     }
     f->link_used = 0;
     return OMK_OK;
