@@ -164,6 +164,11 @@ struct omk_batch {
     // which selection it is of (the forest's and the batch's counts when it was made): an expansion takes leaves,
     // child counts and visit counts from it while nothing has changed them
     int64_t select_calls = 0, gathered_call = -1, gathered_changes = -1;
+    // The gather that a selection of lone traversals has made itself (lone_rows): its call, the forest's changes
+    // before it, its number, and the staging in use then.  read_call: the selection that was read last.
+    int64_t lone_call = -1, lone_changes = -1, read_call = -1;
+    int32_t lone_seq = 0;
+    size_t lone_staged = 0;
     std::vector<int32_t> leaf_table;  // work space of an expansion
     std::vector<int32_t> winners;
     long long *trace = nullptr;  // records of the timeline, kTraceCap of them
@@ -308,12 +313,12 @@ struct Bulk {
 constexpr int64_t kBulkWords = 1 << 18, kBackWords = 1 << 17;
 constexpr int kBulkSlots = 4, kBackSlots = 8;
 static_assert(kBulkWords * kBulkSlots * 4 <= (int64_t)kLinkStaging, "the slots are the staging");
+static_assert(kBackWords * kBackSlots * 4 <= (int64_t)kLinkStaging, "the slots are the staging");
 
 static int bulk_put(omk_forest *f, const Bulk &b) {
     const int64_t words = b.words();
     const bool whole = words <= kBulkWords * kBulkSlots;
     void *staged = nullptr;
-static_assert(kBackWords * kBackSlots * 4 <= (int64_t)kLinkStaging, "the slots are the staging");
     if (int rc = link_stage(f, (size_t)(whole ? words : kBulkWords * kBulkSlots) * 4, &staged)) return rc;
     char *at = (char *)staged;
     if (whole) {
@@ -1170,6 +1175,49 @@ int omk_batch_destroy(omk_batch *b) {
 
 }  // extern "C"
 
+// Where the leaf gather of the batch goes: its pinned buffer, laid out for the paths there are.
+static int gather_room(omk_batch *b, ExportOut *o) {
+    const size_t n = (size_t)b->n, D = (size_t)b->max_depth;
+    // lengths | leaves | their child counts | their visit counts | abort words | paths | actions
+    const size_t need = (n * (2 * D + 5) + 4) * 4;
+    if (need > b->out_bytes) {
+        if (b->out) {
+            HIP_TRY(hipStreamSynchronize(b->f->stream));
+            HIP_TRY(hipHostFree(b->out));
+        }
+        b->out = nullptr;
+        b->out_bytes = 0;
+        const size_t room = ((size_t)b->stride * (2 * D + 5) + 4) * 4;
+        HIP_TRY(hipHostMalloc((void **)&b->out, room, hipHostMallocDefault));
+        b->out_bytes = room;
+    }
+    o->len = b->out;
+    o->leaf = o->len + n;
+    o->children = o->leaf + n;
+    o->visits = o->children + n;
+    o->abort = o->visits + n;
+    o->paths = o->abort + 4;
+    o->actions = o->paths + n * (D + 1);
+    return OMK_OK;
+}
+
+// A selection whose traversals are all alone at their roots, in a batch whose selection before was read: its
+// walkers send their own rows (export_lone), and the read finds them there.  Small batches only: the rows of a
+// large one leave in better pieces by a kernel of their own.
+constexpr int kLoneRowsMax = 1024;
+static int lone_rows(omk_batch *b, LoneOut *out) {
+    memset(out, 0, sizeof(*out));
+    if (b->n_items0 > 0 || b->n > kLoneRowsMax || b->max_depth >= 64 || b->read_call != b->select_calls) return OMK_OK;
+    if (int rc = gather_room(b, &out->rows)) return rc;
+    for (int i = 0; i < 4; i++) out->rows.abort[i] = 0;  // (these kernels wait for nobody)
+    out->sig = link_signal(b->f);
+    b->lone_call = b->select_calls + 1;
+    b->lone_changes = b->f->changes;
+    b->lone_seq = out->sig.seq;
+    b->lone_staged = b->f->link_used;
+    return OMK_OK;
+}
+
 // What a selection of the batch with call number `epoch` is told, the caller's parameters apart.
 static SelectArgs select_args(omk_batch *b, int32_t epoch) {
     SelectArgs a;
@@ -1398,8 +1446,11 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
     a.pw = p->pw;
     a.c_puct = p->c_puct;
     a.rave_k = p->rave_k;
+    LoneOut out;
+    if (int rc = lone_rows(b, &out)) return rc;
     HIP_TRY(launch_select(f->dev(), a, b->n_items0, b->n_singles0, b->n, b->most_visitors, f->max_fanout, p->use_rave != 0,
-                          f->grown, b->n_cus, b->n_hctx0, b->prepared == b->epoch, f->stream));
+                          f->grown, b->n_cus, b->n_hctx0, b->prepared == b->epoch, out,
+                          f->stream));
     b->selected = true;
     b->select_calls++;
     return OMK_OK;
@@ -1485,32 +1536,19 @@ int omk_backup_paths(omk_forest *f, const int32_t *d_paths, const int32_t *d_pat
 // The leaf gather of the last selection into the batch's pinned buffer; waits for it.
 static int gather(omk_batch *b, bool paths, bool actions) {
     omk_forest *f = b->f;
-    const size_t n = (size_t)b->n, D = (size_t)b->max_depth;
-    // lengths | leaves | their child counts | their visit counts | abort words | paths | actions
-    const size_t need = (n * (2 * D + 5) + 4) * 4;
-    if (need > b->out_bytes) {
-        if (b->out) {
-            HIP_TRY(hipStreamSynchronize(f->stream));
-            HIP_TRY(hipHostFree(b->out));
-        }
-        b->out = nullptr;
-        b->out_bytes = 0;
-        const size_t room = ((size_t)b->stride * (2 * D + 5) + 4) * 4;
-        HIP_TRY(hipHostMalloc((void **)&b->out, room, hipHostMallocDefault));
-        b->out_bytes = room;
-    }
     ExportOut &o = b->gathered;
-    o.len = b->out;
-    o.leaf = o.len + n;
-    o.children = o.leaf + n;
-    o.visits = o.children + n;
-    o.abort = o.visits + n;
-    o.paths = paths ? o.abort + 4 : nullptr;
-    o.actions = actions ? o.abort + 4 + n * (D + 1) : nullptr;
     b->gathered_call = -1;
-    HIP_TRY(launch_export(f->dev(), b->paths, b->path_len, b->leaf, b->counters + 3 * kSchedStep + 1, b->n, b->stride,
-                          b->max_depth, o, link_signal(f), f->stream));
-    if (int rc = link_wait(f)) return rc;
+    if (int rc = gather_room(b, &o)) return rc;
+    if (b->lone_call == b->select_calls && b->lone_changes == f->changes) {
+        if (int rc = link_wait_for(f, b->lone_seq)) return rc;
+        if (b->lone_seq == f->link_seq && b->lone_staged == f->link_used) f->link_used = 0;  // as in link_wait
+    } else {
+        if (!paths) o.paths = nullptr;
+        if (!actions) o.actions = nullptr;
+        HIP_TRY(launch_export(f->dev(), b->paths, b->path_len, b->leaf, b->counters + 3 * kSchedStep + 1, b->n, b->stride,
+                              b->max_depth, o, link_signal(f), f->stream));
+        if (int rc = link_wait(f)) return rc;
+    }
     b->gathered_call = b->select_calls;
     b->gathered_changes = f->changes;
     return OMK_OK;
@@ -1663,6 +1701,7 @@ int omk_batch_read(omk_batch *b, int32_t *h_paths, int32_t *h_path_len, int32_t 
     omk_forest *f = b->f;
     if (int rc = use_device(f)) return rc;
     const size_t n = (size_t)b->n, D = (size_t)b->max_depth;
+    b->read_call = b->select_calls;
     if (int rc = gather(b, h_paths != nullptr, h_actions != nullptr)) return rc;
     const ExportOut &o = b->gathered;
     if (h_paths) memcpy(h_paths, o.paths, n * (D + 1) * 4);

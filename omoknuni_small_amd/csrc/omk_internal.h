@@ -114,11 +114,33 @@ struct SelectArgs {
     float rave_k;
 };
 
+// How a kernel tells the waiting host that its results lie in pinned memory: the last block to finish stores
+// `seq` to the host's flag word.  `count` is a device word that is zero between two such kernels.
+struct HostSignal {
+    int32_t *count;
+    int32_t *flag;
+    int32_t seq;
+};
+// Where the leaf gather of a batch goes (pinned host memory that the kernel writes itself; any of the first two
+// may be null): row-major paths [n][max_depth+1] and actions [n][max_depth], -1 padded; per traversal the path
+// length, the leaf, and the leaf's child and visit count; the four abort words of the selection.
+struct ExportOut {
+    int32_t *paths, *actions;
+    int32_t *len, *leaf, *children, *visits;
+    int32_t *abort;
+};
+// The leaf gather that the kernels of lone traversals write themselves; none with sig.flag NULL.  Both path arrays
+// are there and max_depth is below 64.
+struct LoneOut {
+    ExportOut rows;
+    HostSignal sig;
+};
+
 // most_visitors: traversals of the most crowded root; grown: the forest has been expanded since it was uploaded;
 // prepared: launch_set_roots has made the reset
 hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, int n_singles0, int n_traversals,
                          int most_visitors, int max_fanout, bool rave, bool grown, int n_cus, int n_hctx0,
-                         bool prepared, hipStream_t s);
+                         bool prepared, const LoneOut &out, hipStream_t s);
 
 // What omk_batch_set_roots has staged (n visitors | n roots | items | lone traversals) to the batch's arrays.
 // prepare: and what launch_select's reset does for the selection that `a` belongs to.
@@ -128,7 +150,7 @@ hipError_t launch_set_roots(const SelectArgs &a, int32_t *seg0, Item *items0, It
 // The kernels of one fan-out class (rounds of 64 children: 1, 4, 6 or 16), behind the reset launch.
 template <int RMAX, bool RAVE>
 hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a, int n_items0, int most_visitors, int n_traversals,
-                               int n_cus, bool grown, hipStream_t s);
+                               int n_cus, bool grown, const LoneOut &out, hipStream_t s);
 
 hipError_t launch_apply_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                            int max_len, int vl, hipStream_t s);
@@ -143,13 +165,6 @@ hipError_t launch_blend_all(const ForestDev &f, float rave_k, hipStream_t s);
 hipError_t launch_blend_paths(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                               int max_len, float rave_k, hipStream_t s);
 
-// How a kernel tells the waiting host that its results lie in pinned memory: the last block to finish stores
-// `seq` to the host's flag word.  `count` is a device word that is zero between two such kernels.
-struct HostSignal {
-    int32_t *count;
-    int32_t *flag;
-    int32_t seq;
-};
 // Arrays of 32-bit words on the device, read as one stream (omk_link.hip): word start[q] + i of the stream is word
 // i * step[q] of dev[q].
 constexpr int kMaxSegments = 10;
@@ -165,14 +180,6 @@ hipError_t launch_put(const Segments &g, const uint32_t *staged, int64_t first, 
 hipError_t launch_get(const Segments &g, uint32_t *staged, int64_t first, int64_t count, const HostSignal &sig,
                       hipStream_t s);
 
-// Where the leaf gather of a batch goes (pinned host memory that the kernel writes itself; any of the first two
-// may be null): row-major paths [n][max_depth+1] and actions [n][max_depth], -1 padded; per traversal the path
-// length, the leaf, and the leaf's child and visit count; the four abort words of the selection.
-struct ExportOut {
-    int32_t *paths, *actions;
-    int32_t *len, *leaf, *children, *visits;
-    int32_t *abort;
-};
 hipError_t launch_export(const ForestDev &f, const int32_t *paths, const int32_t *path_len, const int32_t *leaf,
                          const int32_t *abort_words, int n, int stride, int max_depth, const ExportOut &out,
                          const HostSignal &sig, hipStream_t s);

@@ -4352,10 +4352,15 @@ __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs
 }
 
 // Single visitors: the rest of the path is private to the visitor, one wavefront walks it.
+// A walk that has ended: lane d (of the first 64) holds the node at depth d, -1 behind the leaf.
+struct LonePath {
+    int t, node, len, leaf, children, visits;
+};
+
 // One lone visitor from its item to its leaf.  MODE 0: plain loads; 1: AHEAD; 2: AHEAD and FAST
 // (select_single).
 template <int RMAX, bool RAVE, int MODE>
-__device__ __forceinline__ void walk_single(const ForestDev &f, const SelectArgs &a, const Item &it, int lane) {
+__device__ __forceinline__ LonePath walk_single(const ForestDev &f, const SelectArgs &a, const Item &it, int lane) {
     constexpr bool AHEAD = MODE >= 1, FAST = MODE >= 2;
     int node = it.node;
     const int t = it.off;
@@ -4369,6 +4374,7 @@ __device__ __forceinline__ void walk_single(const ForestDev &f, const SelectArgs
     constexpr bool kFastWide = FAST && RMAX <= 6;
     bool have_span = false;
     int2 span = int2{0, 0};
+    int mine = lane == d ? node : -1;
     for (;;) {
         NodeCtx c = node_ctx(f, a, node, np, have_span, span);
         int i = -1;
@@ -4388,7 +4394,7 @@ __device__ __forceinline__ void walk_single(const ForestDev &f, const SelectArgs
                 a.path_len[t] = d + 1;
                 if (c.cc > 0 && d >= a.max_depth) atomicAdd(a.truncated, 1);
             }
-            return;
+            return LonePath{t, mine, d + 1, node, c.cc, np};
         }
         int child = c.cb + i;
         if (lane == 0) {
@@ -4399,14 +4405,31 @@ __device__ __forceinline__ void walk_single(const ForestDev &f, const SelectArgs
         node = child;
         np = np_child;
         d++;
+        if (lane == d) mine = node;
     }
+}
+
+// The leaf gather's row of a lone path (ExportOut), written by the wavefront that walked it.
+__device__ __forceinline__ void export_lone(const ForestDev &f, const ExportOut &o, const LonePath &w, int max_depth,
+                                            int lane) {
+    const int act = lane < w.len ? (f.action ? f.action[w.node] : w.node) : -1;
+    if (lane == 0) {
+        host_store(o.len + w.t, w.len);
+        host_store(o.leaf + w.t, w.leaf);
+        host_store(o.children + w.t, w.children);
+        host_store(o.visits + w.t, w.visits);
+    }
+    if (lane <= max_depth) host_store(o.paths + (size_t)w.t * (max_depth + 1) + lane, w.node);
+    if (lane >= 1 && lane <= max_depth) host_store(o.actions + (size_t)w.t * max_depth + lane - 1, act);
 }
 
 // The kernel of a select whose traversals are all alone at their roots (one per tree): the
 // walkers are the `seeded` entries the host prepared, no other launch belongs to the select, and
-// one thread leaves the scheduler words as a reset would have.
-template <int RMAX, bool RAVE, int MODE>
-__global__ __launch_bounds__(256) void k_select_singles(ForestDev f, SelectArgs a, int seeded) {
+// one thread leaves the scheduler words as a reset would have.  With ROWS every walker also sends its path to
+// the host: the gather of the leaves that a search asks for next, without a launch of its own (256 games: 44 -> 37
+// us a batch).  A kernel of its own, because keeping the path costs 32768 walkers a tenth (41 -> 45 us).
+template <int RMAX, bool RAVE, int MODE, bool ROWS>
+__global__ __launch_bounds__(256) void k_select_singles(ForestDev f, SelectArgs a, int seeded, LoneOut out) {
     const int lane = threadIdx.x & 63;
     const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (wave == 0 && lane == 0) {
@@ -4414,8 +4437,11 @@ __global__ __launch_bounds__(256) void k_select_singles(ForestDev f, SelectArgs 
         *a.truncated_next = 0;
         a.sched_wait[1] = 0;
     }
-    if (wave >= seeded) return;
-    walk_single<RMAX, RAVE, MODE>(f, a, a.singles0[wave], lane);
+    if (wave < seeded) {
+        const LonePath w = walk_single<RMAX, RAVE, MODE>(f, a, a.singles0[wave], lane);
+        if (ROWS) export_lone(f, out.rows, w, a.max_depth, lane);
+    }
+    if (ROWS) host_signal(out.sig.count, out.sig.flag, out.sig.seq, gridDim.x);
 }
 
 // The same walk by a whole block, for a batch of few traversals on a wide layout (a legal mask: one slot per
@@ -4435,7 +4461,8 @@ struct SingleSlot {
 };
 
 template <int RMAX, bool RAVE>
-__global__ __launch_bounds__(RMAX * kWave) void k_select_singles_team(ForestDev f, SelectArgs a, int seeded) {
+__global__ __launch_bounds__(RMAX * kWave) void k_select_singles_team(ForestDev f, SelectArgs a, int seeded,
+                                                                       LoneOut out) {
     constexpr int F = RMAX * kWave;
     __shared__ SingleSlot slot[2][RMAX];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -4453,6 +4480,7 @@ __global__ __launch_bounds__(RMAX * kWave) void k_select_singles_team(ForestDev 
         if (threadIdx.x == 0) a.paths[t] = node;
     }
     int2 span = f.span[node];
+    int mine = lane == d ? node : -1;
     for (int level = 0;; level++) {
         const int cb = span.x, cc = span.y;
         int nelig = cc;
@@ -4560,6 +4588,10 @@ __global__ __launch_bounds__(RMAX * kWave) void k_select_singles_team(ForestDev 
                 a.path_len[t] = d + 1;
                 if (cc > 0 && d >= a.max_depth) atomicAdd(a.truncated, 1);
             }
+            if (out.sig.flag) {
+                if (wv == 0) export_lone(f, out.rows, LonePath{t, mine, d + 1, node, cc, np}, a.max_depth, lane);
+                host_signal(out.sig.count, out.sig.flag, out.sig.seq, gridDim.x);
+            }
             return;
         }
         const int child = cb + ci;
@@ -4572,6 +4604,7 @@ __global__ __launch_bounds__(RMAX * kWave) void k_select_singles_team(ForestDev 
         np = np_child;
         span = span_child;
         d++;
+        if (lane == d) mine = node;
     }
 }
 
@@ -4646,7 +4679,7 @@ __device__ __noinline__ void walkers_loop(ForestDev f, SelectArgs a, int lane) {
 
 template <int RMAX, bool RAVE>
 hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_items0, int most_visitors,
-                                 int n_traversals, int n_cus, bool grown, hipStream_t s) {
+                                 int n_traversals, int n_cus, bool grown, const LoneOut &out, hipStream_t s) {
     // Few walkers cannot keep the memory system busy: then the variant that spends bytes to save
     // dependent trips (select_single, FAST).  The number of lone visitors is only known on the
     // device; the number of traversals bounds it.  Measured: it pays on a board layout (legal
@@ -4686,15 +4719,16 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_i
     }
     // every traversal is alone at its root: the walkers are the host's list
     const dim3 grid((n_traversals + 3) / 4), block(256);
-    if (RMAX > 1 && f.legal && n_traversals * RMAX <= kTeamSinglesMaxWaves)
+    if (RMAX > 1 && f.legal && n_traversals * RMAX <= kTeamSinglesMaxWaves) {
         hipLaunchKernelGGL((k_select_singles_team<RMAX, RAVE>), dim3(n_traversals), dim3(RMAX * kWave), 0, s, f, a0,
-                           n_traversals);
-    else if (!f.legal)
-        hipLaunchKernelGGL((k_select_singles<RMAX, RAVE, 0>), grid, block, 0, s, f, a0, n_traversals);
-    else if (fast)
-        hipLaunchKernelGGL((k_select_singles<RMAX, RAVE, 2>), grid, block, 0, s, f, a0, n_traversals);
-    else
-        hipLaunchKernelGGL((k_select_singles<RMAX, RAVE, 1>), grid, block, 0, s, f, a0, n_traversals);
+                           n_traversals, out);
+        return hipGetLastError();
+    }
+    const bool rows = out.sig.flag != nullptr;
+    auto *kernel = !f.legal ? (rows ? k_select_singles<RMAX, RAVE, 0, true> : k_select_singles<RMAX, RAVE, 0, false>)
+                   : fast   ? (rows ? k_select_singles<RMAX, RAVE, 2, true> : k_select_singles<RMAX, RAVE, 2, false>)
+                            : (rows ? k_select_singles<RMAX, RAVE, 1, true> : k_select_singles<RMAX, RAVE, 1, false>);
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, f, a0, n_traversals, out);
     return hipGetLastError();
 }
 

@@ -3,7 +3,7 @@
 
 namespace omk {
 template hipError_t launch_select_class<4, false>(const ForestDev &, const SelectArgs &, int, int, int, int, bool,
-                                                      hipStream_t);
+                                                      const LoneOut &, hipStream_t);
 template hipError_t launch_select_class<4, true>(const ForestDev &, const SelectArgs &, int, int, int, int, bool,
-                                                      hipStream_t);
+                                                      const LoneOut &, hipStream_t);
 }  // namespace omk

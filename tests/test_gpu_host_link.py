@@ -384,3 +384,35 @@ def test_table_hits_on_the_host_and_on_the_device(n, depth):
     for a, b in zip(got[:2], got[2:]):
         assert (a[0] == b[0]).all() and a[1] == b[1]
     assert n == 1 or (got[1][0] >= 0).any()
+
+
+# one traversal per tree, read every time: from the second selection on the walkers send their own rows (up to 1024
+# traversals and a depth bound of 63), which a read finds after whatever was staged in between, twice if it asks
+# twice, and not once a backup has changed what they say
+@pytest.mark.parametrize("n,depth", [(1, 5), (3, 1), (4, 63), (5, 64), (257, 8), (1024, 6), (1025, 6)])
+@pytest.mark.parametrize("mask", [0.0, 0.4])
+def test_lone_walkers_send_their_own_rows(n, depth, mask):
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(n + depth, n_expand=2 * n + 40, fanout=(1, 90 if n < 300 else 9), max_depth=70, n_roots=n, mask_frac=mask)
+    ref = R.RefTree.from_soa(soa)
+    f = omk.Forest.from_soa(soa)
+    b = omk.Batch(f, n, depth)
+    b.set_roots(roots[:n])
+    rng = np.random.default_rng(n)
+    for step in range(6):
+        rpaths, rlen, rleaf, _ = ref.select_batch(roots[:n], R.make_params(c_puct=1.4, virtual_loss=3, max_depth=depth))
+        values = (rng.integers(-64, 65, n) / 64.0).astype(np.float32)
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+        b.set_values(values)
+        if step == 3:
+            ref.backup_batch(rpaths, rlen, values, 3)
+            b.backup(3)
+        for _ in range(0 if step == 4 else 2):
+            paths, plen, leaf, actions = b.read()
+            assert (paths == rpaths).all() and (plen == rlen).all() and (leaf == rleaf).all()
+            assert (actions == ref.gather_actions(rpaths, rlen)).all()
+        if step != 3:
+            ref.backup_batch(rpaths, rlen, values, 3)
+            b.backup(3)
+        got = f.download()
+        assert (got["N"] == ref.N).all() and (got["W"] == ref.W).all() and (got["VL"] == ref.VL).all()
