@@ -15,6 +15,7 @@
 
 #include "omk_internal.h"
 #include "omk_priors.h"
+#include "omk_staging.h"
 
 using namespace omk;
 
@@ -71,8 +72,7 @@ struct omk_forest {
     bool redirected = false;
     // The way between the host and the kernels: one block of pinned memory that both sides address (see link_*).
     char *link = nullptr;
-    size_t link_bytes = 0;
-    size_t link_used = 0;         // staging handed out since the stream was last known to be idle
+    Staging staging;
     int32_t link_seq = 0;         // number of the last call that waited
     int32_t *link_count = nullptr;  // HostSignal::count
     char *scratch = nullptr;  // work space of a compaction, kept for the next (kKeepScratch)
@@ -165,10 +165,11 @@ struct omk_batch {
     // child counts and visit counts from it while nothing has changed them
     int64_t select_calls = 0, gathered_call = -1, gathered_changes = -1;
     // The gather that a selection of lone traversals has made itself (lone_rows): its call, the forest's changes
-    // before it, its number, and the staging in use then.  read_call: the selection that was read last.
+    // before it, its number, and the point of the stream it lies at (Staging::now).  read_call: the selection that
+    // was read last.
     int64_t lone_call = -1, lone_changes = -1, read_call = -1;
     int32_t lone_seq = 0;
-    size_t lone_staged = 0;
+    uint64_t lone_staged = 0;
     std::vector<int32_t> leaf_table;  // work space of an expansion
     std::vector<int32_t> winners;
     long long *trace = nullptr;  // records of the timeline, kTraceCap of them
@@ -235,22 +236,24 @@ static hipError_t link_alloc(omk_forest *f, size_t staging) {
     if (e != hipSuccess) return e;
     if (f->link) (void)hipHostFree(f->link);
     f->link = p;
-    f->link_bytes = kLinkHead + staging;
-    f->link_used = 0;
+    f->staging.replace(staging);
     *(int32_t *)p = f->link_seq;
     return hipSuccess;
 }
 
 // `bytes` of staging, aligned to a cache line; valid until the next call that waits for the stream.
 static int link_stage(omk_forest *f, size_t bytes, void **out) {
-    bytes = (bytes + 127) & ~(size_t)127;
-    if (kLinkHead + f->link_used + bytes > f->link_bytes) {
+    size_t at = f->staging.take(bytes);
+    if (at == Staging::kFull) {
         HIP_TRY(hipStreamSynchronize(f->stream));
-        f->link_used = 0;
-        if (kLinkHead + bytes > f->link_bytes) HIP_TRY(link_alloc(f, bytes + bytes / 2));
+        f->staging.idle();
+        at = f->staging.take(bytes);
+        if (at == Staging::kFull) {
+            HIP_TRY(link_alloc(f, bytes + bytes / 2 + 128));
+            at = f->staging.take(bytes);
+        }
     }
-    *out = f->link + kLinkHead + f->link_used;
-    f->link_used += bytes;
+    *out = f->link + kLinkHead + at;
     return OMK_OK;
 }
 
@@ -278,7 +281,7 @@ static int link_wait_for(omk_forest *f, int32_t seq) {
 // Waits for the last one: everything enqueued has run, and staging starts at the front again.
 static int link_wait(omk_forest *f) {
     if (int rc = link_wait_for(f, f->link_seq)) return rc;
-    f->link_used = 0;
+    f->staging.idle();
     return OMK_OK;
 }
 
@@ -362,7 +365,7 @@ static int bulk_get(omk_forest *f, const Bulk &b) {
                [&](char *h, int64_t off, size_t bytes) { memcpy(h, p + off, bytes); });
         if (c + kBackSlots < pieces) HIP_TRY(ask(c + kBackSlots));
     }
-    f->link_used = 0;
+    f->staging.idle();
     return OMK_OK;
 }
 
@@ -1214,7 +1217,7 @@ static int lone_rows(omk_batch *b, LoneOut *out) {
     b->lone_call = b->select_calls + 1;
     b->lone_changes = b->f->changes;
     b->lone_seq = out->sig.seq;
-    b->lone_staged = b->f->link_used;
+    b->lone_staged = b->f->staging.now();
     return OMK_OK;
 }
 
@@ -1541,7 +1544,7 @@ static int gather(omk_batch *b, bool paths, bool actions) {
     if (int rc = gather_room(b, &o)) return rc;
     if (b->lone_call == b->select_calls && b->lone_changes == f->changes) {
         if (int rc = link_wait_for(f, b->lone_seq)) return rc;
-        if (b->lone_seq == f->link_seq && b->lone_staged == f->link_used) f->link_used = 0;  // as in link_wait
+        f->staging.ran_to(b->lone_staged);  // (link_wait waits for the last call; another batch's may be on their way)
     } else {
         if (!paths) o.paths = nullptr;
         if (!actions) o.actions = nullptr;

@@ -202,3 +202,14 @@ def test_direct_merge_rule_against_the_serial_loop(tmp_path):
     assert out.returncode == 0, out.stdout[-2000:]
     m = re.search(r"merged: (\d+); wrong 0;", out.stdout)
     assert m and int(m.group(1)) > 30000, out.stdout[-500:]
+
+
+def test_staging_is_not_handed_out_over_what_kernels_still_read(tmp_path):
+    """The pinned block's staging (csrc/omk_staging.h) against a stream that runs as late as it can
+    (tests/cpp/staging_check.cpp): after a wrap, an offset that was in use before says nothing about what
+    has run."""
+    exe = str(tmp_path / "staging_check")
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-Wall", os.path.join(ROOT, "tests", "cpp", "staging_check.cpp"),
+                           "-o", exe])
+    out = subprocess.run([exe, "3000"], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0 and out.stdout == "ok 3000\n", out.stdout

@@ -416,3 +416,39 @@ def test_lone_walkers_send_their_own_rows(n, depth, mask):
             b.backup(3)
         got = f.download()
         assert (got["N"] == ref.N).all() and (got["W"] == ref.W).all() and (got["VL"] == ref.VL).all()
+
+
+# two batches on one forest: what one of them has staged, after a wrap of the staging, is still on its way when the
+# other one reads rows its walkers sent before and stages again
+def test_values_staged_behind_a_lone_selection_arrive_whole():
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(81, n_expand=900, fanout=(1, 9), max_depth=6, n_roots=300)
+    ref = R.RefTree.from_soa(soa)
+    f = omk.Forest.from_soa(soa)
+    rng = np.random.default_rng(81)
+    many = 600_000  # 2.4 of the 4 MB: the second time they do not fit behind the first
+    params = omk.SelectParams(c_puct=1.4, virtual_loss=3)
+    lone, other = omk.Batch(f, 256, 6), omk.Batch(f, many, 6)
+    lone.set_roots(roots[:256])
+    other.set_roots(roots[256:])
+    first, second, own = ((rng.integers(-64, 65, n) / 64.0).astype(np.float32) for n in (many, many, 256))
+    for step in range(4):
+        rlone = ref.select_batch(roots[:256], R.make_params(c_puct=1.4, virtual_loss=3, max_depth=6))
+        rother = ref.select_batch(roots[256:], R.make_params(c_puct=1.4, virtual_loss=3, max_depth=6))
+        other.select(params)
+        other.set_values(first)
+        lone.select(params)
+        other.set_values(second)
+        paths, plen, leaf, _ = lone.read()
+        lone.set_values(own)
+        other.backup(3)
+        lone.backup(3)
+        assert (paths == rlone[0]).all() and (plen == rlone[1]).all() and (leaf == rlone[2]).all()
+        ref.backup_batch(rother[0], rother[1], second[:44], 3)
+        ref.backup_batch(rlone[0], rlone[1], own, 3)
+        got = f.download()
+        assert (got["N"] == ref.N).all() and (got["VL"] == ref.VL).all()
+        err = np.abs(got["W"].astype(np.float64) - ref.W) / np.maximum(np.abs(ref.W), 1.0)
+        assert err.max() <= 1e-5, step  # (the trees' own sums are no multiples of 1/64)
+        ref.W[:] = got["W"]
+        first, second = second, first
