@@ -130,6 +130,10 @@ struct omk_batch {
     int32_t n = 0;          // traversals bound by set_roots
     int64_t generation = -1;  // the forest's generation when the roots were set
     bool selected = false;  // paths of a select are on the device
+    // No two of these paths share a node: said by the selection that made them.  (What the forest or the roots are
+    // like when they are settled says nothing: paths that follow transpositions meet in nodes that several trees
+    // hold, and an upload makes the forest a tree again under them.)
+    bool disjoint = false;
     int32_t *paths = nullptr, *path_len = nullptr, *leaf = nullptr;
     float *values = nullptr;
     Item *items0 = nullptr, *items_q = nullptr, *singles0 = nullptr, *singles_q = nullptr;
@@ -1455,12 +1459,10 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
                           f->grown, b->n_cus, b->n_hctx0, b->prepared == b->epoch, out,
                           f->stream));
     b->selected = true;
+    b->disjoint = b->n_items0 == 0;  // a root each, and distinct roots head disjoint trees
     b->select_calls++;
     return OMK_OK;
 }
-
-// Every traversal has a root of its own, and the trees are disjoint (a redirected forest's are not).
-static bool alone(const omk_batch *b) { return b->n_items0 == 0 && !b->f->redirected; }
 
 int omk_backup_batch(omk_batch *b, int32_t virtual_loss) {
     if (!b) return fail(OMK_ERR_INVALID, "omk_backup_batch: null batch");
@@ -1469,7 +1471,7 @@ int omk_backup_batch(omk_batch *b, int32_t virtual_loss) {
     if (int rc = use_device(b->f)) return rc;
     b->f->changes++;
     HIP_TRY(launch_backup(b->f->dev(), b->paths, b->path_len, b->values, b->n, b->stride, b->max_depth + 1,
-                          virtual_loss, alone(b), b->f->stream));
+                          virtual_loss, b->disjoint, b->f->stream));
     // N and W of the nodes on the paths have changed: their RAVE blend with them
     if (b->f->has_rave && b->f->blend_valid)
         HIP_TRY(launch_blend_paths(b->f->dev(), b->paths, b->path_len, b->n, b->stride, b->max_depth + 1, b->f->blend_k,
@@ -1496,7 +1498,7 @@ int omk_revert_vl(omk_batch *b, int32_t virtual_loss) {
     if (int rc = fresh_batch("omk_revert_vl", b)) return rc;
     if (int rc = use_device(b->f)) return rc;
     HIP_TRY(launch_revert_vl(b->f->dev(), b->paths, b->path_len, b->n, b->stride, b->max_depth + 1, virtual_loss,
-                             alone(b), b->f->stream));
+                             b->disjoint, b->f->stream));
     return OMK_OK;
 }
 
@@ -2067,6 +2069,7 @@ int omk_tt_select_redirect(omk_tt *tt, omk_batch *b, const omk_select_params *p,
     a.abort_word = b->counters + 3 * kSchedStep + 1;
     HIP_TRY(launch_select_redirect(f->dev(), a, p->use_rave != 0, s));
     b->selected = true;
+    b->disjoint = false;
     b->select_calls++;
     int32_t status[8];
     if (int rc = tt_counts(tt, status)) return rc;

@@ -154,7 +154,7 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a, int n_it
 
 hipError_t launch_apply_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                            int max_len, int vl, hipStream_t s);
-// alone: no two of the paths share a node (every traversal has a root of its own)
+// alone: no two of the paths share a node
 hipError_t launch_revert_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                             int max_len, int vl, bool alone, hipStream_t s);
 hipError_t launch_backup(const ForestDev &f, const int32_t *paths, const int32_t *path_len, const float *values,

@@ -242,3 +242,42 @@ def test_without_position_keys_or_with_widening_it_refuses():
     b2.set_roots(np.zeros(4, np.int32))
     with pytest.raises(omk.OmkError, match="widening"):
         tt2.select_redirect(b2, omk.SelectParams(pw=True))
+
+
+@pytest.mark.parametrize("how", ["backup", "revert"])
+def test_paths_that_share_nodes_are_settled_after_an_upload_as_before_it(how):
+    # the same game in 96 trees with one table: a traversal of each tree ends up in nodes of the trees before it.
+    # The upload of the same structure makes the forest a tree again and leaves the batch and its paths usable.
+    import omoknuni_small_amd as omk
+    one, trees = stones_tree(np.random.default_rng(91), cells=5, plies=4), 96
+    n = one["n"]
+    shift = np.repeat(np.arange(trees, dtype=np.int32) * n, n)
+    g = dict(n=n * trees, P=np.tile(one["P"], trees), keys=np.tile(one["keys"], trees), action=np.tile(one["action"], trees),
+             cb=np.where(np.tile(one["cc"], trees) > 0, np.tile(one["cb"], trees) + shift, 0).astype(np.int32),
+             cc=np.tile(one["cc"], trees))
+    roots = np.arange(trees, dtype=np.int32) * n
+    f, ref, alias, total, (b, sp, tt) = search_both(g, 91, batches=8, B=trees, max_depth=6, log2=14, roots=roots)
+    assert total[3] > 0
+    rng = np.random.default_rng(92)
+    for step in range(3):
+        b.set_roots(roots)
+        tt.select_redirect(b, sp)
+        paths, plen, _, _ = b.read()
+        met = paths[paths >= 0]
+        assert len(np.unique(met)) < len(met)
+        now = f.download()
+        f.upload(dict(as_soa(g, rng), **now))
+        assert (f.download_redirects() == -1).all()
+        soa = dict(as_soa(g, rng), **{k: v.copy() for k, v in now.items()})
+        again = R.RefTree.from_soa(soa)
+        if how == "backup":
+            values = rng.uniform(-1, 1, trees).astype(np.float32)
+            b.set_values(values)
+            b.backup(3)
+            again.backup_batch(paths, plen, values, 3)
+        else:
+            b.revert_vl(3)
+            again.revert_vl_paths(paths, plen, 3)
+        got = f.download()
+        assert (got["N"] == again.N).all() and (got["VL"] == again.VL).all()
+        assert np.allclose(got["W"], again.W, rtol=0, atol=1e-5 * np.sqrt(trees))
