@@ -162,7 +162,7 @@ struct omk_batch {
     int32_t spin_limit = 1 << 18;  // polls of about a microsecond: a quarter of a second, a selection takes a millisecond
     int32_t n_cus = 0;
     int32_t n_items0 = 0;
-    int32_t *out = nullptr;  // the leaf gather in pinned memory (see gather)
+    int32_t *out = nullptr;  // the leaf gather in pinned memory (see gather): allocated with the batch
     size_t out_bytes = 0;
     ExportOut gathered = {};      // its parts
     // which selection it is of (the forest's and the batch's counts when it was made): an expansion takes leaves,
@@ -170,8 +170,8 @@ struct omk_batch {
     int64_t select_calls = 0, gathered_call = -1, gathered_changes = -1;
     // The gather that a selection of lone traversals has made itself (lone_rows): its call, the forest's changes
     // before it, its number, and the point of the stream it lies at (Staging::now).  read_call: the selection that
-    // was read last.
-    int64_t lone_call = -1, lone_changes = -1, read_call = -1;
+    // was read last, and before the first one as if there had been one.
+    int64_t lone_call = -1, lone_changes = -1, read_call = 0;
     int32_t lone_seq = 0;
     uint64_t lone_staged = 0;
     std::vector<int32_t> leaf_table;  // work space of an expansion
@@ -1100,6 +1100,17 @@ int omk_forest_node_count(omk_forest *f, int64_t *h_nodes, int64_t *h_capacity) 
 
 // ---------------------------------------------------------------- batch
 
+}  // extern "C"
+
+// 32-bit words of a leaf gather: lengths | leaves | their child counts | their visit counts | abort words | paths | actions
+static size_t gather_words(size_t n, size_t depth) { return n * (2 * depth + 5) + 4; }
+// What a batch's pinned buffer holds from the start; a batch whose gather takes more gets the rest when it is read.
+// (Allocated with the batch, 20 us: the first step of a batch of 256 took 65 us when its read had to do that, and 43
+// so, the later ones 37.)
+constexpr size_t kGatherBytes = 16 << 20;
+
+extern "C" {
+
 int omk_batch_create(omk_forest *f, int32_t max_traversals, int32_t max_depth, omk_batch **out) {
     if (!f || !out) return fail(OMK_ERR_INVALID, "omk_batch_create: null argument");
     if (max_traversals <= 0 || max_traversals > (1 << 24))
@@ -1155,6 +1166,8 @@ int omk_batch_create(omk_forest *f, int32_t max_traversals, int32_t max_depth, o
     if (e == hipSuccess) e = hipMemset(b->single_ready, 0, (size_t)std::max(max_traversals, 1) * 4);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&b->n_cus, hipDeviceAttributeMultiprocessorCount, f->device);
     if (e == hipSuccess) e = hipMemset(b->values, 0, (size_t)B * 4);
+    b->out_bytes = std::min(kGatherBytes, gather_words((size_t)B, (size_t)max_depth) * 4);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&b->out, b->out_bytes, hipHostMallocDefault);
     if (e != hipSuccess) {
         int rc = fail(OMK_ERR_HIP, "omk_batch_create: %s", hipGetErrorString(e));
         omk_batch_destroy(b);
@@ -1185,8 +1198,7 @@ int omk_batch_destroy(omk_batch *b) {
 // Where the leaf gather of the batch goes: its pinned buffer, laid out for the paths there are.
 static int gather_room(omk_batch *b, ExportOut *o) {
     const size_t n = (size_t)b->n, D = (size_t)b->max_depth;
-    // lengths | leaves | their child counts | their visit counts | abort words | paths | actions
-    const size_t need = (n * (2 * D + 5) + 4) * 4;
+    const size_t need = gather_words(n, D) * 4;
     if (need > b->out_bytes) {
         if (b->out) {
             HIP_TRY(hipStreamSynchronize(b->f->stream));
@@ -1194,7 +1206,7 @@ static int gather_room(omk_batch *b, ExportOut *o) {
         }
         b->out = nullptr;
         b->out_bytes = 0;
-        const size_t room = ((size_t)b->stride * (2 * D + 5) + 4) * 4;
+        const size_t room = gather_words((size_t)b->stride, D) * 4;
         HIP_TRY(hipHostMalloc((void **)&b->out, room, hipHostMallocDefault));
         b->out_bytes = room;
     }
@@ -1208,8 +1220,8 @@ static int gather_room(omk_batch *b, ExportOut *o) {
     return OMK_OK;
 }
 
-// A selection whose traversals are all alone at their roots, in a batch whose selection before was read: its
-// walkers send their own rows (export_lone), and the read finds them there.  Small batches only: the rows of a
+// A selection whose traversals are all alone at their roots, in a batch whose selection before was read (or that has
+// none before: most batches are read): its walkers send their own rows (export_lone), and the read finds them there.  Small batches only: the rows of a
 // large one leave in better pieces by a kernel of their own.
 constexpr int kLoneRowsMax = 1024;
 static int lone_rows(omk_batch *b, LoneOut *out) {

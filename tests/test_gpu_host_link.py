@@ -452,3 +452,29 @@ def test_values_staged_behind_a_lone_selection_arrive_whole():
         assert err.max() <= 1e-5, step  # (the trees' own sums are no multiples of 1/64)
         ref.W[:] = got["W"]
         first, second = second, first
+
+
+# what a batch needs to be read and expanded it has from its creation: the device's mappings stay as they are
+@pytest.mark.parametrize("n,depth", [(1, 5), (40, 12), (3000, 30)])
+def test_the_first_read_and_expansion_of_a_batch_allocate_nothing(n, depth):
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(3, n_expand=300, fanout=(1, 5), max_depth=10, n_roots=40)
+
+    def mapped():
+        with open("/proc/self/maps") as lines:
+            return {line.split()[0] for line in lines if "/dev/" in line}
+
+    begin = np.arange(n + 1, dtype=np.int32)
+    moves = np.zeros(n, np.int32)
+    f = omk.Forest.from_soa(soa, capacity=len(soa["N"]) + 4 * n)
+    for fresh in (False, True):  # (the first batch brings in the kernels)
+        b = omk.Batch(f, n, depth)
+        b.set_roots(roots[np.arange(n) % 40])
+        before = mapped()
+        for _ in range(2):
+            b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+            b.read()
+            b.expand(begin, moves)
+            b.revert_vl(3)
+        assert not fresh or mapped() == before
+        b.close()
