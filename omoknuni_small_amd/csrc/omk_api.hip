@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -162,8 +163,9 @@ struct omk_batch {
     int32_t spin_limit = 1 << 18;  // polls of about a microsecond: a quarter of a second, a selection takes a millisecond
     int32_t n_cus = 0;
     int32_t n_items0 = 0;
-    int32_t *out = nullptr;  // the leaf gather in pinned memory (see gather): allocated with the batch
+    int32_t *out = nullptr;  // the leaf gather in pinned memory (see gather), out_bytes of it
     size_t out_bytes = 0;
+    std::unique_ptr<int32_t[]> heads;  // the leaves and their counts of a gather that crossed in pieces
     ExportOut gathered = {};      // its parts
     // which selection it is of (the forest's and the batch's counts when it was made): an expansion takes leaves,
     // child counts and visit counts from it while nothing has changed them
@@ -1102,9 +1104,24 @@ int omk_forest_node_count(omk_forest *f, int64_t *h_nodes, int64_t *h_capacity) 
 
 }  // extern "C"
 
-// 32-bit words of a leaf gather: lengths | leaves | their child counts | their visit counts | abort words | paths | actions
-static size_t gather_words(size_t n, size_t depth) { return n * (2 * depth + 5) + 4; }
-// What a batch's pinned buffer holds from the start; a batch whose gather takes more gets the rest when it is read.
+// 32-bit words of the leaf gather of n traversals: lengths | leaves | their child counts | their visit counts | abort
+// words | paths and actions, if they are asked for
+static size_t gather_words(size_t n, size_t depth, bool paths, bool actions) {
+    return n * (4 + (paths ? depth + 1 : 0) + (actions ? depth : 0)) + 4;
+}
+static ExportOut gather_layout(int32_t *at, size_t n, size_t depth, bool paths, bool actions) {
+    ExportOut o = {};
+    o.len = at;
+    o.leaf = o.len + n;
+    o.children = o.leaf + n;
+    o.visits = o.children + n;
+    o.abort = o.visits + n;
+    int32_t *rows = o.abort + 4;
+    if (paths) o.paths = rows;
+    if (actions) o.actions = rows + (paths ? n * (depth + 1) : 0);
+    return o;
+}
+// Pinned memory of a batch for its gather, at most: a larger gather crosses in pieces.
 // (Allocated with the batch, 20 us: the first step of a batch of 256 took 65 us when its read had to do that, and 43
 // so, the later ones 37.)
 constexpr size_t kGatherBytes = 16 << 20;
@@ -1166,7 +1183,7 @@ int omk_batch_create(omk_forest *f, int32_t max_traversals, int32_t max_depth, o
     if (e == hipSuccess) e = hipMemset(b->single_ready, 0, (size_t)std::max(max_traversals, 1) * 4);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&b->n_cus, hipDeviceAttributeMultiprocessorCount, f->device);
     if (e == hipSuccess) e = hipMemset(b->values, 0, (size_t)B * 4);
-    b->out_bytes = std::min(kGatherBytes, gather_words((size_t)B, (size_t)max_depth) * 4);
+    b->out_bytes = std::min(kGatherBytes, gather_words((size_t)B, (size_t)max_depth, true, true) * 4);
     if (e == hipSuccess) e = hipHostMalloc((void **)&b->out, b->out_bytes, hipHostMallocDefault);
     if (e != hipSuccess) {
         int rc = fail(OMK_ERR_HIP, "omk_batch_create: %s", hipGetErrorString(e));
@@ -1195,31 +1212,6 @@ int omk_batch_destroy(omk_batch *b) {
 
 }  // extern "C"
 
-// Where the leaf gather of the batch goes: its pinned buffer, laid out for the paths there are.
-static int gather_room(omk_batch *b, ExportOut *o) {
-    const size_t n = (size_t)b->n, D = (size_t)b->max_depth;
-    const size_t need = gather_words(n, D) * 4;
-    if (need > b->out_bytes) {
-        if (b->out) {
-            HIP_TRY(hipStreamSynchronize(b->f->stream));
-            HIP_TRY(hipHostFree(b->out));
-        }
-        b->out = nullptr;
-        b->out_bytes = 0;
-        const size_t room = gather_words((size_t)b->stride, D) * 4;
-        HIP_TRY(hipHostMalloc((void **)&b->out, room, hipHostMallocDefault));
-        b->out_bytes = room;
-    }
-    o->len = b->out;
-    o->leaf = o->len + n;
-    o->children = o->leaf + n;
-    o->visits = o->children + n;
-    o->abort = o->visits + n;
-    o->paths = o->abort + 4;
-    o->actions = o->paths + n * (D + 1);
-    return OMK_OK;
-}
-
 // A selection whose traversals are all alone at their roots, in a batch whose selection before was read (or that has
 // none before: most batches are read): its walkers send their own rows (export_lone), and the read finds them there.  Small batches only: the rows of a
 // large one leave in better pieces by a kernel of their own.
@@ -1227,7 +1219,8 @@ constexpr int kLoneRowsMax = 1024;
 static int lone_rows(omk_batch *b, LoneOut *out) {
     memset(out, 0, sizeof(*out));
     if (b->n_items0 > 0 || b->n > kLoneRowsMax || b->max_depth >= 64 || b->read_call != b->select_calls) return OMK_OK;
-    if (int rc = gather_room(b, &out->rows)) return rc;
+    static_assert((kLoneRowsMax * (2 * 63 + 5) + 4) * 4 <= kGatherBytes, "the rows fit the batch's pinned buffer");
+    out->rows = gather_layout(b->out, (size_t)b->n, (size_t)b->max_depth, true, true);
     for (int i = 0; i < 4; i++) out->rows.abort[i] = 0;  // (these kernels wait for nobody)
     out->sig = link_signal(b->f);
     b->lone_call = b->select_calls + 1;
@@ -1550,21 +1543,63 @@ int omk_backup_paths(omk_forest *f, const int32_t *d_paths, const int32_t *d_pat
 
 }  // extern "C"
 
-// The leaf gather of the last selection into the batch's pinned buffer; waits for it.
-static int gather(omk_batch *b, bool paths, bool actions) {
+// The leaf gather of the last selection: lengths, leaves and their counts to `gathered`, paths and actions to the
+// caller's arrays (if given); waits for it.  What fits the pinned buffer crosses in one piece.  More crosses in pieces
+// of half of it, the host copying one out while the next is on its way.
+static int gather(omk_batch *b, int32_t *h_paths, int32_t *h_actions) {
     omk_forest *f = b->f;
-    ExportOut &o = b->gathered;
+    const size_t n = (size_t)b->n, D = (size_t)b->max_depth;
+    const bool paths = h_paths != nullptr, actions = h_actions != nullptr;
+    auto copy_rows = [&](const ExportOut &o, size_t t0, size_t m) {
+        if (paths) memcpy(h_paths + t0 * (D + 1), o.paths, m * (D + 1) * 4);
+        if (actions) memcpy(h_actions + t0 * D, o.actions, m * D * 4);
+    };
+    auto ask = [&](const ExportOut &o, size_t t0, size_t m, const HostSignal &sig) {
+        return launch_export(f->dev(), b->paths + t0, b->path_len + t0, b->leaf + t0, b->counters + 3 * kSchedStep + 1,
+                             (int)m, b->stride, b->max_depth, o, sig, f->stream);
+    };
     b->gathered_call = -1;
-    if (int rc = gather_room(b, &o)) return rc;
     if (b->lone_call == b->select_calls && b->lone_changes == f->changes) {
+        b->gathered = gather_layout(b->out, n, D, true, true);
         if (int rc = link_wait_for(f, b->lone_seq)) return rc;
         f->staging.ran_to(b->lone_staged);  // (link_wait waits for the last call; another batch's may be on their way)
-    } else {
-        if (!paths) o.paths = nullptr;
-        if (!actions) o.actions = nullptr;
-        HIP_TRY(launch_export(f->dev(), b->paths, b->path_len, b->leaf, b->counters + 3 * kSchedStep + 1, b->n, b->stride,
-                              b->max_depth, o, link_signal(f), f->stream));
+        copy_rows(b->gathered, 0, n);
+    } else if (gather_words(n, D, paths, actions) * 4 <= b->out_bytes) {
+        b->gathered = gather_layout(b->out, n, D, paths, actions);
+        HIP_TRY(ask(b->gathered, 0, n, link_signal(f)));
         if (int rc = link_wait(f)) return rc;
+        copy_rows(b->gathered, 0, n);
+    } else {
+        const size_t half = b->out_bytes / 8;  // words
+        const size_t most = (half - 4) / (gather_words(1, D, paths, actions) - 4) / 64 * 64;
+        static_assert((kGatherBytes / 8 - 4) / (2 * 4096 + 5) >= 64, "a piece holds 64 traversals at any depth");
+        if (!b->heads) b->heads.reset(new (std::nothrow) int32_t[4 * (size_t)b->stride + 4]);
+        if (!b->heads) return fail(OMK_ERR_INVALID, "out of host memory");
+        const ExportOut all = gather_layout(b->heads.get(), n, D, false, false);
+        const size_t pieces = (n + most - 1) / most;
+        ExportOut o[2];
+        int32_t seq[2] = {0, 0};
+        for (size_t c = 0; c <= pieces; c++) {
+            if (c < pieces) {
+                const size_t m = std::min(most, n - c * most);
+                o[c & 1] = gather_layout(b->out + (c & 1) * half, m, D, paths, actions);
+                const HostSignal sig = link_signal(f);
+                seq[c & 1] = sig.seq;
+                HIP_TRY(ask(o[c & 1], c * most, m, sig));
+            }
+            if (c == 0) continue;
+            const ExportOut &p = o[(c - 1) & 1];
+            const size_t t0 = (c - 1) * most, m = std::min(most, n - t0);
+            if (int rc = link_wait_for(f, seq[(c - 1) & 1])) return rc;
+            copy_rows(p, t0, m);
+            memcpy(all.len + t0, p.len, m * 4);
+            memcpy(all.leaf + t0, p.leaf, m * 4);
+            memcpy(all.children + t0, p.children, m * 4);
+            memcpy(all.visits + t0, p.visits, m * 4);
+            memcpy(all.abort, p.abort, 16);
+        }
+        f->staging.idle();
+        b->gathered = all;
     }
     b->gathered_call = b->select_calls;
     b->gathered_changes = f->changes;
@@ -1613,7 +1648,7 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
     // The leaves with their child and visit counts: a search has just read them (omk_batch_read brings all
     // three), and one that has not gathers them now.
     if (b->gathered_call != b->select_calls || b->gathered_changes != f->changes)
-        if (int rc = gather(b, false, false)) return rc;
+        if (int rc = gather(b, nullptr, nullptr)) return rc;
     const int32_t *leaf = b->gathered.leaf, *children = b->gathered.children, *visits = b->gathered.visits;
     // One job per distinct leaf: the first traversal (in index order) that offers moves wins.  A leaf that has
     // children already (the selection stopped at it because of the depth bound) is left alone and takes no ids.
@@ -1717,12 +1752,10 @@ int omk_batch_read(omk_batch *b, int32_t *h_paths, int32_t *h_path_len, int32_t 
     if (int rc = fresh_batch("omk_batch_read", b)) return rc;
     omk_forest *f = b->f;
     if (int rc = use_device(f)) return rc;
-    const size_t n = (size_t)b->n, D = (size_t)b->max_depth;
+    const size_t n = (size_t)b->n;
     b->read_call = b->select_calls;
-    if (int rc = gather(b, h_paths != nullptr, h_actions != nullptr)) return rc;
+    if (int rc = gather(b, h_paths, h_actions)) return rc;
     const ExportOut &o = b->gathered;
-    if (h_paths) memcpy(h_paths, o.paths, n * (D + 1) * 4);
-    if (h_actions) memcpy(h_actions, o.actions, n * D * 4);
     if (h_path_len) memcpy(h_path_len, o.len, n * 4);
     if (h_leaf) memcpy(h_leaf, o.leaf, n * 4);
     const int32_t *ab = o.abort;  // abort flag and what the wavefront that raised it was waiting for

@@ -455,7 +455,8 @@ def test_values_staged_behind_a_lone_selection_arrive_whole():
 
 
 # what a batch needs to be read and expanded it has from its creation: the device's mappings stay as they are
-@pytest.mark.parametrize("n,depth", [(1, 5), (40, 12), (3000, 30)])
+# (the largest takes more than the 16 MB of pinned memory a batch has for it: it crosses in pieces)
+@pytest.mark.parametrize("n,depth", [(1, 5), (40, 12), (3000, 30), (90_000, 30)])
 def test_the_first_read_and_expansion_of_a_batch_allocate_nothing(n, depth):
     import omoknuni_small_amd as omk
     soa, roots = random_tree(3, n_expand=300, fanout=(1, 5), max_depth=10, n_roots=40)
@@ -478,3 +479,45 @@ def test_the_first_read_and_expansion_of_a_batch_allocate_nothing(n, depth):
             b.revert_vl(3)
         assert not fresh or mapped() == before
         b.close()
+
+
+# a gather of more than 16 MB crosses in pieces of half of that: one traversal short of it, one beyond, pieces that
+# end with the last traversal and that do not, the deepest paths there are
+@pytest.mark.parametrize("n,depth", [(64_527, 30), (64_528, 30), (3 * 32_256, 30), (3 * 32_256 + 1, 30), (577, 4096)])
+def test_gathers_in_pieces(n, depth):
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(9, n_expand=900, fanout=(1, 5), max_depth=40, n_roots=300)
+    ref = R.RefTree.from_soa(soa)
+    troots = roots[np.arange(n) % 300]
+    rpaths, rlen, rleaf, _ = ref.select_batch(troots, R.make_params(c_puct=1.4, virtual_loss=3, max_depth=depth))
+    f = omk.Forest.from_soa(soa, capacity=ref.n + 3 * n)
+    b = omk.Batch(f, n, depth)
+    b.set_roots(troots)
+    b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+    paths, plen, leaf, actions = b.read()
+    assert (paths == rpaths).all() and (plen == rlen).all() and (leaf == rleaf).all()
+    assert (actions == ref.gather_actions(rpaths, rlen)).all()
+    # and what an expansion takes from it
+    begin = np.arange(n + 1, dtype=np.int32) * 3
+    moves = np.tile(np.int32([4, 1, 7]), n)
+    assert (b.expand(begin, moves) == ref.expand_batch(rleaf, begin, moves)).all()
+
+
+# an expansion that has to gather the leaves itself, of so many traversals that they cross in pieces
+def test_an_expansion_of_more_than_a_million_traversals():
+    import omoknuni_small_amd as omk
+    n = (1 << 20) + 77
+    zeros = np.zeros(n, np.int32)
+    soa = dict(N=zeros, W=np.zeros(n, np.float32), P=np.ones(n, np.float32), VL=zeros, child_begin=zeros,
+               child_count=zeros, action=zeros - 1)
+    f = omk.Forest.from_soa(soa, capacity=2 * n)
+    b = omk.Batch(f, n, 3)
+    b.set_roots(np.arange(n, dtype=np.int32))
+    b.select(omk.SelectParams(c_puct=1.4, virtual_loss=1))
+    counts = (np.arange(n) % 3 > 0).astype(np.int32)  # every third position is over
+    begin = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    first = b.expand(begin, np.arange(begin[-1], dtype=np.int32))
+    assert (first == np.where(counts > 0, n + begin[:-1], -1)).all()
+    sx = f.download_structure()
+    assert (sx["child_begin"][:n][counts > 0] == first[counts > 0]).all() and (sx["child_count"][:n] == counts).all()
+    assert (sx["action"][n:] == np.arange(begin[-1])).all()
