@@ -177,7 +177,7 @@ struct omk_batch {
     int32_t lone_seq = 0;
     uint64_t lone_staged = 0;
     std::vector<int32_t> leaf_table;  // work space of an expansion
-    std::vector<int32_t> winners;
+    std::vector<int32_t> winners, counts;
     long long *trace = nullptr;  // records of the timeline, kTraceCap of them
     std::vector<int32_t> order, order_tmp;  // work space of omk_batch_set_roots
     std::vector<Item> items_h, singles_h;
@@ -233,31 +233,27 @@ static hipError_t dalloc(T **p, int64_t count) {
 // So a call's inputs are copied into the staging part of this block, which the kernels read through the host
 // link, and its results come back into pinned memory, followed by the call's number in the flag word.
 // Staging is handed out front to back; once a call has seen its flag everything enqueued before has run, and
-// the next one starts at the front again.
-constexpr size_t kLinkHead = 4096;         // flag word, and behind it (64 bytes on) the results of small calls
-constexpr size_t kLinkStaging = 4 << 20;   // staging a forest starts with (30 us to allocate, like 4 KiB)
-static hipError_t link_alloc(omk_forest *f, size_t staging) {
-    char *p = nullptr;
-    hipError_t e = hipHostMalloc((void **)&p, kLinkHead + staging, hipHostMallocDefault);
+// the next one starts at the front again.  It stays as large as it is: a call with more than that sends it in pieces.
+constexpr size_t kLinkHead = 4096;         // the flag word, on a page of its own
+constexpr size_t kLinkStaging = 4 << 20;   // (30 us to allocate, like 4 KiB)
+constexpr size_t kLinkPiece = 1 << 20;     // what does not fit goes in pieces of this, four of them on their way
+static hipError_t link_alloc(omk_forest *f) {
+    hipError_t e = hipHostMalloc((void **)&f->link, kLinkHead + kLinkStaging, hipHostMallocDefault);
     if (e != hipSuccess) return e;
-    if (f->link) (void)hipHostFree(f->link);
-    f->link = p;
-    f->staging.replace(staging);
-    *(int32_t *)p = f->link_seq;
+    f->staging = Staging(kLinkStaging);
+    *(int32_t *)f->link = f->link_seq;
     return hipSuccess;
 }
 
-// `bytes` of staging, aligned to a cache line; valid until the next call that waits for the stream.
+// `bytes` (at most kLinkStaging) of staging, aligned to a cache line; valid until the next call that waits for the
+// stream.
 static int link_stage(omk_forest *f, size_t bytes, void **out) {
     size_t at = f->staging.take(bytes);
     if (at == Staging::kFull) {
         HIP_TRY(hipStreamSynchronize(f->stream));
         f->staging.idle();
         at = f->staging.take(bytes);
-        if (at == Staging::kFull) {
-            HIP_TRY(link_alloc(f, bytes + bytes / 2 + 128));
-            at = f->staging.take(bytes);
-        }
+        if (at == Staging::kFull) return fail(OMK_ERR_INVALID, "%zu bytes of staging", bytes);
     }
     *out = f->link + kLinkHead + at;
     return OMK_OK;
@@ -375,8 +371,7 @@ static int bulk_get(omk_forest *f, const Bulk &b) {
     return OMK_OK;
 }
 
-// `words` 32-bit words of device memory to the host; waits for the stream.  Up to kLinkStaging bytes through the
-// pinned block (8 us), more by the runtime's copy into pageable memory.
+// `words` 32-bit words of device memory (at most kLinkStaging bytes) to the host; waits for the stream: 8 us.
 static int link_fetch(omk_forest *f, void *h_dst, const void *d_src, size_t words) {
     void *staged = nullptr;
     if (int rc = link_stage(f, words * 4, &staged)) return rc;
@@ -442,7 +437,7 @@ int omk_forest_create(const omk_forest_desc *desc, omk_forest **out) {
     if (e == hipSuccess && f->has_rave) e = dalloc(&f->Q2, n);
     if (e == hipSuccess) e = dalloc(&f->link_count, 64);
     if (e == hipSuccess) e = launch_fill_words(f->link_count, 0u, 64, f->own_stream);
-    if (e == hipSuccess) e = link_alloc(f, kLinkStaging);
+    if (e == hipSuccess) e = link_alloc(f);
     if (e != hipSuccess) {
         int rc = fail(OMK_ERR_HIP, "omk_forest_create: %s", hipGetErrorString(e));
         omk_forest_destroy(f);
@@ -758,13 +753,17 @@ int omk_forest_set_keys(omk_forest *f, const int32_t *h_nodes, const uint64_t *h
     if (n == 0) return OMK_OK;
     int64_t bad = 0;
     for (int64_t i = 0; i < n; i++) bad += h_nodes[i] < 0 || h_nodes[i] >= f->n_nodes;
-    void *staged = nullptr;
-    if (int rc = link_stage(f, (size_t)n * 12, &staged)) return rc;
-    uint64_t *keys = (uint64_t *)staged;
-    int32_t *nodes = (int32_t *)(keys + n);
-    memcpy(keys, h_keys, (size_t)n * 8);
-    memcpy(nodes, h_nodes, (size_t)n * 4);
-    HIP_TRY(launch_set_keys(f->hash, nodes, keys, n, f->n_nodes, s));
+    const int64_t most = (size_t)n * 12 <= kLinkStaging ? n : (int64_t)kLinkPiece / 12;
+    for (int64_t at = 0; at < n; at += most) {
+        const int64_t m = std::min(most, n - at);
+        void *staged = nullptr;
+        if (int rc = link_stage(f, (size_t)m * 12, &staged)) return rc;
+        uint64_t *keys = (uint64_t *)staged;
+        int32_t *nodes = (int32_t *)(keys + m);
+        memcpy(keys, h_keys + at, (size_t)m * 8);
+        memcpy(nodes, h_nodes + at, (size_t)m * 4);
+        HIP_TRY(launch_set_keys(f->hash, nodes, keys, m, f->n_nodes, s));
+    }
     if (bad) return fail(OMK_ERR_INVALID, "omk_forest_set_keys: %lld node ids outside the forest (skipped)", (long long)bad);
     return OMK_OK;
 }
@@ -1370,19 +1369,29 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) {
     // Every path starts at its root: written here once, not by every selection (the wavefront that takes a
     // crowded root would spend its first microseconds on thousands of path entries)
     const size_t words = (size_t)n * 2 + (items.size() + singles.size()) * (sizeof(Item) / 4);
-    void *staged = nullptr;
-    if (int rc = link_stage(f, words * 4, &staged)) return rc;
-    int32_t *at = (int32_t *)staged;
-    memcpy(at, order.data(), (size_t)n * 4);
-    memcpy(at + n, h_roots, (size_t)n * 4);
-    if (!items.empty()) memcpy(at + 2 * (size_t)n, items.data(), items.size() * sizeof(Item));
-    if (!singles.empty())
-        memcpy(at + 2 * (size_t)n + items.size() * (sizeof(Item) / 4), singles.data(), singles.size() * sizeof(Item));
     // The next selection's reset comes along (k_set_roots), unless its call number starts over or, with every
     // traversal alone at its root, it needs none (launch_select).
-    const int32_t next = !items.empty() && b->epoch < (1 << 30) - 2 ? b->epoch + 1 : 0;
-    HIP_TRY(launch_set_roots(select_args(b, next), b->seg0, b->items0, b->singles0, at, n, (int)items.size(),
-                             (int)singles.size(), n_hctx0, next > 0, f->stream));
+    int32_t next = !items.empty() && b->epoch < (1 << 30) - 2 ? b->epoch + 1 : 0;
+    if (words * 4 <= kLinkStaging) {
+        void *staged = nullptr;
+        if (int rc = link_stage(f, words * 4, &staged)) return rc;
+        int32_t *at = (int32_t *)staged;
+        memcpy(at, order.data(), (size_t)n * 4);
+        memcpy(at + n, h_roots, (size_t)n * 4);
+        if (!items.empty()) memcpy(at + 2 * (size_t)n, items.data(), items.size() * sizeof(Item));
+        if (!singles.empty())
+            memcpy(at + 2 * (size_t)n + items.size() * (sizeof(Item) / 4), singles.data(), singles.size() * sizeof(Item));
+        HIP_TRY(launch_set_roots(select_args(b, next), b->seg0, b->items0, b->singles0, at, n, (int)items.size(),
+                                 (int)singles.size(), n_hctx0, next > 0, f->stream));
+    } else {  // in pieces, and the selection makes its own reset
+        next = 0;
+        Bulk up;
+        up.add(b->seg0, 1, order.data(), n);
+        up.add(b->paths, 1, h_roots, n);
+        up.add(b->items0, 1, items.data(), (int64_t)(items.size() * (sizeof(Item) / 4)));
+        up.add(b->singles0, 1, singles.data(), (int64_t)(singles.size() * (sizeof(Item) / 4)));
+        if (int rc = bulk_put(f, up)) return rc;
+    }
     b->prepared = next;
     b->most_visitors = items.empty() ? 1 : items[0].m;
     b->n_items0 = (int32_t)items.size();
@@ -1398,11 +1407,9 @@ int omk_batch_set_values(omk_batch *b, const float *h_values, int32_t n) {
     if (!b || !h_values) return fail(OMK_ERR_INVALID, "omk_batch_set_values: null argument");
     if (n <= 0 || n > b->max_traversals) return fail(OMK_ERR_CAPACITY, "omk_batch_set_values: %d values", n);
     if (int rc = use_device(b->f)) return rc;
-    void *staged = nullptr;
-    if (int rc = link_stage(b->f, (size_t)n * 4, &staged)) return rc;
-    memcpy(staged, h_values, (size_t)n * 4);
-    HIP_TRY(launch_copy_words(b->values, staged, n, b->f->stream));
-    return OMK_OK;
+    Bulk up;
+    up.add(b->values, 1, h_values, n);
+    return bulk_put(b->f, up);
 }
 
 int omk_batch_device(omk_batch *b, omk_batch_dev *out) {
@@ -1655,9 +1662,10 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
     // The leaves met so far: open addressing, at most half full.
     int bits = 4;
     while ((1 << bits) < 2 * n) bits++;
-    std::vector<int32_t> &table = b->leaf_table, &winners = b->winners;
+    std::vector<int32_t> &table = b->leaf_table, &winners = b->winners, &counts = b->counts;
     table.assign((size_t)1 << bits, -1);
     winners.clear();
+    counts.clear();
     int64_t cursor = f->n_nodes;
     for (int t = 0; t < n; t++) {
         const int32_t offered = h_move_begin[t + 1] - h_move_begin[t];
@@ -1668,8 +1676,8 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
         table[h] = leaf[t];
         if (children[t] != 0) continue;
         winners.push_back(t);
-        // MCTSNode::expand: max_reasonable_moves
-        cursor += widened_children(std::min(offered, 1000), visits[t], params);
+        counts.push_back(widened_children(std::min(offered, 1000), visits[t], params));  // expand's max_reasonable_moves
+        cursor += counts.back();
     }
     if (cursor > f->capacity)
         return fail(OMK_ERR_CAPACITY, "omk_expand_batch_ex: %lld nodes needed, capacity %lld", (long long)cursor,
@@ -1678,53 +1686,61 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
     if (h_first_child)
         for (int t = 0; t < n; t++) h_first_child[t] = -1;
     if (winners.empty()) return OMK_OK;
-    // staged for the kernel: jobs | moves | priors
-    const size_t nj = winners.size(), nm = (size_t)(cursor - f->n_nodes);
-    void *staged = nullptr;
-    if (int rc = link_stage(f, nj * sizeof(ExpandJob) + nm * 8, &staged)) return rc;
-    ExpandJob *jobs = (ExpandJob *)staged;
-    int32_t *moves = (int32_t *)(jobs + nj);
-    float *priors = (float *)(moves + nm);
-    bool sorted = f->prior_sorted;  // (once they are not, no later child makes it so)
-    int mf = f->max_fanout;
-    cursor = f->n_nodes;
     f->made_node.clear();
     f->made_count.clear();
-    size_t off = 0;
-    for (size_t wi = 0; wi < nj; wi++) {
-        const int32_t t = winners[wi];
-        const int32_t cnt = widened_children(std::min(h_move_begin[t + 1] - h_move_begin[t], 1000), visits[t], params);
-        // MCTSNode::setPriorProbabilities (:512-593) is only called with a policy that is not empty
-        // (mcts_engine_batch_tree_simple.cpp:256-258); otherwise expand's uniform prior stays
-        const int32_t psize = h_policy_begin ? h_policy_begin[t + 1] - h_policy_begin[t] : 0;
-        const float *pol = psize > 0 ? h_policy + h_policy_begin[t] : nullptr;
-        jobs[wi] = ExpandJob{leaf[t], (int32_t)cursor, cnt, (int32_t)off};
-        const int32_t *mv = h_moves + h_move_begin[t];
-        float *pr = priors + off;
-        if (pol && psize == action_space) {  // a policy over the action space (:537-560); the moves along with it
-            gather_priors(mv, cnt, pol, action_space, moves + off, pr);
-        } else if (pol && psize == cnt) {  // one value per child, by child index (:561-575)
-            memcpy(moves + off, mv, (size_t)cnt * 4);
-            for (int32_t i = 0; i < cnt; i++) pr[i] = std::min(1.0f, std::max(0.0f, pol[i]));
-        } else {  // expand(): uniform prior; a policy of neither size likewise (:576-584)
-            memcpy(moves + off, mv, (size_t)cnt * 4);
-            for (int32_t i = 0; i < cnt; i++) pr[i] = 1.0f / (float)cnt;
+    // staged for the kernel: jobs | moves | priors, in one piece if that fits, else in pieces of whole jobs (8 KB the
+    // largest); the forest has grown with every piece
+    const size_t whole = winners.size() * sizeof(ExpandJob) + (size_t)(cursor - f->n_nodes) * 8;
+    const size_t most = whole <= kLinkStaging ? whole : kLinkPiece;
+    for (size_t w0 = 0; w0 < winners.size();) {
+        size_t w1 = w0, nm = 0;
+        while (w1 < winners.size() && (w1 + 1 - w0) * sizeof(ExpandJob) + (nm + (size_t)counts[w1]) * 8 <= most)
+            nm += (size_t)counts[w1++];
+        const size_t nj = w1 - w0;
+        void *staged = nullptr;
+        if (int rc = link_stage(f, nj * sizeof(ExpandJob) + nm * 8, &staged)) return rc;
+        ExpandJob *jobs = (ExpandJob *)staged;
+        int32_t *moves = (int32_t *)(jobs + nj);
+        float *priors = (float *)(moves + nm);
+        bool sorted = f->prior_sorted;  // (once they are not, no later child makes it so)
+        int mf = f->max_fanout;
+        cursor = f->n_nodes;
+        size_t off = 0;
+        for (size_t wi = 0; wi < nj; wi++) {
+            const int32_t t = winners[w0 + wi], cnt = counts[w0 + wi];
+            // MCTSNode::setPriorProbabilities (:512-593) is only called with a policy that is not empty
+            // (mcts_engine_batch_tree_simple.cpp:256-258); otherwise expand's uniform prior stays
+            const int32_t psize = h_policy_begin ? h_policy_begin[t + 1] - h_policy_begin[t] : 0;
+            const float *pol = psize > 0 ? h_policy + h_policy_begin[t] : nullptr;
+            jobs[wi] = ExpandJob{leaf[t], (int32_t)cursor, cnt, (int32_t)off};
+            const int32_t *mv = h_moves + h_move_begin[t];
+            float *pr = priors + off;
+            if (pol && psize == action_space) {  // a policy over the action space (:537-560); the moves along with it
+                gather_priors(mv, cnt, pol, action_space, moves + off, pr);
+            } else if (pol && psize == cnt) {  // one value per child, by child index (:561-575)
+                memcpy(moves + off, mv, (size_t)cnt * 4);
+                for (int32_t i = 0; i < cnt; i++) pr[i] = std::min(1.0f, std::max(0.0f, pol[i]));
+            } else {  // expand(): uniform prior; a policy of neither size likewise (:576-584)
+                memcpy(moves + off, mv, (size_t)cnt * 4);
+                for (int32_t i = 0; i < cnt; i++) pr[i] = 1.0f / (float)cnt;
+            }
+            for (int32_t i = 1; i < cnt && sorted; i++) sorted = !(pr[i] > pr[i - 1]);
+            if (h_first_child) h_first_child[t] = (int32_t)cursor;
+            f->made_node.push_back(leaf[t]);
+            f->made_count.push_back(cnt);
+            off += (size_t)cnt;
+            cursor += cnt;
+            mf = std::max(mf, (int)cnt);
         }
-        for (int32_t i = 1; i < cnt && sorted; i++) sorted = !(pr[i] > pr[i - 1]);
-        if (h_first_child) h_first_child[t] = (int32_t)cursor;
-        f->made_node.push_back(leaf[t]);
-        f->made_count.push_back(cnt);
-        off += (size_t)cnt;
-        cursor += cnt;
-        mf = std::max(mf, (int)cnt);
+        HIP_TRY(launch_expand(f->mut(), jobs, (int)nj, moves, priors, f->n_nodes, cursor, f->stream));
+        f->n_nodes = cursor;
+        f->changes++;
+        f->grown = true;
+        f->structure_changed = true;  // ids keep their meaning, but an upload of the old arrays would not
+        f->max_fanout = mf;
+        f->prior_sorted = sorted;
+        w0 = w1;
     }
-    HIP_TRY(launch_expand(f->mut(), jobs, (int)nj, moves, priors, f->n_nodes, cursor, f->stream));
-    f->n_nodes = cursor;
-    f->changes++;
-    f->grown = true;
-    f->structure_changed = true;  // ids keep their meaning, but an upload of the old arrays would not
-    f->max_fanout = mf;
-    f->prior_sorted = sorted;
     return OMK_OK;
 }
 

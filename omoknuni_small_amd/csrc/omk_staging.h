@@ -17,11 +17,6 @@ public:
 
     explicit Staging(size_t room = 0) : room_(room) {}
     size_t room() const { return room_; }
-    // another block in the place of the old one, which no kernel reads any more
-    void replace(size_t room) {
-        room_ = room;
-        used_ = 0;
-    }
 
     // `bytes`, rounded up to a cache line: their offset, or kFull when they do not fit behind what is in use
     size_t take(size_t bytes) {

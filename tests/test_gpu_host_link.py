@@ -9,6 +9,12 @@ from tests.helpers import random_tree
 pytestmark = pytest.mark.gpu
 
 
+def mapped():
+    """The process's mappings of device and pinned memory."""
+    with open("/proc/self/maps") as lines:
+        return {line.split()[0] for line in lines if "/dev/" in line}
+
+
 # the gather takes 64 traversals x 32 depths at a time (a path has one node more than the depth bound)
 @pytest.mark.parametrize("depth", [1, 30, 31, 32, 33, 70])
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 300])
@@ -460,11 +466,6 @@ def test_values_staged_behind_a_lone_selection_arrive_whole():
 def test_the_first_read_and_expansion_of_a_batch_allocate_nothing(n, depth):
     import omoknuni_small_amd as omk
     soa, roots = random_tree(3, n_expand=300, fanout=(1, 5), max_depth=10, n_roots=40)
-
-    def mapped():
-        with open("/proc/self/maps") as lines:
-            return {line.split()[0] for line in lines if "/dev/" in line}
-
     begin = np.arange(n + 1, dtype=np.int32)
     moves = np.zeros(n, np.int32)
     f = omk.Forest.from_soa(soa, capacity=len(soa["N"]) + 4 * n)
@@ -521,3 +522,73 @@ def test_an_expansion_of_more_than_a_million_traversals():
     sx = f.download_structure()
     assert (sx["child_begin"][:n][counts > 0] == first[counts > 0]).all() and (sx["child_count"][:n] == counts).all()
     assert (sx["action"][n:] == np.arange(begin[-1])).all()
+
+
+# roots, values and keys beyond the 4 MB of staging cross in pieces, and take no pinned memory beside it
+@pytest.mark.parametrize("doubled", [0, 70_000])
+def test_large_batches_are_handed_over_in_pieces(doubled):
+    import omoknuni_small_amd as omk
+    n_roots, n = 400_000, 400_000 + doubled  # the first roots have two traversals each
+    rng = np.random.default_rng(doubled)
+    nodes = 3 * n_roots
+    soa = dict(N=rng.integers(1, 9, nodes).astype(np.int32), W=rng.integers(-4, 5, nodes).astype(np.float32),
+               P=rng.random(nodes).astype(np.float32), VL=np.zeros(nodes, np.int32), child_begin=np.zeros(nodes, np.int32),
+               child_count=np.zeros(nodes, np.int32), action=np.tile(np.arange(3, dtype=np.int32), n_roots),
+               hash=np.zeros(nodes, np.uint64))
+    soa["child_begin"][:n_roots], soa["child_count"][:n_roots] = n_roots + 2 * np.arange(n_roots), 2
+    troots = rng.permutation(np.arange(n, dtype=np.int32) % n_roots)
+    ref = R.RefTree.from_soa(soa)
+    rpaths, rlen, rleaf, _ = ref.select_batch(troots, R.make_params(c_puct=1.4, virtual_loss=3, max_depth=2))
+    keys = rng.permutation(np.arange(1, nodes + 1, dtype=np.uint64))
+    values = (rng.integers(-64, 65, n) / 64.0).astype(np.float32)
+    for fresh in (False, True):  # (the first forest brings in the kernels)
+        f = omk.Forest.from_soa(soa)
+        b = omk.Batch(f, n, 2)
+        before = mapped()
+        b.set_roots(troots)
+        b.set_values(values)
+        f.set_keys(np.arange(nodes, dtype=np.int32), keys)
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+        paths, plen, leaf, _ = b.read()
+        assert not fresh or mapped() == before
+        assert (paths == rpaths).all() and (plen == rlen).all() and (leaf == rleaf).all()
+        if not fresh:
+            b.close()
+            f.close()
+    table = omk.TranspositionTable(f, 21)
+    table.insert(keys[::3], np.arange(nodes, dtype=np.int32)[::3])
+    assert (table.probe_leaves(b) == np.where(leaf % 3 == 0, leaf, -1)).all()
+    b.backup(3)
+    ref.backup_batch(rpaths, rlen, values, 3)
+    got = f.download()
+    assert (got["N"] == ref.N).all() and (got["VL"] == ref.VL).all() and (got["W"] == ref.W).all()
+
+
+# offers of more than 4 MB: pieces of whole leaves, with a legal mask (whose words pieces share) and without
+@pytest.mark.parametrize("mask", [0.0, 0.3])
+@pytest.mark.parametrize("moves,n", [(1000, 700), (33, 16_500)])
+def test_an_expansion_in_pieces(moves, n, mask):
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(12, n_expand=300, fanout=(1, 3), max_depth=2, n_roots=n, mask_frac=mask, vl_frac=0.0)
+    ref = R.RefTree.from_soa(soa)
+    f = omk.Forest.from_soa(soa, capacity=ref.n + n * moves)
+    b = omk.Batch(f, n, 4)
+    b.set_roots(roots[:n])
+    rleaf = ref.select_batch(roots[:n], R.make_params(c_puct=1.4, virtual_loss=3, max_depth=4))[2]
+    b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+    rng = np.random.default_rng(moves)
+    counts = rng.integers(moves - 3, moves + 1, n)
+    begin = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    mv = rng.integers(0, 1200, begin[-1]).astype(np.int32)
+    policy = rng.random(begin[-1]).astype(np.float32)  # one value a child
+    got = b.expand_ex(begin, mv, begin, policy, 2000)
+    assert (got == ref.expand_batch(rleaf, begin, mv, policy=policy, action_space=2000, policy_begin=begin)).all()
+    st, sx = f.download(), f.download_structure()
+    assert (st["N"] == ref.N).all() and st["P"].tobytes() == ref.P.tobytes() and (st["VL"] == ref.VL).all()
+    assert (sx["child_begin"] == ref.child_begin).all() and (sx["child_count"] == ref.child_count).all()
+    assert (sx["action"] == ref.action).all()
+    # the new children take part in the next selection as the checker has them
+    rpaths, rlen, _, _ = ref.select_batch(roots[:n], R.make_params(c_puct=1.4, virtual_loss=3, max_depth=4))
+    b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+    paths, plen, _, _ = b.read()
+    assert (paths == rpaths).all() and (plen == rlen).all()
