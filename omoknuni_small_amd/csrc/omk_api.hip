@@ -984,9 +984,23 @@ static int compact_in(omk_forest *f, int32_t new_root, int64_t *h_nodes_after, i
     return OMK_OK;
 }
 
-// Scratch of up to this much stays with the forest from one move to the next (a tree of a million nodes); more is
-// given back after the call.
+// Scratch of up to this much stays with the forest from one move to the next; more is given back after the call.
 constexpr size_t kKeepScratch = 64 << 20;
+
+// Words of CompactScratch::tmp for a forest of n nodes: every array at once (eight of 32-bit words and two of 64-bit
+// ones) as long as that stays within kKeepScratch, at least one 64-bit array.  A large tree passes through in more
+// rounds of two launches, which its nodes outweigh (12 M nodes: 9.5 ms, with every array at once 9.6), and takes at
+// most 24 bytes a node.
+constexpr int64_t compact_tmp_words(int64_t n) {
+    const int64_t kept = ((int64_t)kKeepScratch - (int64_t)kCompactFixed - 8 * (n + 63)) / 4;
+    return std::max(2 * n, std::min(12 * n, kept));
+}
+constexpr size_t compact_bytes(int64_t n) {
+    return kCompactFixed + ((size_t)n + 63) / 64 * 64 * 8 + (size_t)compact_tmp_words(n) * 4;
+}
+static_assert(compact_tmp_words(1 << 20) == 12 << 20, "a tree of a million nodes moves at once");
+static_assert(compact_bytes(1500000) <= kKeepScratch && compact_bytes(4000000) <= kKeepScratch, "kept");
+static_assert(compact_bytes(1 << 24) <= 24ull << 24 && compact_bytes(0x7FFFFFF0) <= 24ull * 0x7FFFFFF0, "24 bytes a node");
 
 extern "C" {
 
@@ -997,11 +1011,9 @@ int omk_forest_compact(omk_forest *f, int32_t new_root, int64_t *h_nodes_after, 
     if (int rc = tree_only("omk_forest_compact", f)) return rc;
     if (int rc = use_device(f)) return rc;
     const int64_t n = f->n_nodes;
-    // every array at once: eight of 32-bit words and two of 64-bit ones
     CompactScratch sc;
-    sc.tmp_words = 12 * n;
-    const size_t words = ((size_t)n + 63) / 64 * 64;
-    const size_t bytes = kCompactFixed + words * 8 + (size_t)sc.tmp_words * 4;
+    sc.tmp_words = compact_tmp_words(n);
+    const size_t words = ((size_t)n + 63) / 64 * 64, bytes = compact_bytes(n);
     if (bytes > f->scratch_bytes) {
         if (f->scratch) {
             HIP_TRY(hipStreamSynchronize(f->stream));

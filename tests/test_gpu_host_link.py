@@ -202,6 +202,59 @@ def test_compaction_of_every_shape(shape, static):
     assert (got["child_begin"] == ref.child_begin).all() and (got["child_count"] == ref.child_count).all()
 
 
+# trees whose arrays do not all fit the scratch at once: two rounds, and an array at a time
+@pytest.mark.parametrize("fan", [500, 1399])
+def test_compaction_of_large_trees(fan):
+    import omoknuni_small_amd as omk
+    rng = np.random.default_rng(fan)
+    upper = 1 + 3 + 3000  # the root, its children, theirs; `fan` children each of the latter, in falling order
+    n = upper + 3000 * fan
+    begin, count = np.zeros(n, np.int32), np.zeros(n, np.int32)
+    if fan > 1024:  # (two levels in the place of one)
+        wide = np.array([700, fan - 700])
+        n = upper + 3000 * 2 + 3000 * fan
+        begin, count = np.zeros(n, np.int32), np.zeros(n, np.int32)
+    begin[0], count[0] = 1, 3
+    begin[1:4], count[1:4] = 4 + 1000 * np.arange(3)[::-1], 1000
+    second = np.arange(4, upper)
+    levels = [np.array([0]), np.arange(1, 4), np.concatenate([np.arange(b, b + 1000) for b in begin[1:4]])]
+    if fan > 1024:
+        begin[second], count[second] = upper + 2 * np.arange(3000)[::-1], 2
+        third = np.arange(upper, upper + 6000)
+        count[third] = np.tile(wide, 3000)
+        begin[third] = upper + 6000 + np.concatenate([[0], np.cumsum(count[third])[:-1]])
+    else:
+        begin[second], count[second] = upper + fan * np.arange(3000)[::-1], fan
+    while count[levels[-1]].any():
+        up = levels[-1][count[levels[-1]] > 0]
+        step = np.repeat(begin[up] - np.concatenate([[0], np.cumsum(count[up])[:-1]]), count[up])
+        levels.append(step + np.arange(len(step)))
+    order = np.concatenate(levels)
+    assert len(order) == n
+    new_id = np.empty(n, np.int32)
+    new_id[order] = np.arange(n)
+    soa = dict(N=rng.integers(0, 99, n).astype(np.int32), W=rng.random(n).astype(np.float32), P=rng.random(n).astype(np.float32),
+               VL=rng.integers(0, 5, n).astype(np.int32), child_begin=begin, child_count=count,
+               action=rng.integers(0, 99, n).astype(np.int32), hash=rng.integers(0, 1 << 63, n).astype(np.uint64),
+               rN=rng.integers(0, 9, n).astype(np.int32), rW=rng.random(n).astype(np.float32))
+    f = omk.Forest.from_soa(soa)
+    assert (f.compact(0) == order).all()
+    got = dict(f.download(), **f.download_structure())
+    for k in ("N", "W", "P", "VL", "rN", "rW", "action"):
+        assert got[k].tobytes() == soa[k][order].tobytes(), k
+    assert (got["child_count"] == count[order]).all()
+    inner = count[order] > 0
+    assert (got["child_begin"][inner] == new_id[begin[order][inner]]).all()
+    # the keys have come along: a table filled by the new ids finds the leaves by them
+    table = omk.TranspositionTable(f, 12)
+    b = omk.Batch(f, 500, 5)
+    b.set_roots(np.zeros(500, np.int32))
+    b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+    leaf = np.unique(b.read()[2])
+    table.insert(soa["hash"][order[leaf]], leaf)
+    assert (table.probe_leaves(b) == b.read()[2]).all()
+
+
 # a young tree: the visitors spread over children without visits (up to 64 of them, one entry per lane)
 @pytest.mark.parametrize("children", [65, 130, 225, 362, 700])
 @pytest.mark.parametrize("n", [8, 23, 63, 64, 65])
