@@ -126,9 +126,16 @@ _EVERY_BATCH = {
 }
 
 
+# What the C library's allocator keeps at hand when it is freed, at most (the limit of its dynamic mmap threshold).
+_KEPT_BLOCK = 32 << 20
+
+
 def _together(n, **dtypes):
-    """Arrays of n 32-bit elements each, side by side in one block: one allocation that the C library keeps at hand
-    when it is freed, where several of a few megabytes each are given back and faulted in again every time."""
+    """Arrays of n 32-bit elements each.  Side by side in one block while the C library keeps a block of that size
+    at hand when it is freed, where several of a few megabytes each are given back and faulted in again every time (an
+    array that the caller keeps then keeps the block); larger ones on their own."""
+    if 4 * n * len(dtypes) > _KEPT_BLOCK:
+        return {k: np.empty(n, t) for k, t in dtypes.items()}
     block = np.empty((len(dtypes), n), np.int32)
     return {k: row.view(t) for (k, t), row in zip(dtypes.items(), block)}
 

@@ -213,3 +213,15 @@ def test_staging_is_not_handed_out_over_what_kernels_still_read(tmp_path):
                            "-o", exe])
     out = subprocess.run([exe, "3000"], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0 and out.stdout == "ok 3000\n", out.stdout
+
+
+@pytest.mark.parametrize("n", [0, 1, 300_000, 2_097_152, 2_097_153, 5_000_000])
+def test_one_downloaded_array_does_not_keep_a_large_tree_alive(n):
+    from omoknuni_small_amd import forest
+    got = forest._together(n, N=np.int32, W=np.float32, P=np.float32, VL=np.int32)
+    for k, a in got.items():
+        assert a.shape == (n,) and a.dtype == (np.float32 if k in "WP" else np.int32) and a.flags["C_CONTIGUOUS"]
+        owner = a
+        while owner.base is not None:
+            owner = owner.base
+        assert owner.nbytes <= max(32 << 20, a.nbytes)
