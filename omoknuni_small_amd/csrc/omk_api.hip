@@ -1224,13 +1224,20 @@ int omk_batch_destroy(omk_batch *b) {
 }  // extern "C"
 
 // A selection whose traversals are all alone at their roots, in a batch whose selection before was read (or that has
-// none before: most batches are read): its walkers send their own rows (export_lone), and the read finds them there.  Small batches only: the rows of a
-// large one leave in better pieces by a kernel of their own.
-constexpr int kLoneRowsMax = 1024;
+// none before: most batches are read): its walkers send their own rows (export_lone), and the read finds them there.
+// Small batches only.  A walker's row crosses the host link in pieces of its own, a kernel's in neighbouring lines, and
+// from some number of rows on that costs more than the launch saves; a path that a whole block walks ends with
+// wavefronts to spare for it.  A step with a read, us, rows by the walkers and by the kernel:
+//   walked by a block (a legal mask, more than 64 slots), 225 slots: 64 traversals 20.9 / 24.2, 256 25.9 / 27.4,
+//   350 29.7 / 27.7, 1024 39.8 / 33.6; 362 slots: 256 28.5 / 28.0 (in larger trees 31.0 / 31.6), 1024 54.5 / 38.7;
+//   walked by a wavefront, 225 slots re-laid: 64 22.4 / 24.0, 128 25.5 / 24.6, 256 29.2 / 26.7, 1024 50.3 / 33.0;
+//   chess-like: 64 23.4 / 25.2, 128 25.7 / 26.2, 200 29.7 / 28.0, 1024 53.4 / 38.5
+constexpr int kLoneRowsBlock = 256, kLoneRowsWave = 128;
 static int lone_rows(omk_batch *b, LoneOut *out) {
     memset(out, 0, sizeof(*out));
-    if (b->n_items0 > 0 || b->n > kLoneRowsMax || b->max_depth >= 64 || b->read_call != b->select_calls) return OMK_OK;
-    static_assert((kLoneRowsMax * (2 * 63 + 5) + 4) * 4 <= kGatherBytes, "the rows fit the batch's pinned buffer");
+    const int most = b->f->has_legal && b->f->max_fanout > 64 ? kLoneRowsBlock : kLoneRowsWave;
+    if (b->n_items0 > 0 || b->n > most || b->max_depth >= 64 || b->read_call != b->select_calls) return OMK_OK;
+    static_assert((kLoneRowsBlock * (2 * 63 + 5) + 4) * 4 <= kGatherBytes, "the rows fit the batch's pinned buffer");
     out->rows = gather_layout(b->out, (size_t)b->n, (size_t)b->max_depth, true, true);
     for (int i = 0; i < 4; i++) out->rows.abort[i] = 0;  // (these kernels wait for nobody)
     out->sig = link_signal(b->f);

@@ -4724,10 +4724,12 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_i
                            n_traversals, out);
         return hipGetLastError();
     }
+    // (rows of a wide masked layout are sent by the blocks above: a batch that sends rows is small enough for them)
     const bool rows = out.sig.flag != nullptr;
-    auto *kernel = !f.legal ? (rows ? k_select_singles<RMAX, RAVE, 0, true> : k_select_singles<RMAX, RAVE, 0, false>)
-                   : fast   ? (rows ? k_select_singles<RMAX, RAVE, 2, true> : k_select_singles<RMAX, RAVE, 2, false>)
-                            : (rows ? k_select_singles<RMAX, RAVE, 1, true> : k_select_singles<RMAX, RAVE, 1, false>);
+    auto *kernel = rows     ? (f.legal ? k_select_singles<RMAX, RAVE, RMAX == 1 ? 2 : 0, true> : k_select_singles<RMAX, RAVE, 0, true>)
+                   : !f.legal ? k_select_singles<RMAX, RAVE, 0, false>
+                   : fast     ? k_select_singles<RMAX, RAVE, 2, false>
+                              : k_select_singles<RMAX, RAVE, 1, false>;
     hipLaunchKernelGGL(kernel, grid, block, 0, s, f, a0, n_traversals, out);
     return hipGetLastError();
 }

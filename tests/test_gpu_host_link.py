@@ -645,3 +645,44 @@ def test_an_expansion_in_pieces(moves, n, mask):
     b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
     paths, plen, _, _ = b.read()
     assert (paths == rpaths).all() and (plen == rlen).all()
+
+
+# what an expansion takes from rows that the walkers have sent: the leaves, whether they have children already (the
+# depth bound) and their visits (the widening); sent by blocks up to 256 traversals, by wavefronts up to 128
+@pytest.mark.parametrize("n", [1, 3, 128, 129, 256, 257])
+@pytest.mark.parametrize("fanout,mask", [((1, 6), 0.0), ((1, 6), 0.4), ((60, 90), 0.4)])
+def test_expansion_after_lone_walkers_have_sent_their_rows(n, fanout, mask):
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(n + 17, n_expand=n + 30, fanout=fanout, max_depth=4, n_roots=n, mask_frac=mask, n_max=400, vl_frac=0.0)
+    depth = 2 if fanout[1] < 64 else 1  # so that some leaves have children
+    ref = R.RefTree.from_soa(soa)
+    moves, A = 60, 200
+    f = omk.Forest.from_soa(soa, capacity=ref.n + 3 * n * moves)
+    b = omk.Batch(f, n, depth)
+    b.set_roots(roots[:n])
+    rng = np.random.default_rng(n)
+    kept = widened = 0
+    for step in range(3):
+        rpaths, rlen, rleaf, _ = ref.select_batch(roots[:n], R.make_params(c_puct=1.4, virtual_loss=3, max_depth=depth))
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+        paths, plen, leaf, actions = b.read()
+        assert (paths == rpaths).all() and (plen == rlen).all() and (leaf == rleaf).all()
+        assert (actions == ref.gather_actions(rpaths, rlen)).all()
+        kept += int((ref.child_count[rleaf] > 0).sum())
+        begin = (np.arange(n + 1) * moves).astype(np.int32)
+        mv = np.concatenate([rng.permutation(A)[:moves] for _ in range(n)]).astype(np.int32)
+        policy = rng.random((n, A)).astype(np.float32)
+        at = ref.n
+        want = ref.expand_batch(rleaf, begin, mv, policy=policy, action_space=A, widening=(2.0, 0.5))
+        widened += int((ref.child_count[rleaf[want >= at]] > 8).sum())
+        got = b.expand_ex(begin, mv, (np.arange(n + 1) * A).astype(np.int32), policy, A, widening=(2.0, 0.5))
+        assert (got == want).all()
+        values = (rng.integers(-64, 65, n) / 64.0).astype(np.float32)
+        ref.backup_batch(rpaths, rlen, values, 3)
+        b.set_values(values)
+        b.backup(3)
+        st, sx = f.download(), f.download_structure()
+        ref.W[:] = st["W"]
+        assert (st["N"] == ref.N).all() and st["P"].tobytes() == ref.P.tobytes() and (st["VL"] == ref.VL).all()
+        assert (sx["child_begin"] == ref.child_begin).all() and (sx["child_count"] == ref.child_count).all()
+    assert n < 100 or (kept > 0 and widened > 0)
