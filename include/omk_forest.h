@@ -14,7 +14,9 @@
  *     host buffer it passes;
  *   - pointers named h_* are host pointers, d_* are device pointers;
  *   - all work of a forest is enqueued on one HIP stream (its own by default,
- *     see omk_forest_set_stream); calls that return data to the host wait for it;
+ *     see omk_forest_set_stream); calls that return data to the host wait for what they return;
+ *   - calls that take host arrays leave them free on return; what they carry is on the device in
+ *     stream order, so a consumer on another stream waits for the forest's (omk_sync, or an event);
  *   - one host thread drives a forest at a time.
  *
  * Node ids are int32 indices into the arrays; the children of node v are the ids
@@ -104,9 +106,10 @@ int omk_forest_set_stream(omk_forest *f, void *hip_stream);
 /* The hipStream_t the forest's work is enqueued on (to record events on it). */
 int omk_forest_get_stream(omk_forest *f, void **hip_stream_out);
 /* Checks that the arrays describe a forest (ranges in bounds, every node the child of at
- * most one parent, fan-out <= OMK_MAX_FANOUT) and copies them to the device.  Uploading the same
- * child ranges again (statistics put back) leaves batches usable; after an upload of another
- * structure their roots and paths are stale: OMK_ERR_STATE until omk_batch_set_roots. */
+ * most one parent, fan-out <= OMK_MAX_FANOUT) and copies them to the device, in stream order.
+ * Uploading the same child ranges again (statistics put back) leaves batches usable, their roots and
+ * the paths they hold; after an upload of another structure these are stale: OMK_ERR_STATE until
+ * omk_batch_set_roots. */
 int omk_forest_upload(omk_forest *f, const omk_soa_view *h_view);
 /* Copies N, W, P, VL (and rN, rW) back; structure pointers of the view are ignored. */
 int omk_forest_download(omk_forest *f, omk_soa_view *h_view);
@@ -142,12 +145,15 @@ int omk_soa_compact_legal(const omk_soa_view *h_view, int64_t count, int32_t *N,
 
 /* ---- batch: the per-search buffers of executeBatchedTreeSearch
  *      (leaf_nodes / paths / leaf_states, mcts_engine_batch_tree_simple.cpp:41-57) ---- */
+/* Beside its device memory a batch holds pinned host memory for the leaf gather: two words a path
+ * entry, at most 16 MB (a larger gather crosses in pieces). */
 int omk_batch_create(omk_forest *f, int32_t max_traversals, int32_t max_depth, omk_batch **out);
 int omk_batch_destroy(omk_batch *b);
 /* Traversal t starts at h_roots[t] (the reference: every simulation starts at root_,
  * mcts_engine_batch_tree_simple.cpp:86-92).  Distinct roots must head disjoint trees. */
 int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n_traversals);
-int omk_batch_set_values(omk_batch *b, const float *h_values, int32_t n); /* NetworkOutput::value of each leaf */
+/* NetworkOutput::value of each leaf, written to omk_batch_dev.d_values in stream order. */
+int omk_batch_set_values(omk_batch *b, const float *h_values, int32_t n);
 int omk_batch_device(omk_batch *b, omk_batch_dev *out);
 
 /* Phase 1 of executeBatchedTreeSearch (mcts_engine_batch_tree_simple.cpp:73-185): for
@@ -206,16 +212,16 @@ int omk_forest_reroot_child(omk_forest *f, int32_t root, int32_t last_action, in
  * *h_nodes_after = k; h_old_of_new (NULL or room for the old node count) receives the old id
  * of every new node.  Paths of earlier selections, roots of batches and node ids stored in
  * transposition tables refer to the old numbering: set roots again (a batch refuses to select,
- * back up, expand or read with OMK_ERR_STATE until then), clear the tables.  All
- * of it runs on the device: the renumbering level by level (child counts of a level, an
- * exclusive scan, the children's ids written to the next level), then one gather per array;
- * the host only reads the size of every level. */
+ * back up, expand or read with OMK_ERR_STATE until then), clear the tables.  All of it runs on the
+ * device: the renumbering level by level, twelve levels enqueued before the host looks whether there
+ * are more, then the arrays through scratch memory, as many at a time as it holds.  Scratch of up to
+ * 64 MB stays with the forest; a larger tree's (24 bytes a node at most) is given back. */
 int omk_forest_compact(omk_forest *f, int32_t new_root, int64_t *h_nodes_after, int32_t *h_old_of_new);
 
 /* omk_forest_compact for callers that cannot allocate device memory (code under HIP graph
  * capture around it, tight serving loops, harnesses that forbid hipMalloc); it has no counterpart
  * in the reference.  Same arguments, same result, but every piece of device scratch memory (the
- * breadth-first order, the per-level counts and their scan, the staging array the fields pass
+ * breadth-first order, the sums of a level, the staging array the fields pass
  * through) lives in one array inside the library that each GPU holds for the life of the process
  * (about 25 MiB), and the call makes no hipMalloc / hipFree.  Limit: the forest may hold at most
  * 2^20 = 1048576 nodes when it is called (OMK_ERR_CAPACITY beyond that, and nothing is changed).
@@ -277,7 +283,7 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
  * that do.  Needs a forest created with RAVE arrays.  Asynchronous on the forest's stream. */
 int omk_backup_rave_batch(omk_batch *b);
 
-/* Leaf gather (mcts_engine_batch_tree_simple.cpp:114,166-184): waits for the stream and
+/* Leaf gather (mcts_engine_batch_tree_simple.cpp:114,166-184): waits for the selection and
  * returns, per traversal, the path (row of max_depth+1 ids, -1 padded), its length, the
  * leaf node and the move list to replay on a clone of the root state (row of max_depth
  * actions, -1 padded).  Any pointer may be NULL. */
@@ -321,7 +327,7 @@ int omk_batch_set_trace(omk_batch *b, int32_t enabled);
  * other wavefronts publish.  Every wait is bounded; a wavefront that polls `polls` times in
  * vain raises an abort flag, all wavefronts leave, and omk_batch_read reports OMK_ERR_STATE
  * for that selection (its paths are incomplete; upload the statistics again before the next
- * one).  The default (about four million polls, seconds) is never reached in normal
+ * one).  The default (2^18 polls, about a quarter of a second) is never reached in normal
  * operation; tests of the error path set a tiny limit.  No counterpart in the reference. */
 int omk_batch_set_spin_limit(omk_batch *b, int32_t polls);
 /* The ready marks of the scheduler's queues are the number of the select call on the batch, which starts

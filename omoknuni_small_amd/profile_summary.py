@@ -170,7 +170,7 @@ def timeline(workload, warmup=8, levels=()):
     batch.select(sp)
     tr = batch.debug_trace()
     batch.enable_trace(False)
-    batch.read()  # reports a selection that was given up (and reuses the staging memory the records were in)
+    batch.read()  # reports a selection that was given up
     batch.backup(vl)
     t0 = tr[:, 0].min()
     start = (tr[:, 0] - t0) / 100.0  # microseconds
