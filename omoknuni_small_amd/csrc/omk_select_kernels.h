@@ -2418,7 +2418,10 @@ constexpr int kFewEntries = 4;  // entries of every child it evaluates
 // position, visit) is the serial order; and no child has all its evaluated entries above the threshold (declined),
 // so an entry not evaluated comes after one that is never reached.
 // A function of its own, and only in the kernel for trees that have grown on the device (SPREAD), whose nodes have
-// many children without visits: anywhere else its mere presence cost the other nodes 2 to 4 %.
+// many children without visits.  Where nodes like that are rare its mere presence costs the others (five registers of
+// the wide classes and their spills): launched for uploaded trees too, 64 visitors of a Gomoku tree took 85.3 us a pass
+// in the place of 83.3, 16 on each of 64 Go trees 133.6 in the place of 130.1; in the HEAVY kernels, 16384 on a Go tree
+// with RAVE 377.7 in the place of 365.6 (4096 on a chess-like tree the same).
 // Measured on an MI355X: a search of 64 visitors a batch from the bare root 1.51 -> 1.32 ms, of 48 with RAVE on a Go
 // board 1.74 -> 1.64.
 struct FewLds {
@@ -3185,8 +3188,9 @@ struct Continuation {
 //
 // HEAVY: the kernel for batches in which a node of kHeavyMin visitors can occur.  Without it (every root has fewer) the
 // slices, their boundaries and their joins are left out, and with them registers that the rest of the code then has
-// (narrow class 160 -> 145, four rounds 224 -> 216, six 276 -> 245): 64 visitors of a Gomoku tree 104.3 -> 98.9 us a
-// pass, 16 on each of 64 Go trees 124 -> 119, 8 on a tree 70 -> 68.
+// (vector registers: narrow class 160 -> 145, four rounds 224 -> 215, six 256 -> 245; scalar spills 302 -> 91, 461 -> 198,
+// 570 -> 211).  A pass with and without: 64 visitors of a Gomoku tree 81.9 and 79.3 us, 16 on each of 64 Go trees 134.3
+// and 126.2, 8 on a tree 60.3 and 55.5.
 // SPREAD: the kernel for trees that grow on the device, whose nodes have many children without visits (few_visitors).
 template <int R, bool RAVE, int RMAX, bool HEAVY, bool SPREAD>
 __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs &a, const NodeCtx &c, int lane,
