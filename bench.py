@@ -477,7 +477,8 @@ def measure(omk, synth, name, steps, warmup, seed, cpu_seconds, scale=1.0, parit
             "seeded_repeats": reps,
             "selection_steps": seeded_steps,
             "launch_covers": "the whole selection, HIP events around it on the forest's stream: " +
-                             ("k_select_reset + k_select_groups (teams and walkers in one persistent launch)"
+                             ("k_select_groups (teams and walkers in one persistent launch; its reset comes with "
+                              "omk_batch_set_roots, before the first event)"
                               if has_groups else
                               singles + " alone (no reset launch when every traversal is alone at its root)")
                              + "; rocprofv3's per-kernel averages add up to it",

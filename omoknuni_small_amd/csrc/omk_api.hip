@@ -172,8 +172,8 @@ struct omk_batch {
     int64_t select_calls = 0, gathered_call = -1, gathered_changes = -1;
     // The gather that a selection of lone traversals has made itself (lone_rows): its call, the forest's changes
     // before it, its number, and the point of the stream it lies at (Staging::now).  read_call: the selection that
-    // was read last, and before the first one as if there had been one.
-    int64_t lone_call = -1, lone_changes = -1, read_call = 0;
+    // was read last.
+    int64_t lone_call = -1, lone_changes = -1, read_call = -1;
     int32_t lone_seq = 0;
     uint64_t lone_staged = 0;
     std::vector<int32_t> leaf_table;  // work space of an expansion
@@ -1223,9 +1223,10 @@ int omk_batch_destroy(omk_batch *b) {
 
 }  // extern "C"
 
-// A selection whose traversals are all alone at their roots, in a batch whose selection before was read (or that has
-// none before: most batches are read): its walkers send their own rows (export_lone), and the read finds them there.
-// Small batches only.  A walker's row crosses the host link in pieces of its own, a kernel's in neighbouring lines, and
+// A selection whose traversals are all alone at their roots, in a batch whose selection before was read: its walkers
+// send their own rows (export_lone), and the read finds them there.  (Not in a batch that nobody has read yet: its
+// evaluator may be on the card, the selection part of a captured graph; the first read makes one launch more.)  Small
+// batches only.  A walker's row crosses the host link in pieces of its own, a kernel's in neighbouring lines, and
 // from some number of rows on that costs more than the launch saves; a path that a whole block walks ends with
 // wavefronts to spare for it.  A step with a read, us, rows by the walkers and by the kernel:
 //   walked by a block (a legal mask, more than 64 slots), 225 slots: 64 traversals 20.9 / 24.2, 256 25.9 / 27.4,
@@ -1241,7 +1242,6 @@ static int lone_rows(omk_batch *b, LoneOut *out) {
     out->rows = gather_layout(b->out, (size_t)b->n, (size_t)b->max_depth, true, true);
     for (int i = 0; i < 4; i++) out->rows.abort[i] = 0;  // (these kernels wait for nobody)
     out->sig = link_signal(b->f);
-    b->lone_call = b->select_calls + 1;
     b->lone_changes = b->f->changes;
     b->lone_seq = out->sig.seq;
     b->lone_staged = b->f->staging.now();
@@ -1500,6 +1500,7 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
     b->selected = true;
     b->disjoint = b->n_items0 == 0;  // a root each, and distinct roots head disjoint trees
     b->select_calls++;
+    b->lone_call = out.sig.flag ? b->select_calls : -1;
     return OMK_OK;
 }
 
