@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -35,6 +36,10 @@ static int fail(int code, const char *fmt, ...) {
         hipError_t e_ = (expr);                                                                    \
         if (e_ != hipSuccess) return fail(OMK_ERR_HIP, "%s: %s", #expr, hipGetErrorString(e_));    \
     } while (0)
+
+// No C++ exception crosses the C boundary: what ends the entry points that hold host vectors.
+#define OMK_NO_THROW \
+    catch (const std::exception &e_) { return fail(OMK_ERR_INVALID, "out of host memory (%s)", e_.what()); }
 
 struct omk_forest {
     int device = 0;
@@ -567,7 +572,7 @@ static int validate(const omk_soa_view *v, int64_t n, int *max_fanout, bool *pri
     return OMK_OK;
 }
 
-int omk_forest_upload(omk_forest *f, const omk_soa_view *v) {
+int omk_forest_upload(omk_forest *f, const omk_soa_view *v) try {
     if (!f || !v) return fail(OMK_ERR_INVALID, "omk_forest_upload: null argument");
     const int64_t n = v->n_nodes;
     if (n <= 0 || n > f->capacity)
@@ -633,7 +638,7 @@ int omk_forest_upload(omk_forest *f, const omk_soa_view *v) {
         f->blend_valid = true;
     }
     return OMK_OK;
-}
+} OMK_NO_THROW
 
 int omk_forest_download(omk_forest *f, omk_soa_view *v) {
     if (!f || !v) return fail(OMK_ERR_INVALID, "omk_forest_download: null argument");
@@ -671,7 +676,7 @@ int64_t omk_soa_count_legal(const omk_soa_view *v) {
 
 int omk_soa_compact_legal(const omk_soa_view *v, int64_t count, int32_t *N, float *W, float *P, int32_t *VL,
                           int32_t *rN, float *rW, int32_t *child_begin, int32_t *child_count, int32_t *action,
-                          uint64_t *hash, int32_t *old_to_new, int32_t *new_to_old) {
+                          uint64_t *hash, int32_t *old_to_new, int32_t *new_to_old) try {
     if (!v || !N || !W || !P || !VL || !child_begin || !child_count)
         return fail(OMK_ERR_INVALID, "omk_soa_compact_legal: N, W, P, VL, child_begin, child_count are required");
     const int64_t n = v->n_nodes;
@@ -718,7 +723,7 @@ int omk_soa_compact_legal(const omk_soa_view *v, int64_t count, int32_t *N, floa
         }
     }
     return OMK_OK;
-}
+} OMK_NO_THROW
 
 int omk_forest_download_structure(omk_forest *f, int64_t n_nodes, int32_t *h_child_begin, int32_t *h_child_count,
                                   int32_t *h_action) {
@@ -1326,7 +1331,7 @@ static void order_by_root(const int32_t *roots, int32_t n, std::vector<int32_t> 
 
 extern "C" {
 
-int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) {
+int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) try {
     if (!b || !h_roots) return fail(OMK_ERR_INVALID, "omk_batch_set_roots: null argument");
     if (n <= 0 || n > b->max_traversals)
         return fail(OMK_ERR_CAPACITY, "omk_batch_set_roots: %d traversals, batch holds %d", n, b->max_traversals);
@@ -1420,7 +1425,7 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) {
     b->generation = f->generation;
     b->selected = false;
     return OMK_OK;
-}
+} OMK_NO_THROW
 
 int omk_batch_set_values(omk_batch *b, const float *h_values, int32_t n) {
     if (!b || !h_values) return fail(OMK_ERR_INVALID, "omk_batch_set_values: null argument");
@@ -1662,7 +1667,7 @@ static int32_t widened_children(int32_t legal, int32_t visits, const omk_expand_
 }
 
 int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t *h_moves, const int32_t *h_policy_begin,
-                        const float *h_policy, const omk_expand_params *params, int32_t *h_first_child) {
+                        const float *h_policy, const omk_expand_params *params, int32_t *h_first_child) try {
     if (!b || !h_move_begin || !h_moves || !params) return fail(OMK_ERR_INVALID, "omk_expand_batch_ex: null argument");
     if (!b->selected) return fail(OMK_ERR_STATE, "omk_expand_batch_ex: no selected paths");
     if (int rc = fresh_batch("omk_expand_batch_ex", b)) return rc;
@@ -1770,10 +1775,10 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
         w0 = w1;
     }
     return OMK_OK;
-}
+} OMK_NO_THROW
 
 int omk_expand_batch(omk_batch *b, const int32_t *h_move_begin, const int32_t *h_moves, const float *h_policy,
-                     int32_t action_space, int32_t *h_first_child) {
+                     int32_t action_space, int32_t *h_first_child) try {
     if (!b || !h_move_begin || !h_moves) return fail(OMK_ERR_INVALID, "omk_expand_batch: null argument");
     if (h_policy && action_space <= 0)
         return fail(OMK_ERR_INVALID, "omk_expand_batch: a policy needs action_space > 0 (got %d)", action_space);
@@ -1788,7 +1793,7 @@ int omk_expand_batch(omk_batch *b, const int32_t *h_move_begin, const int32_t *h
         for (int32_t t = 0; t <= b->n; t++) pb[(size_t)t] = t * action_space;
     }
     return omk_expand_batch_ex(b, h_move_begin, h_moves, h_policy ? pb.data() : nullptr, h_policy, &p, h_first_child);
-}
+} OMK_NO_THROW
 
 int omk_batch_read(omk_batch *b, int32_t *h_paths, int32_t *h_path_len, int32_t *h_leaf, int32_t *h_actions) {
     if (!b) return fail(OMK_ERR_INVALID, "omk_batch_read: null batch");

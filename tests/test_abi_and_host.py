@@ -225,3 +225,23 @@ def test_one_downloaded_array_does_not_keep_a_large_tree_alive(n):
         while owner.base is not None:
             owner = owner.base
         assert owner.nbytes <= max(32 << 20, a.nbytes)
+
+
+def test_no_exception_crosses_the_c_boundary():
+    """More nodes than a host vector can hold: a status, not an abort (in a process of its own, should it be one)."""
+    program = """
+import ctypes as C
+import numpy as np
+from omoknuni_small_amd import forest as F
+lib = F.load_library()
+a = dict(N=np.zeros(4, np.int32), W=np.zeros(4, np.float32), P=np.zeros(4, np.float32), VL=np.zeros(4, np.int32), rN=None,
+         rW=None, child_begin=np.zeros(4, np.int32), child_count=np.zeros(4, np.int32), action=None, legal=None, hash=None)
+v = F._view_of(a)
+v.n_nodes = 1 << 61
+i, f = F._ptr(a["N"], F.i32p), F._ptr(a["W"], F.f32p)
+none = C.c_void_p()
+print(lib.omk_soa_compact_legal(C.byref(v), C.c_int64(4), i, f, f, i, none, none, i, i, none, none, none, none),
+      lib.omk_last_error().decode())
+"""
+    r = subprocess.run([sys.executable, "-c", program], capture_output=True, text=True, cwd=ROOT)
+    assert r.returncode == 0 and r.stdout.startswith("-1 out of host memory"), (r.returncode, r.stdout, r.stderr[-500:])
