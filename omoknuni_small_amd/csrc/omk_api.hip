@@ -145,6 +145,7 @@ struct omk_batch {
     Item *items0 = nullptr, *items_q = nullptr, *singles0 = nullptr, *singles_q = nullptr;
     int32_t n_singles0 = 0;
     int32_t most_visitors = 1;  // of one root
+    bool in_order = true;       // the traversals' roots ascend
     int32_t n_hctx0 = 0;  // contexts of heavy roots, handed out when the roots are set
     int32_t *seg0 = nullptr, *seg[2] = {nullptr, nullptr};
     int32_t *sc_child = nullptr, *sc_occ = nullptr;
@@ -1228,22 +1229,33 @@ int omk_batch_destroy(omk_batch *b) {
 
 }  // extern "C"
 
-// A selection whose traversals are all alone at their roots, in a batch whose selection before was read: its walkers
-// send their own rows (export_lone), and the read finds them there.  (Not in a batch that nobody has read yet: its
-// evaluator may be on the card, the selection part of a captured graph; the first read makes one launch more.)  Small
-// batches only.  A walker's row crosses the host link in pieces of its own, a kernel's in neighbouring lines, and
+// A selection whose traversals are all alone at their roots, or few at each, in a batch whose selection before was read:
+// its walkers or blocks send their own rows (export_lone, k_select_blocks), and the read finds them there.  (Not in a
+// batch that nobody has read yet: its evaluator may be on the card, the selection part of a captured graph; the first
+// read makes one launch more.)  Small batches only.  A walker's row crosses the host link in pieces of its own, a kernel's in neighbouring lines, and
 // from some number of rows on that costs more than the launch saves; a path that a whole block walks ends with
 // wavefronts to spare for it.  A step with a read, us, rows by the walkers and by the kernel:
 //   walked by a block (a legal mask, more than 64 slots), 225 slots: 64 traversals 20.9 / 24.2, 256 25.9 / 27.4,
 //   350 29.7 / 27.7, 1024 39.8 / 33.6; 362 slots: 256 28.5 / 28.0 (in larger trees 31.0 / 31.6), 1024 54.5 / 38.7;
 //   walked by a wavefront, 225 slots re-laid: 64 22.4 / 24.0, 128 25.5 / 24.6, 256 29.2 / 26.7, 1024 50.3 / 33.0;
 //   chess-like: 64 23.4 / 25.2, 128 25.7 / 26.2, 200 29.7 / 28.0, 1024 53.4 / 38.5
-constexpr int kLoneRowsBlock = 256, kLoneRowsWave = 128;
+// A batch of few visitors a root (omk_select_blocks.h) sends a root's rows together.  What costs there is a line of the
+// host's memory that blocks on several XCDs write parts of: the rows of 2 to 8 roots whose traversals alternate, and of
+// many roots with less than 8 visitors each, are the kernel's.  A read of traversals on 225 slots, us, rows by the
+// blocks and by the kernel: 1 root x 64 53 / 53; 2 x 32 with the roots in order 37.2 / 38.8, alternating
+// 53.4 / 39.2; 8 x 32 49.6 / 53.1 and 62.6 / 53.4; 16 x 32 55.2 / 59.2 and 53.8 / 58.8; steps of 64 x 16 54.8 / 62.1,
+// 64 x 64 107 / 131, of 256 x 4 46.2 / 45.7, 512 x 2 56 / 48, 1024 x 2 92 / 71.
+constexpr int kLoneRowsBlock = 256, kLoneRowsWave = 128, kBlockRows = 4096;
+constexpr int kBlockRowsRoots = 16, kBlockRowsVisitors = 8;
 static int lone_rows(omk_batch *b, LoneOut *out) {
     memset(out, 0, sizeof(*out));
-    const int most = b->f->has_legal && b->f->max_fanout > 64 ? kLoneRowsBlock : kLoneRowsWave;
-    if (b->n_items0 > 0 || b->n > most || b->max_depth >= 64 || b->read_call != b->select_calls) return OMK_OK;
-    static_assert((kLoneRowsBlock * (2 * 63 + 5) + 4) * 4 <= kGatherBytes, "the rows fit the batch's pinned buffer");
+    const int roots = b->n_items0 + b->n_singles0;
+    const bool whole_lines = roots == 1 || (b->n >= kBlockRowsVisitors * roots && (b->in_order || roots >= kBlockRowsRoots));
+    int most = b->f->has_legal && b->f->max_fanout > 64 ? kLoneRowsBlock : kLoneRowsWave;
+    if (b->n_items0 > 0)
+        most = by_blocks(b->n_items0, b->most_visitors, b->f->max_fanout) && whole_lines ? kBlockRows : 0;
+    if (b->n > most || b->max_depth >= 64 || b->read_call != b->select_calls) return OMK_OK;
+    static_assert((kBlockRows * (2 * 63 + 5) + 4) * 4 <= kGatherBytes, "the rows fit the batch's pinned buffer");
     out->rows = gather_layout(b->out, (size_t)b->n, (size_t)b->max_depth, true, true);
     for (int i = 0; i < 4; i++) out->rows.abort[i] = 0;  // (these kernels wait for nobody)
     out->sig = link_signal(b->f);
@@ -1308,7 +1320,8 @@ static SelectArgs select_args(omk_batch *b, int32_t epoch) {
 // The traversals in ascending order of their roots, those of one root in ascending order: what a stable sort
 // gives.  One root for all, and roots that ascend already (one traversal per tree), are in order as they are; else
 // a radix sort, eleven bits a pass, as many passes as the largest root has digits.
-static void order_by_root(const int32_t *roots, int32_t n, std::vector<int32_t> &order, std::vector<int32_t> &tmp) {
+// Returns whether they ascend already.
+static bool order_by_root(const int32_t *roots, int32_t n, std::vector<int32_t> &order, std::vector<int32_t> &tmp) {
     order.resize((size_t)n);
     bool ascending = true;
     int32_t top = 0;
@@ -1317,7 +1330,7 @@ static void order_by_root(const int32_t *roots, int32_t n, std::vector<int32_t> 
         ascending &= t == 0 || roots[t - 1] <= roots[t];
         top = std::max(top, roots[t]);
     }
-    if (ascending) return;
+    if (ascending) return true;
     tmp.resize((size_t)n);
     for (int shift = 0; shift == 0 || (top >> shift) > 0; shift += 11) {
         int32_t start[2049] = {0};
@@ -1327,6 +1340,7 @@ static void order_by_root(const int32_t *roots, int32_t n, std::vector<int32_t> 
         order.swap(tmp);
         if (shift == 22) break;
     }
+    return false;
 }
 
 extern "C" {
@@ -1343,7 +1357,7 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) try {
                         t, (long long)f->n_nodes);
     // level-0 work items: traversals grouped by root, ascending traversal index inside a group
     std::vector<int32_t> &order = b->order;
-    order_by_root(h_roots, n, order, b->order_tmp);
+    const bool in_order = order_by_root(h_roots, n, order, b->order_tmp);
     std::vector<Item> &items = b->items_h, &singles = b->singles_h;
     items.clear();
     singles.clear();
@@ -1394,8 +1408,9 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) try {
     // crowded root would spend its first microseconds on thousands of path entries)
     const size_t words = (size_t)n * 2 + (items.size() + singles.size()) * (sizeof(Item) / 4);
     // The next selection's reset comes along (k_set_roots), unless its call number starts over or, with every
-    // traversal alone at its root, it needs none (launch_select).
-    int32_t next = !items.empty() && b->epoch < (1 << 30) - 2 ? b->epoch + 1 : 0;
+    // traversal alone at its root or few at each, it needs none (launch_select).
+    const bool blocks = by_blocks((int)items.size(), items.empty() ? 1 : items[0].m, f->max_fanout);
+    int32_t next = !items.empty() && !blocks && b->epoch < (1 << 30) - 2 ? b->epoch + 1 : 0;
     if (words * 4 <= kLinkStaging) {
         void *staged = nullptr;
         if (int rc = link_stage(f, words * 4, &staged)) return rc;
@@ -1422,6 +1437,7 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) try {
     b->n_hctx0 = n_hctx0;
     b->n_singles0 = (int32_t)singles.size();
     b->n = n;
+    b->in_order = in_order;
     b->generation = f->generation;
     b->selected = false;
     return OMK_OK;

@@ -129,7 +129,7 @@ struct ExportOut {
     int32_t *len, *leaf, *children, *visits;
     int32_t *abort;
 };
-// The leaf gather that the kernels of lone traversals write themselves; none with sig.flag NULL.  Both path arrays
+// The leaf gather that the kernels of lone traversals and of few visitors write themselves; none with sig.flag NULL.  Both path arrays
 // are there and max_depth is below 64.
 struct LoneOut {
     ExportOut rows;
@@ -141,6 +141,19 @@ struct LoneOut {
 hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, int n_singles0, int n_traversals,
                          int most_visitors, int max_fanout, bool rave, bool grown, int n_cus, int n_hctx0,
                          bool prepared, const LoneOut &out, hipStream_t s);
+
+// The same for a batch whose roots have few visitors each (omk_select_blocks.h): a block a root, without a reset.  The
+// line lies at a visitor per lane and at the children that fit its registers (with 128 for each of 16 wavefronts).  Below
+// it the blocks are the faster ones throughout, a step with its settling, us, of the queue's kernel and of theirs:
+// Gomoku 1 tree x 8 56 and 38, 1 x 64 76 and 54, 64 x 16 66 and 36, 64 x 64 80 and 75, 256 x 24 79 and 35, 4096 x 2 222
+// and 112; Go 64 x 16 125 and 74, chess-like 64 x 16 98 and 65, 2048 x 4 155 and 87.
+constexpr int kBlockMax = 64;       // visitors of one root, at most
+constexpr int kBlockFanout = 384;   // widest node
+inline bool by_blocks(int n_items0, int most_visitors, int max_fanout) {
+    return n_items0 > 0 && most_visitors <= kBlockMax && max_fanout <= kBlockFanout;
+}
+hipError_t launch_select_blocks(const ForestDev &f, const SelectArgs &a, int n_items, int n_singles, int max_fanout, bool rave,
+                                const LoneOut &out, hipStream_t s);
 
 // What omk_batch_set_roots has staged (n visitors | n roots | items | lone traversals) to the batch's arrays.
 // prepare: and what launch_select's reset does for the selection that `a` belongs to.

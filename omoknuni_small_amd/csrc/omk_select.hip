@@ -95,11 +95,13 @@ hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, 
     // own leaf and path length, so nothing has to be cleared first (the statistics apart).
     // Otherwise the reset launch.
     const bool alone = n_items0 == 0 && n_singles0 == n_traversals;
-    if ((!alone && !prepared) || a.stats || a.trace) {  // (the statistics and the timeline start at zero)
+    const bool blocks = by_blocks(n_items0, most_visitors, max_fanout);
+    if ((!alone && !blocks && !prepared) || a.stats || a.trace) {  // (the statistics and the timeline start at zero)
         int reset_blocks = (n_traversals + 255) / 256;
         hipLaunchKernelGGL(k_select_reset, dim3(reset_blocks), dim3(256), 0, s, a, n_items0, n_singles0,
                            n_traversals - n_singles0, n_traversals, n_hctx0);
     }
+    if (blocks) return launch_select_blocks(f, a, n_items0, n_singles0, max_fanout, rave, out, s);
 #define OMK_DISPATCH(RM)                                                              \
     return rave ? launch_select_class<RM, true>(f, a, n_items0, most_visitors, n_traversals, n_cus, grown, out, s) \
                 : launch_select_class<RM, false>(f, a, n_items0, most_visitors, n_traversals, n_cus, grown, out, s)

@@ -337,6 +337,9 @@ __device__ __forceinline__ int wave_pick(const Kids<R, RAVE> &k, int lane, uint3
     return (int)wave_min_u32(idx);
 }
 
+// A value that is the same in all lanes, for the compiler to know.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 struct NodeCtx {
     int cb;
     int cc;

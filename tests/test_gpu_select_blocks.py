@@ -1,0 +1,83 @@
+"""GPU parity of the selection of batches whose roots have at most 64 visitors each (a block a root) at the edges of what
+it takes: visitors of a root, fan-out classes, roots with one visitor among the others, depth bounds, values without a
+real score; and of the rows the blocks send to the host themselves."""
+import numpy as np
+import pytest
+
+from helpers import random_tree
+from oracle import ref_cpu as R
+from test_gpu_scheduler import layered_forest
+
+pytestmark = pytest.mark.gpu
+
+
+def both(soa, troots, D, vl=3, rave=False, pw=False, steps=4):
+    """Selections and backups on the device and by the checker; from the second on the rows come from the blocks."""
+    import omoknuni_small_amd as omk
+    ref = R.RefTree.from_soa(soa)
+    rp = R.make_params(c_puct=1.4, virtual_loss=vl, use_rave=rave, rave_k=1000.0, pw=pw, max_depth=D)
+    f = omk.Forest.from_soa(soa)
+    b = omk.Batch(f, len(troots), D)
+    b.set_roots(troots)
+    sp = omk.SelectParams(c_puct=1.4, virtual_loss=vl, use_rave=rave, rave_k=1000.0, pw=pw)
+    rng = np.random.default_rng(len(troots))
+    for step in range(steps):
+        rpaths, rlen, rleaf, _ = ref.select_batch(troots, rp, near_ties=False)
+        b.select(sp)
+        paths, plen, leaf, acts = b.read()
+        assert (paths == rpaths).all() and (plen == rlen).all() and (leaf == rleaf).all(), step
+        assert (acts == ref.gather_actions(rpaths, rlen)).all(), step
+        assert b.truncated() == int(((ref.child_count[rleaf] > 0) & (rlen == D + 1)).sum()), step
+        values = (rng.integers(-64, 65, len(troots)) / 64.0).astype(np.float32)
+        ref.backup_batch(rpaths, rlen, values, vl)
+        b.set_values(values)
+        b.backup(vl)
+        got = f.download()
+        assert (got["N"] == ref.N).all() and (got["VL"] == ref.VL).all(), step
+        ref.W[:] = got["W"]
+
+
+@pytest.mark.parametrize("visitors", [2, 3, 17, 63, 64, 65])
+@pytest.mark.parametrize("fan,rave", [(2, False), (64, True), (65, False), (256, False), (257, True), (384, True),
+                                      (385, False)])
+def test_crowds_and_fan_outs(visitors, fan, rave):
+    soa, roots = layered_forest(3 + fan + visitors, [fan, 40, 5], n_trees=3, rave=rave)
+    both(soa, np.repeat(roots, visitors).astype(np.int32), 6, rave=rave)
+
+
+@pytest.mark.parametrize("rave", [False, True])
+@pytest.mark.parametrize("widest,mask", [(12, 0.0), (150, 0.4), (380, 0.3)])
+@pytest.mark.parametrize("D", [1, 7, 63, 64])
+def test_roots_of_all_sizes_in_one_batch(widest, mask, D, rave):
+    """Roots with 1 to 64 visitors side by side (the single ones in blocks of their own), ties, unvisited children, virtual
+    loss from before; rows only where the bound is below 64."""
+    soa, roots = random_tree(D + widest, n_expand=120, fanout=(2, widest), max_depth=9, n_roots=40, mask_frac=mask, rave=rave,
+                             vl_frac=0.1, tie_frac=0.1, n_max=200)
+    rng = np.random.default_rng(D)
+    sizes = np.concatenate([np.ones(19, np.int64), rng.integers(2, 65, 21)])
+    both(soa, rng.permutation(np.repeat(roots, sizes)).astype(np.int32), D, rave=rave)
+
+
+@pytest.mark.parametrize("kind", ["nan prior", "nan sum", "-inf sum", "inf sum of the unvisited", "no virtual loss", "all equal"])
+@pytest.mark.parametrize("rave", [False, True])
+def test_scores_that_are_not_real_and_ties(kind, rave):
+    soa, roots = random_tree(11, n_expand=60, fanout=(2, 130), max_depth=6, n_roots=6, rave=rave, n_max=30)
+    rng = np.random.default_rng(5)
+    some = rng.random(len(soa["N"])) < 0.3
+    some[roots] = False
+    if kind == "nan prior":
+        soa["P"][some] = np.nan
+    elif kind == "nan sum":
+        soa["W"][some] = np.nan
+    elif kind == "-inf sum":
+        soa["W"][some] = -np.inf
+    elif kind == "inf sum of the unvisited":
+        soa["W"][some & (soa["N"] == 0)] = np.inf
+    elif kind == "all equal":
+        soa["N"][:], soa["W"][:], soa["P"][:] = 1, 0.5, 0.25
+    both(soa, np.repeat(roots, 20).astype(np.int32), 8, vl=0 if kind == "no virtual loss" else 2, rave=rave, steps=1)
+
+
+def test_widening_at_the_selection():
+    soa, roots = random_tree(21, n_expand=80, fanout=(2, 200), max_depth=7, n_roots=9, sort_prior=True, n_max=400)
+    both(soa, np.repeat(roots, [1, 2, 5, 9, 16, 33, 48, 63, 64]).astype(np.int32), 8, pw=True)
