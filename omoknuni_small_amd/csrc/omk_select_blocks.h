@@ -17,8 +17,6 @@ namespace omk {
 constexpr int kBlockVisitors = kBlockMax;  // of one root: a lane each
 constexpr int kBlockDepth = 63;     // deepest bound for which the blocks send rows to the host themselves
 constexpr int kBlockWaves = 16;     // wavefronts of a block: 128 registers each
-constexpr int kPlayQueue = 4;       // entries of a child worked out ahead
-constexpr uint32_t kPlayEmpty = 0xFFFFFFFFu;  // above every real key: they have run out
 
 // A node and the visitors that reached it: entries [off, off + m) of the block's list.
 struct BlockItem {
@@ -32,6 +30,8 @@ struct BlockScratch {
     int n[kWave], vl[kWave], sx[kWave], sy[kWave];
     float w[kWave], p[kWave], q2[kWave];
     int start[kWave];        // first place of the child's visitors in the node's list
+    int taken[kWave];        // its visits
+    uint64_t entry[2 * kWave + 8];  // merge_heads: the entries being put in order
     uint32_t order[kWave];   // per visitor: child << 21 | number of the visit
     uint8_t lane_of[RMAX * kWave];  // where child i is listed
 };
@@ -63,138 +63,102 @@ __device__ __forceinline__ void wave_best_fast(uint32_t bk, uint32_t bpos, uint3
     mpos = (uint32_t)__builtin_amdgcn_readlane((int)bpos, __ffsll((long long)tie) - 1);
 }
 
-// m visitors of a node played over the n0 children listed in `s`, one per lane: order[q] for every visitor, and the
-// visits of the lane's child.  It is the serial loop itself (the best of the current entries, first scan before second,
-// lowest child first), but not one visitor at a time:
-//   * every lane has its child's next kPlayQueue entries worked out, independently of each other;
-//   * the next entries that come before every entry after the next are the next visitors', all at once, the best first:
-//     each lane counts the ones before its own;
-//   * a child whose entries run out becomes the leader, with 64 of its entries spread over the lanes: the visitors it
-//     wins in a row are taken at once.
-// Nothing is assumed about the order of a child's entries.  The children that are not listed have no entry above
-// floor_key: false (with `order` overwritten) when an entry at or below it, or none, would be next.
+// m visitors of a node settled over the n0 children listed in `s`, one per lane: order[q] for every visitor, and the
+// visits of the lane's child.  The score a child shows its j-th visitor of this node depends on nothing but j, and where
+// no child's scores increase with j the serial order is the merge of the children's lists.  Twice 64 entries are worked
+// out at once, as many of every child (64 of two children, two of 64), independently of each other where the serial
+// loop waits for two divisions a visitor.  An entry that is not worked out comes after the last one of its child that is:
+// the entries up to the first of these last ones are the next visitors', the best first, and every one finds its place
+// by counting the ones before it.  What is left goes on from there.
+// floor_key: the children that are not listed have no entry above it.
+// False (with `order` overwritten) when a child's entries are not in order, or when an entry at or below floor_key or none
+// would be next: the caller plays one visitor after the other.
 template <int RMAX, bool RAVE>
-__device__ __forceinline__ bool play_heads(BlockScratch<RMAX> &s, int n0, int m, float ep, uint32_t uvl,
-                                           uint32_t floor_key, int lane, int &visits) {
-    constexpr int K = kPlayQueue;
-    int child = 0, cn = 0, cvl = 0, cnt = 0;
+__device__ __forceinline__ bool merge_heads(BlockScratch<RMAX> &s, int n0, int m, float ep, uint32_t uvl,
+                                            uint32_t floor_key, int lane, int &visits) {
+    visits = 0;
+    if (n0 == 0) return false;
+    const int log_e = n0 <= 1 ? 6 : 6 - (32 - __clz(n0 - 1));  // a child's lanes: the largest power of two that fits
+    const int E = 1 << log_e;
+    const int c = lane >> log_e, j0 = lane & (E - 1);
+    const bool mine = c < n0;
+    int cn = 0, cvl = 0;
     float cw = 0.0f, cp = 0.0f, cq2 = 0.0f;
-    if (lane < n0) {
-        child = s.child[lane];
-        cn = s.n[lane];
-        cw = s.w[lane];
-        cp = s.p[lane];
-        cvl = s.vl[lane];
-        if (RAVE) cq2 = s.q2[lane];
+    if (mine) {
+        cn = s.n[c];
+        cw = s.w[c];
+        cp = s.p[c];
+        cvl = s.vl[c];
+        if (RAVE) cq2 = s.q2[c];
     }
-    uint32_t q[K], second = 0u;  // bit j of `second`: entry j is a candidate of the second scan
-    int lead = -1;               // lane of the leader, whose queue holds nothing
-    auto refill = [&]() {
-        second = 0u;
-#pragma unroll
-        for (int j = 0; j < K; j++) {
-            uint32_t pos;
-            entry_key<1, RAVE>(cn, cw, cp, cvl, cq2, ep, uvl, cnt + j, 0, q[j], pos);
-            if (lane >= n0 || lane == lead) q[j] = 0u;
-            second |= pos != 0u ? 1u << j : 0u;
-        }
-    };
-    int l_child = 0, l_n = 0, l_vl = 0, l_base = 0, l_pos = 0;  // the leader; entry l_base + l_pos is its next
-    float l_w = 0.0f, l_p = 0.0f, l_q2 = 0.0f;
-    uint32_t l_key = 0u;                // entry l_base + lane
-    uint64_t l_second = 0u, l_ok = 0u;  // which of them are of the second scan, and above floor_key
-    auto lead_entries = [&]() {
-        uint32_t pos;
-        entry_key<1, RAVE>(l_n, l_w, l_p, l_vl, l_q2, ep, uvl, l_base + lane, 0, l_key, pos);
-        l_second = __ballot(pos != 0u);
-        l_ok = __ballot(l_key > floor_key);
-        l_pos = 0;
-    };
-    refill();
-    const uint32_t id = (uint32_t)lane;
+    const bool proven =
+        __ballot(mine && !keys_provably_monotone<RAVE>(cn, cw, cp, cvl, cq2, ep, uvl, m - 1)) == 0ull;
+    s.taken[lane] = 0;
+    wave_sync_memory();
+    int base = 0;  // visits of the lane's child so far
     for (int done = 0; done < m;) {
-        const uint32_t after = (uint32_t)uniform((int)wave_max_all(q[1]));
-        if (after == kPlayEmpty) {  // somebody's entries run out
-            const int x = __ffsll((long long)__ballot(q[1] == kPlayEmpty)) - 1;
-            if (lane == lead) cnt = l_base + l_pos;
-            lead = x;
-            l_child = __builtin_amdgcn_readlane(child, x);
-            l_n = __builtin_amdgcn_readlane(cn, x);
-            l_vl = __builtin_amdgcn_readlane(cvl, x);
-            l_w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cw), x));
-            l_p = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cp), x));
-            if (RAVE) l_q2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cq2), x));
-            l_base = __builtin_amdgcn_readlane(cnt, x);
-            refill();
-            lead_entries();
-            continue;
+        const int need = m - done;
+        uint32_t key[2] = {0u, 0u}, pos[2] = {0u, 0u};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if (h == 1 && E >= need) break;  // uniform: nobody gets more than the first E
+            entry_key<1, RAVE>(cn, cw, cp, cvl, cq2, ep, uvl, base + h * E + j0, 0, key[h], pos[h]);
+            key[h] = mine && h * E + j0 < need ? key[h] : 0u;  // (nobody gets more than `need`)
         }
-        // the next entries above all entries after the next, above the leader's and above floor_key
-        uint32_t bar = after > floor_key ? after : floor_key;
-        if (lead >= 0) {
-            const uint32_t l_next = (uint32_t)__builtin_amdgcn_readlane((int)l_key, l_pos);
-            bar = bar > l_next ? bar : l_next;
+        if (!proven) {
+            const uint32_t p0 = (uint32_t)__shfl_up((int)key[0], 1, kWave), q0 = (uint32_t)__shfl_up((int)pos[0], 1, kWave);
+            const uint32_t l0 = (uint32_t)__shfl((int)key[0], lane + E - 1, kWave), m0 = (uint32_t)__shfl((int)pos[0], lane + E - 1, kWave);
+            const uint32_t p1 = (uint32_t)__shfl_up((int)key[1], 1, kWave), q1 = (uint32_t)__shfl_up((int)pos[1], 1, kWave);
+            bool bad = j0 > 0 && comes_before(key[0], pos[0], p0, q0);
+            if (key[1] != 0u) bad |= j0 > 0 ? comes_before(key[1], pos[1], p1, q1) : comes_before(key[1], pos[1], l0, m0);
+            if (__ballot(mine && bad)) return false;
         }
-        const uint64_t set = __ballot(q[0] > bar);
-        if (set) {
-            const uint64_t mine = ((uint64_t)q[0] << 32) | ((second & 1u) ? 63u - id : 127u - id);  // larger: earlier
+        // ---- up to the first of the children's last entries (those that can be needed are all there, or it counts) ----
+        // (equal keys: first scan before second, then the children's order, then the visits')
+        uint32_t low[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) low[h] = (pos[h] << 24) | (uint32_t)(c << 16) | (uint32_t)(base + h * E + j0);
+        const uint32_t last = j0 == E - 1 && 2 * E < need ? key[1] : 0u;
+        const uint32_t bar = (uint32_t)uniform((int)wave_max_all(last));
+        const uint32_t bar_low = bar == 0u ? 0u : wave_min_u32(last == bar ? low[1] : 0xFFFFFFFFu);
+        bool in[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) in[h] = key[h] > floor_key && (key[h] > bar || (key[h] == bar && low[h] <= bar_low));
+        const uint64_t in0 = __ballot(in[0]), in1 = __ballot(in[1]);
+        const int n_in0 = __popcll(in0), total = n_in0 + __popcll(in1);
+        if (total == 0) return false;
+        const uint64_t below = (1ull << lane) - 1ull;
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (in[h])
+                s.entry[h == 0 ? __popcll(in0 & below) : n_in0 + __popcll(in1 & below)] = ((uint64_t)~key[h] << 32) | low[h];
+        if (lane < 8) s.entry[total + lane] = ~0ull;
+        wave_sync_memory();
+        // smaller = played earlier, all different; a lane has one of them, or two
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if (h * kWave >= total) break;  // uniform
+            const int at = h * kWave + lane;
+            const uint64_t e = at < total ? s.entry[at] : ~0ull;
             int rank = 0;
-            for (uint64_t rest = set; rest; rest &= rest - 1ull) {
-                const int x = __ffsll((long long)rest) - 1;
-                const uint64_t other = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(mine >> 32), x) << 32) |
-                                       (uint32_t)__builtin_amdgcn_readlane((int)mine, x);
-                rank += other > mine ? 1 : 0;
-            }
-            if (q[0] > bar && rank < m - done) {
-                s.order[done + rank] = ((uint32_t)child << 21) | (uint32_t)cnt;
+            for (int e0 = 0; e0 < total; e0 += 8) {
+                uint64_t o[8];
 #pragma unroll
-                for (int j = 0; j + 1 < K; j++) q[j] = q[j + 1];
-                q[K - 1] = kPlayEmpty;
-                second >>= 1;
-                cnt++;
-            }
-            done += __popcll(set);
-            continue;
-        }
-        // one at a time: the best of the next entries, or the leader's as long as they come before it
-        const uint32_t best = wave_max_all(q[0]);
-        const uint64_t tied = __ballot(q[0] == best), first = __ballot(q[0] == best && !(second & 1u));
-        const int x = __ffsll((long long)(first ? first : tied)) - 1;
-        const uint32_t key = (uint32_t)uniform((int)best);
-        if (lead >= 0) {
-            uint64_t wins = __ballot(l_key > key);
-            const uint64_t same = __ballot(l_key == key);
-            if (same) {
-                const uint64_t lower = lead < x ? ~0ull : 0ull;
-                wins |= same & (first ? ~l_second & lower : ~l_second | lower);
-            }
-            const uint64_t lost = ~(wins & l_ok) & (~0ull << l_pos);
-            int run = (lost ? __ffsll((long long)lost) - 1 : kWave) - l_pos;
-            run = run < m - done ? run : m - done;
-            if (run > 0) {
-                if (lane >= l_pos && lane < l_pos + run)
-                    s.order[done + lane - l_pos] = ((uint32_t)l_child << 21) | (uint32_t)(l_base + lane);
-                done += run;
-                l_pos += run;
-                if (l_pos == kWave && done < m) {
-                    l_base += kWave;
-                    lead_entries();
-                }
-                continue;
-            }
-        }
-        if (key <= floor_key) return false;
-        if (lane == x) {
-            s.order[done] = ((uint32_t)child << 21) | (uint32_t)cnt;
+                for (int u = 0; u < 8; u++) o[u] = s.entry[e0 + u];
 #pragma unroll
-            for (int j = 0; j + 1 < K; j++) q[j] = q[j + 1];
-            q[K - 1] = kPlayEmpty;
-            second >>= 1;
-            cnt++;
+                for (int u = 0; u < 8; u++) rank += o[u] < e ? 1 : 0;
+            }
+            if (at < total && rank < need) {
+                const int w = (int)((e >> 16) & 63u);
+                s.order[done + rank] = ((uint32_t)s.child[w] << 21) | (uint32_t)(e & 0xFFFFu);
+                atomicAdd(&s.taken[w], 1);
+            }
         }
-        done++;
+        wave_sync_memory();
+        base = s.taken[c];
+        done += total < need ? total : need;
     }
-    visits = lane == lead ? l_base + l_pos : cnt;
+    visits = s.taken[lane];
     return true;
 }
 
@@ -345,20 +309,10 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                 wave_best_fast(bk, bpos, hk, hp);
                 const int best = (int)(hp >= (uint32_t)F ? hp - (uint32_t)F : hp);
                 serial = true;
-                uint32_t lk = 0u;  // the best child's entry for the last visitor, where others come before it
                 if (hk != 0u && (m == 1 || a.vl <= 0)) {
                     run_child = best;
                 } else if (hk != 0u && !odd) {
                     // ---- does the best child win every time?  (single_run) ----
-                    uint32_t ok = 0u, opos = 0xFFFFFFFFu;
-#pragma unroll
-                    for (int r = 0; r < RMAX; r++)
-                        if (r * kWave + lane != best && k.k1[r] > ok) { ok = k.k1[r]; opos = (uint32_t)(r * kWave + lane); }
-#pragma unroll
-                    for (int r = 0; r < RMAX; r++)
-                        if (r * kWave + lane != best && k.k2[r] > ok) { ok = k.k2[r]; opos = (uint32_t)(F + r * kWave + lane); }
-                    uint32_t sk, spos, lp;
-                    wave_best_fast(ok, opos, sk, spos);
                     int tn = 0, tvl = 0;
                     float tw = 0.0f, tp = 0.0f, tq2 = 0.0f;
 #pragma unroll
@@ -376,28 +330,25 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                     const float bw = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tw), bl));
                     const float bp = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tp), bl));
                     const float bq2 = RAVE ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tq2), bl)) : 0.0f;
+                    uint32_t lk, lp;
                     entry_key<RMAX, RAVE>(bn, bw, bp, bvl, bq2, ep, uvl, m - 1, best, lk, lp);
                     lk = (uint32_t)uniform((int)lk);
-                    lp = (uint32_t)uniform((int)lp);
-                    if (lk != 0u && (sk == 0u || comes_before(lk, lp, sk, spos))) {
-                        if (entries_in_order<RMAX, RAVE>(bn, bw, bp, bvl, bq2, ep, uvl, best, m, lane)) run_child = best;
-                        lk = 0u;
-                    }
+                    auto heads = [&](uint32_t T) {
+                        int c = 0;
+#pragma unroll
+                        for (int r = 0; r < RMAX; r++) c += __popcll(__ballot(umax32(k.k1[r], k.k2[r]) >= T));
+                        return c;
+                    };
+                    // its entry for the last visitor comes before every other child's next one, and they are in order
+                    uint32_t from = lk < hk ? lk : hk, floor_key = from - 1u;
+                    int n_heads = from != 0u ? heads(from) : 0;
+                    if (n_heads == 1 && entries_in_order<RMAX, RAVE>(bn, bw, bp, bvl, bq2, ep, uvl, best, m, lane))
+                        run_child = best;
                     if (run_child < 0) {
                         // ---- the children that can be chosen, one per lane ----
-                        // those whose next entry is not below lk (with the best child's entries in order nobody else
-                        // is; play_heads sees to it), or, if there are too many or no lk, the m best
-                        uint32_t from = lk < hk ? lk : hk, floor_key = from - 1u;
-                        auto heads = [&](uint32_t T) {
-                            int c = 0;
-#pragma unroll
-                            for (int r = 0; r < RMAX; r++) c += __popcll(__ballot(umax32(k.k1[r], k.k2[r]) >= T));
-                            return c;
-                        };
-                        if (RMAX == 1) {
-                            from = 1u;
-                            floor_key = 0u;
-                        } else if (from == 0u || heads(from) > kWave) {
+                        // those whose next entry is not below that one (with the best child's entries in order nobody
+                        // else is; merge_heads sees to it), or, if there are too many or it is not real, the m best
+                        if (from == 0u || n_heads > kWave) {
                             from = first_heads<RMAX, RAVE>(k, bk, m);
                             floor_key = 0u;
                         }
@@ -421,7 +372,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                                 n0 += __popcll(cm);
                             }
                             wave_sync_memory();
-                            serial = !play_heads<RMAX, RAVE>(my, n0, m, ep, uvl, floor_key, lane, visits);
+                            serial = !merge_heads<RMAX, RAVE>(my, n0, m, ep, uvl, floor_key, lane, visits);
                         }
                     }
                 }
