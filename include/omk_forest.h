@@ -294,13 +294,12 @@ int omk_batch_truncated(omk_batch *b, int32_t *h_count);
  * [1] of these settled by the parallel paths, [2] visitors settled by them, [3] visitors
  * settled one at a time, [4] nodes replayed one visitor at a time because the parallel
  * path's exactness checks did not hold, [5] threshold probes, [6] single-visitor selection
- * steps, [7] nodes settled by merging a few entries of other children into the list of the child
- * that takes nearly every visitor, [8] when the first block of the persistent launch started,
+ * steps, [7] nodes settled by merging the lists of their children's entries, [8] when the first block of the persistent launch started,
  * [9] when its last team of wavefronts left, [10] when its last walker left (low 31 bits of the
  * device's 100 MHz clock; these three are kept whether or not the counters are on), [11] the number
- * of walks of lone visitors inside that launch, [12] nodes of more than 64 child slots settled through
- * the few children that can be chosen at all, one per lane (RAVE layouts), [13] nodes of at most 64 visitors that
- * spread over many children, settled at once (trees grown by omk_expand_batch*), [14] unused (0), [15] nodes
+ * of walks of lone visitors inside that launch, [12] of the nodes of [7], those of
+ * layouts with RAVE and more than 64 child slots a node, [13] of them, those of at most 64 visitors (of such layouts, and
+ * of batches with at most 64 visitors a root), [14] unused (0), [15] nodes
  * cut into slices for several wavefronts.  (Nodes taken by the walk down one-winner nodes count in [0]..[2].) */
 int omk_batch_stats(omk_batch *b, int32_t *h_stats16);
 /* The counters above cost one atomic per processed node (and per single-visitor step), all on

@@ -48,7 +48,6 @@ struct omk_forest {
     bool has_rave = false;
     bool uploaded = false;
     bool prior_sorted = false;
-    bool grown = false;  // expanded since the last upload: most children have no visits
     // What the last call changed the structure by, if it was an expansion: node made_node[i] has made_count[i] children
     std::vector<int32_t> made_node, made_count;
     int max_fanout = 0;
@@ -626,7 +625,6 @@ int omk_forest_upload(omk_forest *f, const omk_soa_view *v) try {
     }
     f->n_nodes = n;
     f->max_fanout = mf;
-    f->grown = false;
     f->made_node.clear();
     f->made_count.clear();
     f->prior_sorted = sorted;
@@ -1516,7 +1514,7 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
     LoneOut out;
     if (int rc = lone_rows(b, &out)) return rc;
     HIP_TRY(launch_select(f->dev(), a, b->n_items0, b->n_singles0, b->n, b->most_visitors, f->max_fanout, p->use_rave != 0,
-                          f->grown, b->n_cus, b->n_hctx0, b->prepared == b->epoch, out,
+                          b->n_cus, b->n_hctx0, b->prepared == b->epoch, out,
                           f->stream));
     b->selected = true;
     b->disjoint = b->n_items0 == 0;  // a root each, and distinct roots head disjoint trees
@@ -1784,7 +1782,6 @@ int omk_expand_batch_ex(omk_batch *b, const int32_t *h_move_begin, const int32_t
         HIP_TRY(launch_expand(f->mut(), jobs, (int)nj, moves, priors, f->n_nodes, cursor, f->stream));
         f->n_nodes = cursor;
         f->changes++;
-        f->grown = true;
         f->structure_changed = true;  // ids keep their meaning, but an upload of the old arrays would not
         f->max_fanout = mf;
         f->prior_sorted = sorted;

@@ -40,7 +40,11 @@ struct Item {
 };
 
 constexpr int kHeavyCtxInts = 16 + 1024;  // 16 + the widest fan-out
-constexpr int kHeavyMin = 1024;          // visitors from which a node is settled by several wavefronts
+// Visitors from which a node is cut into slices for several blocks.  Below, the helpers of one block are as fast
+// (team_merge): its batch holds 2048 entries, up to 1475 visitors of a node with 384 children.  4096 visitors on a
+// chess-like tree and 16384 on a Go tree with RAVE: 261 and 382 us with 1024, 245 and 348 with 1536, 251 and 358 with 2048,
+// 278 and 364 with 3072.
+constexpr int kHeavyMin = 1536;
 constexpr int kMaxSlices = 64;           // slices (and parts of the partition) of such a node, at most
 constexpr int kHeavyFanout = 384;        // widest node settled that way (register budget)
 constexpr int kSliceEntries = 192;       // visitors per slice of such a node, about
@@ -136,10 +140,9 @@ struct LoneOut {
     HostSignal sig;
 };
 
-// most_visitors: traversals of the most crowded root; grown: the forest has been expanded since it was uploaded;
-// prepared: launch_set_roots has made the reset
+// most_visitors: traversals of the most crowded root; prepared: launch_set_roots has made the reset
 hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, int n_singles0, int n_traversals,
-                         int most_visitors, int max_fanout, bool rave, bool grown, int n_cus, int n_hctx0,
+                         int most_visitors, int max_fanout, bool rave, int n_cus, int n_hctx0,
                          bool prepared, const LoneOut &out, hipStream_t s);
 
 // The same for a batch whose roots have few visitors each (omk_select_blocks.h): a block a root, without a reset.  The
@@ -163,7 +166,7 @@ hipError_t launch_set_roots(const SelectArgs &a, int32_t *seg0, Item *items0, It
 // The kernels of one fan-out class (rounds of 64 children: 1, 4, 6 or 16), behind the reset launch.
 template <int RMAX, bool RAVE>
 hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a, int n_items0, int most_visitors, int n_traversals,
-                               int n_cus, bool grown, const LoneOut &out, hipStream_t s);
+                               int n_cus, const LoneOut &out, hipStream_t s);
 
 hipError_t launch_apply_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                            int max_len, int vl, hipStream_t s);

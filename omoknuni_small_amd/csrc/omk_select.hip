@@ -88,7 +88,7 @@ __global__ void k_select_reset(SelectArgs a, int n_items0, int n_singles0, int o
 }
 
 hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, int n_singles0, int n_traversals,
-                         int most_visitors, int max_fanout, bool rave, bool grown, int n_cus, int n_hctx0,
+                         int most_visitors, int max_fanout, bool rave, int n_cus, int n_hctx0,
                          bool prepared, const LoneOut &out, hipStream_t s) {
     // Every traversal alone at its root (one per tree: leaf-parallel self-play): the single-visitor
     // kernel is the whole select and takes its walkers from the host's list; every walker writes its
@@ -103,8 +103,8 @@ hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, 
     }
     if (blocks) return launch_select_blocks(f, a, n_items0, n_singles0, max_fanout, rave, out, s);
 #define OMK_DISPATCH(RM)                                                              \
-    return rave ? launch_select_class<RM, true>(f, a, n_items0, most_visitors, n_traversals, n_cus, grown, out, s) \
-                : launch_select_class<RM, false>(f, a, n_items0, most_visitors, n_traversals, n_cus, grown, out, s)
+    return rave ? launch_select_class<RM, true>(f, a, n_items0, most_visitors, n_traversals, n_cus, out, s) \
+                : launch_select_class<RM, false>(f, a, n_items0, most_visitors, n_traversals, n_cus, out, s)
     if (max_fanout <= 64) { OMK_DISPATCH(1); }
     if (max_fanout <= 256) { OMK_DISPATCH(4); }
     if (max_fanout <= 384) { OMK_DISPATCH(6); }

@@ -20,7 +20,8 @@
 //  * few visitors: they are played one after another on register-resident statistics --
 //    score, DPP arg-max with lowest-index tie-break, bump the chosen child's virtual loss,
 //    next visitor.  That is the serial order itself.
-//  * many visitors ("water level"): the score child i shows to its j-th visitor of this
+//  * eight visitors or more: the helpers of the block merge the children's descending lists (team_merge).
+//  * what that declines, and the slices of a heavy node ("water level"): the score child i shows to its j-th visitor of this
 //    batch depends on nothing but j.  If every child's scores do not increase with j, the
 //    serial winner sequence is the merge of these descending lists, i.e. the m best
 //    entries (i, j) in the order (score descending, candidate position ascending, j
@@ -34,7 +35,7 @@
 //    produces exactly this sequence; if either fails the node is replayed one visitor at a
 //    time.  A long run of one child (its score hardly moves with virtual loss) is emitted
 //    without sorting.
-//  * a thousand visitors or more: the node is cut into slices of its winner order that
+//  * kHeavyMin visitors or more: the node is cut into slices of its winner order that
 //    several wavefronts settle side by side, and the partition is shared out the same way
 //    (see select_group).
 //
@@ -100,7 +101,7 @@ struct Kids {
 
 // What the owner wavefront of a block asks of its helpers; first member of the LDS scratch,
 // so that it sits at the same place for every fan-out class.
-enum { kOpExit = 0, kOpOrder = 1, kOpEmit = 2, kOpRun = 3, kOpPartition = 4, kOpLoad = 5, kOpChain = 6 };
+enum { kOpExit = 0, kOpOrder = 1, kOpEmit = 2, kOpRun = 3, kOpPartition = 4, kOpLoad = 5, kOpChain = 6, kOpMerge = 7 };
 struct TeamCmd {
     int op;
     int rounds;  // R of the node's fan-out class: 1, or the kernel's RMAX
@@ -124,6 +125,9 @@ struct TeamCmd {
     int pre_node, pre_np, pre_cb, pre_cc;
     // kOpChain: the node a chain walk starts at (chain_walk), its N, child range, depth, and its visitors
     int c_node, c_np, c_cb, c_cc, c_depth, c_off, c_m;
+    // kOpMerge (`total` visitors): whether the helpers settled the node; -1 while they are at it, then the number of
+    // block barriers they took
+    int merged, n_barriers;
 };
 
 // What that helper reads, at the same place for every fan-out class: the owner's next node
@@ -153,6 +157,7 @@ struct WaveLds {
     int st_j0[R * kWave];  // visits already settled / visit count, by phase
     int hist[kSortBins * (kBatchCap / kWave + 1) > R * kWave ? kSortBins * (kBatchCap / kWave + 1) : R * kWave];  // sort: entries per (digit value, block of 64); emit: visits per child
     uint32_t pay[R * kWave];      // per child: entries of the batch
+    uint32_t slots[2][2 * kTeamWaves];  // team_merge: what the wavefronts tell each other
     alignas(16) uint32_t key[2][kBatchCap];  // entries of the batch being ordered: inverted score key ...
     alignas(16) uint32_t pay2[2][kBatchCap];  // ... and pass flag, child, visit number; two buffers, ping-pong
 };
@@ -477,19 +482,19 @@ __device__ __forceinline__ int predict_count(int n, float w, float p, int vl, fl
     const float x0 = (float)n + (float)vl;
     const float A = w + (float)n;
     const float cc = p * ep;
-    const float inv_step = __frcp_rn((float)uvl);
+    const float inv_step = __builtin_amdgcn_rcpf((float)uvl);
     float xs = -1.0f;  // largest x with score >= tau
     const float a2 = tau + 1.0f;
     if (a2 > 1e-12f) {
         const float b2 = a2 - A - cc;
         const float disc = b2 * b2 + 4.0f * a2 * A;
-        if (disc >= 0.0f) xs = (-b2 + __fsqrt_rn(disc)) * __frcp_rn(2.0f * a2);
+        if (disc >= 0.0f) xs = (-b2 + __builtin_amdgcn_sqrtf(disc)) * __builtin_amdgcn_rcpf(2.0f * a2);
     } else {
         xs = 3.0e38f;
     }
     if (RAVE) {
         const float d = tau - q2;
-        float x2 = d > 1e-12f ? cc * __frcp_rn(d) - 1.0f : 3.0e38f;
+        float x2 = d > 1e-12f ? cc * __builtin_amdgcn_rcpf(d) - 1.0f : 3.0e38f;
         xs = fmaxf(xs, x2);
     }
     float cnt = floorf((xs - x0) * inv_step) + 1.0f;
@@ -504,10 +509,7 @@ struct ChainLds {
     int nodes[kChainMaxLevels];  // the child taken at every one of them
     int e_node, e_np, e_cb, e_cc, e_depth;  // where the walk stands: a node that has not been settled
     int e_kids;       // that node's children are in the LDS scratch (it failed the one-winner test), with:
-    int e_contested;  // single_run's verdict: the best child's entry for the last visitor is real but not first,
-    int e_best0;      // that child,
-    uint32_t e_lk0;   // that entry's key,
-    int e_second;     // and whether it is a candidate of the second scan
+    int e_contested;  // single_run's verdict: the best child's entry for the last visitor is real but not first
     int n_barriers;   // -1 while a walk is under way, then the number of block barriers it took
 };
 typedef __attribute__((address_space(3))) unsigned char *LdsBytesP;
@@ -578,20 +580,22 @@ __device__ __forceinline__ bool wait_list(const SelectArgs &a, int off, int dept
 // to return at once, or 0.
 template <typename Est, typename Plateau>
 __device__ __forceinline__ uint32_t search_threshold(uint32_t lo_key, uint32_t hi_key, int target, int acc_hi,
-                                                     int acc_below, int &evals, Est est, Plateau plateau) {
+                                                     int acc_below, int &evals, Est est, Plateau plateau,
+                                                     float lo_count = -1.0f) {
     uint32_t klo = lo_key, khi = hi_key;
     auto y_of = [](uint32_t k) {
         float d = key_score(k) + 1.0f;
         d = d > 1e-6f ? d : 1e-6f;
-        return __frcp_rn(d);
+        return __builtin_amdgcn_rcpf(d);
     };
     float ylo = y_of(klo), yhi = y_of(khi);
     const float aim = (float)target + 0.5f * (float)(acc_hi - target);
     float flo = aim, fhi = -aim;  // count minus aim at the two ends: made up until an end has been evaluated
+    if (lo_count >= 0.0f) flo = lo_count - aim;
     int last = 0;                 // which end the last step moved: +1 the low one, -1 the high one
     for (int it = 0; it < 48 && khi - klo > 1u; it++) {
-        const float ym = (ylo * fhi - yhi * flo) * __frcp_rn(fhi - flo);
-        uint32_t kmid = score_key(__frcp_rn(ym) - 1.0f);
+        const float ym = (ylo * fhi - yhi * flo) * __builtin_amdgcn_rcpf(fhi - flo);
+        uint32_t kmid = score_key(__builtin_amdgcn_rcpf(ym) - 1.0f);
         if (!(kmid > klo)) kmid = klo + 1u;
         if (!(kmid < khi)) kmid = khi - 1u;
         // the dense sliver: once false position stops moving off an end, halve the key interval
@@ -2016,8 +2020,8 @@ __device__ __forceinline__ bool entries_in_order(int bn, float bw, float bp, int
 template <int R, bool RAVE>
 __device__ __forceinline__ bool single_run(const SelectArgs &a, const NodeCtx &c, int lane, const Kids<R, RAVE> &k,
                                            uint32_t bk, uint32_t bpos, int off, int m, bool to_global, int (&cnt)[R],
-                                           int &run_child, bool &contested, int &best0, uint32_t &lk0, uint32_t &lp0) {
-    // contested: the best child's entry for the last visitor, (lk0, lp0), is real but does not come first
+                                           int &run_child, bool &contested) {
+    // contested: the best child's entry for the last visitor is real but does not come first
     contested = false;
     constexpr int F = R * kWave;
     const uint32_t uvl = (uint32_t)a.vl;
@@ -2061,10 +2065,7 @@ __device__ __forceinline__ bool single_run(const SelectArgs &a, const NodeCtx &c
     entry_key<R, RAVE>(bn, bw, bp, bvl, bq2, c.ep, uvl, m - 1, best, lk, lp);
     if (lk == 0u) return false;
     if (sk != 0u && !comes_before(lk, lp, sk, spos)) {
-        contested = true;  // other children get a look in: the caller may still find that they are few
-        best0 = best;
-        lk0 = lk;
-        lp0 = lp;
+        contested = true;  // other children get a look in
         return false;
     }
     // when the order of the child's keys is proven beforehand, the entries in between need no look
@@ -2133,10 +2134,380 @@ __device__ __forceinline__ int count_before(int n, float w, float p, int vl, flo
     return lo_c;
 }
 
-constexpr int kSparseMax = 64;  // entries of other children a nearly-one-winner node may hold (one per lane)
-constexpr int kSparseMin = 8;    // visitors from which that direct merge is tried
-enum { kMergeNo = 0, kMergeDone = 1, kMergeMany = 2 };
-static_assert(2 * kHeavyMin <= kBatchCap, "the (key, position) list of the dominant child fits one sort buffer");
+// ---- A contested node settled by the three helpers ----
+// The score a child shows the j-th of a node's visitors that choose it depends on nothing but j, and where no child's
+// scores increase with j the serial order is the merge of the children's lists by (key, position).  The helpers work out
+// a prefix of every list side by side, a few more entries than the closed form says lie at or above a threshold with
+// enough of them.  An entry that was not worked out comes after the last one of its child that was (or is a child's very
+// next one): the entries up to the first of these are the next visitors', whatever the estimate was worth, and what is
+// left goes on from there.  They are put in order by buckets, every one finds its place among the others of its bucket.
+// Without RAVE their number is nearly a straight line in y = 1 / (score + 1), and the buckets are equal steps of y: one or
+// two entries each.  With RAVE most lie close above the threshold (blends that hardly move with virtual loss): 64 buckets
+// for every halving of the distance in y to it.
+// What bounds it: the dependent steps of one wavefront and some 15 block barriers; no memory.  Three wavefronts and not the
+// owner's as well: its code is the kernel's largest, and a part of it that only waits costs it no registers.
+// Measured on an MI355X, in the place of the counts and the sort of one wavefront (water_level), the whole node: 246 visitors of a chess-like node 15.6 -> 11.5 us, 75 to 190 of a Go node with
+// RAVE 23 to 33 -> 13 to 15, 944 of one 45 -> 20; 4096 on the chess-like tree 270 -> 245 us a selection, 16384 on the Go
+// tree with RAVE 373 -> 348 (with the higher kHeavyMin, which it makes worth while), a search of 500 a batch 2.96 -> 2.76 ms.
+constexpr int kMergeMin = 8;  // visitors from which a contested node is settled that way (5 and 14: the same)
+constexpr int kMergeThreads = (kTeamWaves - 1) * kWave;
+constexpr int kMergeOwn = 6;  // buckets a thread adds up
+constexpr int kMergeBuckets = kMergeThreads * kMergeOwn;
+constexpr int kMergePasses = 12;
+constexpr int kMergeCount = 32;  // entries of a bucket that are ranked by counting whoever they belong to
+static_assert(2 * kMergeBuckets + 1 + 2 * kBatchCap + 1024 <= kSortBins * (kBatchCap / kWave + 1), "buckets and arrivals fit the sort's table");
+
+// t: number of the helper thread.  On success (cmd.merged) order[] holds (child << 21) | visit number of the m visitors and
+// st_j0[] the visits per child.  The owner takes the barriers with them.
+template <int R, bool RAVE>
+__device__ __forceinline__ void team_merge(WaveLds<R> &lds, uint32_t *order, int t, int m, float ep, uint32_t uvl) {
+    constexpr int F = R * kWave, NT = kMergeThreads, W = NT / kWave;
+    constexpr int K = (F + NT - 1) / NT;  // children of a thread: t, t + NT ..
+    const int lane = t & 63, wv = uniform(t >> 6);
+    uint64_t *ent = reinterpret_cast<uint64_t *>(lds.key[0]);    // in (child, visit) order; smaller = played earlier
+    uint64_t *ent2 = reinterpret_cast<uint64_t *>(lds.pay2[0]);  // by bucket
+    uint32_t *own = lds.pay2[0];                                 // (before that: the child of every entry)
+    int *bucket = lds.hist;
+    uint32_t *arrival = reinterpret_cast<uint32_t *>(lds.hist) + kMergeBuckets + 1;
+    int *runs = lds.hist + kMergeBuckets + 1 + kBatchCap;      // of a bucket: children with entries in it
+    int *seg_end = runs + kMergeBuckets;                       // of a child: behind its last entry
+    uint32_t *run_at = reinterpret_cast<uint32_t *>(seg_end) + F;  // by bucket: first entry of each of these, end of the child's
+    int par = 0, barriers = 0;
+    auto sync = [&]() {
+        __syncthreads();
+        barriers++;
+    };
+    auto tell = [&](uint32_t a, uint32_t b) {
+        if (lane == 0) {
+            lds.slots[par][2 * wv] = a;
+            lds.slots[par][2 * wv + 1] = b;
+        }
+        sync();
+    };
+    auto told = [&](int w, int h) { return (uint32_t)uniform((int)lds.slots[par][2 * w + h]); };
+    auto y_of = [](uint32_t k) {
+        const float d = key_score(k) + 1.0f;
+        return __frcp_rn(d > 1e-6f ? d : 1e-6f);
+    };
+    int cn[K], cvl[K];
+    float cw[K], cp[K], cq2[K];
+    bool part[K];
+#pragma unroll
+    for (int q = 0; q < K; q++) {
+        const int i = t + q * NT;
+        part[q] = false;
+        cn[q] = cvl[q] = 0;
+        cw[q] = cp[q] = cq2[q] = 0.0f;
+        if (i < F) {
+            part[q] = lds.pay[i] != 0u;
+            cn[q] = lds.st_n[i];
+            cw[q] = lds.st_w[i];
+            cp[q] = lds.st_p[i];
+            cvl[q] = lds.st_vl[i];
+            if (RAVE) cq2[q] = lds.st_q2[i];
+        }
+    }
+    bool ok = true;
+    int done = 0;
+    for (int pass = 0; done < m; pass++) {
+        const int need = m - done;
+        // ---- the children's next entries, and the key no useful threshold lies below: a child alone has `need` entries
+        // at or above the last one it could be asked for ----
+        uint32_t hk[K], hp[K];
+        uint32_t lmax = 0u, hmax = 0u;
+        int tk[K];
+#pragma unroll
+        for (int q = 0; q < K; q++) {
+            const int i = t + q * NT;
+            hk[q] = 0u;
+            hp[q] = 0u;
+            tk[q] = i < F ? lds.st_j0[i] : 0;
+            if (q * NT < F && part[q]) {
+                uint32_t zk, zp;
+                entry_key<R, RAVE>(cn[q], cw[q], cp[q], cvl[q], cq2[q], ep, uvl, tk[q], i, hk[q], hp[q]);
+                entry_key<R, RAVE>(cn[q], cw[q], cp[q], cvl[q], cq2[q], ep, uvl, tk[q] + need - 1, i, zk, zp);
+                if (hk[q] != 0u) lmax = umax32(lmax, zk);
+                hmax = umax32(hmax, hk[q]);
+            }
+        }
+        for (int b = t; b <= kMergeBuckets; b += NT) bucket[b] = 0;
+        tell(wave_max_all(lmax), wave_max_all(hmax));
+        uint32_t lo_key = 0u, hi_key = 0u;
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            lo_key = umax32(lo_key, told(w, 0));
+            hi_key = umax32(hi_key, told(w, 1));
+        }
+        par ^= 1;
+        if (lo_key == 0u || lo_key > hi_key || pass >= kMergePasses) {
+            ok = false;
+            break;
+        }
+        // ---- a threshold with some more than `need` entries at or above it, by the closed form ----
+        // (whether the next entry does is known; the closed form does not hold for a child without visits)
+        auto entries_from = [&](int q, uint32_t key) {
+            if (hk[q] < key) return 0;
+            const int n = predict_count<RAVE>(cn[q], cw[q], cp[q], (int)((uint32_t)cvl[q] + (uint32_t)tk[q] * uvl), cq2[q], ep,
+                                              uvl, key_score(key), need);
+            return n > 1 ? n : 1;
+        };
+        auto estimate = [&](uint32_t key) {
+            int est = 0;
+#pragma unroll
+            for (int q = 0; q < K; q++) est += entries_from(q, key);
+            tell((uint32_t)wave_sum_i32(est), 0u);
+            est = 0;
+#pragma unroll
+            for (int w = 0; w < W; w++) est += (int)told(w, 0);
+            par ^= 1;
+            return est;
+        };
+        constexpr int kMost = kBatchCap - F;  // (every child gets one more)
+        int target = need + (need >> 3) + 4;
+        if (target > kMost) target = kMost;
+        int acc_hi = target + (target >> 1);
+        if (acc_hi < 2 * NT) acc_hi = 2 * NT;  // (two entries a thread cost hardly more than one)
+        if (acc_hi > kMost) acc_hi = kMost;
+        uint32_t T = lo_key;
+        const int at_lo = estimate(lo_key);
+        if (at_lo > acc_hi) {
+            int n_evals = 0;
+            T = search_threshold(lo_key, hi_key, target, acc_hi, target, n_evals, estimate,
+                                 [](uint32_t, uint32_t) { return 0u; }, (float)at_lo);
+        }
+        // ---- the entries of every child that are worked out ----
+        int c[K];
+        int sum = 0;
+#pragma unroll
+        for (int q = 0; q < K; q++) {
+            const int n = entries_from(q, T);
+            c[q] = n > 0 && n < need ? n + 1 : n;
+            sum += c[q];
+        }
+        int inc = wave_inclusive_sum(sum, lane);
+        tell((uint32_t)__builtin_amdgcn_readlane(inc, 63), 0u);
+        int total = 0, before = 0;
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const int n = (int)told(w, 0);
+            before += w < wv ? n : 0;
+            total += n;
+        }
+        par ^= 1;
+        if (total > kBatchCap) {
+            // (the closed form jumps over the window: many entries on one key)  In proportion, and one at least
+            const float f = (float)kMost * __frcp_rn((float)total) * 0.999f;
+            sum = 0;
+#pragma unroll
+            for (int q = 0; q < K; q++) {
+                if (c[q] > 1) c[q] = 1 + (int)((float)(c[q] - 1) * f);
+                sum += c[q];
+            }
+            inc = wave_inclusive_sum(sum, lane);
+            tell((uint32_t)__builtin_amdgcn_readlane(inc, 63), 0u);
+            total = before = 0;
+#pragma unroll
+            for (int w = 0; w < W; w++) {
+                const int n = (int)told(w, 0);
+                before += w < wv ? n : 0;
+                total += n;
+            }
+            par ^= 1;
+            if (total > kBatchCap) {
+                ok = false;
+                break;
+            }
+        }
+        int at[K];
+        int run = before + inc - sum;
+#pragma unroll
+        for (int q = 0; q < K; q++) {
+            const int i = t + q * NT;
+            at[q] = run;
+            run += c[q];
+            if (i < F) {
+                lds.offs[i] = at[q];
+                seg_end[i] = run;
+            }
+            constexpr int kLone = 8;  // entries a thread marks by itself
+            for (int e = 0; e < kLone; e++) {
+                if (__ballot(e < c[q]) == 0ull) break;
+                if (e < c[q]) own[at[q] + e] = (uint32_t)i;
+            }
+            uint64_t many = __ballot(c[q] > kLone);
+            while (many != 0ull) {
+                const int src = __ffsll((long long)many) - 1;
+                many &= many - 1ull;
+                const int n = __builtin_amdgcn_readlane(c[q], src), a0 = __builtin_amdgcn_readlane(at[q], src);
+                const uint32_t who = (uint32_t)__builtin_amdgcn_readlane(i, src);
+                for (int e = kLone + lane; e < n; e += kWave) own[a0 + e] = who;
+            }
+        }
+        sync();
+        // ---- work them out ----
+        for (int e = t; e < total; e += NT) {
+            const int i = (int)own[e];
+            const int j = lds.st_j0[i] + e - lds.offs[i];
+            uint32_t kk, pp;
+            entry_key<R, RAVE>(lds.st_n[i], lds.st_w[i], lds.st_p[i], lds.st_vl[i], lds.st_q2[i], ep, uvl, j, i, kk, pp);
+            ent[e] = ((uint64_t)~kk << 32) | (pp >= (uint32_t)F ? 0x80000000u : 0u) | ((uint32_t)i << 21) | (uint32_t)j;
+        }
+        sync();
+        // ---- every child's entries in order?  And the first entry behind which one may be missing ----
+        bool bad = false;
+        for (int e = t; e < total; e += NT) {
+            if (e == 0) continue;
+            const uint64_t p = ent[e - 1], x = ent[e];
+            if (((p ^ x) & 0x7FE00000ull) == 0ull && x < p) bad = true;
+        }
+        uint32_t bk = 0u, bl = 0xFFFFFFFFu;  // as a key (larger = earlier) and the rest of the entry
+#pragma unroll
+        for (int q = 0; q < K; q++) {
+            const int i = t + q * NT;
+            uint64_t last = ~0ull;
+            if (c[q] > 0 && c[q] < need) last = ent[at[q] + c[q] - 1];
+            else if (c[q] == 0 && hk[q] != 0u)
+                last = ((uint64_t)~hk[q] << 32) | (hp[q] >= (uint32_t)F ? 0x80000000u : 0u) | ((uint32_t)i << 21) | (uint32_t)tk[q];
+            const uint32_t lk = ~(uint32_t)(last >> 32), ll = (uint32_t)last;
+            if (lk > bk || (lk == bk && ll < bl)) {
+                bk = lk;
+                bl = ll;
+            }
+        }
+        {
+            const uint32_t top = wave_max_all(bk);
+            const uint32_t low = wave_min_u32(bk == top ? bl : 0xFFFFFFFFu);
+            if (__ballot(bad) != 0ull) tell(0xFFFFFFFFu, 0u);  // (no score has that key)
+            else tell(top, low);
+        }
+        uint64_t bar = ~0ull;
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const uint64_t b = ((uint64_t)~told(w, 0) << 32) | told(w, 1);
+            bar = b < bar ? b : bar;
+        }
+        par ^= 1;
+        if ((bar >> 32) == 0ull) {
+            ok = false;
+            break;
+        }
+        // ---- the entries up to there, in order ----
+        const float y0 = y_of(hi_key), y1 = y_of(umax32(T, ~(uint32_t)(bar >> 32)));
+        const float scale = y1 > y0 ? (RAVE ? 1.0f : (float)kMergeBuckets) * __frcp_rn(y1 - y0) : 0.0f;
+        for (int e = t; e < total; e += NT) {
+            const uint64_t x = ent[e];
+            if (x > bar) continue;
+            const float y = y_of(~(uint32_t)(x >> 32));
+            int b;
+            if (RAVE) {
+                const float d = (y1 - y) * scale;  // 1 .. 0
+                b = kMergeBuckets - 1 - ((int)(__float_as_uint(d > 0.0f ? d : 0.0f) >> 17) - (0x3F800000 >> 17) + kMergeBuckets);
+                b = b < 0 ? 0 : (b > kMergeBuckets - 1 ? kMergeBuckets - 1 : b);
+            } else {
+                float fb = (y - y0) * scale;
+                fb = fb > 0.0f ? fb : 0.0f;
+                b = fb < (float)(kMergeBuckets - 1) ? (int)fb : kMergeBuckets - 1;
+            }
+            arrival[e] = ((uint32_t)b << 16) | (uint32_t)atomicAdd(&bucket[b], 1);
+        }
+        sync();
+        int own_n[kMergeOwn], lsum = 0, fullest = 0;
+#pragma unroll
+        for (int u = 0; u < kMergeOwn; u++) {
+            own_n[u] = bucket[t * kMergeOwn + u];
+            runs[t * kMergeOwn + u] = 0;
+            lsum += own_n[u];
+            fullest = own_n[u] > fullest ? own_n[u] : fullest;
+        }
+        const int binc = wave_inclusive_sum(lsum, lane);
+        tell((uint32_t)__builtin_amdgcn_readlane(binc, 63), __ballot(fullest > kMergeCount) != 0ull ? 1u : 0u);
+        int n_in = 0, start = binc - lsum;
+        bool piled = false;  // a child whose key hardly moves with virtual loss puts its entries in one bucket
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const int n = (int)told(w, 0);
+            start += w < wv ? n : 0;
+            n_in += n;
+            piled |= told(w, 1) != 0u;
+        }
+        par ^= 1;
+#pragma unroll
+        for (int u = 0; u < kMergeOwn; u++) {
+            bucket[t * kMergeOwn + u] = start;
+            start += own_n[u];
+        }
+        if (t == NT - 1) bucket[kMergeBuckets] = start;
+        sync();
+        if (n_in == 0) {
+            ok = false;
+            break;
+        }
+        for (int e = t; e < total; e += NT) {
+            const uint64_t x = ent[e];
+            if (x > bar) continue;
+            const uint32_t w = arrival[e];
+            const int b = (int)(w >> 16), b0 = bucket[b];
+            ent2[b0 + (int)(w & 0xFFFFu)] = x;
+            if (piled) {
+                const int i = (int)((uint32_t)x >> 21) & 1023;
+                if (e == lds.offs[i] || (int)(arrival[e - 1] >> 16) != b)
+                    run_at[b0 + atomicAdd(&runs[b], 1)] = (uint32_t)e | ((uint32_t)seg_end[i] << 16);
+            }
+        }
+        sync();
+        bad = false;
+        for (int e = t; e < total; e += NT) {
+            const uint64_t x = ent[e];
+            if (x > bar) continue;
+            const int b = (int)(arrival[e] >> 16);
+            const int b0 = bucket[b], b1 = bucket[b + 1];
+            if (b0 >= need) continue;
+            int rank = b0;
+            const int n_runs = b1 - b0 > kMergeCount ? runs[b] : b1 - b0;
+            if (b1 - b0 > kMergeCount && 8 * n_runs < b1 - b0) {
+                // few children, each with its entries here in order and next to each other
+                for (int r = 0; r < n_runs; r++) {
+                    const uint32_t d = run_at[b0 + r];
+                    const int first = (int)(d & 0xFFFFu);
+                    int lo = first, hi = (int)(d >> 16);
+                    hi = hi < first + (b1 - b0) ? hi : first + (b1 - b0);
+                    while (lo < hi) {
+                        const int mid = (lo + hi) >> 1;
+                        if (ent[mid] < x) lo = mid + 1;
+                        else hi = mid;
+                    }
+                    rank += lo - first;
+                }
+            } else {
+                int o = b0;
+                for (; o + 8 <= b1; o += 8) {
+                    uint64_t v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) v[u] = ent2[o + u];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) rank += v[u] < x ? 1 : 0;
+                }
+                for (; o < b1; o++) rank += ent2[o] < x ? 1 : 0;
+            }
+            if (rank >= need) continue;
+            if ((x >> 32) == 0xFFFFFFFFull) bad = true;  // no key
+            const uint32_t pay = (uint32_t)x & 0x7FFFFFFFu;
+            order[done + rank] = pay;
+            atomicMax(&lds.st_j0[pay >> 21], (int)(pay & 0x1FFFFFu) + 1);
+        }
+        tell(__ballot(bad) != 0ull ? 1u : 0u, 0u);
+#pragma unroll
+        for (int w = 0; w < W; w++) ok = ok && told(w, 0) == 0u;
+        par ^= 1;
+        if (!ok) break;
+        done += n_in < need ? n_in : need;
+    }
+    if (t == 0) {
+        lds.cmd.merged = ok ? 1 : 0;
+        lds.cmd.n_barriers = barriers;
+    }
+    __syncthreads();
+}
 
 
 // A lower end of the key range with at least `least` and at most 64 of the keys that `count` counts at or above it,
@@ -2167,517 +2538,6 @@ __device__ __forceinline__ uint32_t first_heads(const Kids<R, RAVE> &k, uint32_t
     };
     if (heads(1u) <= kWave) return 1u;
     return halve_to_lanes(heads, wave_max_u32(best_key), m);
-}
-
-// A node where one child wins ALMOST every time: the winner order is that child's list with
-// a few entries of other children merged in.  The child, A, is the one that holds out longest,
-// the one with the best entry (lk, lp) for the node's LAST visitor (not always the one with the
-// best next entry: a child whose score is mostly exploration starts high and drops at once).
-// Only a child whose next entry comes before the last-visitor entry (lk0, lp0) of the child
-// with the best next entry can be A or get an entry in (A's last entry is at or before that
-// one), so these few are listed one per lane first.  Every other child's entries that can get
-// in come before (lk, lp); when there are at most 64 of them in all, each finds its place
-// directly: the number of A's entries that come before it (a bisection on A's list, evaluated
-// once into LDS) plus the number of such entries of other children that do.  No threshold
-// search, no sort.  Exactness rests on: A's entries 0 .. m-1 in order (checked one by one);
-// every other child's used entries in order and its first unused one either not before
-// (lk, lp) (count_before brackets the count by two exact evaluations) or looked at and placed
-// behind the m-th winner (checked).  Then the best head at any step is never one of the heads
-// left out, and merging the lists by (key, position) is the serial order.
-// On success (kMergeDone): order[q] = (child << 21) | visit number for the m visitors, cnt[] the visits
-// per child.  kMergeMany: the entries of the others are too many for one per lane.  On failure nothing the caller relies on has changed (order[] is scratch).
-template <int R, bool RAVE>
-__device__ __forceinline__ int sparse_merge(const SelectArgs &a, const NodeCtx &c, int lane, const Kids<R, RAVE> &k,
-                                             int best0, uint32_t lk0, uint32_t lp0, int m, WaveLds<R> &lds,
-                                             uint32_t *order, int (&cnt)[R], bool &pending) {
-    constexpr int F = R * kWave;
-    const uint32_t uvl = (uint32_t)a.vl;
-    // ---- the children that matter, one per lane ----
-    int n0 = 0;
-    bool listed[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int i = r * kWave + lane;
-        uint32_t hk = k.k1[r], hp = (uint32_t)i;
-        if (k.k2[r] > k.k1[r]) {
-            hk = k.k2[r];
-            hp = (uint32_t)(F + i);
-        }
-        listed[r] = hk != 0u && (i == best0 || comes_before(hk, hp, lk0, lp0));
-        const uint64_t cm = __ballot(listed[r]);
-        if (listed[r]) {
-            const int cl = n0 + __popcll(cm & ((1ull << lane) - 1ull));
-            if (cl < kSparseMax) {
-                lds.st_j0[cl] = i;
-                lds.st_n[cl] = k.n[r];
-                lds.st_w[cl] = k.w[r];
-                lds.st_p[cl] = k.p[r];
-                lds.st_vl[cl] = k.vl[r];
-                lds.st_q2[cl] = k.q2[r];
-            }
-        }
-        n0 += __popcll(cm);
-    }
-    if (n0 < 2) return kMergeNo;
-    if (n0 > kSparseMax) return kMergeMany;
-    wave_sync_memory();
-    int ci = -1, cn = 0, cvl = 0;
-    float cw = 0.0f, cp = 0.0f, cq2 = 0.0f;
-    uint32_t hk = 0u, hp = 0xFFFFFFFFu, zk = 0u, zp = 0xFFFFFFFFu;  // the child's next entry and its last-visitor entry
-    if (lane < n0) {
-        ci = lds.st_j0[lane];
-        cn = lds.st_n[lane];
-        cw = lds.st_w[lane];
-        cp = lds.st_p[lane];
-        cvl = lds.st_vl[lane];
-        cq2 = lds.st_q2[lane];
-        entry_key<R, RAVE>(cn, cw, cp, cvl, cq2, c.ep, uvl, 0, ci, hk, hp);
-        entry_key<R, RAVE>(cn, cw, cp, cvl, cq2, c.ep, uvl, m - 1, ci, zk, zp);
-    }
-    // ---- A: the child that holds out longest ----
-    uint32_t lk, lp;
-    wave_best(zk, zp, lk, lp);
-    if (lk == 0u) return kMergeNo;
-    const uint64_t am = __ballot(lane < n0 && zk == lk && zp == lp);
-    if (am == 0ull) return kMergeNo;
-    const int a_lane = __ffsll((long long)am) - 1;
-    const int a_child = __builtin_amdgcn_readlane(ci, a_lane);
-    const int a_n = __builtin_amdgcn_readlane(cn, a_lane);
-    const int a_vl = __builtin_amdgcn_readlane(cvl, a_lane);
-    const float a_w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cw), a_lane));
-    const float a_p = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cp), a_lane));
-    const float a_q2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cq2), a_lane));
-    // ---- the others that can get an entry in: next entry before (lk, lp) ----
-    const bool is_cand = lane < n0 && lane != a_lane && hk != 0u && comes_before(hk, hp, lk, lp);
-    if (__ballot(is_cand) == 0ull) return kMergeNo;
-    {
-        // Far too many entries by the estimates: leave before anything exact is paid for.  An entry
-        // of a child gets in only if fewer than m entries come before it; the child's next entry has
-        // r0 of A's entries before it, so its entry number t has at least r0 + t, and no more than
-        // m - r0 of its entries can get in, however many come before (lk, lp) (two children whose
-        // scores hardly move with virtual loss, a RAVE blend that dominates both, can have hundreds
-        // there and still only meet at the very end).
-        int est = 0;
-        if (is_cand) {
-            const int r0 = predict_count<RAVE>(a_n, a_w, a_p, a_vl, a_q2, c.ep, uvl, key_score(hk), m);
-            const int room = m - r0 > 1 ? m - r0 : 1;
-            est = predict_count<RAVE>(cn, cw, cp, cvl, cq2, c.ep, uvl, key_score(lk), kSparseMax + 1);
-            est = est < room ? est : room;
-        }
-        // (a little below the capacity: the exact counts tend to come out above the estimates, and
-        // a refusal after them costs three times what one here does)
-        if (wave_sum_i32(est) > kSparseMax - 4) return kMergeMany;
-    }
-    // ---- A's entries, all m of them, evaluated once into LDS and checked: none may come before its
-    // predecessor (its head then stays at or before (lk, lp) throughout) ----
-    // as one 64-bit number per entry, smaller = played earlier: inverted key above the position
-    unsigned long long *akp = reinterpret_cast<unsigned long long *>(lds.key[0]);  // m < kHeavyMin = kBatchCap / 2 entries
-    {
-        bool bad_a = false;
-        uint32_t carry_k = 0xFFFFFFFFu, carry_p = 0u;  // entry before the chunk
-        for (int base = 0; base < m; base += kWave) {
-            const int j = base + lane;
-            uint32_t kk = 0u, pp = 0xFFFFFFFFu;
-            if (j < m) {
-                entry_key<R, RAVE>(a_n, a_w, a_p, a_vl, a_q2, c.ep, uvl, j, a_child, kk, pp);
-                akp[j] = ((unsigned long long)~kk << 32) | pp;
-            }
-            uint32_t pk = (uint32_t)__shfl_up((int)kk, 1, kWave);
-            uint32_t ppos = (uint32_t)__shfl_up((int)pp, 1, kWave);
-            if (lane == 0) {
-                pk = carry_k;
-                ppos = carry_p;
-            }
-            if (j < m && (kk == 0u || comes_before(kk, pp, pk, ppos))) bad_a = true;
-            carry_k = (uint32_t)__builtin_amdgcn_readlane((int)kk, 63);
-            carry_p = (uint32_t)__builtin_amdgcn_readlane((int)pp, 63);
-        }
-        if (__ballot(bad_a) != 0ull) return kMergeNo;
-    }
-    wave_sync_memory();
-    // how many of A's entries come before the entry (tk, tp): the list is in order, so a bisection
-    // on the exact keys
-    auto rank_in_a = [&](uint32_t tk, uint32_t tp) {
-        const unsigned long long t64 = ((unsigned long long)~tk << 32) | tp;
-        int lo = 0, hi = m;
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (akp[mid] < t64) lo = mid + 1;
-            else hi = mid;
-        }
-        return lo;
-    };
-    // ---- how many entries each of the others has before (lk, lp), at most m - r0 (see above) ----
-    int cc = 0, cap = 1;
-    if (is_cand) {
-        cap = m - rank_in_a(hk, hp);  // at least 1: A's last entry does not come before this one
-        if (cap > kSparseMax + 1) cap = kSparseMax + 1;
-        if (cap < 1) cap = 1;
-        cc = count_before<R, RAVE>(cn, cw, cp, cvl, cq2, c.ep, uvl, ci, lk, lp, cap, true);
-    }
-    const int inc = wave_inclusive_sum(cc, lane);
-    const int total = __builtin_amdgcn_readlane(inc, 63);
-    if (total > kSparseMax) return kMergeMany;
-    const int start = inc - cc;
-    // ---- one lane per entry: (lane of its child, visit number) ----
-    for (int t = 0; t < cc; t++) lds.hist[start + t] = lane | (t << 8);  // start + cc <= total <= 64
-    wave_sync_memory();
-    int bad = 0;  // nonzero: the merge is refused
-    uint32_t ek = 0u, epos = 0xFFFFFFFFu;
-    int e_child = -1, e_t = 0, rank_a = m;
-    if (lane < total) {
-        const uint32_t w0 = (uint32_t)lds.hist[lane];
-        const int e_cl = (int)(w0 & 255u);
-        e_t = (int)(w0 >> 8);
-        e_child = lds.st_j0[e_cl];
-        entry_key<R, RAVE>(lds.st_n[e_cl], lds.st_w[e_cl], lds.st_p[e_cl], lds.st_vl[e_cl], lds.st_q2[e_cl], c.ep, uvl,
-                           e_t, e_child, ek, epos);
-        if (ek == 0u) bad = 1;
-        rank_a = rank_in_a(ek, epos);
-    }
-    {
-        // a child's entries sit in neighbouring lanes, in visit order: none may come before its predecessor
-        const uint32_t pk = (uint32_t)__shfl_up((int)ek, 1, kWave);
-        const uint32_t pp = (uint32_t)__shfl_up((int)epos, 1, kWave);
-        if (lane < total && e_t > 0 && comes_before(ek, epos, pk, pp)) bad = 2;
-    }
-    // ---- the other entries before each of them (equal keys at one position: one child, visit order) ----
-    // as 64-bit numbers again, with the lane below the position: all different, a child's entries in visit order
-    unsigned long long *ekp = reinterpret_cast<unsigned long long *>(lds.key[1]);  // all lanes read all entries: through LDS
-    const unsigned long long e64 =
-        lane < total ? ((unsigned long long)~ek << 32) | ((unsigned long long)epos << 8) | (unsigned)lane : ~0ull;
-    ekp[lane] = e64;
-    wave_sync_memory();
-    int fr = 0;
-    // (eight reads in flight at a time: one wavefront alone waits out every LDS access it depends on)
-    for (int e0 = 0; e0 < total; e0 += 8) {
-        unsigned long long o[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) o[u] = ekp[e0 + u];  // lanes past `total` hold the largest number: before nothing
-#pragma unroll
-        for (int u = 0; u < 8; u++) fr += o[u] < e64 ? 1 : 0;
-    }
-    const int posn = rank_a + fr;
-    const bool valid = lane < total && posn < m;
-    {
-        // of a child's entries the ones that get in are the first ones
-        const int pv = __shfl_up(valid ? 1 : 0, 1, kWave);
-        if (valid && e_t > 0 && pv == 0) bad = 3;
-    }
-    const uint64_t vmask = __ballot(valid);
-    const int nfv = __popcll(vmask);
-    int mine_in = 0;  // entries of this lane's child that get in
-    if (is_cand) {
-        const uint64_t mine = cc >= 64 ? ~0ull : ((1ull << cc) - 1ull);
-        mine_in = __popcll((vmask >> start) & mine);
-        // a child all of whose counted entries get in, counted up to its limit: its next entry was
-        // not looked at
-        if (mine_in == cc && cc == cap) bad = 4;
-    }
-    {
-        const int why = (int)wave_max_u32((uint32_t)bad);
-        if (why != 0) return kMergeNo;
-    }
-    // ---- the winner order: the others' entries at their places, A's in between ----
-    close_pending(pending);  // the previous node's partition may still read the order buffer
-    for (int q = lane; q < m; q += kWave) order[q] = 0u;
-    wave_sync_memory();
-    if (valid) order[posn] = 0x80000000u | ((uint32_t)e_child << 21) | (uint32_t)e_t;
-    wave_sync_memory();
-    int seen = 0;
-    for (int base = 0; base < m; base += kWave) {
-        const int q = base + lane;
-        const uint32_t v = q < m ? order[q] : 0u;
-        const bool other = (v >> 31) != 0u;
-        const uint64_t om = __ballot(other);
-        const int below = seen + __popcll(om & ((1ull << lane) - 1ull));
-        if (q < m) order[q] = other ? (v & 0x7FFFFFFFu) : (((uint32_t)a_child << 21) | (uint32_t)(q - below));
-        seen += __popcll(om);
-    }
-    if (seen != nfv) return kMergeNo;  // two entries at one place: cannot happen when the checks hold
-    // ---- visits per child, back to the lanes that hold the children ----
-    if (lane < n0) lds.hist[kSparseMax + lane] = lane == a_lane ? m - nfv : mine_in;
-    wave_sync_memory();
-    int cl_run = 0;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const uint64_t cm = __ballot(listed[r]);
-        cnt[r] = listed[r] ? lds.hist[kSparseMax + cl_run + __popcll(cm & ((1ull << lane) - 1ull))] : 0;
-        cl_run += __popcll(cm);
-    }
-    return kMergeDone;
-}
-
-
-constexpr int kFewMax = 64;  // visitors of a node that few_visitors settles, at most
-constexpr int kFewEntries = 4;  // entries of every child it evaluates
-
-// A contested node of at most 64 visitors that spread out (more entries of other children than the merge above has
-// lanes for), settled at once.  Only the children with the m first heads matter (first_heads), one per lane.  Every
-// lane evaluates its child's next kFewEntries entries, independently of each other where the serial loop waits for a
-// division chain per visitor; a threshold with at least m and at most 64 of all these entries above it is found by
-// halving the key range, and the entries above it, one per lane, find their places by counting the ones before them.
-// Exact because: every child's entries used are in order (checked), so the merge of the lists in the order (key,
-// position, visit) is the serial order; and no child has all its evaluated entries above the threshold (declined),
-// so an entry not evaluated comes after one that is never reached.
-// A function of its own, and only in the kernel for trees that have grown on the device (SPREAD), whose nodes have
-// many children without visits.  Where nodes like that are rare its mere presence costs the others (five registers of
-// the wide classes and their spills): launched for uploaded trees too, 64 visitors of a Gomoku tree took 85.3 us a pass
-// in the place of 83.3, 16 on each of 64 Go trees 133.6 in the place of 130.1; in the HEAVY kernels, 16384 on a Go tree
-// with RAVE 377.7 in the place of 365.6 (4096 on a chess-like tree the same).
-// Measured on an MI355X: a search of 64 visitors a batch from the bare root 1.51 -> 1.32 ms, of 48 with RAVE on a Go
-// board 1.74 -> 1.64.
-struct FewLds {
-    int child[kWave];  // the children that matter, one per lane, in child order: index in the node ...
-    int n[kWave];      // ... and statistics
-    float w[kWave], p[kWave], q2[kWave];
-    int vl[kWave];
-    unsigned long long entry[kWave];  // the entries above the threshold: smaller = played earlier, all different
-    int who[kWave];                   // lane of the child | number of the visit << 8
-    uint32_t order[kWave];            // (child << 21) | number of the visit, per visitor
-    int count[kWave];                 // visits per child
-};
-__shared__ FewLds g_few;
-
-template <bool RAVE>
-__device__ __noinline__ bool few_order(int n0, int m, float ep, uint32_t uvl, uint32_t top, int lane) {
-    constexpr int K = kFewEntries;
-    uint32_t ek[K];
-    bool second[K];
-#pragma unroll
-    for (int j = 0; j < K; j++) {
-        ek[j] = 0u;
-        second[j] = false;
-    }
-    if (lane < n0) {
-        const int cn = g_few.n[lane], cvl = g_few.vl[lane];
-        const float cw = g_few.w[lane], cp = g_few.p[lane], cq2 = RAVE ? g_few.q2[lane] : 0.0f;
-#pragma unroll
-        for (int j = 0; j < K; j++) {
-            uint32_t pos;
-            entry_key<1, RAVE>(cn, cw, cp, cvl, cq2, ep, uvl, j, lane, ek[j], pos);
-            second[j] = pos >= (uint32_t)kWave;
-        }
-    }
-    auto entries = [&](uint32_t T) {
-        int n = 0;
-#pragma unroll
-        for (int j = 0; j < K; j++) n += __popcll(__ballot(ek[j] >= T));
-        return n;
-    };
-    const int all = entries(1u);
-    if (all < m) return false;
-    const uint32_t T = all <= kWave ? 1u : halve_to_lanes(entries, top, m);
-    if (T == 0u) return false;
-    int mine = 0;
-    bool bad = ek[K - 1] >= T;
-#pragma unroll
-    for (int j = 0; j < K; j++) {
-        const bool in = ek[j] >= T;
-        mine += in ? 1 : 0;
-        // (an entry of the second scan at the key of the one of the first scan before it is in order)
-        if (j > 0 && in && (ek[j] > ek[j - 1] || (ek[j] == ek[j - 1] && second[j - 1] && !second[j]))) bad = true;
-    }
-    if (__ballot(bad) != 0ull) return false;
-    const int inc = wave_inclusive_sum(mine, lane);
-    const int start = inc - mine, total = __builtin_amdgcn_readlane(inc, 63);
-    g_few.entry[lane] = ~0ull;
-    wave_sync_memory();
-#pragma unroll
-    for (int j = 0; j < K; j++) {
-        if (j < mine) {
-            const uint32_t pos = (uint32_t)((second[j] ? kWave : 0) + lane);
-            g_few.entry[start + j] = ((unsigned long long)~ek[j] << 32) | (pos << 8) | (unsigned)(start + j);
-            g_few.who[start + j] = lane | (j << 8);
-        }
-    }
-    wave_sync_memory();
-    const unsigned long long e64 = g_few.entry[lane];
-    int rank = 0;
-    for (int e0 = 0; e0 < total; e0 += 8) {
-        unsigned long long o[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) o[u] = g_few.entry[e0 + u];
-#pragma unroll
-        for (int u = 0; u < 8; u++) rank += o[u] < e64 ? 1 : 0;
-    }
-    const bool valid = lane < total && rank < m;
-    const uint64_t vmask = __ballot(valid);
-    if (valid) {
-        const int who = g_few.who[lane];
-        g_few.order[rank] = ((uint32_t)g_few.child[who & 255] << 21) | (uint32_t)(who >> 8);
-    }
-    g_few.count[lane] = __popcll((vmask >> (start & 63)) & ((1ull << mine) - 1ull));  // (mine < 64; none: 0)
-    wave_sync_memory();
-    return true;
-}
-
-// Returns false with nothing the caller relies on changed.
-template <int R, bool RAVE>
-__device__ __forceinline__ bool few_visitors(const SelectArgs &a, const NodeCtx &c, int lane, const Kids<R, RAVE> &k,
-                                             uint32_t best_key, int best, int m, uint32_t *order, int (&cnt)[R],
-                                             bool &pending) {
-    // Only where the visitors are sure to spread: m children's next entries come before the second entry of the best
-    // one.  (Where they do not, finding that out below costs 5 us; this test a twentieth of a node.)
-    {
-        int bn = 0, bvl = 0;
-        float bw = 0.0f, bp = 0.0f, bq2 = 0.0f;
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            if (r == (best >> 6)) {
-                bn = k.n[r];
-                bw = k.w[r];
-                bp = k.p[r];
-                bvl = k.vl[r];
-                bq2 = k.q2[r];
-            }
-        }
-        uint32_t key, pos;
-        entry_key<1, RAVE>(bn, bw, bp, bvl, bq2, c.ep, (uint32_t)a.vl, 1, 0, key, pos);
-        key = (uint32_t)__builtin_amdgcn_readlane((int)key, best & 63);
-        int before = 0;
-#pragma unroll
-        for (int r = 0; r < R; r++) before += __popcll(__ballot(umax32(k.k1[r], k.k2[r]) > key));
-        if (before < m) return false;
-    }
-    const uint32_t T0 = first_heads<R, RAVE>(k, best_key, m);
-    if (T0 == 0u) return false;
-    int n0 = 0;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const bool in = umax32(k.k1[r], k.k2[r]) >= T0;
-        const uint64_t cm = __ballot(in);
-        if (in) {
-            const int cl = n0 + __popcll(cm & ((1ull << lane) - 1ull));
-            g_few.child[cl] = r * kWave + lane;
-            g_few.n[cl] = k.n[r];
-            g_few.w[cl] = k.w[r];
-            g_few.p[cl] = k.p[r];
-            g_few.vl[cl] = k.vl[r];
-            if (RAVE) g_few.q2[cl] = k.q2[r];
-        }
-        n0 += __popcll(cm);
-    }
-    wave_sync_memory();
-    if (!few_order<RAVE>(n0, m, c.ep, (uint32_t)a.vl, wave_max_u32(best_key), lane)) return false;
-    close_pending(pending);  // the previous node's partition may still read the order buffer
-    if (lane < m) order[lane] = g_few.order[lane];
-    int base = 0;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const bool in = umax32(k.k1[r], k.k2[r]) >= T0;
-        const uint64_t cm = __ballot(in);
-        cnt[r] = in ? g_few.count[base + __popcll(cm & ((1ull << lane) - 1ull))] : 0;
-        base += __popcll(cm);
-    }
-    wave_sync_memory();
-    return true;
-}
-
-// A wide node (more than 64 child slots) whose visitors split, settled as a narrow one.  Of all its
-// children only those can be chosen whose next entry comes before the entry (lk0, lp0) that the child
-// with the best next entry, B, shows its LAST visitor, provided B's entries are in order: B's head is
-// then at or before (lk0, lp0) at every step, so a child whose head does not come before that entry is
-// never the best.  Where B's order is provable (keys_provably_monotone) and these children are at most
-// 64, they are moved to one lane each, in child order (positions keep their order, and every first-scan
-// candidate still comes before every second-scan one), and the water level of the narrow class settles
-// them: its probes walk one round of children instead of R.  The winner order comes back with the
-// children's own indices, the visits per child to the lanes that hold them.  Returns false with nothing
-// the caller relies on changed (cnt[] zero).
-template <int R, bool RAVE>
-__device__ __forceinline__ bool narrow_water_level(const SelectArgs &a, const NodeCtx &c, int lane,
-                                                   const Kids<R, RAVE> &k, int soff, int best0, uint32_t lk0,
-                                                   uint32_t lp0, int m, WaveLds<R> &lds, int (&cnt)[R], int &lds_cur,
-                                                   uint32_t *order, bool &pending) {
-    static_assert(R > 1, "a narrow node is settled as it is");
-    constexpr int F = R * kWave;
-    const uint32_t uvl = (uint32_t)a.vl;
-    int n0 = 0;
-    bool listed[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int i = r * kWave + lane;
-        uint32_t hk = k.k1[r], hp = (uint32_t)i;
-        if (k.k2[r] > k.k1[r]) {
-            hk = k.k2[r];
-            hp = (uint32_t)(F + i);
-        }
-        listed[r] = hk != 0u && (i == best0 || comes_before(hk, hp, lk0, lp0));
-        const uint64_t cm = __ballot(listed[r]);
-        if (listed[r]) {
-            const int cl = n0 + __popcll(cm & ((1ull << lane) - 1ull));
-            if (cl < kWave) {
-                lds.st_j0[cl] = i;
-                lds.st_n[cl] = k.n[r];
-                lds.st_w[cl] = k.w[r];
-                lds.st_p[cl] = k.p[r];
-                lds.st_vl[cl] = k.vl[r];
-                lds.st_q2[cl] = k.q2[r];
-            }
-        }
-        n0 += __popcll(cm);
-    }
-    if (n0 < 2 || n0 > kWave) return false;
-    wave_sync_memory();
-    Kids<1, RAVE> kc;
-    int orig = -1;
-    kc.part[0] = lane < n0;
-    kc.n[0] = 0;
-    kc.w[0] = 0.0f;
-    kc.p[0] = 0.0f;
-    kc.vl[0] = 0;
-    kc.q2[0] = 0.0f;
-    if (lane < n0) {
-        orig = lds.st_j0[lane];
-        kc.n[0] = lds.st_n[lane];
-        kc.w[0] = lds.st_w[lane];
-        kc.p[0] = lds.st_p[lane];
-        kc.vl[0] = lds.st_vl[lane];
-        kc.q2[0] = lds.st_q2[lane];
-    }
-    score_round<1, RAVE>(kc, 0, c.ep);
-    {
-        const bool b_ok = orig == best0 && keys_provably_monotone<RAVE>(kc.n[0], kc.w[0], kc.p[0], kc.vl[0], kc.q2[0],
-                                                                       c.ep, uvl, m - 1);
-        if (__ballot(b_ok) == 0ull) return false;
-    }
-    wave_sync_memory();  // every lane has read its child: the scratch changes hands
-    WaveLds<1> &l1 = reinterpret_cast<WaveLds<1> &>(lds);
-    NodeCtx c1 = c;
-    c1.cc = n0;
-    c1.nelig = n0;
-    int cnt1[1] = {0};
-    const int zero1[1] = {0};
-    int cur = -1;
-    if (!water_level<1, RAVE>(a, c1, lane, kc, soff, 0, m, zero1, l1, cnt1, true, cur, false, zero1, order, pending))
-        return false;
-    // ---- back to the node's own child indices ----
-    // (every lane takes part in the exchange, whether it has an entry in this pass or not)
-    if (cur >= 0) {
-        for (int base = 0; base < m; base += kWave) {
-            const int q = base + lane;
-            const uint32_t v = q < m ? order[q] : 0u;
-            const int i = __shfl(orig, (int)((v >> 21) & 63u), kWave);
-            if (q < m) order[q] = (v & 0x80000000u) | ((uint32_t)i << 21) | (v & 0x1FFFFFu);
-        }
-    } else {
-        for (int base = 0; base < m; base += kWave) {
-            const int q = base + lane;
-            const int cl = q < m ? a.sc_child[soff + q] : 0;
-            const int i = __shfl(orig, cl & 63, kWave);
-            if (q < m) a.sc_child[soff + q] = i;
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) lds.st_j0[r * kWave + lane] = 0;
-    wave_sync_memory();
-    if (lane < n0) lds.st_j0[orig] = cnt1[0];
-    wave_sync_memory();
-#pragma unroll
-    for (int r = 0; r < R; r++) cnt[r] = lds.st_j0[r * kWave + lane];
-    lds_cur = cur;
-    wave_sync_memory();
-    return true;
 }
 
 // ---- Chains of nodes whose visitors all follow one child ----
@@ -2767,8 +2627,7 @@ __device__ __noinline__ int chain_walk(KernArgsP ka, LdsBytesP scratch, int wi, 
     long long *const trace = ka->a.trace;
     int level = 1;  // level 0 is the node settled before, whose child this walk starts at
     int bars = 0;   // block barriers taken
-    int kids = 0, contested = 0, best0 = -1, second = 0;
-    uint32_t lk0 = 0u;
+    int kids = 0, contested = 0;
     auto eligible = [&](int np_, int cc_) {
         int e = cc_;
         if (pw) {
@@ -2985,9 +2844,6 @@ __device__ __noinline__ int chain_walk(KernArgsP ka, LdsBytesP scratch, int wi, 
             } else if (sk != 0u && !comes_before(lk, lp, sk, spos)) {
                 one = false;
                 contested = 1;
-                best0 = best;
-                lk0 = lk;
-                second = lp >= (uint32_t)F ? 1 : 0;
             } else if (!entries_in_order<RMAX, RAVE>(bn, bw, bp, bvl, bq2, ep, uvl, best, m, lane)) {
                 one = false;
             }
@@ -3056,9 +2912,6 @@ __device__ __noinline__ int chain_walk(KernArgsP ka, LdsBytesP scratch, int wi, 
         g_chain.e_depth = depth;
         g_chain.e_kids = kids;
         g_chain.e_contested = contested;
-        g_chain.e_best0 = best0;
-        g_chain.e_lk0 = lk0;
-        g_chain.e_second = second;
         // the owner counts the block barriers it takes with the walk: it leaves after the one that follows these
         g_chain.n_barriers = bars;
     }
@@ -3191,11 +3044,9 @@ struct Continuation {
 //
 // HEAVY: the kernel for batches in which a node of kHeavyMin visitors can occur.  Without it (every root has fewer) the
 // slices, their boundaries and their joins are left out, and with them registers that the rest of the code then has
-// (vector registers: narrow class 160 -> 145, four rounds 224 -> 215, six 256 -> 245; scalar spills 302 -> 91, 461 -> 198,
-// 570 -> 211).  A pass with and without: 64 visitors of a Gomoku tree 81.9 and 79.3 us, 16 on each of 64 Go trees 134.3
-// and 126.2, 8 on a tree 60.3 and 55.5.
-// SPREAD: the kernel for trees that grow on the device, whose nodes have many children without visits (few_visitors).
-template <int R, bool RAVE, int RMAX, bool HEAVY, bool SPREAD>
+// (scalar spills of the narrow class 417 -> 95, of four rounds 403 -> 193, of six 533 -> 230, whose vector registers go
+// 271 -> 244).
+template <int R, bool RAVE, int RMAX, bool HEAVY>
 __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs &a, const NodeCtx &c, int lane,
                                             const Item &item, const int32_t *seg_in, int32_t *seg_out,
                                             WaveLds<R> &lds, PartLds<RMAX> &pl, bool &pending, Continuation &next,
@@ -3340,34 +3191,50 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
         settled = true;
     }
     bool contested = false;
-    int best0 = -1;
-    uint32_t lk0 = 0u, lp0 = 0xFFFFFFFFu;
     if (preload == 2) {
         // the walk has made the one-winner test on these very children, and it failed
         contested = __builtin_amdgcn_readfirstlane(g_chain.e_contested) != 0;
-        best0 = __builtin_amdgcn_readfirstlane(g_chain.e_best0);
-        lk0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)g_chain.e_lk0);
-        lp0 = (uint32_t)(__builtin_amdgcn_readfirstlane(g_chain.e_second) ? R * kWave + best0 : best0);
     } else if (!as_slice && !just_boundary && !settled && m >= kRunMin && a.vl > 0 && !odd)
-        settled = single_run<R, RAVE>(a, c, lane, k, bk, bpos, soff, m, m >= kRunShareMin, cnt, run_child, contested, best0,
-                                      lk0, lp0);
-    if (!settled && contested && m >= kSparseMin && !heavy && !odd) {
-        const int merged =
-            sparse_merge<R, RAVE>(a, c, lane, k, best0, lk0, lp0, m, lds, pl.order, cnt, pending);
-        settled = merged == kMergeDone;
-        if (settled) {
-            if (a.stats && lane == 0) atomicAdd(a.stats + 7, 1);
-        } else if constexpr (SPREAD && R > 1) {
-            if (merged == kMergeMany && m <= kFewMax) {
-                settled = few_visitors<R, RAVE>(a, c, lane, k, bk, best0, m, pl.order, cnt, pending);
-                if (settled && a.stats && lane == 0) atomicAdd(a.stats + 13, 1);
-            }
+        settled = single_run<R, RAVE>(a, c, lane, k, bk, bpos, soff, m, m >= kRunShareMin, cnt, run_child, contested);
+    if (!settled && contested && m >= kMergeMin && !heavy && !odd) {
+        close_pending(pending);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int i = r * kWave + lane;
+            lds.st_n[i] = k.n[r];
+            lds.st_w[i] = k.w[r];
+            lds.st_p[i] = k.p[r];
+            lds.st_vl[i] = k.vl[r];
+            if (RAVE) lds.st_q2[i] = k.q2[r];
+            lds.st_j0[i] = 0;
+            lds.pay[i] = k.part[r] ? 1u : 0u;
         }
+        if (lane == 0) {
+            TeamCmd &cm = lds.cmd;
+            cm.op = kOpMerge;
+            cm.rounds = R;
+            cm.total = m;
+            cm.ep = c.ep;
+            cm.uvl = uvl;
+            cm.n_barriers = -1;
+        }
+        __syncthreads();  // the request is open
+        for (int taken = 1;; taken++) {
+            __syncthreads();
+            int nb = -1;
+            if (lane == 0) nb = __hip_atomic_load(&lds.cmd.n_barriers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (uniform(nb) + 1 == taken && uniform(nb) >= 0) break;
+        }
+        settled = uniform(lds.cmd.merged) != 0;
         if (settled) {
             lds_cur = 0;
-        } else {
 #pragma unroll
-            for (int r = 0; r < R; r++) cnt[r] = 0;
+            for (int r = 0; r < R; r++) cnt[r] = lds.st_j0[r * kWave + lane];
+            if (a.stats && lane == 0) {
+                atomicAdd(a.stats + 7, 1);
+                if (R > 1 && RAVE) atomicAdd(a.stats + 12, 1);
+                if (R > 1 && m <= kWave) atomicAdd(a.stats + 13, 1);
+            }
         }
     }
     if (HEAVY && R * kWave <= kHeavyFanout) {
@@ -3538,21 +3405,6 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
         }
     }
     if (just_boundary) return kStepParked;  // (a fan-out class that is never cut into slices)
-    // (with RAVE, where every probe of the water level scores two scans per child; without it the path's code
-    // costs the kernel more than its shorter probes save)
-    if constexpr (R > 1 && RAVE) {
-        if (!settled && contested && m >= kWaterLevelMin && !heavy && a.vl > 0 && !odd && !as_slice &&
-            !as_scatter) {
-            settled = narrow_water_level<R, RAVE>(a, c, lane, k, soff, best0, lk0, lp0, m, lds, cnt, lds_cur, pl.order,
-                                                  pending);
-            if (settled && a.stats && lane == 0) atomicAdd(a.stats + 12, 1);
-            if (!settled) {
-                lds_cur = -1;
-#pragma unroll
-                for (int r = 0; r < R; r++) cnt[r] = 0;
-            }
-        }
-    }
     if (!settled && m >= kWaterLevelMin && m <= kWaterLevelMaxJ && a.vl > 0 && !odd) {
         int zero[R];
 #pragma unroll
@@ -4012,7 +3864,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
 //
 // A block is a team: its first wavefront (the owner) runs this loop, the other wavefronts
 // wait at a block barrier until the owner shares out the batch work of a node (team_help).
-template <int RMAX, bool RAVE, bool HEAVY, bool SPREAD>
+template <int RMAX, bool RAVE, bool HEAVY>
 __device__ __forceinline__ void owner_loop(const ForestDev &f, const SelectArgs &a, WaveLds<RMAX> &s_lds,
                                            PartLds<RMAX> &s_part, bool &pending, int lane) {
     for (;;) {
@@ -4098,11 +3950,11 @@ __device__ __forceinline__ void owner_loop(const ForestDev &f, const SelectArgs 
             next.chain_open = false;
             if (c.cc > 0 && depth < a.max_depth) {
                 if (c.cc <= kWave)
-                    status = select_group<1, RAVE, RMAX, HEAVY, SPREAD>(f, a, c, lane, it, seg_in, seg_out,
+                    status = select_group<1, RAVE, RMAX, HEAVY>(f, a, c, lane, it, seg_in, seg_out,
                                                          reinterpret_cast<WaveLds<1> &>(s_lds), s_part, pending,
                                                          next, preload_now == 2 ? 2 : 0);
                 else
-                    status = select_group<RMAX, RAVE, RMAX, HEAVY, SPREAD>(f, a, c, lane, it, seg_in, seg_out, s_lds, s_part, pending,
+                    status = select_group<RMAX, RAVE, RMAX, HEAVY>(f, a, c, lane, it, seg_in, seg_out, s_lds, s_part, pending,
                                                             next, preload_now);
             }
             if (a.trace && lane == 0) {
@@ -4285,7 +4137,7 @@ __device__ __forceinline__ void team_help(const ForestDev &f, const SelectArgs &
 template <int RMAX, bool RAVE>
 __device__ void walkers_loop(ForestDev f, SelectArgs a, int lane);
 
-template <int RMAX, bool RAVE, bool HEAVY, bool SPREAD>
+template <int RMAX, bool RAVE, bool HEAVY>
 __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs a) {
     __shared__ WaveLds<RMAX> s_lds;
     __shared__ PartLds<RMAX> s_part;
@@ -4301,7 +4153,7 @@ __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs
     if (tid < kWave) {
         // every path out of the owner's loop comes back here: the helpers are always released
         bool pending = false;
-        owner_loop<RMAX, RAVE, HEAVY, SPREAD>(f, a, s_lds, s_part, pending, tid);
+        owner_loop<RMAX, RAVE, HEAVY>(f, a, s_lds, s_part, pending, tid);
         close_pending(pending);
         if (tid == 0) atomicMax(a.times + 1, (int)(wall_clock64() & 0x7FFFFFFF));
         if (tid == 0) s_lds.cmd.op = kOpExit;
@@ -4339,6 +4191,14 @@ __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs
             if (RMAX > 1) chain_finish(ka, tid - kWave, kChainWalkers * kWave, levels, c_depth - 1, c_off, c_m);
             else if (wi == 0) chain_finish(ka, tid & 63, kWave, levels, c_depth - 1, c_off, c_m);
             __syncthreads();  // the request is done
+            continue;
+        }
+        if (op == kOpMerge) {
+            // (its last barrier ends the request)
+            if (rounds == 1)
+                team_merge<1, RAVE>(reinterpret_cast<WaveLds<1> &>(s_lds), s_part.order, tid - kWave, total, ep, uvl);
+            else
+                team_merge<RMAX, RAVE>(s_lds, s_part.order, tid - kWave, total, ep, uvl);
             continue;
         }
         if (RMAX > 1 && (op == kOpPartition || op == kOpLoad) && (tid >> 6) >= 2) {
@@ -4686,7 +4546,7 @@ __device__ __noinline__ void walkers_loop(ForestDev f, SelectArgs a, int lane) {
 
 template <int RMAX, bool RAVE>
 hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_items0, int most_visitors,
-                                 int n_traversals, int n_cus, bool grown, const LoneOut &out, hipStream_t s) {
+                                 int n_traversals, int n_cus, const LoneOut &out, hipStream_t s) {
     // Few walkers cannot keep the memory system busy: then the variant that spends bytes to save
     // dependent trips (select_single, FAST).  The number of lone visitors is only known on the
     // device; the number of traversals bounds it.  Measured: it pays on a board layout (legal
@@ -4717,11 +4577,9 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_i
         a.fast_singles = fast ? 1 : 0;
         const dim3 grid(teams + walkers), block(kTeam);
         if (most_visitors >= kHeavyMin)
-            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, true, false>), grid, block, 0, s, f, a);
-        else if (RMAX > 1 && grown)
-            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, false, (RMAX > 1)>), grid, block, 0, s, f, a);
+            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, true>), grid, block, 0, s, f, a);
         else
-            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, false, false>), grid, block, 0, s, f, a);
+            hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, false>), grid, block, 0, s, f, a);
         return hipGetLastError();
     }
     // every traversal is alone at its root: the walkers are the host's list

@@ -2,8 +2,8 @@
 #include "omk_select_kernels.h"
 
 namespace omk {
-template hipError_t launch_select_class<4, false>(const ForestDev &, const SelectArgs &, int, int, int, int, bool,
+template hipError_t launch_select_class<4, false>(const ForestDev &, const SelectArgs &, int, int, int, int,
                                                       const LoneOut &, hipStream_t);
-template hipError_t launch_select_class<4, true>(const ForestDev &, const SelectArgs &, int, int, int, int, bool,
+template hipError_t launch_select_class<4, true>(const ForestDev &, const SelectArgs &, int, int, int, int,
                                                       const LoneOut &, hipStream_t);
 }  // namespace omk
