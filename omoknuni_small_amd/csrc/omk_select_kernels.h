@@ -125,8 +125,10 @@ struct TeamCmd {
     int pre_node, pre_np, pre_cb, pre_cc;
     // kOpChain: the node a chain walk starts at (chain_walk), its N, child range, depth, and its visitors
     int c_node, c_np, c_cb, c_cc, c_depth, c_off, c_m;
-    // kOpMerge (`total` visitors): whether the helpers settled the node; -1 while they are at it, then the number of
-    // block barriers they took
+    // kOpMerge (`total` visitors, their winners to sc_child / sc_occ from `goff` on, or to LDS if that is negative):
+    // the threshold above which the entries counted in offs[] lie, of a slice (0: to be found); whether the helpers
+    // settled it; -1 while they are at it, then the number of block barriers they took
+    uint32_t floor_key;
     int merged, n_barriers;
 };
 
@@ -2146,9 +2148,10 @@ __device__ __forceinline__ int count_before(int n, float w, float p, int vl, flo
 // for every halving of the distance in y to it.
 // What bounds it: the dependent steps of one wavefront and some 15 block barriers; no memory.  Three wavefronts and not the
 // owner's as well: its code is the kernel's largest, and a part of it that only waits costs it no registers.
-// Measured on an MI355X, in the place of the counts and the sort of one wavefront (water_level), the whole node: 246 visitors of a chess-like node 15.6 -> 11.5 us, 75 to 190 of a Go node with
-// RAVE 23 to 33 -> 13 to 15, 944 of one 45 -> 20; 4096 on the chess-like tree 270 -> 245 us a selection, 16384 on the Go
-// tree with RAVE 373 -> 348 (with the higher kHeavyMin, which it makes worth while), a search of 500 a batch 2.96 -> 2.76 ms.
+// Measured on an MI355X, in the place of the counts and the sort of one wavefront (water_level), the whole node: 246
+// visitors of a chess-like node 15.6 -> 11.5 us, 75 to 190 of a Go node with RAVE 23 to 33 -> 13 to 15, 944 of one 45 -> 20;
+// 4096 on the chess-like tree 270 -> 245 us a selection, 16384 on the Go tree with RAVE 373 -> 348 (with the higher
+// kHeavyMin, which it makes worth while), a search of 500 a batch 2.96 -> 2.76 ms.
 constexpr int kMergeMin = 8;  // visitors from which a contested node is settled that way (5 and 14: the same)
 constexpr int kMergeThreads = (kTeamWaves - 1) * kWave;
 constexpr int kMergeOwn = 6;  // buckets a thread adds up
@@ -2157,10 +2160,15 @@ constexpr int kMergePasses = 12;
 constexpr int kMergeCount = 32;  // entries of a bucket that are ranked by counting whoever they belong to
 static_assert(2 * kMergeBuckets + 1 + 2 * kBatchCap + 1024 <= kSortBins * (kBatchCap / kWave + 1), "buckets and arrivals fit the sort's table");
 
+// A slice of a heavy node goes the same way from the visits the children have had before it (st_j0[]), with the entries
+// that its two thresholds count (offs[]) in the place of the estimate.
+// Measured (the batch of a slice of 192 visitors): chess-like 7.3 -> 5.5 us, Go with RAVE 11.5 -> 6.3; 4096 visitors on the
+// chess-like tree 245 -> 238 us a selection, 16384 on the Go tree with RAVE 348 -> 328.
 // t: number of the helper thread.  On success (cmd.merged) order[] holds (child << 21) | visit number of the m visitors and
 // st_j0[] the visits per child.  The owner takes the barriers with them.
 template <int R, bool RAVE>
-__device__ __forceinline__ void team_merge(WaveLds<R> &lds, uint32_t *order, int t, int m, float ep, uint32_t uvl) {
+__device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds, uint32_t *order, int t, int m, int goff,
+                                           float ep, uint32_t uvl) {
     constexpr int F = R * kWave, NT = kMergeThreads, W = NT / kWave;
     constexpr int K = (F + NT - 1) / NT;  // children of a thread: t, t + NT ..
     const int lane = t & 63, wv = uniform(t >> 6);
@@ -2192,9 +2200,12 @@ __device__ __forceinline__ void team_merge(WaveLds<R> &lds, uint32_t *order, int
     int cn[K], cvl[K];
     float cw[K], cp[K], cq2[K];
     bool part[K];
+    int slice_n[K];
+    const uint32_t floor_key = (uint32_t)uniform((int)lds.cmd.floor_key);
 #pragma unroll
     for (int q = 0; q < K; q++) {
         const int i = t + q * NT;
+        slice_n[q] = i < F ? lds.offs[i] : 0;
         part[q] = false;
         cn[q] = cvl[q] = 0;
         cw[q] = cp[q] = cq2[q] = 0.0f;
@@ -2211,6 +2222,7 @@ __device__ __forceinline__ void team_merge(WaveLds<R> &lds, uint32_t *order, int
     int done = 0;
     for (int pass = 0; done < m; pass++) {
         const int need = m - done;
+        const bool counted = pass == 0 && floor_key != 0u;
         // ---- the children's next entries, and the key no useful threshold lies below: a child alone has `need` entries
         // at or above the last one it could be asked for ----
         uint32_t hk[K], hp[K];
@@ -2225,8 +2237,10 @@ __device__ __forceinline__ void team_merge(WaveLds<R> &lds, uint32_t *order, int
             if (q * NT < F && part[q]) {
                 uint32_t zk, zp;
                 entry_key<R, RAVE>(cn[q], cw[q], cp[q], cvl[q], cq2[q], ep, uvl, tk[q], i, hk[q], hp[q]);
-                entry_key<R, RAVE>(cn[q], cw[q], cp[q], cvl[q], cq2[q], ep, uvl, tk[q] + need - 1, i, zk, zp);
-                if (hk[q] != 0u) lmax = umax32(lmax, zk);
+                if (!counted) {
+                    entry_key<R, RAVE>(cn[q], cw[q], cp[q], cvl[q], cq2[q], ep, uvl, tk[q] + need - 1, i, zk, zp);
+                    if (hk[q] != 0u) lmax = umax32(lmax, zk);
+                }
                 hmax = umax32(hmax, hk[q]);
             }
         }
@@ -2239,6 +2253,7 @@ __device__ __forceinline__ void team_merge(WaveLds<R> &lds, uint32_t *order, int
             hi_key = umax32(hi_key, told(w, 1));
         }
         par ^= 1;
+        if (counted) lo_key = floor_key < hi_key ? floor_key : hi_key;
         if (lo_key == 0u || lo_key > hi_key || pass >= kMergePasses) {
             ok = false;
             break;
@@ -2269,7 +2284,7 @@ __device__ __forceinline__ void team_merge(WaveLds<R> &lds, uint32_t *order, int
         if (acc_hi < 2 * NT) acc_hi = 2 * NT;  // (two entries a thread cost hardly more than one)
         if (acc_hi > kMost) acc_hi = kMost;
         uint32_t T = lo_key;
-        const int at_lo = estimate(lo_key);
+        const int at_lo = counted ? 0 : estimate(lo_key);
         if (at_lo > acc_hi) {
             int n_evals = 0;
             T = search_threshold(lo_key, hi_key, target, acc_hi, target, n_evals, estimate,
@@ -2280,7 +2295,7 @@ __device__ __forceinline__ void team_merge(WaveLds<R> &lds, uint32_t *order, int
         int sum = 0;
 #pragma unroll
         for (int q = 0; q < K; q++) {
-            const int n = entries_from(q, T);
+            const int n = counted ? (slice_n[q] < need ? slice_n[q] : need) : entries_from(q, T);
             c[q] = n > 0 && n < need ? n + 1 : n;
             sum += c[q];
         }
@@ -2492,7 +2507,12 @@ __device__ __forceinline__ void team_merge(WaveLds<R> &lds, uint32_t *order, int
             if (rank >= need) continue;
             if ((x >> 32) == 0xFFFFFFFFull) bad = true;  // no key
             const uint32_t pay = (uint32_t)x & 0x7FFFFFFFu;
-            order[done + rank] = pay;
+            if (goff >= 0) {
+                a.sc_child[goff + done + rank] = (int)(pay >> 21);
+                a.sc_occ[goff + done + rank] = (int)(pay & 0x1FFFFFu);
+            } else {
+                order[done + rank] = pay;
+            }
             atomicMax(&lds.st_j0[pay >> 21], (int)(pay & 0x1FFFFFu) + 1);
         }
         tell(__ballot(bad) != 0ull ? 1u : 0u, 0u);
@@ -3013,6 +3033,46 @@ __device__ __forceinline__ void prefetch_boundaries(const ForestDev &f, const Se
         __hip_atomic_store(a.q_ready + at + j, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The owner's part of a merge: what the helpers read (team_merge), and their barriers.  False when they decline.
+template <int R, bool RAVE>
+__device__ __forceinline__ bool ask_merge(WaveLds<R> &lds, const Kids<R, RAVE> &k, int lane, int m, int goff, float ep,
+                                          uint32_t uvl, uint32_t floor_key, const int (&had)[R], const int (&counted)[R],
+                                          bool &pending) {
+    close_pending(pending);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int i = r * kWave + lane;
+        lds.st_n[i] = k.n[r];
+        lds.st_w[i] = k.w[r];
+        lds.st_p[i] = k.p[r];
+        lds.st_vl[i] = k.vl[r];
+        if (RAVE) lds.st_q2[i] = k.q2[r];
+        lds.st_j0[i] = had[r];
+        lds.offs[i] = counted[r];
+        lds.pay[i] = k.part[r] ? 1u : 0u;
+    }
+    if (lane == 0) {
+        TeamCmd &cm = lds.cmd;
+        cm.op = kOpMerge;
+        cm.rounds = R;
+        cm.total = m;
+        cm.goff = goff;
+        cm.ep = ep;
+        cm.uvl = uvl;
+        cm.floor_key = floor_key;
+        cm.n_barriers = -1;
+    }
+    __syncthreads();  // the request is open
+    for (int taken = 1;; taken++) {
+        __syncthreads();
+        int nb = -1;
+        if (lane == 0) nb = __hip_atomic_load(&lds.cmd.n_barriers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        nb = uniform(nb);
+        if (nb >= 0 && taken == nb + 1) break;
+    }
+    return uniform(lds.cmd.merged) != 0;
+}
+
 struct Continuation {
     int node;
     int off;
@@ -3197,35 +3257,10 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
     } else if (!as_slice && !just_boundary && !settled && m >= kRunMin && a.vl > 0 && !odd)
         settled = single_run<R, RAVE>(a, c, lane, k, bk, bpos, soff, m, m >= kRunShareMin, cnt, run_child, contested);
     if (!settled && contested && m >= kMergeMin && !heavy && !odd) {
-        close_pending(pending);
+        int zero[R];
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            const int i = r * kWave + lane;
-            lds.st_n[i] = k.n[r];
-            lds.st_w[i] = k.w[r];
-            lds.st_p[i] = k.p[r];
-            lds.st_vl[i] = k.vl[r];
-            if (RAVE) lds.st_q2[i] = k.q2[r];
-            lds.st_j0[i] = 0;
-            lds.pay[i] = k.part[r] ? 1u : 0u;
-        }
-        if (lane == 0) {
-            TeamCmd &cm = lds.cmd;
-            cm.op = kOpMerge;
-            cm.rounds = R;
-            cm.total = m;
-            cm.ep = c.ep;
-            cm.uvl = uvl;
-            cm.n_barriers = -1;
-        }
-        __syncthreads();  // the request is open
-        for (int taken = 1;; taken++) {
-            __syncthreads();
-            int nb = -1;
-            if (lane == 0) nb = __hip_atomic_load(&lds.cmd.n_barriers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            if (uniform(nb) + 1 == taken && uniform(nb) >= 0) break;
-        }
-        settled = uniform(lds.cmd.merged) != 0;
+        for (int r = 0; r < R; r++) zero[r] = 0;
+        settled = ask_merge<R, RAVE>(lds, k, lane, m, -1, c.ep, uvl, 0u, zero, zero, pending);
         if (settled) {
             lds_cur = 0;
 #pragma unroll
@@ -3352,8 +3387,14 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
                         int between[R];  // entries of every child between the two thresholds
 #pragma unroll
                         for (int r = 0; r < R; r++) between[r] = ct_lo[r] - ct_hi[r];
-                        ok = water_level<R, RAVE>(a, c, lane, k, soff, rank_hi, todo, ct_hi, lds, cnt, false, unused_cur,
-                                                  preset_ok, between, pl.order, pending);
+                        if (preset_ok && ask_merge<R, RAVE>(lds, k, lane, todo, soff + rank_hi, c.ep, uvl, T_lo, ct_hi, between,
+                                                            pending)) {
+#pragma unroll
+                            for (int r = 0; r < R; r++) cnt[r] = lds.st_j0[r * kWave + lane];
+                        } else {
+                            ok = water_level<R, RAVE>(a, c, lane, k, soff, rank_hi, todo, ct_hi, lds, cnt, false, unused_cur,
+                                                      preset_ok, between, pl.order, pending);
+                        }
                     }
                 } else {
 #pragma unroll
@@ -4196,9 +4237,9 @@ __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs
         if (op == kOpMerge) {
             // (its last barrier ends the request)
             if (rounds == 1)
-                team_merge<1, RAVE>(reinterpret_cast<WaveLds<1> &>(s_lds), s_part.order, tid - kWave, total, ep, uvl);
+                team_merge<1, RAVE>(a, reinterpret_cast<WaveLds<1> &>(s_lds), s_part.order, tid - kWave, total, goff, ep, uvl);
             else
-                team_merge<RMAX, RAVE>(s_lds, s_part.order, tid - kWave, total, ep, uvl);
+                team_merge<RMAX, RAVE>(a, s_lds, s_part.order, tid - kWave, total, goff, ep, uvl);
             continue;
         }
         if (RMAX > 1 && (op == kOpPartition || op == kOpLoad) && (tid >> 6) >= 2) {
