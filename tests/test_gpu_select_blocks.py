@@ -81,3 +81,18 @@ def test_scores_that_are_not_real_and_ties(kind, rave):
 def test_widening_at_the_selection():
     soa, roots = random_tree(21, n_expand=80, fanout=(2, 200), max_depth=7, n_roots=9, sort_prior=True, n_max=400)
     both(soa, np.repeat(roots, [1, 2, 5, 9, 16, 33, 48, 63, 64]).astype(np.int32), 8, pw=True)
+
+
+@pytest.mark.parametrize("kind", ["nan sum", "no score at all", "all equal"])
+@pytest.mark.parametrize("widest,rave", [(60, False), (250, True), (380, False), (380, True)])
+def test_lone_visitors_of_masked_trees(widest, rave, kind):
+    """One visitor a root, a block a visitor with a wavefront for every 64 children: ties across wavefronts, wavefronts
+    without a real score, nodes without one (the least visited child is taken)."""
+    soa, roots = random_tree(31, n_expand=90, fanout=(2, widest), max_depth=6, n_roots=30, mask_frac=0.3, rave=rave, n_max=30)
+    some = np.random.default_rng(6).random(len(soa["N"])) < 0.5
+    some[roots] = False
+    if kind == "all equal":
+        soa["N"][:], soa["W"][:], soa["P"][:] = 1, 0.5, 0.25
+    else:
+        soa["P" if kind == "no score at all" else "W"][some if kind == "nan sum" else slice(None)] = np.nan
+    both(soa, np.array(roots, np.int32), 8, vl=2, rave=rave, steps=1)
