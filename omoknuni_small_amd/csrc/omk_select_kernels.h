@@ -3109,8 +3109,8 @@ struct Continuation {
 //
 // HEAVY: the kernel for batches in which a node of kHeavyMin visitors can occur.  Without it (every root has fewer) the
 // slices, their boundaries and their joins are left out, and with them registers that the rest of the code then has
-// (scalar spills of the narrow class 417 -> 95, of four rounds 403 -> 193, of six 533 -> 230, whose vector registers go
-// 271 -> 244).
+// (scalar spills of the narrow class 332 -> 93, of four rounds 404 -> 190, of six 649 -> 229, whose vector registers go
+// 277 -> 262).
 template <int R, bool RAVE, int RMAX, bool HEAVY>
 __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs &a, const NodeCtx &c, int lane,
                                             const Item &item, const int32_t *seg_in, int32_t *seg_out,
