@@ -77,7 +77,6 @@ constexpr int kCountSortLone = 2, kCountSortTeam = 1;
 constexpr int kRunShortcutMin = 128;      // entries from which a run of one child is emitted without sorting
 constexpr int kScatterPart = 256;         // visitors per part of a heavy node's partition, about
 constexpr int kScatterUnroll = 8;         // chunks of 64 visitors whose loads the partition issues together
-constexpr int kFewRoots = 16, kFewRootsTeams = 128;  // teams of the persistent launch for few roots, at most
 constexpr int kMaxWalkerBlocks = 16;         // blocks of walkers of the persistent launch, at most
 constexpr int kTeamSinglesMaxWaves = 4096;  // wavefronts up to which a batch of lone traversals is walked by blocks (one round of children per wavefront)
 constexpr int kFastSinglesMax = 16384;    // traversals up to which the single-visitor kernel trades bytes for latency
@@ -4693,11 +4692,6 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_i
         int teams = capacity - walkers;
         const int most = n_traversals / 2;
         if (teams > most) teams = most;
-        // Teams without work poll, and every poll is a trip to memory that the walkers' own wait behind.  A few trees do
-        // not have work for all: 4096 visitors on a chess-like tree and 16384 on a Go tree with RAVE 234 and 319 us with a
-        // team on every compute unit, 231 and 317 with 128 (before the partition was shared 238 and 327, 236 and 324 with
-        // 160, 232 and 328 with 96), 128 on each of 16 Gomoku trees 105 and 100; on each of 64 167 and 183.
-        if (n_items0 <= kFewRoots && teams > kFewRootsTeams) teams = kFewRootsTeams;
         if (teams < 1) teams = 1;
         SelectArgs a = a0;
         a.n_team_blocks = teams;
