@@ -216,9 +216,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
     BlockScratch<RMAX> &my = s.scratch[wv];
     const uint32_t uvl = a.vl > 0 ? (uint32_t)a.vl : 0u;
     for (;;) {
-        int ticket = 0;
-        if (lane == 0) ticket = atomicAdd(&s.head, 1);
-        ticket = uniform(ticket);
+        const int ticket = take_ticket(&s.head, lane);
         bool got = false;
         for (;;) {  // (ends: a visitor goes down one level with every node settled)
             const int open = uniform(__hip_atomic_load(&s.open, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));

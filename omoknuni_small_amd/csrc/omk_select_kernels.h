@@ -53,9 +53,9 @@
 // walkers behind the teams of the same persistent launch take such visitors as the teams
 // create them (one wavefront per walk, no LDS); a batch whose traversals are all alone at
 // their roots is one launch of the single-visitor kernel instead.
-#include <algorithm>
 #pragma once
 
+#include <algorithm>
 #include <cstddef>
 
 #include "omk_internal.h"
@@ -350,6 +350,19 @@ __device__ __forceinline__ int wave_pick(const Kids<R, RAVE> &k, int lane, uint3
 
 // A value that is the same in all lanes, for the compiler to know.
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// The next number of a counter that wavefronts draw from, the same in every lane.  Lane 0 draws it, at the head of a loop
+// whose body may end in another branch of lane 0's own (a count of what is done).  The compiler joins two such branches
+// across the loop's edge when it can: lane 0 then goes straight from one to the other, and the other lanes go round
+// without the number (seen in the partition's loop, which did not end).  It may not copy a barrier of the wavefront,
+// which costs no instruction: one on each side of the branch, here for every loop.
+__device__ __forceinline__ int take_ticket(int *counter, int lane) {
+    int ticket = 0;
+    __builtin_amdgcn_wave_barrier();
+    if (lane == 0) ticket = atomicAdd(counter, 1);
+    __builtin_amdgcn_wave_barrier();
+    return uniform(ticket);
+}
 
 struct NodeCtx {
     int cb;
@@ -3915,9 +3928,7 @@ template <int RMAX, bool RAVE, bool HEAVY>
 __device__ __forceinline__ void owner_loop(const ForestDev &f, const SelectArgs &a, WaveLds<RMAX> &s_lds,
                                            PartLds<RMAX> &s_part, bool &pending, int lane) {
     for (;;) {
-        int ticket = 0;
-        if (lane == 0) ticket = atomicAdd(a.sched_head, 1);
-        ticket = __builtin_amdgcn_readfirstlane(ticket);
+        const int ticket = take_ticket(a.sched_head, lane);
         if (ticket >= a.q_cap) return;
         bool got = false;
         for (int spins = 0;; spins++) {
@@ -4096,17 +4107,11 @@ template <int RMAX>
 __device__ __forceinline__ void partition_chunks(const SelectArgs &a, const TeamCmd &cm, PartLds<RMAX> &pl, int n_chunks,
                                                  int lone0, int lane) {
     for (;;) {
-        int chunk = 0;
-        if (lane == 0) chunk = atomicAdd(&pl.next, 1);
-        __builtin_amdgcn_wave_barrier();
-        chunk = uniform(chunk);
+        const int chunk = take_ticket(&pl.next, lane);
         if (chunk >= n_chunks) return;
         partition_chunk(a, cm, pl, chunk, lone0, lane);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         if (lane == 0) atomicAdd(&pl.finished, 1);
-        // the lanes go round together: without this the compiler joins lane 0's branch to the next round's, and the others
-        // read a ticket that lane 0 has not drawn
-        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -4607,9 +4612,7 @@ __global__ __launch_bounds__(RMAX * kWave) void k_select_singles_team(ForestDev 
 template <int RMAX, bool RAVE>
 __device__ __noinline__ void walkers_loop(ForestDev f, SelectArgs a, int lane) {
     for (;;) {
-        int ticket = 0;
-        if (lane == 0) ticket = atomicAdd(a.singles_head, 1);
-        ticket = __builtin_amdgcn_readfirstlane(ticket);
+        const int ticket = take_ticket(a.singles_head, lane);
         bool got = false;
         for (int spins = 0;; spins++) {
             int rdy = 0, open = 1, ab = 0, n = 0;

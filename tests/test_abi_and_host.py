@@ -204,6 +204,22 @@ def test_direct_merge_rule_against_the_serial_loop(tmp_path):
     assert m and int(m.group(1)) > 30000, out.stdout[-500:]
 
 
+def test_tickets_are_drawn_between_barriers_of_the_wavefront():
+    """Lane 0 draws a wavefront's next ticket at the head of loops that may end in another branch of lane 0's own.  Without a
+    barrier of the wavefront the compiler may join the two across the loop's edge, and the other lanes go round without the
+    ticket: every loop draws through the one function that has them (take_ticket)."""
+    import re
+    csrc = os.path.join(ROOT, "omoknuni_small_amd", "csrc")
+    text = ""
+    for name in ("omk_select_kernels.h", "omk_select_blocks.h"):
+        with open(os.path.join(csrc, name)) as f:
+            text += f.read()
+    body = re.search(r"int take_ticket\(.*?\n}\n", text, re.S).group(0)
+    assert re.search(r"wave_barrier\(\);\s*if \(lane == 0\) ticket = atomicAdd\(counter, 1\);\s*__builtin_amdgcn_wave_barrier\(\);", body)
+    assert not re.search(r"atomicAdd\(\s*&?[\w.>-]*\b(head|next|sched_head|singles_head)\s*,", text)
+    assert len(re.findall(r"= take_ticket\(", text)) == 4
+
+
 def test_staging_is_not_handed_out_over_what_kernels_still_read(tmp_path):
     """The pinned block's staging (csrc/omk_staging.h) against a stream that runs as late as it can
     (tests/cpp/staging_check.cpp): after a wrap, an offset that was in use before says nothing about what
