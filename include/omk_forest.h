@@ -297,10 +297,12 @@ int omk_batch_truncated(omk_batch *b, int32_t *h_count);
  * steps, [7] nodes settled by merging the lists of their children's entries, [8] when the first block of the persistent launch started,
  * [9] when its last team of wavefronts left, [10] when its last walker left (low 31 bits of the
  * device's 100 MHz clock; these three are kept whether or not the counters are on), [11] the number
- * of walks of lone visitors inside that launch, [12] of the nodes of [7], those of
- * layouts with RAVE and more than 64 child slots a node, [13] of them, those of at most 64 visitors (of such layouts, and
- * of batches with at most 64 visitors a root), [14] unused (0), [15] nodes
- * cut into slices for several wavefronts.  (Nodes taken by the walk down one-winner nodes count in [0]..[2].) */
+ * of walks of lone visitors inside that launch, [12] of the nodes of [7], those settled by the helpers of a team,
+ * [13] those settled by one wavefront of a root's block, [14] unused (0), [15] nodes
+ * cut into slices for several wavefronts.  (Nodes taken by the walk down one-winner nodes count in [0]..[2].)
+ * A batch of at most 64 visitors a root, on nodes of at most 384 child slots, has a block for each crowded root in the
+ * place of the persistent launch: [8] and [9] are of those blocks, their rows for the host included, [10] and [11] stay
+ * 0, and what they replay is in [3] alone.  A batch of lone visitors has neither: [8] to [11] are 0. */
 int omk_batch_stats(omk_batch *b, int32_t *h_stats16);
 /* The counters above cost one atomic per processed node (and per single-visitor step), all on
  * the same few addresses, so they are off unless switched on here (enabled != 0); with

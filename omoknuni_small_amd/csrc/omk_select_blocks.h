@@ -423,7 +423,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                         visits = lane < n0 ? my.vl[lane] : 0;
                     }
                 }
-                if (a.stats && lane == 0 && m > 1) {
+                if (a.stats && lane == 0 && m > 1 && !leaf) {
                     atomicAdd(a.stats + 0, 1);
                     atomicAdd(a.stats + 1, serial && run_child < 0 ? 0 : 1);
                     atomicAdd(a.stats + 2, serial && run_child < 0 ? 0 : m);

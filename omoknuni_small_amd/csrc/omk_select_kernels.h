@@ -3284,8 +3284,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
             for (int r = 0; r < R; r++) cnt[r] = lds.st_j0[r * kWave + lane];
             if (a.stats && lane == 0) {
                 atomicAdd(a.stats + 7, 1);
-                if (R > 1 && RAVE) atomicAdd(a.stats + 12, 1);
-                if (R > 1 && m <= kWave) atomicAdd(a.stats + 13, 1);
+                atomicAdd(a.stats + 12, 1);
             }
         }
     }

@@ -255,7 +255,8 @@ def test_compaction_of_large_trees(fan):
     assert (table.probe_leaves(b) == b.read()[2]).all()
 
 
-# a young tree: the visitors spread over children without visits (up to 64 of them, one entry per lane)
+# a young tree: the visitors spread over children without visits, whose first entries are nearly all of the merge that the
+# root's block makes, or beyond 64 visitors or 384 children the helpers of a team
 @pytest.mark.parametrize("children", [65, 130, 225, 362, 700])
 @pytest.mark.parametrize("n", [8, 23, 63, 64, 65])
 @pytest.mark.parametrize("rave", [False, True])
@@ -270,7 +271,7 @@ def test_visitors_spread_over_a_fresh_node(children, n, rave):
     b = omk.Batch(f, n, 6)
     b.enable_stats()
     rng = np.random.default_rng(children + n)
-    spread = 0
+    spread, teams = 0, n > 64 or children > 384
     for step in range(4):
         k = 1 if step == 0 else n
         roots = np.zeros(k, np.int32)
@@ -280,7 +281,9 @@ def test_visitors_spread_over_a_fresh_node(children, n, rave):
         b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3, use_rave=rave, rave_k=1000.0))
         paths, plen, leaf, _ = b.read()
         assert (paths == rpaths).all() and (plen == rlen).all() and (leaf == rleaf).all(), step
-        spread += b.stats()["spread_nodes"]
+        st = b.stats()
+        spread += st["merged_by_teams" if teams else "merged_by_blocks"]
+        assert st["merged_by_blocks" if teams else "merged_by_teams"] == 0, st
         begin = (np.arange(k + 1) * children).astype(np.int32)
         moves = np.tile(np.arange(children, dtype=np.int32), k)
         policy = rng.random((k, children)).astype(np.float32)
@@ -292,7 +295,7 @@ def test_visitors_spread_over_a_fresh_node(children, n, rave):
         b.set_values(values)
         b.backup(3)
     assert (f.download()["N"] == ref.N).all()
-    if not rave and n in (23, 63, 64):
+    if not rave and n >= 23:
         assert spread > 0
 
 

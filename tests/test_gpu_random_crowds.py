@@ -112,20 +112,20 @@ def test_the_widest_fan_out_class_with_crowds():
         select_both(soa, roots[tr], len(lay) + 1, rave=rave, steps=2, vl=int(rng.integers(1, 5)))
 
 
-def test_wide_nodes_with_rave_settled_through_the_children_that_can_be_chosen():
-    """With RAVE, a node of more than 64 child slots whose 24 to 1023 visitors split is settled through the few
-    children that can be chosen at all, moved to one lane each (the counter says how often).  Forests with the
-    statistics of the Go workload (a few children dominate a node) at several sizes of crowd, and random shapes
-    of 65 to 380 slots with masks, plateaus and pre-existing virtual loss."""
+def test_wide_nodes_with_rave_whose_visitors_split():
+    """With RAVE, a node of more than 64 child slots whose 8 to 1535 visitors split is settled by the helpers of a team
+    (the counter says how often): the blends hardly move with virtual loss, so that the entries pile up close above the
+    threshold.  Forests with the statistics of the Go workload (a few children dominate a node) at several sizes of crowd,
+    and random shapes of 65 to 380 slots with masks, plateaus and pre-existing virtual loss."""
     from omoknuni_small_amd import synth
-    narrowed = 0
+    merged = 0
     for seed, B in enumerate((2000, 5000, 9000, 16000)):
         soa, roots, meta = synth.generate("c4", seed=40 + seed, nodes_per_tree=600_000)
         st = select_both(soa, synth.traversal_roots(roots, B), int(meta["max_depth"]), rave=True, steps=3,
                          vl=int(meta["virtual_loss"]) if seed % 2 else 1, rave_k=float(meta.get("rave_k", 3000.0)))
-        narrowed += st["narrowed_nodes"]
-    print("nodes settled that way:", narrowed)
-    assert narrowed >= 5, narrowed  # (the full-size Go workload has 20 to 30 such nodes a selection)
+        merged += st["merged_by_teams"]  # (every expanded node of these forests has 362 slots)
+    print("nodes settled that way:", merged)
+    assert merged >= 5, merged  # (the full-size Go workload has 20 to 30 such nodes a selection)
     for seed in range(12):
         rng = np.random.default_rng(1000 + seed)
         if seed % 3 == 2:

@@ -83,6 +83,31 @@ def test_widening_at_the_selection():
     both(soa, np.repeat(roots, [1, 2, 5, 9, 16, 33, 48, 63, 64]).astype(np.int32), 8, pw=True)
 
 
+@pytest.mark.parametrize("sizes", [[64], [2, 64, 17, 1, 1, 1, 40], [1] * 50, [65], [700, 3, 1, 1], [5000, 80, 1]])
+@pytest.mark.parametrize("fan,rave", [(48, False), (300, True)])
+def test_work_counters(sizes, fan, rave):
+    """The counters against the paths: a node with several visitors that go on from it is one processed node, a lone
+    visitor's step is one, and every merge has been made by a team or by a block."""
+    import omoknuni_small_amd as omk
+    soa, roots = layered_forest(fan, [fan, 30, 6], n_trees=len(sizes), rave=rave)
+    troots = np.repeat(roots, sizes).astype(np.int32)
+    b = omk.Batch(omk.Forest.from_soa(soa), len(troots), 6)
+    b.set_roots(troots)
+    b.enable_stats()
+    for _ in range(3):  # (the rows of the last two come from the blocks)
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3, use_rave=rave, rave_k=1000.0))
+        paths, plen, _, _ = b.read()
+        st = b.stats()
+        went_on = paths[:, :-1][np.arange(paths.shape[1] - 1)[None, :] < plen[:, None] - 1]
+        visitors = np.bincount(went_on)
+        assert st["group_nodes"] == (visitors > 1).sum()
+        assert st["settled_by_water_level"] + st["settled_one_by_one"] == visitors[visitors > 1].sum()
+        assert st["single_visitor_steps"] == (visitors == 1).sum()
+        assert st["merged_by_teams"] + st["merged_by_blocks"] == st["merged_nodes"]
+        assert (st["merged_by_blocks"] > 0) == (1 < max(sizes) <= 64) and (st["merged_by_teams"] > 0) == (max(sizes) > 64)
+        b.backup(3)
+
+
 @pytest.mark.parametrize("kind", ["nan sum", "no score at all", "all equal"])
 @pytest.mark.parametrize("widest,rave", [(60, False), (250, True), (380, False), (380, True)])
 def test_lone_visitors_of_masked_trees(widest, rave, kind):
