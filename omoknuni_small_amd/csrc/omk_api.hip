@@ -139,6 +139,7 @@ struct omk_batch {
     // like when they are settled says nothing: paths that follow transpositions meet in nodes that several trees
     // hold, and an upload makes the forest a tree again under them.)
     bool disjoint = false;
+    bool stamped = false;  // the last selection has left its time stamps
     int32_t *paths = nullptr, *path_len = nullptr, *leaf = nullptr;
     float *values = nullptr;
     Item *items0 = nullptr, *items_q = nullptr, *singles0 = nullptr, *singles_q = nullptr;
@@ -1518,6 +1519,7 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
                           f->stream));
     b->selected = true;
     b->disjoint = b->n_items0 == 0;  // a root each, and distinct roots head disjoint trees
+    b->stamped = b->n_items0 > 0 && (!by_blocks(b->n_items0, b->most_visitors, f->max_fanout) || a.stats || a.trace);
     b->select_calls++;
     b->lone_call = out.sig.flag ? b->select_calls : -1;
     return OMK_OK;
@@ -1890,8 +1892,7 @@ int omk_batch_stats(omk_batch *b, int32_t *h_stats16) {
     int32_t times[3] = {0, 0, 0};
     HIP_TRY(hipMemcpyAsync(times, b->counters + 26, sizeof(times), hipMemcpyDeviceToHost, b->f->stream));
     HIP_TRY(hipStreamSynchronize(b->f->stream));
-    // the three time stamps are kept whether or not the counters are on
-    for (int i = 0; i < 3; i++) h_stats8[8 + i] = times[i];
+    for (int i = 0; i < 3; i++) h_stats8[8 + i] = b->stamped ? times[i] : 0;
     return OMK_OK;
 }
 
@@ -2177,6 +2178,7 @@ int omk_tt_select_redirect(omk_tt *tt, omk_batch *b, const omk_select_params *p,
     HIP_TRY(launch_select_redirect(f->dev(), a, p->use_rave != 0, s));
     b->selected = true;
     b->disjoint = false;
+    b->stamped = false;
     b->select_calls++;
     int32_t status[8];
     if (int rc = tt_counts(tt, status)) return rc;

@@ -175,7 +175,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
         *a.n_singles = n_singles;
         *a.truncated_next = 0;
         a.sched_wait[1] = 0;
-        a.times[0] = (int)(wall_clock64() & 0x7FFFFFFF);
+        if (a.stats || a.trace) a.times[0] = (int)(wall_clock64() & 0x7FFFFFFF);
     }
     // ---- the block's visitors ----
     int n_here = 0;
@@ -568,8 +568,13 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
             }
         }
     }
-    if (threadIdx.x == 0) a.times[1] = a.times[2] = (int)(wall_clock64() & 0x7FFFFFFF);
-    if (!ROWS) return;
+    auto left = [&]() {  // (stamps of every launch, with the call in their upper half, cost it up to 3 %)
+        if ((a.stats || a.trace) && threadIdx.x == 0) atomicMax(a.times + 1, (int)(wall_clock64() & 0x7FFFFFFF));
+    };
+    if (!ROWS) {
+        left();
+        return;
+    }
     // ---- the rows, straight into pinned host memory (see k_export) ----
     __syncthreads();
     n_here = (int)blockIdx.x < n_items ? a.items0[blockIdx.x].m
@@ -590,6 +595,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
         if (lane >= 1 && lane <= a.max_depth) host_store(o.actions + (size_t)t * a.max_depth + lane - 1, act);
     }
     host_signal(out.sig.count, out.sig.flag, out.sig.seq, gridDim.x);
+    left();
 }
 
 }  // namespace omk

@@ -108,6 +108,40 @@ def test_work_counters(sizes, fan, rave):
         b.backup(3)
 
 
+def test_time_stamps():
+    """When the first block started and the last one left: around all work of the timeline, of this selection and not of an
+    earlier one, whether the rows come from the blocks or not; with the counters and the timeline off only the persistent
+    launch keeps them."""
+    import omoknuni_small_amd as omk
+    soa, roots = random_tree(77, n_expand=900, fanout=(2, 150), max_depth=9, n_roots=300, n_max=200)
+    f = omk.Forest.from_soa(soa)
+    few = np.repeat(roots, np.r_[64, np.full(149, 6), np.ones(150, np.int64)]).astype(np.int32)
+    many = np.repeat(roots[:3], 70).astype(np.int32)
+    b = omk.Batch(f, len(few), 12)
+    before = None
+    for troots, trace, read in [(few, True, False), (few, True, True), (few, True, True), (many, False, True), (few, False, True),
+                                (roots.astype(np.int32), True, True), (many, True, True), (few, True, True)]:
+        b.set_roots(troots)
+        b.enable_trace(trace)
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=3))
+        if read:
+            b.read()
+        st = b.stats()
+        b.revert_vl(3)
+        first, last = st["t_first_block"], max(st["t_last_team"], st["t_last_walker"])
+        if len(troots) == 300 or troots is few and not trace:
+            assert first == last == 0
+            continue
+        assert (st["t_last_walker"] != 0) == (troots is many)
+        assert before is None or (first - before) % (1 << 31) < 1 << 30
+        assert 0 < (last - first) % (1 << 31) < 10_000_000  # (a tenth of a second)
+        if trace:  # (the block numbered first need not be the first to start: 10 us)
+            tr = b.debug_trace()
+            assert len(tr) > 0 and ((tr[:, 0] - first + 1000) % (1 << 31) < 1 << 30).all()
+            assert ((last - tr[:, 1]) % (1 << 31) < 1 << 30).all()
+        before = last
+
+
 @pytest.mark.parametrize("kind", ["nan sum", "no score at all", "all equal"])
 @pytest.mark.parametrize("widest,rave", [(60, False), (250, True), (380, False), (380, True)])
 def test_lone_visitors_of_masked_trees(widest, rave, kind):
