@@ -109,12 +109,6 @@ __device__ __forceinline__ int wave_inclusive_sum(int x, int lane) {
     return (int)(v + add);
 }
 
-__device__ __forceinline__ float wave_sum_f32(float v) {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, kWave);
-    return v;
-}
-
 // smallest k >= 1 with k*k >= n
 __device__ __forceinline__ int ceil_sqrt_i32(int n) {
     if (n <= 1) return 1;

@@ -2104,55 +2104,6 @@ __device__ __forceinline__ bool single_run(const SelectArgs &a, const NodeCtx &c
     return true;
 }
 
-// How many of a child's entries 0 .. cap-1 come before the entry (tk, tp), given that the child's
-// keys do not increase (the caller checks the entries it then uses): the closed-form estimate,
-// the two entries around it tested with the exact arithmetic, and a gallop away from it plus a
-// bisection when it is further off.  first_known: entry 0 is known to come before (tk, tp).  On
-// return c: entry c-1 was seen to come before (tk, tp) (or c == 0, or c == 1 with first_known),
-// entry c was seen not to (or c == cap).
-template <int R, bool RAVE>
-__device__ __forceinline__ int count_before(int n, float w, float p, int vl, float q2, float ep, uint32_t uvl,
-                                            int child, uint32_t tk, uint32_t tp, int cap, bool first_known) {
-    uint32_t kk, pp;
-    if (!first_known) {
-        entry_key<R, RAVE>(n, w, p, vl, q2, ep, uvl, 0, child, kk, pp);
-        if (!(kk != 0u && comes_before(kk, pp, tk, tp))) return 0;
-    }
-    int lo_c = 1, hi_c = cap;
-    if (hi_c < lo_c) return lo_c;
-    int g = predict_count<RAVE>(n, w, p, vl, q2, ep, uvl, key_score(tk), cap);
-    g = g < lo_c ? lo_c : (g > hi_c ? hi_c : g);
-    if (g > lo_c) {
-        entry_key<R, RAVE>(n, w, p, vl, q2, ep, uvl, g - 1, child, kk, pp);
-        if (kk != 0u && comes_before(kk, pp, tk, tp)) lo_c = g;
-        else hi_c = g - 1;
-    }
-    if (lo_c == g && g < hi_c) {
-        entry_key<R, RAVE>(n, w, p, vl, q2, ep, uvl, g, child, kk, pp);
-        if (kk != 0u && comes_before(kk, pp, tk, tp)) lo_c = g + 1;
-        else hi_c = g;
-    }
-    if (lo_c < hi_c) {
-        const bool up = lo_c > g;
-        for (int step = 2; lo_c < hi_c; step <<= 1) {
-            int t = up ? lo_c + step : hi_c - step + 1;
-            t = t > hi_c ? hi_c : (t <= lo_c ? lo_c + 1 : t);
-            entry_key<R, RAVE>(n, w, p, vl, q2, ep, uvl, t - 1, child, kk, pp);
-            const bool before = kk != 0u && comes_before(kk, pp, tk, tp);
-            if (before) lo_c = t;
-            else hi_c = t - 1;
-            if (before != up) break;
-        }
-    }
-    while (lo_c < hi_c) {
-        const int t = (lo_c + hi_c + 1) >> 1;
-        entry_key<R, RAVE>(n, w, p, vl, q2, ep, uvl, t - 1, child, kk, pp);
-        if (kk != 0u && comes_before(kk, pp, tk, tp)) lo_c = t;
-        else hi_c = t - 1;
-    }
-    return lo_c;
-}
-
 // ---- A contested node settled by the three helpers ----
 // The score a child shows the j-th of a node's visitors that choose it depends on nothing but j, and where no child's
 // scores increase with j the serial order is the merge of the children's lists by (key, position).  The helpers work out
@@ -2545,7 +2496,6 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
     }
     __syncthreads();
 }
-
 
 // A lower end of the key range with at least `least` and at most 64 of the keys that `count` counts at or above it,
 // found by halving; `top`: no key lies above it; 0: there is none (keys tied).

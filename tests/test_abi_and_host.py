@@ -187,11 +187,10 @@ def test_proof_of_non_increasing_keys_against_brute_force(tmp_path):
     assert int(m.group(1)) > 100000 and int(m.group(2)) > 100000
 
 
-def test_direct_merge_rule_against_the_serial_loop(tmp_path):
-    """The rule by which the selection kernel settles a node where one child takes nearly every
-    visitor (merge the few entries of the others into that child's list by rank: no threshold search,
-    no sort), restated step by step on the host with the kernel's own score arithmetic
-    (tests/cpp/merge_check.cpp): every node it accepts must come out as the serial loop plays it."""
+def test_merge_rules_against_the_serial_loop(tmp_path):
+    """The rules by which the selection kernels settle a node whose visitors split (a root's block up to 64 of them, the
+    helpers of a team any number), restated step by step on the host with the kernels' own score arithmetic
+    (tests/cpp/merge_check.cpp): every node they accept must come out as the serial loop plays it."""
     import re
     import subprocess
     exe = str(tmp_path / "merge_check")
@@ -200,8 +199,8 @@ def test_direct_merge_rule_against_the_serial_loop(tmp_path):
                            os.path.join(ROOT, "tests", "cpp", "merge_check.cpp"), "-o", exe])
     out = subprocess.run([exe, "60000", "7"], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0, out.stdout[-2000:]
-    m = re.search(r"merged: (\d+); wrong 0;", out.stdout)
-    assert m and int(m.group(1)) > 30000, out.stdout[-500:]
+    m = re.search(r"blocks: merged (\d+), declined \d+; teams: merged (\d+), declined \d+; wrong 0", out.stdout)
+    assert m and int(m.group(1)) > 30000 and int(m.group(2)) > 30000, out.stdout[-500:]
 
 
 def test_tickets_are_drawn_between_barriers_of_the_wavefront():
