@@ -29,11 +29,17 @@ def both(soa, troots, D, vl=3, rave=False, pw=False, steps=4):
         assert (acts == ref.gather_actions(rpaths, rlen)).all(), step
         assert b.truncated() == int(((ref.child_count[rleaf] > 0) & (rlen == D + 1)).sum()), step
         values = (rng.integers(-64, 65, len(troots)) / 64.0).astype(np.float32)
+        was, visits = ref.W.astype(np.float64), ref.N.copy()
         ref.backup_batch(rpaths, rlen, values, vl)
         b.set_values(values)
         b.backup(vl)
         got = f.download()
         assert (got["N"] == ref.N).all() and (got["VL"] == ref.VL).all(), step
+        # k values of at most 1 added to W in two orders: every partial sum is at most |W| + k and rounds by 2^-24 of it
+        k, finite = ref.N - visits, np.isfinite(was)
+        bound = 2.0 ** -23 * k[finite] * (np.abs(was[finite]) + k[finite])
+        assert (np.abs(got["W"][finite].astype(np.float64) - ref.W[finite]) <= bound).all(), step
+        assert np.array_equal(got["W"][~finite], ref.W[~finite], equal_nan=True), step
         ref.W[:] = got["W"]
 
 
@@ -56,6 +62,19 @@ def test_roots_of_all_sizes_in_one_batch(widest, mask, D, rave):
     rng = np.random.default_rng(D)
     sizes = np.concatenate([np.ones(19, np.int64), rng.integers(2, 65, 21)])
     both(soa, rng.permutation(np.repeat(roots, sizes)).astype(np.int32), D, rave=rave)
+
+
+@pytest.mark.parametrize("crowds", [[64, 2, 33], [2], [65]])
+@pytest.mark.parametrize("widest,mask,rave,n_expand", [(12, 0.0, False, 5000), (150, 0.4, True, 1500)])
+@pytest.mark.parametrize("alternating", [False, True])
+def test_few_crowded_roots_among_thousands_of_lone_ones(crowds, widest, mask, rave, n_expand, alternating):
+    """Up to 64 visitors a root the lone ones are walked by blocks of 16 beside the crowds' own; from 65 on by the walkers
+    of the persistent launch."""
+    lone = 2503
+    soa, roots = random_tree(n_expand, n_expand=n_expand, fanout=(2, widest), max_depth=6, n_roots=len(crowds) + lone,
+                             mask_frac=mask, rave=rave, tie_frac=0.1, n_max=200)
+    troots = np.repeat(roots, crowds + [1] * lone).astype(np.int32)
+    both(soa, np.random.default_rng(lone).permutation(troots) if alternating else troots, 9, rave=rave, steps=2)
 
 
 @pytest.mark.parametrize("kind", ["nan prior", "nan sum", "-inf sum", "inf sum of the unvisited", "no virtual loss", "all equal"])
@@ -89,7 +108,7 @@ def test_work_counters(sizes, fan, rave):
     """The counters against the paths: a node with several visitors that go on from it is one processed node, a lone
     visitor's step is one, and every merge has been made by a team or by a block."""
     import omoknuni_small_amd as omk
-    soa, roots = layered_forest(fan, [fan, 30, 6], n_trees=len(sizes), rave=rave)
+    soa, roots = layered_forest(fan, [fan, 8, 4], n_trees=len(sizes), rave=rave)
     troots = np.repeat(roots, sizes).astype(np.int32)
     b = omk.Batch(omk.Forest.from_soa(soa), len(troots), 6)
     b.set_roots(troots)
