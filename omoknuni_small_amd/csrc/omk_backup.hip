@@ -782,7 +782,7 @@ __global__ __launch_bounds__(256) void k_tt_hits(ForestDev f, const TTSlot *slot
     const uint64_t any = __ballot(out >= 0);
     if (any && (threadIdx.x & 63) == 0) atomicAdd(d_status + 6, __popcll(any));
     // host_signal with the counters before the flag: eight lanes take them, one round trip instead of eight
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    wait_stores();
     __syncthreads();
     if (threadIdx.x >= 64) return;
     int before = 0;
@@ -792,7 +792,7 @@ __global__ __launch_bounds__(256) void k_tt_hits(ForestDev f, const TTSlot *slot
     if (threadIdx.x < 8)
         host_store(h_status + threadIdx.x,
                    __hip_atomic_exchange(d_status + threadIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    wait_stores();
     if (threadIdx.x == 0) host_store(sig.flag, sig.seq);
 }
 

@@ -126,6 +126,11 @@ __device__ __forceinline__ void host_store(T *p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Until this wavefront's own stores have been acknowledged.  For a wavefront that hands what it stored to another one, whose
+// release of agent scope announces it to other blocks: that one waits for its own stores only, and a release of workgroup
+// scope or a block barrier waits for none in memory.
+__device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // The end of a kernel whose results the host waits for (all threads of all blocks take part): every wavefront
 // waits until its own host_stores have been acknowledged, and the last of the grid's `blocks` blocks stores the
 // call's number to the host's flag.  The host polls that word.  Measured on an MI355X from the launch to the
@@ -133,7 +138,7 @@ __device__ __forceinline__ void host_store(T *p, T v) {
 // second kernel that raises the flag costs 1.6 us more, a release of system scope per block 27 % more at 1 MB.
 // One kernel and hipStreamSynchronize take 11 us, a copy back into pageable memory 14 more.
 __device__ __forceinline__ void host_signal(int32_t *count, int32_t *flag, int32_t seq, int blocks) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    wait_stores();
     __syncthreads();
     if (threadIdx.x != 0) return;
     if (blocks > 1) {

@@ -2494,6 +2494,7 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
         lds.cmd.merged = ok ? 1 : 0;
         lds.cmd.n_barriers = barriers;
     }
+    if (goff >= 0) wait_stores();  // (the owner's join announces a slice's winners to other blocks)
     __syncthreads();
 }
 
@@ -4059,6 +4060,7 @@ __device__ __forceinline__ void partition_chunks(const SelectArgs &a, const Team
         const int chunk = take_ticket(&pl.next, lane);
         if (chunk >= n_chunks) return;
         partition_chunk(a, cm, pl, chunk, lone0, lane);
+        wait_stores();  // (the helper that counts the chunks announces the lists and the lone visitors to other blocks)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         if (lane == 0) atomicAdd(&pl.finished, 1);
     }
@@ -4257,6 +4259,7 @@ __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs
             __syncthreads();  // the walk has stopped
             if (RMAX > 1) chain_finish(ka, tid - kWave, kChainWalkers * kWave, levels, c_depth - 1, c_off, c_m);
             else if (wi == 0) chain_finish(ka, tid & 63, kWave, levels, c_depth - 1, c_off, c_m);
+            if (HEAVY) wait_stores();
             __syncthreads();  // the request is done
             continue;
         }
@@ -4281,6 +4284,8 @@ __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs
                                      ep, uvl);
         else
             team_help<RMAX, RAVE, RMAX>(f, a, s_lds, s_part, tid, op, total, keep, goff, cur, ep, uvl);
+        // a heavy node's list and the winners of its slices are read by other blocks once the owner has announced them
+        if (HEAVY) wait_stores();
         __syncthreads();  // the request is done
     }
 }

@@ -219,6 +219,22 @@ def test_tickets_are_drawn_between_barriers_of_the_wavefront():
     assert len(re.findall(r"= take_ticket\(", text)) == 4
 
 
+def test_stores_for_other_blocks_are_waited_for_by_who_made_them():
+    """A helper's stores that its owner, or another helper, announces to other blocks with a release of agent scope: that
+    release waits for the announcing wavefront's own stores, a release of workgroup scope and a block barrier for none in
+    memory.  The helper waits before it says that it is done."""
+    import re
+    with open(os.path.join(ROOT, "omoknuni_small_amd", "csrc", "omk_select_kernels.h")) as f:
+        text = re.sub(r"//[^\n]*", "", f.read())
+    body = lambda name: re.search(r"void %s\(.*?\n}\n" % name, text, re.S).group(0)
+    before = r"wait_stores\(\);\s*"
+    assert re.search(before + r'__builtin_amdgcn_fence\(__ATOMIC_RELEASE, "workgroup"\);\s*if \(lane == 0\) atomicAdd\(&pl.finished',
+                     body("partition_chunks"))
+    assert re.search(r"if \(goff >= 0\) " + before + r"__syncthreads\(\);\s*}\s*$", body("team_merge"))
+    helpers = body("k_select_groups").split("for (;;)", 1)[1]
+    assert len(re.findall(r"if \(HEAVY\) " + before + r"__syncthreads\(\);", helpers)) == 2
+
+
 def test_staging_is_not_handed_out_over_what_kernels_still_read(tmp_path):
     """The pinned block's staging (csrc/omk_staging.h) against a stream that runs as late as it can
     (tests/cpp/staging_check.cpp): after a wrap, an offset that was in use before says nothing about what
