@@ -302,8 +302,8 @@ int omk_batch_truncated(omk_batch *b, int32_t *h_count);
  * cut into slices for several wavefronts.  (Nodes taken by the walk down one-winner nodes count in [0]..[2].)
  * A batch of at most 64 visitors a root, on nodes of at most 384 child slots, has a block for each crowded root in the
  * place of the persistent launch: [8] and [9] are of those blocks, their rows for the host included, and kept only with
- * the counters or the timeline on (0 else); [10] and [11] are 0, and what they replay is in [3] alone.  A batch of lone
- * visitors has neither launch: [8] to [11] are 0. */
+ * the counters or the timeline on (0 else); [10] and [11] are 0, and [4] counts
+ * the contested nodes with real scores that no merge settled.  A batch of lone visitors has neither launch: [8] to [11] are 0. */
 int omk_batch_stats(omk_batch *b, int32_t *h_stats16);
 /* The counters above cost one atomic per processed node (and per single-visitor step), all on
  * the same few addresses, so they are off unless switched on here (enabled != 0); with

@@ -428,6 +428,8 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                     atomicAdd(a.stats + 1, serial && run_child < 0 ? 0 : 1);
                     atomicAdd(a.stats + 2, serial && run_child < 0 ? 0 : m);
                     atomicAdd(a.stats + 3, serial && run_child < 0 ? m : 0);
+                    // (without a real score, or with values that are not finite, no merge was tried)
+                    if (serial && run_child < 0 && hk != 0u && !odd) atomicAdd(a.stats + 4, 1);
                     if (!serial) {
                         atomicAdd(a.stats + 7, 1);
                         atomicAdd(a.stats + 13, 1);

@@ -11,8 +11,9 @@ from test_gpu_scheduler import layered_forest
 pytestmark = pytest.mark.gpu
 
 
-def both(soa, troots, D, vl=3, rave=False, pw=False, steps=4):
-    """Selections and backups on the device and by the checker; from the second on the rows come from the blocks."""
+def both(soa, troots, D, vl=3, rave=False, pw=False, steps=4, count=False):
+    """Selections and backups on the device and by the checker; from the second on the rows come from the blocks.  With
+    `count` the work counters are on, and their sums are returned."""
     import omoknuni_small_amd as omk
     ref = R.RefTree.from_soa(soa)
     rp = R.make_params(c_puct=1.4, virtual_loss=vl, use_rave=rave, rave_k=1000.0, pw=pw, max_depth=D)
@@ -21,12 +22,16 @@ def both(soa, troots, D, vl=3, rave=False, pw=False, steps=4):
     b.set_roots(troots)
     sp = omk.SelectParams(c_puct=1.4, virtual_loss=vl, use_rave=rave, rave_k=1000.0, pw=pw)
     rng = np.random.default_rng(len(troots))
+    b.enable_stats(count)
+    total = {}
     for step in range(steps):
         rpaths, rlen, rleaf, _ = ref.select_batch(troots, rp, near_ties=False)
         b.select(sp)
         paths, plen, leaf, acts = b.read()
         assert (paths == rpaths).all() and (plen == rlen).all() and (leaf == rleaf).all(), step
         assert (acts == ref.gather_actions(rpaths, rlen)).all(), step
+        if count:
+            total = {k: v + total.get(k, 0) for k, v in b.stats().items()}
         assert b.truncated() == int(((ref.child_count[rleaf] > 0) & (rlen == D + 1)).sum()), step
         values = (rng.integers(-64, 65, len(troots)) / 64.0).astype(np.float32)
         was, visits = ref.W.astype(np.float64), ref.N.copy()
@@ -41,6 +46,7 @@ def both(soa, troots, D, vl=3, rave=False, pw=False, steps=4):
         assert (np.abs(got["W"][finite].astype(np.float64) - ref.W[finite]) <= bound).all(), step
         assert np.array_equal(got["W"][~finite], ref.W[~finite], equal_nan=True), step
         ref.W[:] = got["W"]
+    return total
 
 
 @pytest.mark.parametrize("visitors", [2, 3, 17, 63, 64, 65])
@@ -49,6 +55,28 @@ def both(soa, troots, D, vl=3, rave=False, pw=False, steps=4):
 def test_crowds_and_fan_outs(visitors, fan, rave):
     soa, roots = layered_forest(3 + fan + visitors, [fan, 40, 5], n_trees=3, rave=rave)
     both(soa, np.repeat(roots, visitors).astype(np.int32), 6, rave=rave)
+
+
+@pytest.mark.parametrize("visitors", [8, 33, 64])
+@pytest.mark.parametrize("fan,rave", [(3, False), (64, True), (256, False), (384, True)])
+@pytest.mark.parametrize("rising", [False, True])
+def test_contested_nodes_are_merged_unless_scores_rise(visitors, fan, rave, rising):
+    """What spreads is merged and nothing is replayed; children whose scores rise with virtual loss (a value sum below minus
+    the visit count) are not in order, and their node is replayed: with the same paths."""
+    soa, roots = layered_forest(fan + visitors, [fan, 20, 4], n_trees=3, rave=rave)
+    if rising:
+        soa["N"] = np.maximum(soa["N"], 1)
+        soa["W"] = (-np.random.default_rng(fan).uniform(1.5, 2.5, len(soa["N"])) * soa["N"]).astype(np.float32)
+        soa["P"][:] = 0.0
+        if rave:  # (and the blend is no better)
+            soa["rN"] = np.maximum(soa["rN"], 1)
+            soa["rW"] = (-5.0 * soa["rN"]).astype(np.float32)
+    st = both(soa, np.repeat(roots, visitors).astype(np.int32), 6, rave=rave, count=True)
+    if rising:
+        assert st["replayed_nodes"] >= 1, st
+    else:
+        assert st["merged_by_blocks"] >= 1 and st["replayed_nodes"] == 0, st
+    assert st["settled_one_by_one"] >= 2 * st["replayed_nodes"], st
 
 
 @pytest.mark.parametrize("rave", [False, True])
