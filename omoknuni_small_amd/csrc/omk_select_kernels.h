@@ -495,9 +495,11 @@ __device__ __forceinline__ float key_score(uint32_t key) {
 // of the score as a function of x = N + VL:  s1(x) = (W+N)/x - 1 + c/(1+x)  (c = P * ep) and,
 // with RAVE, s2(x) = q2 + c/(1+x).  Fast approximate arithmetic on purpose: the result only
 // seeds the exact search, which tests the two entries around it.
+// half_ulp: half the distance from tau to the next lower score.  A sum rounded to the nearest reaches tau from there on:
+// where a blend hardly moves, that is most of its entries.
 template <bool RAVE>
 __device__ __forceinline__ int predict_count(int n, float w, float p, int vl, float q2, float ep, uint32_t uvl,
-                                             float tau, int cap) {
+                                             float tau, int cap, float half_ulp = 0.0f) {
     const float x0 = (float)n + (float)vl;
     const float A = w + (float)n;
     const float cc = p * ep;
@@ -512,7 +514,7 @@ __device__ __forceinline__ int predict_count(int n, float w, float p, int vl, fl
         xs = 3.0e38f;
     }
     if (RAVE) {
-        const float d = tau - q2;
+        const float d = (tau - q2) - half_ulp;
         float x2 = d > 1e-12f ? cc * __builtin_amdgcn_rcpf(d) - 1.0f : 3.0e38f;
         xs = fmaxf(xs, x2);
     }
@@ -2187,13 +2189,13 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
         }
     }
     bool ok = true;
-    int done = 0;
+    int done = 0, more = 0;  // more: entries a child gets on top of the estimate
     for (int pass = 0; done < m; pass++) {
         const int need = m - done;
         const bool counted = pass == 0 && floor_key != 0u;
         // ---- the children's next entries, and the key no useful threshold lies below: a child alone has `need` entries
         // at or above the last one it could be asked for ----
-        uint32_t hk[K], hp[K];
+        uint32_t hk[K], hp[K], tail[K];  // tail: the last entry it could be asked for
         uint32_t lmax = 0u, hmax = 0u;
         int tk[K];
 #pragma unroll
@@ -2201,13 +2203,14 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
             const int i = t + q * NT;
             hk[q] = 0u;
             hp[q] = 0u;
+            tail[q] = 0u;
             tk[q] = i < F ? lds.st_j0[i] : 0;
             if (q * NT < F && part[q]) {
-                uint32_t zk, zp;
+                uint32_t zp;
                 entry_key<R, RAVE>(cn[q], cw[q], cp[q], cvl[q], cq2[q], ep, uvl, tk[q], i, hk[q], hp[q]);
                 if (!counted) {
-                    entry_key<R, RAVE>(cn[q], cw[q], cp[q], cvl[q], cq2[q], ep, uvl, tk[q] + need - 1, i, zk, zp);
-                    if (hk[q] != 0u) lmax = umax32(lmax, zk);
+                    entry_key<R, RAVE>(cn[q], cw[q], cp[q], cvl[q], cq2[q], ep, uvl, tk[q] + need - 1, i, tail[q], zp);
+                    if (hk[q] != 0u) lmax = umax32(lmax, tail[q]);
                 }
                 hmax = umax32(hmax, hk[q]);
             }
@@ -2227,11 +2230,15 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
             break;
         }
         // ---- a threshold with some more than `need` entries at or above it, by the closed form ----
-        // (whether the next entry does is known; the closed form does not hold for a child without visits)
+        // (whether the next entry and the last one do is known; the closed form does not hold for a child without visits.
+        // A RAVE blend may stop moving after a few of a node's visitors, and its other entries all lie on one key.  Two
+        // such children of a Go node, 256 visitors: 12 passes, all but the first of two entries, then declined, 90 us; now 13.5)
         auto entries_from = [&](int q, uint32_t key) {
             if (hk[q] < key) return 0;
+            if (tail[q] >= key) return need;
+            const float tau = key_score(key);
             const int n = predict_count<RAVE>(cn[q], cw[q], cp[q], (int)((uint32_t)cvl[q] + (uint32_t)tk[q] * uvl), cq2[q], ep,
-                                              uvl, key_score(key), need);
+                                              uvl, tau, need, RAVE ? 0.5f * (tau - key_score(key - 1u)) : 0.0f);
             return n > 1 ? n : 1;
         };
         auto estimate = [&](uint32_t key) {
@@ -2264,7 +2271,7 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
 #pragma unroll
         for (int q = 0; q < K; q++) {
             const int n = counted ? (slice_n[q] < need ? slice_n[q] : need) : entries_from(q, T);
-            c[q] = n > 0 && n < need ? n + 1 : n;
+            c[q] = n > 0 && n < need ? (n + 1 + more < need ? n + 1 + more : need) : n;
             sum += c[q];
         }
         int inc = wave_inclusive_sum(sum, lane);
@@ -2488,6 +2495,7 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
         for (int w = 0; w < W; w++) ok = ok && told(w, 0) == 0u;
         par ^= 1;
         if (!ok) break;
+        if (4 * n_in < need) more = more == 0 ? 16 : 4 * more;  // the estimate is worth little here
         done += n_in < need ? n_in : need;
     }
     if (t == 0) {
