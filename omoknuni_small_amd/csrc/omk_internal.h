@@ -95,7 +95,7 @@ struct SelectArgs {
     int32_t trace_cap;
     int32_t *times;        // [0] when the first block of the persistent launch started, [1] when the last team
                            // left, [2] when the last walker left (100 MHz clock, low 31 bits); of a launch of blocks [0]
-                           // and [1], with the statistics or the timeline on, whose reset clears them
+                           // and [1], with the statistics or the timeline on, whose reset clears them (else NULL there)
     int32_t spin_limit;    // polls of a waiting wavefront before it raises the abort flag
     int32_t *single_ready;  // per entry of the single-visitor queue: number of the select call that wrote it
     int32_t *singles_head;  // tickets of the walkers of the persistent launch

@@ -175,7 +175,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
         *a.n_singles = n_singles;
         *a.truncated_next = 0;
         a.sched_wait[1] = 0;
-        if (a.stats || a.trace) a.times[0] = (int)(wall_clock64() & 0x7FFFFFFF);
+        if (a.times) a.times[0] = (int)(wall_clock64() & 0x7FFFFFFF);
     }
     // ---- the block's visitors ----
     int n_here = 0;
@@ -286,6 +286,10 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                         k.k1[r] = k.part[r] ? k.k1[r] : 0u;
                         k.k2[r] = k.part[r] ? k.k2[r] : 0u;
                     }
+                    // All of them have arrived, the child ranges too (vmcnt(0)), and the compiler knows it.  Else it may wait
+                    // for a round that was skipped where the loop comes round, and with it for the stores and atomics of
+                    // the level before its next loads: 8 visitors of a Gomoku tree 35 or 38 us, by how registers fall.
+                    __builtin_amdgcn_s_waitcnt(0x0F70);
                 }
                 const float ep = a.c_puct * sqrtf((float)np);
                 bool odd = false;  // (select_group: such a node is played one visitor after the other)
@@ -570,8 +574,9 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
             }
         }
     }
-    auto left = [&]() {  // (stamps of every launch, with the call in their upper half, cost it up to 3 %)
-        if ((a.stats || a.trace) && threadIdx.x == 0) atomicMax(a.times + 1, (int)(wall_clock64() & 0x7FFFFFFF));
+    // (NULL unless somebody reads them: stamps of every launch, with the call in their upper half, cost it up to 3 %)
+    auto left = [&]() {
+        if (a.times && threadIdx.x == 0) atomicMax(a.times + 1, (int)(wall_clock64() & 0x7FFFFFFF));
     };
     if (!ROWS) {
         left();

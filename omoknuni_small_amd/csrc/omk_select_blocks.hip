@@ -12,8 +12,10 @@ static hipError_t launch_class(const ForestDev &f, const SelectArgs &a, int n_it
     return hipGetLastError();
 }
 
-hipError_t launch_select_blocks(const ForestDev &f, const SelectArgs &a, int n_items, int n_singles, int max_fanout, bool rave,
+hipError_t launch_select_blocks(const ForestDev &f, const SelectArgs &a0, int n_items, int n_singles, int max_fanout, bool rave,
                                 const LoneOut &out, hipStream_t s) {
+    SelectArgs a = a0;
+    if (!a.stats && !a.trace) a.times = nullptr;  // nobody has cleared them, nobody reads them
     if (max_fanout <= 64)
         return rave ? launch_class<1, true>(f, a, n_items, n_singles, out, s)
                     : launch_class<1, false>(f, a, n_items, n_singles, out, s);
