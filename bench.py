@@ -422,17 +422,19 @@ def measure(omk, synth, name, steps, warmup, seed, cpu_seconds, scale=1.0, parit
     par = parity_check(omk, soa, meta, forest, batch, tt, tt_ids, troots, values, params) if parity else None
 
     # selection = 1 reset + 1 persistent launch (teams over a work queue of multi-visitor items, and
-    # walkers for the lone visitors) when any traversals share a root, else 1 launch of the
-    # single-visitor kernel; the roofline is quoted for the kernel that carries the work, with the
-    # whole selection phase (HIP events around it on the forest's stream) as its launch duration
-    has_groups = len(np.unique(troots)) < B
+    # walkers for the lone visitors) when any traversals share a root, 1 launch of a block a root when
+    # no root has more than 64, 1 launch of the single-visitor kernel when every one is alone; the
+    # roofline is quoted for the kernel that carries the work, with the whole selection phase (HIP
+    # events around it on the forest's stream) as its launch duration
+    most_at_a_root = int(np.unique(troots, return_counts=True)[1].max())
     # (the library walks a small batch of lone traversals on a wide layout with a legal mask by blocks, one round
     # of 64 child slots per wavefront: the same rule as its launch code)
     fan = int(np.max(soa["child_count"]))
     rounds = 1 if fan <= 64 else 4 if fan <= 256 else 6 if fan <= 384 else 16
     singles = ("k_select_singles_team" if rounds > 1 and soa.get("legal") is not None and B * rounds <= 4096
                else "k_select_singles")
-    dominant = "k_select_groups" if has_groups else singles
+    dominant = (singles if most_at_a_root == 1 else
+                "k_select_blocks" if most_at_a_root <= 64 and fan <= 384 else "k_select_groups")
     sel_ms_step = sel_ms / K
     bak_ms_step = bak_ms / K
     achieved_timed = sel_bytes / (sel_ms * 1e-3) / 1e9
@@ -479,8 +481,8 @@ def measure(omk, synth, name, steps, warmup, seed, cpu_seconds, scale=1.0, parit
             "launch_covers": "the whole selection, HIP events around it on the forest's stream: " +
                              ("k_select_groups (teams and walkers in one persistent launch; its reset comes with "
                               "omk_batch_set_roots, before the first event)"
-                              if has_groups else
-                              singles + " alone (no reset launch when every traversal is alone at its root)")
+                              if dominant == "k_select_groups" else
+                              dominant + " alone (no reset launch when no root has more than 64 traversals)")
                              + "; rocprofv3's per-kernel averages add up to it",
             # the same figures over the K timed steps, whose statistics drift with every backup (they depend on
             # --steps / --warmup; kept as information)

@@ -41,9 +41,11 @@ struct Item {
 
 constexpr int kHeavyCtxInts = 16 + 1024;  // 16 + the widest fan-out
 // Visitors from which a node is cut into slices for several blocks.  Below, the helpers of one block are as fast
-// (team_merge): its batch holds 2048 entries, up to 1475 visitors of a node with 384 children.  4096 visitors on a
-// chess-like tree and 16384 on a Go tree with RAVE: 261 and 382 us with 1024, 245 and 348 with 1536, 251 and 358 with 2048,
-// 278 and 364 with 3072.
+// (team_merge): its batch holds 2048 entries, up to 1475 visitors of a node with 384 children.  A selection and its
+// reverting with 1024, 1536 and 2048, us, over trees of three seeds: 1100 to 1500 visitors (Gomoku, chess-like, Go with RAVE
+// and re-laid, 1 and 4 trees) 1 to 30 % more with 1024 in 51 of 54; 2000 on one tree with 2048 up to 13 % more (Go with
+// RAVE 146 / 129 / 146, Gomoku 118 / 118 / 126, chess-like 206 / 205 / 211), 1700 within 6 % but for one (4 Go trees with
+// RAVE 131 / 167 / 158), 4096 and 8192 within 4 % of 1024's and up to 10 % under 2048's.
 constexpr int kHeavyMin = 1536;
 constexpr int kMaxSlices = 64;           // slices (and parts of the partition) of such a node, at most
 constexpr int kHeavyFanout = 384;        // widest node settled that way (register budget)
@@ -148,9 +150,10 @@ hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, 
 
 // The same for a batch whose roots have few visitors each (omk_select_blocks.h): a block a root, without a reset.  The
 // line lies at a visitor per lane and at the children that fit its registers (with 128 for each of 16 wavefronts).  Below
-// it the blocks are the faster ones throughout, a step with its settling, us, of the queue's kernel and of theirs:
-// Gomoku 1 tree x 8 56 and 38, 1 x 64 76 and 54, 64 x 16 66 and 36, 64 x 64 80 and 75, 256 x 24 79 and 35, 4096 x 2 222
-// and 112; Go 64 x 16 125 and 74, chess-like 64 x 16 98 and 65, 2048 x 4 155 and 87.
+// it the blocks are the faster ones throughout but for crowds with RAVE that stay together (32 % faster to 11 % slower at 64
+// visitors, where two entries of each of many children settle few of them a pass).  A selection and its reverting, us, of
+// the queue's kernel and of theirs: Gomoku 1 tree x 8 43 and 25, 1 x 64 75 and 55, 64 x 16 66 and 37, 64 x 64 106 and 71,
+// 256 x 24 146 and 31, 4096 x 2 298 and 98; Go re-laid 64 x 16 72 and 42, chess-like 64 x 16 98 and 46, 2048 x 4 206 and 73.
 constexpr int kBlockMax = 64;       // visitors of one root, at most
 constexpr int kBlockFanout = 384;   // widest node
 inline bool by_blocks(int n_items0, int most_visitors, int max_fanout) {

@@ -39,8 +39,10 @@ struct BlockScratch {
 template <int RMAX, bool ROWS>
 struct BlockLds {
     int head, tail, open;  // tickets taken, items handed out, visitors that have not reached their leaf
-    int ready[kBlockVisitors];  // item i lies in slot i % kBlockVisitors once this is i + 1 (an item has a visitor of its
-                                // own, so that a slot is free again when its turn comes)
+    int ready[kBlockVisitors];  // item i lies in slot i once this is i + 1.  A block hands out at most kBlockVisitors items in
+                                // all: each but the first (of the lone roots: their own) makes one group more of the
+                                // visitors, who are in no more groups than they are.  So no slot is used twice, and the
+                                // tickets beyond wait at slots that never hold their number
     BlockItem item[kBlockVisitors];
     int list[kBlockVisitors];  // visitors by number, partitioned in place
     int trav[kBlockVisitors];  // traversal of a visitor

@@ -2119,9 +2119,11 @@ __device__ __forceinline__ bool single_run(const SelectArgs &a, const NodeCtx &c
 // What bounds it: the dependent steps of one wavefront and some 15 block barriers; no memory.  Three wavefronts and not the
 // owner's as well: its code is the kernel's largest, and a part of it that only waits costs it no registers.
 // Measured on an MI355X, in the place of the counts and the sort of one wavefront (water_level), the whole node: 246
-// visitors of a chess-like node 15.6 -> 11.5 us, 75 to 190 of a Go node with RAVE 23 to 33 -> 13 to 15, 944 of one 45 -> 20;
-// 4096 on the chess-like tree 270 -> 245 us a selection, 16384 on the Go tree with RAVE 373 -> 348 (with the higher
-// kHeavyMin, which it makes worth while), a search of 500 a batch 2.96 -> 2.76 ms.
+// visitors of a chess-like node 15.6 -> 11.5 us, 75 to 190 of a Go node with RAVE 23 to 33 -> 13 to 15, 944 of one 45 -> 20.
+// A selection, with the higher kHeavyMin, which it makes worth while (what that is worth by itself: there), and all paths for
+// special cases that it replaced, us: Gomoku 1 x 256 142 -> 120, 1 x 1024 167 -> 137, chess-like 1 x 500 157 -> 138, 1 x 4096
+// 223 -> 202, Go with RAVE 1 x 1024 151 -> 101, 1 x 16384 215 -> 186.  Slower: crowds with RAVE of 65 to 256 that one child
+// dominates, 11.5 a node where a path of their own took 10.3 (1 x 100 of one tree 105 -> 112, 1 x 256 76 -> 82).
 constexpr int kMergeMin = 8;  // visitors from which a contested node is settled that way (5 and 14: the same)
 constexpr int kMergeThreads = (kTeamWaves - 1) * kWave;
 constexpr int kMergeOwn = 6;  // buckets a thread adds up
@@ -3080,7 +3082,7 @@ struct Continuation {
 //
 // HEAVY: the kernel for batches in which a node of kHeavyMin visitors can occur.  Without it (every root has fewer) the
 // slices, their boundaries and their joins are left out, and with them registers that the rest of the code then has
-// (scalar spills of the narrow class 332 -> 93, of four rounds 404 -> 190, of six 649 -> 229, whose vector registers go
+// (scalar spills of the narrow class 331 -> 92, of four rounds 404 -> 190, of six 649 -> 229, whose vector registers go
 // 277 -> 262).
 template <int R, bool RAVE, int RMAX, bool HEAVY>
 __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs &a, const NodeCtx &c, int lane,

@@ -71,6 +71,14 @@ def stats(path, skip=0):
                                                   float(r["AverageNs"]) / 1e3, float(r["Percentage"])))
 
 
+def copy_factor(rows, counter, copy_bytes):
+    """Counts of one copy of copy_bytes, and bytes per count.  That copy is the largest dispatch of k_copy_words, which
+    also takes leaf values to the card."""
+    counts = [float(r["Counter_Value"]) for r in rows
+              if r["Counter_Name"] == counter and short(r["Kernel_Name"]) == "k_copy_words"]
+    return (max(counts), copy_bytes / max(counts)) if counts else (0.0, None)
+
+
 def pmc(path, counter, copy_bytes=None, skip=0):
     rows = skipped(list(csv.DictReader(open(path))), skip, "Kernel_Name")
     if skip:
@@ -85,9 +93,9 @@ def pmc(path, counter, copy_bytes=None, skip=0):
         calls[k] += 1
     factor = None
     if copy_bytes and calls.get("k_copy_words"):
-        factor = copy_bytes * calls["k_copy_words"] / tot["k_copy_words"]
-        print("calibration: k_copy_words moved %d bytes per launch, %s read %.1f per launch -> %.2f bytes per count"
-              % (copy_bytes, counter, tot["k_copy_words"] / calls["k_copy_words"], factor))
+        count, factor = copy_factor(rows, counter, copy_bytes)
+        print("calibration: k_copy_words moved %d bytes in its largest launch, %s read %.1f -> %.2f bytes per count"
+              % (copy_bytes, counter, count, factor))
     print("%-44s %8s %16s %16s %s" % ("kernel", "calls", counter + "_sum", "per_call", "bytes_per_call" if factor else ""))
     for k in sorted(tot, key=lambda x: -tot[x]):
         line = "%-44s %8d %16.1f %16.1f" % (k[:44], calls[k], tot[k], tot[k] / calls[k])
@@ -122,7 +130,7 @@ def scaled_bytes(path, counter, copy_bytes, skip=0):
         if r["Counter_Name"] == counter:
             tot[short(r["Kernel_Name"])] += float(r["Counter_Value"])
             calls[short(r["Kernel_Name"])] += 1
-    factor = copy_bytes * calls["k_copy_words"] / tot["k_copy_words"]
+    factor = copy_factor(rows, counter, copy_bytes)[1]
     return {k: int(tot[k] / calls[k] * factor) for k in tot if k.startswith("k_") or "k_select" in k}, factor
 
 
