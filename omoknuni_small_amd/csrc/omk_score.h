@@ -120,4 +120,32 @@ OMK_HD bool keys_provably_monotone(int n, float w, float p, int vl0, float q2, f
     return lhs >= rhs;
 }
 
+// Bounds of a child's score (the larger of its two candidates), for a caller that has approximate reciprocals rx of
+// float(ev) and r1 of 1 + float(ev), each within two units in its last place, where child_keys divides.  With a numerator
+// rounded as there, each quotient is off by less than 2^-21 of itself, the rounding of the sums and of a second scan's
+// own divisor included; the slack is eight times that of both terms together, and a term of the size of the smallest
+// normal numbers for quotients that underflow.  What is not finite gives bounds that are not finite.
+constexpr float kBoundSlack = 3.814697265625e-6f;  // 2^-18
+template <bool RAVE>
+OMK_HD void score_about(int n, float w, float p, int vl, float q2, float ep, float rx, float r1, float &s, float &size) {
+    const int ev = (int)((uint32_t)n + (uint32_t)vl);
+    const float q = ev > 0 ? (w - (float)vl) * rx : 0.0f;
+    const float u = (p * ep) * r1;
+    s = q + u;
+    size = fabsf(q) + fabsf(u);
+    if (RAVE) {
+        const float s2 = q2 + u, size2 = fabsf(q2) + fabsf(u);
+        s = s2 > s ? s2 : s;
+        size = size2 > size ? size2 : size;
+    }
+}
+
+// keys_provably_monotone for the children most nodes turn on: values that stay positive, counts well within what binary32
+// holds exactly.  (The caller knows that q2 is finite.)
+OMK_HD bool in_order_at_once(int n, float w, float p, int vl0, float ep, uint32_t uvl, int j_last) {
+    const uint32_t vl_last = (uint32_t)vl0 + (uint32_t)j_last * uvl;  // (j_last * uvl: at most 2^16)
+    return (uint32_t)n < (1u << 23) && (uint32_t)vl0 < (1u << 22) && (uint32_t)j_last <= 63u && uvl - 1u < 1024u && n + vl0 > 0 &&
+           w >= (float)(int)vl_last && w < 3.0e38f && p * ep >= 0.0f && p * ep < 3.0e38f;
+}
+
 }  // namespace omk

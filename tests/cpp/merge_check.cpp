@@ -1,4 +1,4 @@
-// Host check of the two rules by which the selection settles a node whose visitors split: merge_heads
+// Host check of the rules by which the selection settles a node whose visitors split: pick_few, merge_heads and merge_rest
 // (csrc/omk_select_blocks.h, up to 64 visitors) and team_merge (csrc/omk_select_kernels.h).  The same steps, one "lane" at
 // a time, with the score arithmetic of csrc/omk_score.h, on random nodes; what a rule accepts is played one visitor at a
 // time as well (the serial loop of the reference, mcts_engine_batch_tree_simple.cpp:73-185 applied to one node) and must
@@ -56,17 +56,62 @@ struct Played {
     std::vector<int> taken;  // per child
 };
 
-// ---- up to 64 visitors: a lane a child, 128 entries at once ----
+// ---- up to 64 visitors: a lane a child ----
+// What is left after `out`: a prefix of every child's list, of whatever lengths, 128 entries in all; the next entry of a
+// child of which there is none is not above a bound of its own, here a little above it.
+template <typename Lengths, typename Slack>
+static bool merge_rest(const std::vector<Kid> &k, const std::vector<int> &L, int m, float ep, uint32_t uvl, uint32_t floor_key,
+                       Lengths &&lengths, Slack &&slack, Played &out) {
+    while ((int)out.order.size() < m) {
+        const int need = m - (int)out.order.size();
+        std::vector<int> c;
+        int total = 0;
+        for (int i : L) {
+            const int n = std::min(need, lengths(i, out.taken[i], need));
+            c.push_back(n > 0 && n < need ? n + 1 : n);
+            total += c.back();
+        }
+        if (total > 128) {
+            total = 0;
+            for (int &n : c) {
+                n = n > 1 ? 1 + (int)((float)(n - 1) * 0.1f) : n;
+                total += n;
+            }
+        }
+        if (total == 0 || total > 128) return false;
+        std::vector<Entry> all;
+        Entry bar{0u, 0};
+        for (size_t q = 0; q < L.size(); q++) {
+            Entry last{0u, 0};
+            for (int j = 0; j < c[q]; j++) {
+                const Entry e = entry(k, L[q], out.taken[L[q]] + j, ep, uvl);
+                if (j > 0 && e.before(last)) return false;  // not in order
+                all.push_back(last = e);
+            }
+            if (c[q] == 0) last = Entry{entry(k, L[q], out.taken[L[q]], ep, uvl).key + slack(), 0};
+            if (c[q] < need && last.key != 0u && (bar.key == 0u || last.before(bar))) bar = last;
+        }
+        std::vector<Entry> in;
+        for (const Entry &e : all)
+            if (e.key > floor_key && !bar.before(e)) in.push_back(e);
+        if (in.empty()) return false;
+        std::sort(in.begin(), in.end(), [](const Entry &a, const Entry &b) { return a.before(b); });
+        for (int r = 0; r < (int)in.size() && r < need; r++) {
+            out.order.push_back(in[r]);
+            out.taken[in[r].child()]++;
+        }
+    }
+    return true;
+}
+// At first 128 entries, as many of every child; where that settles less than a quarter, as above.
+template <typename Lengths, typename Slack>
 static bool merge_heads(const std::vector<Kid> &k, const std::vector<int> &L, int m, float ep, uint32_t uvl, uint32_t floor_key,
-                        Played &out) {
+                        Lengths &&lengths, Slack &&slack, Played &out) {
     const int n0 = (int)L.size();
-    if (n0 == 0) return false;
     int E = 64;
     while (E * n0 > 64) E >>= 1;
     bool proven = true;
     for (int c : L) proven = proven && monotone(k[c], ep, uvl, m - 1);
-    out.order.clear();
-    out.taken.assign(k.size(), 0);
     while ((int)out.order.size() < m) {
         const int need = m - (int)out.order.size();
         std::vector<Entry> all;
@@ -92,42 +137,64 @@ static bool merge_heads(const std::vector<Kid> &k, const std::vector<int> &L, in
             out.order.push_back(in[r]);
             out.taken[in[r].child()]++;
         }
+        if (4 * (int)in.size() < need) return merge_rest(k, L, m, ep, uvl, floor_key, lengths, slack, out);
     }
     return true;
 }
-// Which children a root's block lists for it.
-static bool by_block(const std::vector<Kid> &k, int m, float ep, uint32_t uvl, Played &out) {
-    auto heads = [&](uint32_t T) {
-        int n = 0;
-        for (const Kid &c : k) n += c.head() >= T;
-        return n;
-    };
+// Three visitors or fewer: the serial loop over the listed children, while their entries are in order and above the floor.
+static bool pick_few(const std::vector<Kid> &k, const std::vector<int> &L, int m, float ep, uint32_t uvl, uint32_t floor_key,
+                     Played &out) {
+    for (int v = 0; v < m; v++) {
+        Entry b{0u, 0};
+        for (int i : L) {
+            const Entry e = entry(k, i, out.taken[i], ep, uvl), next = entry(k, i, out.taken[i] + 1, ep, uvl);
+            if (next.before(e)) return false;
+            if (e.key != 0u && (b.key == 0u || e.before(b))) b = e;
+        }
+        if (b.key <= floor_key) return false;
+        out.order.push_back(b);
+        out.taken[b.child()]++;
+    }
+    return true;
+}
+// Which children a root's block lists for it: those that a bound a little above their next entry's score does not rule out
+// against `from`, which lies a little below the best child's last entry (or its first, if that is lower), or where that
+// leaves more than 64, with at least m of them.
+template <typename Lengths, typename Slack>
+static bool by_block(const std::vector<Kid> &k, int m, float ep, uint32_t uvl, Lengths &&lengths, Slack &&slack, Played &out) {
+    out.order.clear();
+    out.taken.assign(k.size(), 0);
+    std::vector<uint32_t> ceiling(k.size(), 0u);
     int best = -1;
     for (int i = 0; i < (int)k.size(); i++)
-        if (k[i].head() && (best < 0 || entry(k, i, 0, ep, uvl).before(entry(k, best, 0, ep, uvl)))) best = i;
-    if (best < 0) return false;
-    const uint32_t hk = k[best].head(), lk = entry(k, best, m - 1, ep, uvl).key;
-    uint32_t from = std::min(lk, hk), floor_key = from - 1u;
-    if (from == 0u || heads(from) > 64) {
-        floor_key = 0u;
-        from = 1u;
-        if (heads(1u) > 64) {  // at least m and at most 64 heads, found by halving
-            uint32_t lo = 1u, hi = hk + 1u;
-            from = 0u;
-            while (from == 0u && hi - lo > 1u) {
-                const uint32_t mid = lo + ((hi - lo) >> 1);
-                const int n = heads(mid);
-                if (n < m) hi = mid;
-                else if (n > 64) lo = mid;
-                else from = mid;
-            }
+        if (k[i].head()) {
+            ceiling[i] = k[i].head() + slack();
+            if (best < 0 || ceiling[i] > ceiling[best]) best = i;
         }
+    if (best < 0) return false;
+    auto listed = [&](uint32_t T) {
+        int n = 0;
+        for (uint32_t c : ceiling) n += c >= T;
+        return n;
+    };
+    const uint32_t low = std::min(entry(k, best, m - 1, ep, uvl).key, k[best].head());
+    uint32_t from = low > 64u ? low - slack() : 1u;
+    if (listed(from) > 64) {
+        uint32_t lo = from, hi = ceiling[best];
+        while (hi - lo > 1u) {
+            const uint32_t mid = lo + ((hi - lo) >> 1);
+            const int n = listed(mid);
+            (n < m ? hi : lo) = mid;
+            if (n >= m && n <= 64) break;
+        }
+        if (listed(lo) > 64) return false;
+        from = lo;
     }
-    if (from == 0u) return false;
     std::vector<int> L;
     for (int i = 0; i < (int)k.size(); i++)
-        if (k[i].head() >= from) L.push_back(i);
-    return merge_heads(k, L, m, ep, uvl, floor_key, out);
+        if (ceiling[i] >= from) L.push_back(i);
+    if (m <= 3) return pick_few(k, L, m, ep, uvl, from - 1u, out);
+    return merge_heads(k, L, m, ep, uvl, from - 1u, lengths, slack, out);
 }
 
 // ---- any number of visitors: a prefix of every child's list, of whatever lengths ----
@@ -254,7 +321,6 @@ int main(int argc, char **argv) {
                 printf("WRONG: %s, case %ld, rave %d, %d children, %d visitors, virtual loss %u\n", who, cs, (int)RAVE, nk, m, uvl);
         };
         Played got;
-        if (m <= 64) hold(by_block(k, m, ep, uvl, got), got, "block", block_yes, block_no);
         // lengths about right, far too short, far too long
         const int how = (int)(rng() % 3);
         auto lengths = [&](int i, int had, int need) {
@@ -263,6 +329,8 @@ int main(int argc, char **argv) {
             if (how == 1) return right / (int)(1 + rng() % 4) + (rng() % 8 == 0);
             return right + (int)(rng() % (need + 1));
         };
+        auto slack = [&]() { return (uint32_t)(rng() % 17); };
+        if (m <= 64) hold(by_block(k, m, ep, uvl, lengths, slack, got), got, "block", block_yes, block_no);
         hold(team_merge(k, m, ep, uvl, lengths, got), got, "team", team_yes, team_no);
     }
     printf("blocks: merged %ld, declined %ld; teams: merged %ld, declined %ld; wrong %ld\n", block_yes, block_no, team_yes, team_no,

@@ -203,6 +203,22 @@ def test_merge_rules_against_the_serial_loop(tmp_path):
     assert m and int(m.group(1)) > 30000 and int(m.group(2)) > 30000, out.stdout[-500:]
 
 
+def test_bounds_of_scores_hold_the_exact_ones(tmp_path):
+    """Children are ruled out by bounds worked out with approximate reciprocals (score_about): over the whole range of counts,
+    sums, priors and blends, with reciprocals off by a unit in the last place either way, the exact score lies between them
+    (tests/cpp/bound_check.cpp)."""
+    import re
+    import subprocess
+    exe = str(tmp_path / "bound_check")
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-fno-fast-math", "-I",
+                           os.path.join(ROOT, "omoknuni_small_amd", "csrc"),
+                           os.path.join(ROOT, "tests", "cpp", "bound_check.cpp"), "-o", exe])
+    out = subprocess.run([exe, "1000000"], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout[-2000:]
+    m = re.search(r"bounds: (\d+) held, wrong 0", out.stdout)
+    assert m and int(m.group(1)) > 1800000, out.stdout[-500:]
+
+
 def test_tickets_are_drawn_between_barriers_of_the_wavefront():
     """Lane 0 draws a wavefront's next ticket at the head of loops that may end in another branch of lane 0's own.  Without a
     barrier of the wavefront the compiler may join the two across the loop's edge, and the other lanes go round without the

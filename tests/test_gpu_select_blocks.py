@@ -105,6 +105,27 @@ def test_few_crowded_roots_among_thousands_of_lone_ones(crowds, widest, mask, ra
     both(soa, np.random.default_rng(lone).permutation(troots) if alternating else troots, 9, rave=rave, steps=2)
 
 
+@pytest.mark.parametrize("visitors", [1, 2, 3, 4, 13, 64])
+@pytest.mark.parametrize("fan,rave", [(3, False), (64, True), (65, False), (225, False), (384, True)])
+def test_scores_closer_than_their_bounds(visitors, fan, rave):
+    """Scores that differ by nothing or by a few units in the last place, which the bounds (2^-18 wide) cannot tell apart,
+    among children with and without visits: crowds, and lone visitors beside them."""
+    soa, roots = layered_forest(fan + 7 * visitors, [fan, 30, 5], n_trees=4, rave=rave)
+    rng = np.random.default_rng(fan + visitors)
+    n = len(soa["N"])
+    near = rng.random(n) < 0.8
+    near[roots] = False
+    soa["N"] = np.where(near, np.where(rng.random(n) < 0.3, 0, 200), soa["N"]).astype(np.int32)
+    soa["W"] = np.where(near, soa["N"] / 4.0, soa["W"]).astype(np.float32)
+    p = np.float32(1.0 / fan)
+    steps = rng.integers(-3, 4, n)
+    soa["P"] = np.where(near, p * (np.float32(1) + steps.astype(np.float32) * np.float32(2.0 ** -23)), soa["P"]).astype(np.float32)
+    if rave:
+        soa["rN"] = np.where(near, 0, soa["rN"]).astype(np.int32)
+        soa["rW"] = np.where(near, 0.0, soa["rW"]).astype(np.float32)
+    both(soa, np.repeat(roots, [visitors, 1, max(1, visitors - 1), visitors]).astype(np.int32), 6, rave=rave)
+
+
 @pytest.mark.parametrize("kind", ["nan prior", "nan sum", "-inf sum", "inf sum of the unvisited", "no virtual loss", "all equal"])
 @pytest.mark.parametrize("rave", [False, True])
 def test_scores_that_are_not_real_and_ties(kind, rave):
