@@ -68,9 +68,20 @@ constexpr int kWaterLevelMaxJ = 1 << 21;  // entries per child representable in 
 constexpr int kBatchCap = 2048;           // entries put in winner order at a time (LDS resident)
 constexpr int kSortBits = 8;              // widest radix digit of that sort
 constexpr int kSortBins = 1 << kSortBits;
-constexpr int kTeamWaves = 4;             // wavefronts per block of the multi-visitor kernel: one owner that
-                                          // takes the items, three helpers for the batch work of its node
-constexpr int kTeam = kTeamWaves * 64;
+// Wavefronts per block of the multi-visitor kernel: one owner that takes the items, and helpers for the batch work of its
+// node: three, or seven in the kernel for crowds (HEAVY).  A helper works on its share of the entries, an instruction every 5
+// cycles, and waits for the others some ten times, for which seven take longer: a merge of 1100 visitors of a Go node with
+// RAVE 37000 -> 25000 cycles with seven, of 564 of a chess-like one 22900 -> 19200, but of 40 12000 -> 13100.  So the line
+// lies at kWideTeamMin visitors of the most crowded root; a layout of narrow nodes gains nothing below kHeavyMin, where that
+// kernel is needed.  A selection and its reverting, us, one tree of three seeds with three and seven: 1024 visitors Gomoku 137,
+// 133, 136 and 133, 130, 134, Go with RAVE 101, 104, 103 and 95, 101, 99, chess-like (with seven) 162, 149, 187 and 169, 155,
+// 190; 1600 Gomoku 150, 145, 161 and 140, 140, 150, Go re-laid 137, 152, 168 and 134, 141, 155, chess-like 203, 175, 196 and
+// 194, 176, 195; 4096 Gomoku 181, 207, 199 and 167, 198, 188, Go with RAVE 151, 160, 124 and 142, 164, 129.
+constexpr int kWideTeamMin = 1024;
+static_assert(kWideTeamMin <= kHeavyMin, "what nodes of kHeavyMin visitors need is in that kernel");
+template <bool HEAVY>
+constexpr int kTeamWaves = HEAVY ? 8 : 4;
+constexpr int kMostTeamWaves = 8;
 constexpr int kTeamMin = 96;              // batch entries from which the helpers are called in
 // a batch of at most this many entries per thread is ordered by counting: a lone wavefront, the block
 constexpr int kCountSortLone = 2, kCountSortTeam = 1;
@@ -153,7 +164,6 @@ template <int R>
 struct WaveLds {
     TeamCmd cmd;
     uint32_t red[4];       // team reductions: smallest / largest inverted key, flags
-    int wsum[kTeamWaves];  // team prefix scan: totals of the wavefronts
     int offs[R * kWave];   // exclusive prefix of the visit counts in child order
     int st_n[R * kWave];   // statistics of every child, readable by any lane
     float st_w[R * kWave];
@@ -163,7 +173,8 @@ struct WaveLds {
     int st_j0[R * kWave];  // visits already settled / visit count, by phase
     int hist[kSortBins * (kBatchCap / kWave + 1) > R * kWave ? kSortBins * (kBatchCap / kWave + 1) : R * kWave];  // sort: entries per (digit value, block of 64); emit: visits per child
     uint32_t pay[R * kWave];      // per child: entries of the batch
-    uint32_t slots[2][2 * kTeamWaves];  // team_merge: what the wavefronts tell each other
+    uint32_t slots[2][2 * kMostTeamWaves];  // team_merge: what the wavefronts tell each other
+    int wsum[kMostTeamWaves];     // team prefix scan: totals of the wavefronts
     alignas(16) uint32_t key[2][kBatchCap];  // entries of the batch being ordered: inverted score key ...
     alignas(16) uint32_t pay2[2][kBatchCap];  // ... and pass flag, child, visit number; two buffers, ping-pong
 };
@@ -1131,13 +1142,13 @@ __device__ __forceinline__ void active_counts(const ActiveSet<R> &s, float ep, u
 // The visitors settled are those with ranks [rank0, rank0 + todo) of the node's winner
 // order, starting from the state in which child i has had tk0[i] visits already (all zero
 // and rank0 = 0 for a whole node; a slice of a heavy node otherwise).
-template <int R, bool RAVE>
+template <int R, bool RAVE, bool HEAVY>
 __device__ __forceinline__ bool water_level(const SelectArgs &a, const NodeCtx &c, int lane, const Kids<R, RAVE> &k,
                                             int off, int rank0, int todo, const int (&tk0)[R], WaveLds<R> &lds,
                                             int (&cnt)[R], bool allow_lds, int &lds_cur, bool use_preset,
                                             const int (&preset)[R], uint32_t *order, bool &pending) {
     lds_cur = -1;
-    constexpr int F = R * kWave;
+    constexpr int F = R * kWave, kTeam = kTeamWaves<HEAVY> * kWave;
     const uint32_t uvl = (uint32_t)a.vl;
     const int m = todo;
     off += rank0;
@@ -2106,7 +2117,7 @@ __device__ __forceinline__ bool single_run(const SelectArgs &a, const NodeCtx &c
     return true;
 }
 
-// ---- A contested node settled by the three helpers ----
+// ---- A contested node settled by the helpers ----
 // The score a child shows the j-th of a node's visitors that choose it depends on nothing but j, and where no child's
 // scores increase with j the serial order is the merge of the children's lists by (key, position).  The helpers work out
 // a prefix of every list side by side, a few more entries than the closed form says lie at or above a threshold with
@@ -2116,8 +2127,8 @@ __device__ __forceinline__ bool single_run(const SelectArgs &a, const NodeCtx &c
 // Without RAVE their number is nearly a straight line in y = 1 / (score + 1), and the buckets are equal steps of y: one or
 // two entries each.  With RAVE most lie close above the threshold (blends that hardly move with virtual loss): 64 buckets
 // for every halving of the distance in y to it.
-// What bounds it: the dependent steps of one wavefront and some 15 block barriers; no memory.  Three wavefronts and not the
-// owner's as well: its code is the kernel's largest, and a part of it that only waits costs it no registers.
+// What bounds it: the dependent steps of one wavefront and some 15 block barriers; no memory.  The helpers and not the
+// owner as well: its code is the kernel's largest, and a part of it that only waits costs it no registers.
 // Measured on an MI355X, in the place of the counts and the sort of one wavefront (water_level), the whole node: 246
 // visitors of a chess-like node 15.6 -> 11.5 us, 75 to 190 of a Go node with RAVE 23 to 33 -> 13 to 15, 944 of one 45 -> 20.
 // A selection, with the higher kHeavyMin, which it makes worth while (what that is worth by itself: there), and all paths for
@@ -2125,12 +2136,14 @@ __device__ __forceinline__ bool single_run(const SelectArgs &a, const NodeCtx &c
 // 223 -> 202, Go with RAVE 1 x 1024 151 -> 101, 1 x 16384 215 -> 186.  Slower: crowds with RAVE of 65 to 256 that one child
 // dominates, 11.5 a node where a path of their own took 10.3 (1 x 100 of one tree 105 -> 112, 1 x 256 76 -> 82).
 constexpr int kMergeMin = 8;  // visitors from which a contested node is settled that way (5 and 14: the same)
-constexpr int kMergeThreads = (kTeamWaves - 1) * kWave;
-constexpr int kMergeOwn = 6;  // buckets a thread adds up
-constexpr int kMergeBuckets = kMergeThreads * kMergeOwn;
+// buckets a thread adds up: 1152 and 1344 in all
+template <bool HEAVY>
+constexpr int kMergeOwn = HEAVY ? 3 : 6;
+template <bool HEAVY>
+constexpr int kMergeBuckets = (kTeamWaves<HEAVY> - 1) * kWave * kMergeOwn<HEAVY>;
 constexpr int kMergePasses = 12;
 constexpr int kMergeCount = 32;  // entries of a bucket that are ranked by counting whoever they belong to
-static_assert(2 * kMergeBuckets + 1 + 2 * kBatchCap + 1024 <= kSortBins * (kBatchCap / kWave + 1), "buckets and arrivals fit the sort's table");
+static_assert(2 * kMergeBuckets<true> + 1 + 2 * kBatchCap + 1024 <= kSortBins * (kBatchCap / kWave + 1), "buckets and arrivals fit the sort's table");
 
 // A slice of a heavy node goes the same way from the visits the children have had before it (st_j0[]), with the entries
 // that its two thresholds count (offs[]) in the place of the estimate.
@@ -2138,19 +2151,19 @@ static_assert(2 * kMergeBuckets + 1 + 2 * kBatchCap + 1024 <= kSortBins * (kBatc
 // chess-like tree 245 -> 238 us a selection, 16384 on the Go tree with RAVE 348 -> 328.
 // t: number of the helper thread.  On success (cmd.merged) order[] holds (child << 21) | visit number of the m visitors and
 // st_j0[] the visits per child.  The owner takes the barriers with them.
-template <int R, bool RAVE>
+template <int R, bool RAVE, bool HEAVY>
 __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds, uint32_t *order, int t, int m, int goff,
                                            float ep, uint32_t uvl) {
-    constexpr int F = R * kWave, NT = kMergeThreads, W = NT / kWave;
+    constexpr int F = R * kWave, W = kTeamWaves<HEAVY> - 1, NT = W * kWave, OWN = kMergeOwn<HEAVY>, B = kMergeBuckets<HEAVY>;
     constexpr int K = (F + NT - 1) / NT;  // children of a thread: t, t + NT ..
     const int lane = t & 63, wv = uniform(t >> 6);
     uint64_t *ent = reinterpret_cast<uint64_t *>(lds.key[0]);    // in (child, visit) order; smaller = played earlier
     uint64_t *ent2 = reinterpret_cast<uint64_t *>(lds.pay2[0]);  // by bucket
     uint32_t *own = lds.pay2[0];                                 // (before that: the child of every entry)
     int *bucket = lds.hist;
-    uint32_t *arrival = reinterpret_cast<uint32_t *>(lds.hist) + kMergeBuckets + 1;
-    int *runs = lds.hist + kMergeBuckets + 1 + kBatchCap;      // of a bucket: children with entries in it
-    int *seg_end = runs + kMergeBuckets;                       // of a child: behind its last entry
+    uint32_t *arrival = reinterpret_cast<uint32_t *>(lds.hist) + B + 1;
+    int *runs = lds.hist + B + 1 + kBatchCap;      // of a bucket: children with entries in it
+    int *seg_end = runs + B;                       // of a child: behind its last entry
     uint32_t *run_at = reinterpret_cast<uint32_t *>(seg_end) + F;  // by bucket: first entry of each of these, end of the child's
     int par = 0, barriers = 0;
     auto sync = [&]() {
@@ -2217,7 +2230,7 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
                 hmax = umax32(hmax, hk[q]);
             }
         }
-        for (int b = t; b <= kMergeBuckets; b += NT) bucket[b] = 0;
+        for (int b = t; b <= B; b += NT) bucket[b] = 0;
         tell(wave_max_all(lmax), wave_max_all(hmax));
         uint32_t lo_key = 0u, hi_key = 0u;
 #pragma unroll
@@ -2258,7 +2271,7 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
         int target = need + (need >> 3) + 4;
         if (target > kMost) target = kMost;
         int acc_hi = target + (target >> 1);
-        if (acc_hi < 2 * NT) acc_hi = 2 * NT;  // (two entries a thread cost hardly more than one)
+        if (acc_hi < 384) acc_hi = 384;  // (one or two entries a thread)
         if (acc_hi > kMost) acc_hi = kMost;
         uint32_t T = lo_key;
         const int at_lo = counted ? 0 : estimate(lo_key);
@@ -2385,7 +2398,7 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
         }
         // ---- the entries up to there, in order ----
         const float y0 = y_of(hi_key), y1 = y_of(umax32(T, ~(uint32_t)(bar >> 32)));
-        const float scale = y1 > y0 ? (RAVE ? 1.0f : (float)kMergeBuckets) * __frcp_rn(y1 - y0) : 0.0f;
+        const float scale = y1 > y0 ? (RAVE ? 1.0f : (float)B) * __frcp_rn(y1 - y0) : 0.0f;
         for (int e = t; e < total; e += NT) {
             const uint64_t x = ent[e];
             if (x > bar) continue;
@@ -2393,21 +2406,21 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
             int b;
             if (RAVE) {
                 const float d = (y1 - y) * scale;  // 1 .. 0
-                b = kMergeBuckets - 1 - ((int)(__float_as_uint(d > 0.0f ? d : 0.0f) >> 17) - (0x3F800000 >> 17) + kMergeBuckets);
-                b = b < 0 ? 0 : (b > kMergeBuckets - 1 ? kMergeBuckets - 1 : b);
+                b = B - 1 - ((int)(__float_as_uint(d > 0.0f ? d : 0.0f) >> 17) - (0x3F800000 >> 17) + B);
+                b = b < 0 ? 0 : (b > B - 1 ? B - 1 : b);
             } else {
                 float fb = (y - y0) * scale;
                 fb = fb > 0.0f ? fb : 0.0f;
-                b = fb < (float)(kMergeBuckets - 1) ? (int)fb : kMergeBuckets - 1;
+                b = fb < (float)(B - 1) ? (int)fb : B - 1;
             }
             arrival[e] = ((uint32_t)b << 16) | (uint32_t)atomicAdd(&bucket[b], 1);
         }
         sync();
-        int own_n[kMergeOwn], lsum = 0, fullest = 0;
+        int own_n[OWN], lsum = 0, fullest = 0;
 #pragma unroll
-        for (int u = 0; u < kMergeOwn; u++) {
-            own_n[u] = bucket[t * kMergeOwn + u];
-            runs[t * kMergeOwn + u] = 0;
+        for (int u = 0; u < OWN; u++) {
+            own_n[u] = bucket[t * OWN + u];
+            runs[t * OWN + u] = 0;
             lsum += own_n[u];
             fullest = own_n[u] > fullest ? own_n[u] : fullest;
         }
@@ -2424,11 +2437,11 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
         }
         par ^= 1;
 #pragma unroll
-        for (int u = 0; u < kMergeOwn; u++) {
-            bucket[t * kMergeOwn + u] = start;
+        for (int u = 0; u < OWN; u++) {
+            bucket[t * OWN + u] = start;
             start += own_n[u];
         }
-        if (t == NT - 1) bucket[kMergeBuckets] = start;
+        if (t == NT - 1) bucket[B] = start;
         sync();
         if (n_in == 0) {
             ok = false;
@@ -3369,7 +3382,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
 #pragma unroll
                             for (int r = 0; r < R; r++) cnt[r] = lds.st_j0[r * kWave + lane];
                         } else {
-                            ok = water_level<R, RAVE>(a, c, lane, k, soff, rank_hi, todo, ct_hi, lds, cnt, false, unused_cur,
+                            ok = water_level<R, RAVE, HEAVY>(a, c, lane, k, soff, rank_hi, todo, ct_hi, lds, cnt, false, unused_cur,
                                                       preset_ok, between, pl.order, pending);
                         }
                     }
@@ -3427,7 +3440,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
         int zero[R];
 #pragma unroll
         for (int r = 0; r < R; r++) zero[r] = 0;
-        settled = water_level<R, RAVE>(a, c, lane, k, soff, 0, m, zero, lds, cnt, !heavy, lds_cur, false, zero,
+        settled = water_level<R, RAVE, HEAVY>(a, c, lane, k, soff, 0, m, zero, lds, cnt, !heavy, lds_cur, false, zero,
                                        pl.order, pending);
         if (!settled) st_replay = 1;
     }
@@ -4184,10 +4197,11 @@ __device__ __forceinline__ void partition_async(const ForestDev &f, const Select
 }
 
 // What a helper wavefront does with one request of its owner.
-template <int R, bool RAVE, int RMAX>
+template <int R, bool RAVE, int RMAX, bool HEAVY>
 __device__ __forceinline__ void team_help(const ForestDev &f, const SelectArgs &a, WaveLds<R> &lds, PartLds<RMAX> &pl,
                                           int tid, int op, int total, int keep, int goff, int cur, float ep,
                                           uint32_t uvl) {
+    constexpr int kTeam = kTeamWaves<HEAVY> * kWave;
     uint32_t *order = pl.order;
     if (op == kOpPartition) {
         if ((tid >> 6) == 1) partition_async<R, RMAX>(f, a, lds.cmd, pl, tid & 63);
@@ -4217,7 +4231,7 @@ template <int RMAX, bool RAVE>
 __device__ void walkers_loop(ForestDev f, SelectArgs a, int lane);
 
 template <int RMAX, bool RAVE, bool HEAVY>
-__global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs a) {
+__global__ __launch_bounds__(kTeamWaves<HEAVY> * kWave) void k_select_groups(ForestDev f, SelectArgs a) {
     __shared__ WaveLds<RMAX> s_lds;
     __shared__ PartLds<RMAX> s_part;
     const int tid = threadIdx.x;
@@ -4261,6 +4275,17 @@ __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs
             const int c_depth = __builtin_amdgcn_readfirstlane(cm.c_depth), c_m = __builtin_amdgcn_readfirstlane(cm.c_m);
             const int c_off = __builtin_amdgcn_readfirstlane(cm.c_off);
             int levels = 0;
+            if (HEAVY && RMAX > 1 && wi >= kChainWalkers) {  // (takes the walk's barriers with it, like the owner)
+                for (int taken = 1;; taken++) {
+                    __syncthreads();
+                    int nb = -1;
+                    if ((tid & 63) == 0) nb = __hip_atomic_load(&g_chain.n_barriers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    nb = uniform(nb);
+                    if (nb >= 0 && taken == nb + 1) break;
+                }
+                __syncthreads();  // the request is done
+                continue;
+            }
             if (RMAX > 1 || wi == 0)
                 levels = chain_walk<RMAX, RAVE>(ka, (LdsBytesP)&s_lds, wi, tid & 63, __builtin_amdgcn_readfirstlane(cm.c_node),
                                                 __builtin_amdgcn_readfirstlane(cm.c_np),
@@ -4276,12 +4301,12 @@ __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs
         if (op == kOpMerge) {
             // (its last barrier ends the request)
             if (rounds == 1)
-                team_merge<1, RAVE>(a, reinterpret_cast<WaveLds<1> &>(s_lds), s_part.order, tid - kWave, total, goff, ep, uvl);
+                team_merge<1, RAVE, HEAVY>(a, reinterpret_cast<WaveLds<1> &>(s_lds), s_part.order, tid - kWave, total, goff, ep, uvl);
             else
-                team_merge<RMAX, RAVE>(a, s_lds, s_part.order, tid - kWave, total, goff, ep, uvl);
+                team_merge<RMAX, RAVE, HEAVY>(a, s_lds, s_part.order, tid - kWave, total, goff, ep, uvl);
             continue;
         }
-        if (RMAX > 1 && (op == kOpPartition || op == kOpLoad) && (tid >> 6) >= 2) {
+        if (RMAX > 1 && (op == kOpPartition || op == kOpLoad) && (tid >> 6) >= 2 && (!HEAVY || (tid >> 6) <= 3)) {
             const int pn = __builtin_amdgcn_readfirstlane(s_lds.cmd.pre_node);
             if (pn >= 0)
                 load_ahead<RMAX, RAVE>(f, a, s_lds, pn, __builtin_amdgcn_readfirstlane(s_lds.cmd.pre_np),
@@ -4290,10 +4315,10 @@ __global__ __launch_bounds__(kTeam) void k_select_groups(ForestDev f, SelectArgs
                                        tid & 63);
         }
         if (rounds == 1)
-            team_help<1, RAVE, RMAX>(f, a, reinterpret_cast<WaveLds<1> &>(s_lds), s_part, tid, op, total, keep, goff, cur,
+            team_help<1, RAVE, RMAX, HEAVY>(f, a, reinterpret_cast<WaveLds<1> &>(s_lds), s_part, tid, op, total, keep, goff, cur,
                                      ep, uvl);
         else
-            team_help<RMAX, RAVE, RMAX>(f, a, s_lds, s_part, tid, op, total, keep, goff, cur, ep, uvl);
+            team_help<RMAX, RAVE, RMAX, HEAVY>(f, a, s_lds, s_part, tid, op, total, keep, goff, cur, ep, uvl);
         // a heavy node's list and the winners of its slices are read by other blocks once the owner has announced them
         if (HEAVY) wait_stores();
         __syncthreads();  // the request is done
@@ -4650,7 +4675,9 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_i
         // on the 4 M-node chess-like tree: 0.247 ms a selection with two blocks per unit, 0.222 with one.
         int capacity = n_cus;
         if (capacity < 2) capacity = 2;
-        int walkers = n_traversals / 4;
+        const bool heavy = most_visitors >= (RMAX > 1 ? kWideTeamMin : kHeavyMin);
+        const int waves = heavy ? kTeamWaves<true> : kTeamWaves<false>;
+        int walkers = n_traversals / waves;
         if (walkers > capacity / 4) walkers = capacity / 4;
         if (walkers > kMaxWalkerBlocks) walkers = kMaxWalkerBlocks;  // idle walkers poll: more of them slow the teams
         // (a wavefront per visitor while that is at most kMaxWalkerBlocks: the root of a young tree leaves nearly
@@ -4663,8 +4690,8 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_i
         SelectArgs a = a0;
         a.n_team_blocks = teams;
         a.fast_singles = fast ? 1 : 0;
-        const dim3 grid(teams + walkers), block(kTeam);
-        if (most_visitors >= kHeavyMin)
+        const dim3 grid(teams + walkers), block(waves * kWave);
+        if (heavy)
             hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, true>), grid, block, 0, s, f, a);
         else
             hipLaunchKernelGGL((k_select_groups<RMAX, RAVE, false>), grid, block, 0, s, f, a);

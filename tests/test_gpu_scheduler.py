@@ -368,6 +368,19 @@ def test_chain_whose_capacity_is_exceeded_by_one_visitor(fan, rave, m):
     assert st["replayed_nodes"] == 0, st
 
 
+@pytest.mark.parametrize("fan,rave,m", [(40, False, 1535), (40, False, 1536), (225, False, 1023), (225, False, 1024),
+                                        (362, True, 1024), (362, True, 1535), (700, False, 1024)])
+def test_crowds_on_both_sides_of_the_wider_teams(fan, rave, m):
+    """Crowds of 1024 visitors (1536 of narrow nodes) are settled by teams of eight wavefronts: contested nodes of all
+    sizes, and a chain of nodes whose visitors stay together, which three of the helpers walk and the others wait out."""
+    soa, roots = layered_forest(31, [fan, 60, 20], rave=rave, plateau=rave)
+    st = select_both(soa, np.zeros(m, np.int32), 4, rave=rave)
+    assert st["replayed_nodes"] == 0, st
+    soa = capacity_chain(fan, 9, 5, m, rave)
+    st = select_both(soa, np.zeros(m, np.int32), 11, rave=rave)
+    assert st["replayed_nodes"] == 0, st
+
+
 def test_boundaries_of_heavy_children_are_worked_out_ahead_of_time():
     """A heavy root with heavy children: the children's slice boundaries are queued as items of their own
     (kind 4 in the timeline) while the root is still being settled, the root's own when the roots are set;
