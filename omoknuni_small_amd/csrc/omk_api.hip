@@ -135,10 +135,11 @@ struct omk_batch {
     int32_t n = 0;          // traversals bound by set_roots
     int64_t generation = -1;  // the forest's generation when the roots were set
     bool selected = false;  // paths of a select are on the device
-    // No two of these paths share a node: said by the selection that made them.  (What the forest or the roots are
+    // What the selection that made them says of the paths.  (What the forest or the roots are
     // like when they are settled says nothing: paths that follow transpositions meet in nodes that several trees
     // hold, and an upload makes the forest a tree again under them.)
-    bool disjoint = false;
+    PathsAre paths_are = PathsAre::kAny;
+    bool one_root = false;  // of all traversals
     bool stamped = false;  // the last selection has left its time stamps
     int32_t *paths = nullptr, *path_len = nullptr, *leaf = nullptr;
     float *values = nullptr;
@@ -1378,6 +1379,7 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) try {
         }
         i = j;
     }
+    const bool one_root = items.size() + singles.size() == 1;
     // the most crowded roots head the longest chains of work: start them first
     std::stable_sort(items.begin(), items.end(), [](const Item &x, const Item &y) { return x.m > y.m; });
     // A root that will be cut into slices (kHeavyMin visitors or more): its boundaries depend on its statistics
@@ -1435,6 +1437,7 @@ int omk_batch_set_roots(omk_batch *b, const int32_t *h_roots, int32_t n) try {
     b->n_items0 = (int32_t)items.size();
     b->n_hctx0 = n_hctx0;
     b->n_singles0 = (int32_t)singles.size();
+    b->one_root = one_root;
     b->n = n;
     b->in_order = in_order;
     b->generation = f->generation;
@@ -1518,7 +1521,9 @@ int omk_select_batch(omk_batch *b, const omk_select_params *p) {
                           b->n_cus, b->n_hctx0, b->prepared == b->epoch, out,
                           f->stream));
     b->selected = true;
-    b->disjoint = b->n_items0 == 0;  // a root each, and distinct roots head disjoint trees
+    b->paths_are = b->n_items0 == 0 ? PathsAre::kDisjoint  // a root each, and distinct roots head disjoint trees
+                   : b->one_root    ? PathsAre::kOneTree
+                                    : PathsAre::kAny;
     b->stamped = b->n_items0 > 0 && (!by_blocks(b->n_items0, b->most_visitors, f->max_fanout) || a.stats || a.trace);
     b->select_calls++;
     b->lone_call = out.sig.flag ? b->select_calls : -1;
@@ -1531,12 +1536,9 @@ int omk_backup_batch(omk_batch *b, int32_t virtual_loss) {
     if (int rc = fresh_batch("omk_backup_batch", b)) return rc;
     if (int rc = use_device(b->f)) return rc;
     b->f->changes++;
+    // N and W of the nodes on the paths change: their RAVE blend with them
     HIP_TRY(launch_backup(b->f->dev(), b->paths, b->path_len, b->values, b->n, b->stride, b->max_depth + 1,
-                          virtual_loss, b->disjoint, b->f->stream));
-    // N and W of the nodes on the paths have changed: their RAVE blend with them
-    if (b->f->has_rave && b->f->blend_valid)
-        HIP_TRY(launch_blend_paths(b->f->dev(), b->paths, b->path_len, b->n, b->stride, b->max_depth + 1, b->f->blend_k,
-                                   b->f->stream));
+                          virtual_loss, b->paths_are, b->f->has_rave && b->f->blend_valid, b->f->blend_k, b->f->stream));
     return OMK_OK;
 }
 
@@ -1559,7 +1561,7 @@ int omk_revert_vl(omk_batch *b, int32_t virtual_loss) {
     if (int rc = fresh_batch("omk_revert_vl", b)) return rc;
     if (int rc = use_device(b->f)) return rc;
     HIP_TRY(launch_revert_vl(b->f->dev(), b->paths, b->path_len, b->n, b->stride, b->max_depth + 1, virtual_loss,
-                             b->disjoint, b->f->stream));
+                             b->paths_are, b->f->stream));
     return OMK_OK;
 }
 
@@ -1582,7 +1584,8 @@ int omk_apply_vl_paths(omk_forest *f, const int32_t *d_paths, const int32_t *d_p
 int omk_revert_vl_paths(omk_forest *f, const int32_t *d_paths, const int32_t *d_path_len, int32_t n, int32_t stride,
                         int32_t max_len, int32_t virtual_loss) {
     if (int rc = check_paths_args("omk_revert_vl_paths", f, d_paths, d_path_len, n, stride, max_len)) return rc;
-    HIP_TRY(launch_revert_vl(f->dev(), d_paths, d_path_len, n, stride, max_len, virtual_loss, false, f->stream));
+    HIP_TRY(launch_revert_vl(f->dev(), d_paths, d_path_len, n, stride, max_len, virtual_loss, PathsAre::kAny,
+                             f->stream));
     return OMK_OK;
 }
 
@@ -1591,9 +1594,8 @@ int omk_backup_paths(omk_forest *f, const int32_t *d_paths, const int32_t *d_pat
     if (int rc = check_paths_args("omk_backup_paths", f, d_paths, d_path_len, n, stride, max_len)) return rc;
     if (!d_values) return fail(OMK_ERR_INVALID, "omk_backup_paths: null values");
     f->changes++;
-    HIP_TRY(launch_backup(f->dev(), d_paths, d_path_len, d_values, n, stride, max_len, virtual_loss, false, f->stream));
-    if (f->has_rave && f->blend_valid)
-        HIP_TRY(launch_blend_paths(f->dev(), d_paths, d_path_len, n, stride, max_len, f->blend_k, f->stream));
+    HIP_TRY(launch_backup(f->dev(), d_paths, d_path_len, d_values, n, stride, max_len, virtual_loss, PathsAre::kAny,
+                          f->has_rave && f->blend_valid, f->blend_k, f->stream));
     return OMK_OK;
 }
 
@@ -2177,7 +2179,7 @@ int omk_tt_select_redirect(omk_tt *tt, omk_batch *b, const omk_select_params *p,
     a.abort_word = b->counters + 3 * kSchedStep + 1;
     HIP_TRY(launch_select_redirect(f->dev(), a, p->use_rave != 0, s));
     b->selected = true;
-    b->disjoint = false;
+    b->paths_are = PathsAre::kAny;
     b->stamped = false;
     b->select_calls++;
     int32_t status[8];

@@ -54,6 +54,7 @@ __global__ __launch_bounds__(256) void k_apply_vl(ForestDev f, const int32_t *pa
 // (one per wavefront where it sat on one node), 4.5 combined; of 16384 of 9 nodes 29 and 4.6.  (Blocks of 1024
 // traversals, with a quarter of these sets, take the same time.)
 constexpr int kSettleSlots = 512;  // two per thread: the table never fills
+constexpr int kSettleTree = 256;   // paths of one tree up to which k_settle_tree settles them
 
 template <bool BACKUP>
 __global__ __launch_bounds__(256) void k_settle(ForestDev f, const int32_t *paths, const int32_t *path_len,
@@ -110,7 +111,68 @@ __global__ __launch_bounds__(256) void k_settle(ForestDev f, const int32_t *path
     }
 }
 
-// The same for paths that share no node (omk_batch::disjoint): every node has one visitor and nothing has to be atomic
+// The same for paths of one tree (PathsAre::kOneTree), as many as a block has threads: a block takes all visits of a
+// depth, and a node of a tree lies at one depth only, so that nobody else touches what the block has combined.  Nothing is
+// atomic in memory, and the RAVE blend of a node, a function of what its thread has just written, is kept up on the spot
+// (blend; k_blend_paths was a launch of its own for it).  What bounds it is a chain of four trips to memory and the launch.
+// Measured on an MI355X: 48 paths of a young Go tree with RAVE 3.4 and 2.7 us -> 4.1, 64 of a Gomoku tree 3.9 -> 3.6.  The
+// line lies at 256 paths: 500 of a chess-like tree, by blocks of 512 threads, 5.1 -> 5.8.
+template <bool BACKUP>
+__global__ __launch_bounds__(kSettleTree) void k_settle_tree(ForestDev f, const int32_t *paths, const int32_t *path_len,
+                                                             const float *values, int n, int stride, int vl, bool blend,
+                                                             float rave_k) {
+    __shared__ int s_key[2 * kSettleTree];
+    __shared__ int s_cnt[2 * kSettleTree];
+    __shared__ float s_w[BACKUP ? 2 * kSettleTree : 1];
+    constexpr int threads = kSettleTree, slots = 2 * threads;
+    static_assert(slots == 512, "the hash gives nine bits");
+    const int t = threadIdx.x, d = blockIdx.y;
+    const int len = t < n ? path_len[t] : 0;
+    const bool act = d < len;
+    int node = t < n ? paths[(size_t)d * stride + t] : -1;  // (not looked at beyond the path's end)
+    float v = 0.0f;
+    if (BACKUP && t < n) v = values[t];
+    if (__syncthreads_or(act ? 1 : 0) == 0) return;  // nothing this deep
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        s_key[u * threads + t] = -1;
+        s_cnt[u * threads + t] = 0;
+        if (BACKUP) s_w[u * threads + t] = 0.0f;
+    }
+    __syncthreads();
+    if (act) {
+        if ((len - 1 - d) & 1) v = -v;  // the leaf receives +value, every ply up flips it
+        uint32_t h = ((uint32_t)node * 2654435761u) >> 23;
+        for (;;) {
+            const int prev = atomicCAS(&s_key[h], -1, node);
+            if (prev == -1 || prev == node) break;
+            h = (h + 1u) & (uint32_t)(slots - 1);
+        }
+        atomicAdd(&s_cnt[h], 1);
+        if (BACKUP) atomicAdd(&s_w[h], v);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int at = s_key[u * threads + t];
+        if (at < 0) continue;
+        const int cnt = s_cnt[u * threads + t], x = f.VL[at];
+        const int taken = (int)((uint32_t)(BACKUP ? vl + 1 : vl) * (uint32_t)cnt);
+        int left = (int)((uint32_t)x - (uint32_t)taken);  // (as vl_sub_clamp)
+        if (x < taken) left = max(left, 0);
+        if (BACKUP) {
+            const int visits = (int)((uint32_t)f.N[at] + (uint32_t)cnt);
+            const float w = f.W[at] + s_w[u * threads + t];
+            if (vl <= 0) left = x > 0 ? (x > cnt ? x - cnt : 0) : x;  // (as vl_dec_if_positive)
+            f.N[at] = visits;
+            f.W[at] = w;
+            if (blend) f.q2[at] = combined_value(visits, w, f.rN[at], f.rW[at], rave_k);
+        }
+        f.VL[at] = left;
+    }
+}
+
+// The same for paths that share no node (PathsAre::kDisjoint): every node has one visitor and nothing has to be atomic
 // (four atomics a visit, one of them waiting for
 // another: 14 us for the 72 k nodes of 32768 paths, 7.7 us without; of 256 paths of 8 nodes 7.0 and 4.4).
 template <bool BACKUP>
@@ -339,9 +401,11 @@ hipError_t launch_root_noise(const ForestMut &f, int32_t root, const float *nois
 // action occurs among the path's actions gets rN += 1, rW += the node's signed value ----
 constexpr int kRaveMaxLen = 4097;  // longest path the ABI accepts
 
-// One wavefront per (traversal, depth): the path's actions go to LDS, the node's children are
-// spread over the lanes.
-__global__ __launch_bounds__(64) void k_rave_backup(ForestMut f, const int32_t *paths, const int32_t *path_len,
+// One block per (traversal, depth): the path's actions go to LDS, the node's children are spread over the threads.  What bounds
+// it is a chain of trips to memory (length, node, children's range, their actions); a wavefront alone made the last of them
+// six times for the 362 children of a Go node.  48 paths: 6.2 -> 3.8 us.
+constexpr int kRaveThreads = 256;
+__global__ __launch_bounds__(kRaveThreads) void k_rave_backup(ForestMut f, const int32_t *paths, const int32_t *path_len,
                                                     const float *values, int n, int stride) {
     __shared__ int s_pa[kRaveMaxLen];
     const int t = blockIdx.x, d = blockIdx.y, lane = threadIdx.x;
@@ -350,17 +414,18 @@ __global__ __launch_bounds__(64) void k_rave_backup(ForestMut f, const int32_t *
     const int node = paths[(size_t)d * stride + t];
     const int2 sp = f.span[node];
     if (sp.y <= 0) return;
-    for (int e = lane; e < len; e += 64) {
+    for (int e = lane; e < len; e += kRaveThreads) {
         const int pn = paths[(size_t)e * stride + t];
         s_pa[e] = f.action ? f.action[pn] : pn;
     }
     __syncthreads();
     float v = values[t];
     if ((len - 1 - d) & 1) v = -v;  // the leaf's children see +value, every ply up flips it
-    for (int i = lane; i < sp.y; i += 64) {
+    for (int i = lane; i < sp.y; i += kRaveThreads) {
         const int id = sp.x + i;
-        if (f.legal && !((f.legal[(uint32_t)id >> 5] >> ((uint32_t)id & 31u)) & 1u)) continue;
+        const uint32_t word = f.legal ? f.legal[(uint32_t)id >> 5] : ~0u;
         const int a = f.action ? f.action[id] : id;
+        if (!((word >> ((uint32_t)id & 31u)) & 1u)) continue;
         bool hit = false;
         for (int e = 0; e < len && !hit; e++) hit = s_pa[e] != -1 && s_pa[e] == a;
         if (hit) {
@@ -373,7 +438,7 @@ __global__ __launch_bounds__(64) void k_rave_backup(ForestMut f, const int32_t *
 hipError_t launch_rave_backup(const ForestMut &f, const int32_t *paths, const int32_t *path_len, const float *values,
                               int n, int stride, int max_len, hipStream_t s) {
     if (n <= 0 || max_len <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_rave_backup, dim3(n, max_len), dim3(64), 0, s, f, paths, path_len, values, n, stride);
+    hipLaunchKernelGGL(k_rave_backup, dim3(n, max_len), dim3(kRaveThreads), 0, s, f, paths, path_len, values, n, stride);
     return hipGetLastError();
 }
 
@@ -426,28 +491,24 @@ hipError_t launch_apply_vl(const ForestDev &f, const int32_t *paths, const int32
     return hipGetLastError();
 }
 
+static bool settled_by_depth(PathsAre are, int n) { return are == PathsAre::kOneTree && n <= kSettleTree; }
+
 template <bool BACKUP>
 static hipError_t launch_settle(const ForestDev &f, const int32_t *paths, const int32_t *path_len, const float *values,
-                                int n, int stride, int max_len, int vl, bool alone, hipStream_t s) {
+                                int n, int stride, int max_len, int vl, PathsAre are, bool blend, float rave_k,
+                                hipStream_t s) {
     if (n <= 0 || max_len <= 0) return hipSuccess;
     const dim3 grid((n + 255) / 256, max_len), block(256);
-    if (alone)
+    if (settled_by_depth(are, n)) {
+        hipLaunchKernelGGL((k_settle_tree<BACKUP>), dim3(1, max_len), dim3(kSettleTree), 0, s, f, paths, path_len, values, n,
+                           stride, vl, blend && f.q2, rave_k);
+    } else if (are == PathsAre::kDisjoint)
         hipLaunchKernelGGL((k_settle_alone<BACKUP>), grid, block, 0, s, f, paths, path_len, values, n, stride, vl);
     else
         hipLaunchKernelGGL((k_settle<BACKUP>), grid, block, 0, s, f, paths, path_len, values, n, stride, vl);
     return hipGetLastError();
 }
 
-hipError_t launch_revert_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
-                            int max_len, int vl, bool alone, hipStream_t s) {
-    if (vl <= 0) return hipSuccess;
-    return launch_settle<false>(f, paths, path_len, nullptr, n, stride, max_len, vl, alone, s);
-}
-
-hipError_t launch_backup(const ForestDev &f, const int32_t *paths, const int32_t *path_len, const float *values,
-                         int n, int stride, int max_len, int vl, bool alone, hipStream_t s) {
-    return launch_settle<true>(f, paths, path_len, values, n, stride, max_len, vl, alone, s);
-}
 
 // ---- the RAVE blend kept per node ----
 // MCTSNode::getCombinedValue (reference src/mcts/mcts_node.cpp:657-678) is a function of the node's own N, W,
@@ -477,9 +538,16 @@ hipError_t launch_blend_all(const ForestDev &f, float rave_k, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_blend_paths(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
-                              int max_len, float rave_k, hipStream_t s) {
-    if (!f.q2 || n <= 0 || max_len <= 0) return hipSuccess;
+hipError_t launch_revert_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
+                            int max_len, int vl, PathsAre are, hipStream_t s) {
+    if (vl <= 0) return hipSuccess;
+    return launch_settle<false>(f, paths, path_len, nullptr, n, stride, max_len, vl, are, false, 0.0f, s);
+}
+
+hipError_t launch_backup(const ForestDev &f, const int32_t *paths, const int32_t *path_len, const float *values,
+                         int n, int stride, int max_len, int vl, PathsAre are, bool blend, float rave_k, hipStream_t s) {
+    const hipError_t e = launch_settle<true>(f, paths, path_len, values, n, stride, max_len, vl, are, blend, rave_k, s);
+    if (e != hipSuccess || !blend || !f.q2 || n <= 0 || max_len <= 0 || settled_by_depth(are, n)) return e;
     hipLaunchKernelGGL(k_blend_paths, dim3((n + 255) / 256, max_len), dim3(256), 0, s, f, paths, path_len, n, stride,
                        rave_k);
     return hipGetLastError();

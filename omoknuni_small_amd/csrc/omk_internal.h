@@ -172,18 +172,18 @@ template <int RMAX, bool RAVE>
 hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a, int n_items0, int most_visitors, int n_traversals,
                                int n_cus, const LoneOut &out, hipStream_t s);
 
+// What is known of the paths that are settled: no two share a node; all lie in one tree, from one root, so that a node is at
+// one depth of all of them; nothing.
+enum class PathsAre { kDisjoint, kOneTree, kAny };
 hipError_t launch_apply_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                            int max_len, int vl, hipStream_t s);
-// alone: no two of the paths share a node
 hipError_t launch_revert_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
-                            int max_len, int vl, bool alone, hipStream_t s);
+                            int max_len, int vl, PathsAre are, hipStream_t s);
+// blend: the RAVE blend of the nodes on the paths is kept up, for the constant rave_k
 hipError_t launch_backup(const ForestDev &f, const int32_t *paths, const int32_t *path_len, const float *values,
-                         int n, int stride, int max_len, int vl, bool alone, hipStream_t s);
-// The per-node RAVE blend f.q2 from the node's statistics as they are: of every node, or of the nodes on the
-// paths given (after a backup has changed their N and W).
+                         int n, int stride, int max_len, int vl, PathsAre are, bool blend, float rave_k, hipStream_t s);
+// The per-node RAVE blend f.q2 of every node from its statistics as they are.
 hipError_t launch_blend_all(const ForestDev &f, float rave_k, hipStream_t s);
-hipError_t launch_blend_paths(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
-                              int max_len, float rave_k, hipStream_t s);
 
 // Arrays of 32-bit words on the device, read as one stream (omk_link.hip): word start[q] + i of the stream is word
 // i * step[q] of dev[q].

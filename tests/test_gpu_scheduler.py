@@ -381,6 +381,35 @@ def test_crowds_on_both_sides_of_the_wider_teams(fan, rave, m):
     assert st["replayed_nodes"] == 0, st
 
 
+@pytest.mark.parametrize("n", [2, 64, 255, 256, 257])
+@pytest.mark.parametrize("vl,rave", [(3, True), (3, False), (0, True)])
+def test_paths_of_one_tree_are_settled_by_depth(n, vl, rave):
+    """Up to 256 paths from one root are settled by a block a depth without an atomic, and the RAVE blends with them: the
+    statistics, and the next selections, which read the blends, are the checker's.  From two roots, one below the other,
+    a node lies at two depths of the paths, which are settled otherwise."""
+    soa, _ = layered_forest(33, [30, 9, 7, 5], rave=rave)
+    select_both(soa, np.zeros(n, np.int32), 6, vl=vl, rave=rave, steps=3)
+    import omoknuni_small_amd as omk
+    soa, _ = layered_forest(34, [12, 9, 7], rave=rave)
+    f = omk.Forest.from_soa(soa)
+    b = omk.Batch(f, n, 5)
+    b.set_roots(np.where(np.arange(n) % 2 == 0, 0, 1).astype(np.int32))    # node 1 is a child of node 0
+    before = f.download()
+    b.select(omk.SelectParams(c_puct=1.4, virtual_loss=vl, use_rave=rave, rave_k=1000.0))
+    paths, plen, _, _ = b.read()
+    values = (np.random.default_rng(5).integers(-64, 65, n) / 64.0).astype(np.float32)
+    b.set_values(values)
+    b.backup(vl)
+    after = f.download()
+    N, W = before["N"].copy(), before["W"].astype(np.float64)
+    for t in range(n):
+        for d in range(plen[t]):
+            N[paths[t, d]] += 1
+            W[paths[t, d]] += values[t] if (plen[t] - 1 - d) % 2 == 0 else -values[t]
+    assert (after["N"] == N).all()
+    assert np.abs(after["W"] - W).max() <= 1e-3    # at most 257 additions of 1/64ths to sums below 2048: half an ulp, 2^-14, each
+
+
 def test_boundaries_of_heavy_children_are_worked_out_ahead_of_time():
     """A heavy root with heavy children: the children's slice boundaries are queued as items of their own
     (kind 4 in the timeline) while the root is still being settled, the root's own when the roots are set;
