@@ -79,8 +79,11 @@ constexpr int kSortBins = 1 << kSortBits;
 // 194, 176, 195; 4096 Gomoku 181, 207, 199 and 167, 198, 188, Go with RAVE 151, 160, 124 and 142, 164, 129.
 constexpr int kWideTeamMin = 1024;
 static_assert(kWideTeamMin <= kHeavyMin, "what nodes of kHeavyMin visitors need is in that kernel");
-template <bool HEAVY>
-constexpr int kTeamWaves = HEAVY ? 8 : 4;
+// (Eight wavefronts have 256 registers each: the widest class, of sixteen rounds, would keep 735 of its 512 in memory.)
+template <int RMAX, bool HEAVY>
+constexpr bool kWideTeams = HEAVY && RMAX <= 6;
+template <bool WIDE>
+constexpr int kTeamWaves = WIDE ? 8 : 4;
 constexpr int kMostTeamWaves = 8;
 constexpr int kTeamMin = 96;              // batch entries from which the helpers are called in
 // a batch of at most this many entries per thread is ordered by counting: a lone wavefront, the block
@@ -1142,13 +1145,13 @@ __device__ __forceinline__ void active_counts(const ActiveSet<R> &s, float ep, u
 // The visitors settled are those with ranks [rank0, rank0 + todo) of the node's winner
 // order, starting from the state in which child i has had tk0[i] visits already (all zero
 // and rank0 = 0 for a whole node; a slice of a heavy node otherwise).
-template <int R, bool RAVE, bool HEAVY>
+template <int R, bool RAVE, bool WIDE>
 __device__ __forceinline__ bool water_level(const SelectArgs &a, const NodeCtx &c, int lane, const Kids<R, RAVE> &k,
                                             int off, int rank0, int todo, const int (&tk0)[R], WaveLds<R> &lds,
                                             int (&cnt)[R], bool allow_lds, int &lds_cur, bool use_preset,
                                             const int (&preset)[R], uint32_t *order, bool &pending) {
     lds_cur = -1;
-    constexpr int F = R * kWave, kTeam = kTeamWaves<HEAVY> * kWave;
+    constexpr int F = R * kWave, kTeam = kTeamWaves<WIDE> * kWave;
     const uint32_t uvl = (uint32_t)a.vl;
     const int m = todo;
     off += rank0;
@@ -2137,10 +2140,10 @@ __device__ __forceinline__ bool single_run(const SelectArgs &a, const NodeCtx &c
 // dominates, 11.5 a node where a path of their own took 10.3 (1 x 100 of one tree 105 -> 112, 1 x 256 76 -> 82).
 constexpr int kMergeMin = 8;  // visitors from which a contested node is settled that way (5 and 14: the same)
 // buckets a thread adds up: 1152 and 1344 in all
-template <bool HEAVY>
-constexpr int kMergeOwn = HEAVY ? 3 : 6;
-template <bool HEAVY>
-constexpr int kMergeBuckets = (kTeamWaves<HEAVY> - 1) * kWave * kMergeOwn<HEAVY>;
+template <bool WIDE>
+constexpr int kMergeOwn = WIDE ? 3 : 6;
+template <bool WIDE>
+constexpr int kMergeBuckets = (kTeamWaves<WIDE> - 1) * kWave * kMergeOwn<WIDE>;
 constexpr int kMergePasses = 12;
 constexpr int kMergeCount = 32;  // entries of a bucket that are ranked by counting whoever they belong to
 static_assert(2 * kMergeBuckets<true> + 1 + 2 * kBatchCap + 1024 <= kSortBins * (kBatchCap / kWave + 1), "buckets and arrivals fit the sort's table");
@@ -2151,10 +2154,10 @@ static_assert(2 * kMergeBuckets<true> + 1 + 2 * kBatchCap + 1024 <= kSortBins * 
 // chess-like tree 245 -> 238 us a selection, 16384 on the Go tree with RAVE 348 -> 328.
 // t: number of the helper thread.  On success (cmd.merged) order[] holds (child << 21) | visit number of the m visitors and
 // st_j0[] the visits per child.  The owner takes the barriers with them.
-template <int R, bool RAVE, bool HEAVY>
+template <int R, bool RAVE, bool WIDE>
 __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds, uint32_t *order, int t, int m, int goff,
                                            float ep, uint32_t uvl) {
-    constexpr int F = R * kWave, W = kTeamWaves<HEAVY> - 1, NT = W * kWave, OWN = kMergeOwn<HEAVY>, B = kMergeBuckets<HEAVY>;
+    constexpr int F = R * kWave, W = kTeamWaves<WIDE> - 1, NT = W * kWave, OWN = kMergeOwn<WIDE>, B = kMergeBuckets<WIDE>;
     constexpr int K = (F + NT - 1) / NT;  // children of a thread: t, t + NT ..
     const int lane = t & 63, wv = uniform(t >> 6);
     uint64_t *ent = reinterpret_cast<uint64_t *>(lds.key[0]);    // in (child, visit) order; smaller = played earlier
@@ -3093,10 +3096,10 @@ struct Continuation {
 // and walks on, every other returns kStepParked.  Any failed check sends the whole node
 // back to the one-wavefront path.
 //
-// HEAVY: the kernel for batches in which a node of kHeavyMin visitors can occur.  Without it (every root has fewer) the
+// HEAVY: the kernel for batches in which a node of kHeavyMin visitors can occur, and for crowds (kWideTeamMin).  Without it the
 // slices, their boundaries and their joins are left out, and with them registers that the rest of the code then has
-// (scalar spills of the narrow class 331 -> 92, of four rounds 404 -> 190, of six 649 -> 229, whose vector registers go
-// 277 -> 262).
+// (scalar spills of the narrow class 275 -> 92, of four rounds 458 -> 190, of six 556 -> 229, which has 256 vector registers
+// with its teams of eight and ten more in memory).
 template <int R, bool RAVE, int RMAX, bool HEAVY>
 __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs &a, const NodeCtx &c, int lane,
                                             const Item &item, const int32_t *seg_in, int32_t *seg_out,
@@ -3382,7 +3385,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
 #pragma unroll
                             for (int r = 0; r < R; r++) cnt[r] = lds.st_j0[r * kWave + lane];
                         } else {
-                            ok = water_level<R, RAVE, HEAVY>(a, c, lane, k, soff, rank_hi, todo, ct_hi, lds, cnt, false, unused_cur,
+                            ok = water_level<R, RAVE, kWideTeams<RMAX, HEAVY>>(a, c, lane, k, soff, rank_hi, todo, ct_hi, lds, cnt, false, unused_cur,
                                                       preset_ok, between, pl.order, pending);
                         }
                     }
@@ -3440,7 +3443,7 @@ __device__ __forceinline__ int select_group(const ForestDev &f, const SelectArgs
         int zero[R];
 #pragma unroll
         for (int r = 0; r < R; r++) zero[r] = 0;
-        settled = water_level<R, RAVE, HEAVY>(a, c, lane, k, soff, 0, m, zero, lds, cnt, !heavy, lds_cur, false, zero,
+        settled = water_level<R, RAVE, kWideTeams<RMAX, HEAVY>>(a, c, lane, k, soff, 0, m, zero, lds, cnt, !heavy, lds_cur, false, zero,
                                        pl.order, pending);
         if (!settled) st_replay = 1;
     }
@@ -4201,7 +4204,7 @@ template <int R, bool RAVE, int RMAX, bool HEAVY>
 __device__ __forceinline__ void team_help(const ForestDev &f, const SelectArgs &a, WaveLds<R> &lds, PartLds<RMAX> &pl,
                                           int tid, int op, int total, int keep, int goff, int cur, float ep,
                                           uint32_t uvl) {
-    constexpr int kTeam = kTeamWaves<HEAVY> * kWave;
+    constexpr int kTeam = kTeamWaves<kWideTeams<RMAX, HEAVY>> * kWave;
     uint32_t *order = pl.order;
     if (op == kOpPartition) {
         if ((tid >> 6) == 1) partition_async<R, RMAX>(f, a, lds.cmd, pl, tid & 63);
@@ -4231,7 +4234,7 @@ template <int RMAX, bool RAVE>
 __device__ void walkers_loop(ForestDev f, SelectArgs a, int lane);
 
 template <int RMAX, bool RAVE, bool HEAVY>
-__global__ __launch_bounds__(kTeamWaves<HEAVY> * kWave) void k_select_groups(ForestDev f, SelectArgs a) {
+__global__ __launch_bounds__((kTeamWaves<kWideTeams<RMAX, HEAVY>> * kWave)) void k_select_groups(ForestDev f, SelectArgs a) {
     __shared__ WaveLds<RMAX> s_lds;
     __shared__ PartLds<RMAX> s_part;
     const int tid = threadIdx.x;
@@ -4301,9 +4304,9 @@ __global__ __launch_bounds__(kTeamWaves<HEAVY> * kWave) void k_select_groups(For
         if (op == kOpMerge) {
             // (its last barrier ends the request)
             if (rounds == 1)
-                team_merge<1, RAVE, HEAVY>(a, reinterpret_cast<WaveLds<1> &>(s_lds), s_part.order, tid - kWave, total, goff, ep, uvl);
+                team_merge<1, RAVE, kWideTeams<RMAX, HEAVY>>(a, reinterpret_cast<WaveLds<1> &>(s_lds), s_part.order, tid - kWave, total, goff, ep, uvl);
             else
-                team_merge<RMAX, RAVE, HEAVY>(a, s_lds, s_part.order, tid - kWave, total, goff, ep, uvl);
+                team_merge<RMAX, RAVE, kWideTeams<RMAX, HEAVY>>(a, s_lds, s_part.order, tid - kWave, total, goff, ep, uvl);
             continue;
         }
         if (RMAX > 1 && (op == kOpPartition || op == kOpLoad) && (tid >> 6) >= 2 && (!HEAVY || (tid >> 6) <= 3)) {
@@ -4675,8 +4678,8 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_i
         // on the 4 M-node chess-like tree: 0.247 ms a selection with two blocks per unit, 0.222 with one.
         int capacity = n_cus;
         if (capacity < 2) capacity = 2;
-        const bool heavy = most_visitors >= (RMAX > 1 ? kWideTeamMin : kHeavyMin);
-        const int waves = heavy ? kTeamWaves<true> : kTeamWaves<false>;
+        const bool heavy = most_visitors >= (RMAX > 1 && kWideTeams<RMAX, true> ? kWideTeamMin : kHeavyMin);
+        const int waves = heavy ? kTeamWaves<kWideTeams<RMAX, true>> : kTeamWaves<false>;
         int walkers = n_traversals / waves;
         if (walkers > capacity / 4) walkers = capacity / 4;
         if (walkers > kMaxWalkerBlocks) walkers = kMaxWalkerBlocks;  // idle walkers poll: more of them slow the teams
