@@ -54,7 +54,7 @@ __global__ __launch_bounds__(256) void k_apply_vl(ForestDev f, const int32_t *pa
 // (one per wavefront where it sat on one node), 4.5 combined; of 16384 of 9 nodes 29 and 4.6.  (Blocks of 1024
 // traversals, with a quarter of these sets, take the same time.)
 constexpr int kSettleSlots = 512;  // two per thread: the table never fills
-constexpr int kSettleTree = 256;   // paths of one tree up to which k_settle_tree settles them
+constexpr int kSettleTree = 256;   // paths of one tree up to which k_settle_tree backs them up
 
 template <bool BACKUP>
 __global__ __launch_bounds__(256) void k_settle(ForestDev f, const int32_t *paths, const int32_t *path_len,
@@ -111,33 +111,32 @@ __global__ __launch_bounds__(256) void k_settle(ForestDev f, const int32_t *path
     }
 }
 
-// The same for paths of one tree (PathsAre::kOneTree), as many as a block has threads: a block takes all visits of a
-// depth, and a node of a tree lies at one depth only, so that nobody else touches what the block has combined.  Nothing is
-// atomic in memory, and the RAVE blend of a node, a function of what its thread has just written, is kept up on the spot
-// (blend; k_blend_paths was a launch of its own for it).  What bounds it is a chain of four trips to memory and the launch.
-// Measured on an MI355X: 48 paths of a young Go tree with RAVE 3.4 and 2.7 us -> 4.1, 64 of a Gomoku tree 3.9 -> 3.6.  The
-// line lies at 256 paths: 500 of a chess-like tree, by blocks of 512 threads, 5.1 -> 5.8.
-template <bool BACKUP>
+// The backup of paths of one tree (PathsAre::kOneTree), as many as a block has threads, with the RAVE blends of their nodes: a
+// block takes all visits of a depth, and a node of a tree lies at one depth only, so that nobody else touches what the block
+// has combined.  Nothing is atomic in memory, and the blend of a node, a function of what its thread has just written, is kept
+// up on the spot, where it took a launch of its own (k_blend_paths).  What bounds it is a chain of four trips to memory.
+// Measured on an MI355X: 48 paths of a young Go tree with RAVE 3.4 and 2.7 us -> 4.1; a selection and the backup of 64 on a Go
+// tree, three seeds, 57, 60, 61 -> 53, 58, 56.  Without a blend the atomics are the faster ones, although their kernel takes
+// longer (64 paths of a Gomoku tree 3.9 and 3.6 us, a pass 51 and 54): plain stores have to leave the caches between two
+// launches.  The line lies at 256 paths: 500, by blocks of 512 threads, 5.1 -> 5.8.
 __global__ __launch_bounds__(kSettleTree) void k_settle_tree(ForestDev f, const int32_t *paths, const int32_t *path_len,
-                                                             const float *values, int n, int stride, int vl, bool blend,
-                                                             float rave_k) {
-    __shared__ int s_key[2 * kSettleTree];
-    __shared__ int s_cnt[2 * kSettleTree];
-    __shared__ float s_w[BACKUP ? 2 * kSettleTree : 1];
+                                                             const float *values, int n, int stride, int vl, float rave_k) {
     constexpr int threads = kSettleTree, slots = 2 * threads;
     static_assert(slots == 512, "the hash gives nine bits");
+    __shared__ int s_key[slots];
+    __shared__ int s_cnt[slots];
+    __shared__ float s_w[slots];
     const int t = threadIdx.x, d = blockIdx.y;
     const int len = t < n ? path_len[t] : 0;
     const bool act = d < len;
-    int node = t < n ? paths[(size_t)d * stride + t] : -1;  // (not looked at beyond the path's end)
-    float v = 0.0f;
-    if (BACKUP && t < n) v = values[t];
+    const int node = t < n ? paths[(size_t)d * stride + t] : -1;  // (not looked at beyond the path's end)
+    float v = t < n ? values[t] : 0.0f;
     if (__syncthreads_or(act ? 1 : 0) == 0) return;  // nothing this deep
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         s_key[u * threads + t] = -1;
         s_cnt[u * threads + t] = 0;
-        if (BACKUP) s_w[u * threads + t] = 0.0f;
+        s_w[u * threads + t] = 0.0f;
     }
     __syncthreads();
     if (act) {
@@ -149,7 +148,7 @@ __global__ __launch_bounds__(kSettleTree) void k_settle_tree(ForestDev f, const 
             h = (h + 1u) & (uint32_t)(slots - 1);
         }
         atomicAdd(&s_cnt[h], 1);
-        if (BACKUP) atomicAdd(&s_w[h], v);
+        atomicAdd(&s_w[h], v);
     }
     __syncthreads();
 #pragma unroll
@@ -157,18 +156,20 @@ __global__ __launch_bounds__(kSettleTree) void k_settle_tree(ForestDev f, const 
         const int at = s_key[u * threads + t];
         if (at < 0) continue;
         const int cnt = s_cnt[u * threads + t], x = f.VL[at];
-        const int taken = (int)((uint32_t)(BACKUP ? vl + 1 : vl) * (uint32_t)cnt);
-        int left = (int)((uint32_t)x - (uint32_t)taken);  // (as vl_sub_clamp)
-        if (x < taken) left = max(left, 0);
-        if (BACKUP) {
-            const int visits = (int)((uint32_t)f.N[at] + (uint32_t)cnt);
-            const float w = f.W[at] + s_w[u * threads + t];
-            if (vl <= 0) left = x > 0 ? (x > cnt ? x - cnt : 0) : x;  // (as vl_dec_if_positive)
-            f.N[at] = visits;
-            f.W[at] = w;
-            if (blend) f.q2[at] = combined_value(visits, w, f.rN[at], f.rW[at], rave_k);
+        const int visits = (int)((uint32_t)f.N[at] + (uint32_t)cnt);
+        const float w = f.W[at] + s_w[u * threads + t];
+        int left;
+        if (vl > 0) {  // (as vl_sub_clamp)
+            const int taken = (int)((uint32_t)(vl + 1) * (uint32_t)cnt);
+            left = (int)((uint32_t)x - (uint32_t)taken);
+            if (x < taken) left = max(left, 0);
+        } else {  // (as vl_dec_if_positive)
+            left = x > 0 ? (x > cnt ? x - cnt : 0) : x;
         }
+        f.N[at] = visits;
+        f.W[at] = w;
         f.VL[at] = left;
+        f.q2[at] = combined_value(visits, w, f.rN[at], f.rW[at], rave_k);
     }
 }
 
@@ -491,24 +492,17 @@ hipError_t launch_apply_vl(const ForestDev &f, const int32_t *paths, const int32
     return hipGetLastError();
 }
 
-static bool settled_by_depth(PathsAre are, int n) { return are == PathsAre::kOneTree && n <= kSettleTree; }
-
 template <bool BACKUP>
 static hipError_t launch_settle(const ForestDev &f, const int32_t *paths, const int32_t *path_len, const float *values,
-                                int n, int stride, int max_len, int vl, PathsAre are, bool blend, float rave_k,
-                                hipStream_t s) {
+                                int n, int stride, int max_len, int vl, PathsAre are, hipStream_t s) {
     if (n <= 0 || max_len <= 0) return hipSuccess;
     const dim3 grid((n + 255) / 256, max_len), block(256);
-    if (settled_by_depth(are, n)) {
-        hipLaunchKernelGGL((k_settle_tree<BACKUP>), dim3(1, max_len), dim3(kSettleTree), 0, s, f, paths, path_len, values, n,
-                           stride, vl, blend && f.q2, rave_k);
-    } else if (are == PathsAre::kDisjoint)
+    if (are == PathsAre::kDisjoint)
         hipLaunchKernelGGL((k_settle_alone<BACKUP>), grid, block, 0, s, f, paths, path_len, values, n, stride, vl);
     else
         hipLaunchKernelGGL((k_settle<BACKUP>), grid, block, 0, s, f, paths, path_len, values, n, stride, vl);
     return hipGetLastError();
 }
-
 
 // ---- the RAVE blend kept per node ----
 // MCTSNode::getCombinedValue (reference src/mcts/mcts_node.cpp:657-678) is a function of the node's own N, W,
@@ -541,13 +535,19 @@ hipError_t launch_blend_all(const ForestDev &f, float rave_k, hipStream_t s) {
 hipError_t launch_revert_vl(const ForestDev &f, const int32_t *paths, const int32_t *path_len, int n, int stride,
                             int max_len, int vl, PathsAre are, hipStream_t s) {
     if (vl <= 0) return hipSuccess;
-    return launch_settle<false>(f, paths, path_len, nullptr, n, stride, max_len, vl, are, false, 0.0f, s);
+    return launch_settle<false>(f, paths, path_len, nullptr, n, stride, max_len, vl, are, s);
 }
 
 hipError_t launch_backup(const ForestDev &f, const int32_t *paths, const int32_t *path_len, const float *values,
                          int n, int stride, int max_len, int vl, PathsAre are, bool blend, float rave_k, hipStream_t s) {
-    const hipError_t e = launch_settle<true>(f, paths, path_len, values, n, stride, max_len, vl, are, blend, rave_k, s);
-    if (e != hipSuccess || !blend || !f.q2 || n <= 0 || max_len <= 0 || settled_by_depth(are, n)) return e;
+    blend = blend && f.q2 && n > 0 && max_len > 0;
+    if (blend && are == PathsAre::kOneTree && n <= kSettleTree) {
+        hipLaunchKernelGGL(k_settle_tree, dim3(1, max_len), dim3(kSettleTree), 0, s, f, paths, path_len, values, n, stride, vl,
+                           rave_k);
+        return hipGetLastError();
+    }
+    const hipError_t e = launch_settle<true>(f, paths, path_len, values, n, stride, max_len, vl, are, s);
+    if (e != hipSuccess || !blend) return e;
     hipLaunchKernelGGL(k_blend_paths, dim3((n + 255) / 256, max_len), dim3(256), 0, s, f, paths, path_len, n, stride,
                        rave_k);
     return hipGetLastError();
