@@ -117,8 +117,8 @@ __global__ __launch_bounds__(256) void k_settle(ForestDev f, const int32_t *path
 // up on the spot, where it took a launch of its own (k_blend_paths).  What bounds it is a chain of four trips to memory.
 // Measured on an MI355X: 48 paths of a young Go tree with RAVE 3.4 and 2.7 us -> 4.1; a selection and the backup of 64 on a Go
 // tree, three seeds, 57, 60, 61 -> 53, 58, 56.  Without a blend the atomics are the faster ones, although their kernel takes
-// longer (64 paths of a Gomoku tree 3.9 and 3.6 us, a pass 51 and 54): plain stores have to leave the caches between two
-// launches.  The line lies at 256 paths: 500, by blocks of 512 threads, 5.1 -> 5.8.
+// longer (64 paths of a Gomoku tree 3.9 and 3.6 us, a pass with the plain stores 0 to 2 us longer over nine shapes): these have
+// to leave the caches between two launches.  The line lies at 256 paths: 500, by blocks of 512 threads, 5.1 -> 5.8.
 __global__ __launch_bounds__(kSettleTree) void k_settle_tree(ForestDev f, const int32_t *paths, const int32_t *path_len,
                                                              const float *values, int n, int stride, int vl, float rave_k) {
     constexpr int threads = kSettleTree, slots = 2 * threads;
