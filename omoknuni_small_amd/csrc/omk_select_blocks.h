@@ -653,6 +653,9 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                 auto bound = [&](int r, bool in) {
                     const float c = score_ceiling<RAVE>(k.n[r], k.w[r], k.p[r], k.vl[r], k.q2[r], ep);
                     odd = fmaf(c, 0.0f, odd);  // not a number from the first value on that is not finite
+                    // (an unvisited child's score does not look at its sum, its later ones do: when those of the first scan run
+                    // out, the blends of the second must not decide)
+                    if (RAVE) odd = fmaf(k.w[r], 0.0f, odd);
                     in = in && ((word[r] >> ((uint32_t)(cb + r * kWave + lane) & 31u)) & 1u);
                     ceil[r] = in ? c : -__builtin_inff();
                     c2 = __builtin_amdgcn_fmed3f(c1, c2, ceil[r]);

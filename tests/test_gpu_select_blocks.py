@@ -4,7 +4,7 @@ real score; and of the rows the blocks send to the host themselves."""
 import numpy as np
 import pytest
 
-from helpers import random_tree
+from helpers import random_tree, star
 from oracle import ref_cpu as R
 from test_gpu_scheduler import layered_forest
 
@@ -144,6 +144,17 @@ def test_scores_that_are_not_real_and_ties(kind, rave):
     elif kind == "all equal":
         soa["N"][:], soa["W"][:], soa["P"][:] = 1, 0.5, 0.25
     both(soa, np.repeat(roots, 20).astype(np.int32), 8, vl=0 if kind == "no virtual loss" else 2, rave=rave, steps=1)
+
+
+@pytest.mark.parametrize("visitors", [1, 2, 3, 4, 20, 64])
+@pytest.mark.parametrize("fan", [2, 5, 63, 70])
+def test_unvisited_children_whose_sums_are_not_finite(visitors, fan):
+    """A child nobody has visited is scored without its sum, and with it from its first visitor on: where no sum is finite
+    the first scan has a real score for the first `fan` visitors only, and the others take the least visited child, although
+    the RAVE blends of the second scan stay real."""
+    for bad in (np.nan, np.inf, -np.inf):
+        soa = star(200, [[0, bad, 7.1e-8 * (1 + i / 1000), 0, 10, 5] for i in range(fan)], rave=True)
+        both(soa, np.zeros(visitors, np.int32), 2, rave=True, steps=1)
 
 
 def test_widening_at_the_selection():
