@@ -42,6 +42,10 @@ struct BlockScratch {
     uint32_t order[kWave];   // per visitor: listed child << 16 | number of the visit
 };
 
+// The ceiling of a lane without a child: the least finite number, so that the sum that looks for others passes over it.  Children
+// are listed from kLeastScore on at the lowest, which no lane without a child reaches; what lies below is left to the serial loop.
+constexpr float kNoChild = -3.402823466e38f, kLeastScore = -3.0e38f;
+
 template <int RMAX, bool ROWS>
 struct BlockLds {
     int head, tail, open;  // tickets taken, items handed out, visitors that have not reached their leaf
@@ -647,17 +651,17 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                 __builtin_amdgcn_s_waitcnt(0x0F70);
                 const float ep = __int_as_float(uniform(__float_as_int(ep_ahead)));
                 // ---- no child's score is above ceil[] (score_ceiling): the lane's two highest ----
-                float ceil[RMAX], c1 = -__builtin_inff(), c2 = -__builtin_inff(), odd = 0.0f;
+                float ceil[RMAX], c1 = kNoChild, c2 = kNoChild, odd = 0.0f;
                 int r1 = 0, tn = 0, tvl = 0, tx = 0, ty = 0;  // the highest: its round and statistics
                 float tw = 0.0f, tp = 0.0f, tq2 = 0.0f;
                 auto bound = [&](int r, bool in) {
-                    const float c = score_ceiling<RAVE>(k.n[r], k.w[r], k.p[r], k.vl[r], k.q2[r], ep);
-                    odd = fmaf(c, 0.0f, odd);  // not a number from the first value on that is not finite
+                    float c = score_ceiling<RAVE>(k.n[r], k.w[r], k.p[r], k.vl[r], k.q2[r], ep);
                     // (an unvisited child's score does not look at its sum, its later ones do: when those of the first scan run
                     // out, the blends of the second must not decide)
-                    if (RAVE) odd = fmaf(k.w[r], 0.0f, odd);
+                    if (RAVE) c = fmaf(k.w[r], 0.0f, c);
+                    odd = fmaf(c, 0.0f, odd);  // not a number from the first value on that is not finite
                     in = in && ((word[r] >> ((uint32_t)(cb + r * kWave + lane) & 31u)) & 1u);
-                    ceil[r] = in ? c : -__builtin_inff();
+                    ceil[r] = in ? c : kNoChild;
                     c2 = __builtin_amdgcn_fmed3f(c1, c2, ceil[r]);
                     const bool up = ceil[r] > c1;
                     r1 = up ? r : r1;
@@ -676,7 +680,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                 } else {
 #pragma unroll
                     for (int r = 0; r < RMAX; r++) {
-                        ceil[r] = -__builtin_inff();
+                        ceil[r] = kNoChild;
                         if (r * kWave < nelig) bound(r, r * kWave + lane < nelig);  // uniform
                     }
                 }
@@ -689,8 +693,14 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                 const uint64_t in_order = __ballot(together || in_order_at_once(tn, tw, tp, tvl, ep, uvl, j_last));
                 const uint32_t lane_top = ordered_bits(c1), top = (uint32_t)uniform((int)wave_max_all(lane_top));
                 const uint64_t tops = __ballot(lane_top == top);
+                if (__builtin_expect_with_probability(__ballot(!(odd == 0.0f)) != 0ull, 0, 0.999)) {
+                    // (not of what stands in an empty slot: in the loop above that would put up to 61 registers into memory)
+                    odd = 0.0f;
+#pragma unroll
+                    for (int r = 0; r < RMAX; r++) odd = fmaf(ceil[r], 0.0f, odd);
+                }
                 serial = true;
-                if (__builtin_expect_with_probability(__ballot(!(odd == 0.0f)) == 0ull && top != ordered_bits(-__builtin_inff()), 1, 0.999)) {
+                if (__builtin_expect_with_probability(__ballot(!(odd == 0.0f)) == 0ull && top > ordered_bits(kLeastScore), 1, 0.999)) {
                     // ---- does that child win every time?  Its last entry comes before every other child's next one ----
                     const int bl = __ffsll((long long)tops) - 1;
                     const float last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lane_last), bl));
@@ -709,7 +719,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                         // ---- the children that can be chosen, one per lane: no other has a score of `from` or more, and m
                         // entries of these have (that child's, or, where too many would be left, the heads of m) ----
                         const float first = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lane_first), bl));
-                        float from = last < first ? last : first;
+                        float from = fmaxf(last < first ? last : first, kLeastScore);
                         const bool few = together || m <= kPickFew;
                         // (a lane's highest child is the only one of its that can: nothing needs to be moved)
                         const bool direct = __ballot(c2 >= from) == 0ull;

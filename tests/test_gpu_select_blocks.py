@@ -157,6 +157,26 @@ def test_unvisited_children_whose_sums_are_not_finite(visitors, fan):
         both(soa, np.zeros(visitors, np.int32), 2, rave=True, steps=1)
 
 
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("field", ["P", "W"])
+@pytest.mark.parametrize("fan,rave", [(9, False), (225, False), (362, True)])
+def test_empty_slots_whose_values_are_not_finite(fan, rave, field, value):
+    """What stands in a slot without a legal move is looked at by nobody: crowds and lone visitors are settled as if it were
+    zero there, and no more of them one after the other."""
+    soa, roots = layered_forest(fan + rave, [fan, 20, 4], n_trees=3, rave=rave)
+    n = len(soa["N"])
+    legal = np.random.default_rng(fan).random((n + 31) // 32 * 32) < 0.6
+    legal[roots] = True
+    legal[soa["child_begin"][soa["child_count"] > 0]] = True
+    soa["legal"] = np.packbits(legal.reshape(-1, 32), axis=1, bitorder="little").view("<u4").reshape(-1).copy()
+    sums = []
+    for v in (0.0, value):
+        soa[field] = np.where(legal[:n], soa[field], np.float32(v)).astype(np.float32)
+        st = both(soa, np.repeat(roots, [64, 1, 9]).astype(np.int32), 6, rave=rave, count=True)
+        sums.append({k: c for k, c in st.items() if not k.startswith("t_")})
+    assert sums[0] == sums[1] and sums[1]["settled_one_by_one"] == 0, sums
+
+
 def test_widening_at_the_selection():
     soa, roots = random_tree(21, n_expand=80, fanout=(2, 200), max_depth=7, n_roots=9, sort_prior=True, n_max=400)
     both(soa, np.repeat(roots, [1, 2, 5, 9, 16, 33, 48, 63, 64]).astype(np.int32), 8, pw=True)
