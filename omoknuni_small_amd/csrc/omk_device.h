@@ -124,21 +124,21 @@ __device__ __forceinline__ uint32_t ordered_bits(float x) {
     return b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);
 }
 
-// No score of the child is above this (score_about; v_rcp_f32 is within one unit in the last place) ..
+// No score of the child is above this and kBoundTiny (score_about; v_rcp_f32 is within one unit in the last place) ..
 template <bool RAVE>
 __device__ __forceinline__ float score_ceiling(int n, float w, float p, int vl, float q2, float ep) {
     const float x = (float)(int)((uint32_t)n + (uint32_t)vl);
     float s, size;
     score_about<RAVE>(n, w, p, vl, q2, ep, __builtin_amdgcn_rcpf(x), __builtin_amdgcn_rcpf(1.0f + x), s, size);
-    return fmaf(size, kBoundSlack, s);
+    return ceiling_of(s, size);
 }
-// .. and none below this.  (The term for what underflows is on this side only: floors are few.)
+// .. and none below this.
 template <bool RAVE>
 __device__ __forceinline__ float score_floor(int n, float w, float p, int vl, float q2, float ep) {
     const float x = (float)(int)((uint32_t)n + (uint32_t)vl);
     float s, size;
     score_about<RAVE>(n, w, p, vl, q2, ep, __builtin_amdgcn_rcpf(x), __builtin_amdgcn_rcpf(1.0f + x), s, size);
-    return fmaf(size, -kBoundSlack, s) - 1.0e-37f;
+    return floor_of(s, size);
 }
 
 // Results for a host that polls: pinned memory is written with stores of system scope, which go past the L2 of

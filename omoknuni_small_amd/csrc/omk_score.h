@@ -123,9 +123,10 @@ OMK_HD bool keys_provably_monotone(int n, float w, float p, int vl0, float q2, f
 // Bounds of a child's score (the larger of its two candidates), for a caller that has approximate reciprocals rx of
 // float(ev) and r1 of 1 + float(ev), each within two units in its last place, where child_keys divides.  With a numerator
 // rounded as there, each quotient is off by less than 2^-21 of itself, the rounding of the sums and of a second scan's
-// own divisor included; the slack is eight times that of both terms together, and a term of the size of the smallest
-// normal numbers for quotients that underflow.  What is not finite gives bounds that are not finite.
+// own divisor included; the slack is eight times that of both terms together.  Quotients that underflow are off by up to a few
+// units of 2^-149 instead, which kBoundTiny covers.  What is not finite gives bounds that are not finite.
 constexpr float kBoundSlack = 3.814697265625e-6f;  // 2^-18
+constexpr float kBoundTiny = 1.0e-37f;
 template <bool RAVE>
 OMK_HD void score_about(int n, float w, float p, int vl, float q2, float ep, float rx, float r1, float &s, float &size) {
     const int ev = (int)((uint32_t)n + (uint32_t)vl);
@@ -139,6 +140,13 @@ OMK_HD void score_about(int n, float w, float p, int vl, float q2, float ep, flo
         size = size2 > size ? size2 : size;
     }
 }
+
+// No score is above the ceiling and kBoundTiny (ceilings are many, and few of them need it), none below the floor, which is
+// lower by twice that: what lies above it still does where kBoundTiny is added to it.
+OMK_HD float ceiling_of(float s, float size) { return fmaf(size, kBoundSlack, s); }
+OMK_HD float floor_of(float s, float size) { return fmaf(size, -kBoundSlack, s) - 2.0f * kBoundTiny; }
+// Children whose ceiling is below `from` have no entry above this key; the child from whose floor on they are ruled out has.
+OMK_HD uint32_t floor_key_of(float from) { return score_key(from + kBoundTiny) - 1u; }
 
 // keys_provably_monotone for the children most nodes turn on: values that stay positive, counts well within what binary32
 // holds exactly.  (The caller knows that q2 is finite.)

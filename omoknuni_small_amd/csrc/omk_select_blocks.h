@@ -131,7 +131,7 @@ __device__ __forceinline__ bool merge_rest(BlockScratch<RMAX> &s, int n0, int m,
                 if (RAVE) cq2 = s.q2[lane];
             }
             // (its next entry is not above `head`)
-            float head = score_ceiling<RAVE>(cn, cw, cp, cvl, cq2, ep);
+            float head = score_ceiling<RAVE>(cn, cw, cp, cvl, cq2, ep) + kBoundTiny;
             if (!mine) head = -__builtin_inff();
             auto entries_from = [&](uint32_t key) {
                 const float tau = key_score(key);
@@ -762,7 +762,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                             }
                             wave_sync_memory();
                         }
-                        const uint32_t floor_key = score_key(from) - 1u;
+                        const uint32_t floor_key = floor_key_of(from);
                         if (direct && !few) {
                             const bool in = c1 >= from;
                             int cl = 0;  // (in child order, which the merge goes by where keys are equal)

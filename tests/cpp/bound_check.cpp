@@ -1,8 +1,9 @@
 // Host check of the bounds by which the selection rules children out without dividing (score_about, in_order_at_once,
-// csrc/omk_score.h): with reciprocals off by up to a unit in the last place either way the exact score (child_keys) lies
+// csrc/omk_score.h): with reciprocals off by up to two units in the last place either way the exact score (child_keys) lies
 // between floor and ceiling, and what in_order_at_once says keys_provably_monotone says too.  Inputs over their whole
 // range: counts to 2^31, sums and priors of any magnitude, blends, children without visits, values that are not finite.
 //   bound_check [cases [seed]]
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -12,8 +13,9 @@
 using namespace omk;
 
 static float off(float x, std::mt19937_64 &rng) {
-    const int by = (int)(rng() % 3) - 1;
-    return by == 0 || !std::isfinite(x) ? x : std::nextafter(x, by < 0 ? -INFINITY : INFINITY);
+    for (int by = (int)(rng() % 5) - 2; by != 0 && std::isfinite(x); by += by < 0 ? 1 : -1)
+        x = std::nextafter(x, by < 0 ? -INFINITY : INFINITY);
+    return x;
 }
 
 template <bool RAVE>
@@ -33,14 +35,23 @@ static long run(long cases, uint64_t seed, long *decided) {
         if (rng() % 50 == 0) (rng() % 2 ? w : p) = rng() % 3 == 0 ? NAN : rng() % 2 ? INFINITY : -INFINITY;
         if (rng() % 50 == 0) w = std::ldexp(w, 100);
         if (rng() % 50 == 0) p = std::ldexp(p, -140);
+        if (rng() % 50 == 0) {  // nothing but quotients that underflow
+            w = rng() % 2 ? 0.0f : std::ldexp((float)(rng() % 64), -149);
+            p = std::ldexp((float)(rng() % 64), -149);
+            q2 = 0.0f;
+            ep = (float)(1 + rng() % 40);
+        }
         const float x = (float)(int)((uint32_t)n + (uint32_t)vl);
         float s, size;
         score_about<RAVE>(n, w, p, vl, q2, ep, off(1.0f / x, rng), off(1.0f / (1.0f + x), rng), s, size);
-        const float ceiling = std::fma(size, kBoundSlack, s), floor = std::fma(size, -kBoundSlack, s) - 1.0e-37f;
+        const float ceiling = ceiling_of(s, size), floor = floor_of(s, size);
         if (!(ceiling * 0.0f == 0.0f)) continue;  // not finite: settled without the bounds
         uint32_t k1, k2;
         child_keys<RAVE>(n, w, p, vl, q2, ep, k1, k2);
-        const uint32_t key = k1 > k2 ? k1 : k2, lo = score_key(floor), hi = score_key(ceiling + 1.0e-37f);
+        // a child that is ruled out by the least `from` above its ceiling has no entry above the floor that goes with it; one
+        // from whose floor on others are listed is above the floor that goes with that; and none is above the ceiling and kBoundTiny
+        const uint32_t key = k1 > k2 ? k1 : k2, lo = floor_key_of(floor) + 1u;
+        const uint32_t hi = std::min(floor_key_of(std::nextafter(ceiling, INFINITY)), score_key(ceiling + kBoundTiny));
         (*decided)++;
         if (k1 == 0u || key < lo || key > hi) {
             if (++bad < 5) printf("outside: rave %d n %d vl %d w %a p %a q2 %a ep %a: %08x not in %08x .. %08x\n", (int)RAVE, n, vl, w, p, q2, ep, key, lo, hi);

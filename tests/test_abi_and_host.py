@@ -205,7 +205,7 @@ def test_merge_rules_against_the_serial_loop(tmp_path):
 
 def test_bounds_of_scores_hold_the_exact_ones(tmp_path):
     """Children are ruled out by bounds worked out with approximate reciprocals (score_about): over the whole range of counts,
-    sums, priors and blends, with reciprocals off by a unit in the last place either way, the exact score lies between them
+    sums, priors and blends, with reciprocals off by two units in the last place either way, the exact score lies between them
     (tests/cpp/bound_check.cpp)."""
     import re
     import subprocess

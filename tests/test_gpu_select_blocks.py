@@ -126,7 +126,8 @@ def test_scores_closer_than_their_bounds(visitors, fan, rave):
     both(soa, np.repeat(roots, [visitors, 1, max(1, visitors - 1), visitors]).astype(np.int32), 6, rave=rave)
 
 
-@pytest.mark.parametrize("kind", ["nan prior", "nan sum", "-inf sum", "inf sum of the unvisited", "no virtual loss", "all equal"])
+@pytest.mark.parametrize("kind", ["nan prior", "nan sum", "-inf sum", "inf sum of the unvisited", "no virtual loss", "all equal",
+                                  "next to nothing"])
 @pytest.mark.parametrize("rave", [False, True])
 def test_scores_that_are_not_real_and_ties(kind, rave):
     soa, roots = random_tree(11, n_expand=60, fanout=(2, 130), max_depth=6, n_roots=6, rave=rave, n_max=30)
@@ -143,6 +144,10 @@ def test_scores_that_are_not_real_and_ties(kind, rave):
         soa["W"][some & (soa["N"] == 0)] = np.inf
     elif kind == "all equal":
         soa["N"][:], soa["W"][:], soa["P"][:] = 1, 0.5, 0.25
+    elif kind == "next to nothing":  # quotients that underflow, which the bounds cannot tell apart
+        soa["W"][:], soa["P"] = 0.0, (rng.integers(0, 64, len(some)) * 2.0 ** -149).astype(np.float32)
+        if rave:
+            soa["rW"][:] = 0.0
     both(soa, np.repeat(roots, 20).astype(np.int32), 8, vl=0 if kind == "no virtual loss" else 2, rave=rave, steps=1)
 
 
