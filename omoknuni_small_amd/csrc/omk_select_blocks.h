@@ -480,7 +480,7 @@ __device__ __forceinline__ bool pick_few(uint32_t *order, bool mine, int child, 
             entry_key<1, RAVE>(cn, cw, cp, cvl, cq2, ep, uvl, visits + g, 0, key[g], pos[g]);
             key[g] = mine ? key[g] : 0u;
         }
-        if (__ballot(comes_before(key[1], pos[1], key[0], pos[0]))) return false;
+        if (__ballot(mine && comes_before(key[1], pos[1], key[0], pos[0]))) return false;
         int used = 0;
         for (bool left = true; left && done < m; done++) {
             const uint32_t top = (uint32_t)uniform((int)wave_max_all(key[0]));

@@ -182,6 +182,19 @@ def test_empty_slots_whose_values_are_not_finite(fan, rave, field, value):
     assert sums[0] == sums[1] and sums[1]["settled_one_by_one"] == 0, sums
 
 
+@pytest.mark.parametrize("visitors", [2, 3])
+@pytest.mark.parametrize("fan", [3, 64, 65, 130, 380])
+def test_few_visitors_look_at_the_listed_children_only(fan, visitors):
+    """Two or three visitors who split between the first and the last child (from 65 children on of one lane, or of two); the
+    others are ruled out, and that one of them would do better with every visit is no reason to replay the node."""
+    kids = [[100, 90.0, 0.3, 0, 0, 0.0]] + [[0, 10.0, 0.0, 0, 100, 1.0]] * (fan - 2) + [[100, 90.0, 0.3, 0, 0, 0.0]]
+    for last in (fan - 1, 64):  # the same lane and the next one, or the last
+        if last < fan:
+            kids[fan - 1], kids[last] = kids[last], kids[fan - 1]
+            st = both(star(400, kids, rave=True), np.zeros(visitors, np.int32), 2, rave=True, steps=1, count=True)
+            assert st["replayed_nodes"] == 0 and st["settled_one_by_one"] == 0, st
+
+
 def test_widening_at_the_selection():
     soa, roots = random_tree(21, n_expand=80, fanout=(2, 200), max_depth=7, n_roots=9, sort_prior=True, n_max=400)
     both(soa, np.repeat(roots, [1, 2, 5, 9, 16, 33, 48, 63, 64]).astype(np.int32), 8, pw=True)
