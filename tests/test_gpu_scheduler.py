@@ -383,31 +383,49 @@ def test_crowds_on_both_sides_of_the_wider_teams(fan, rave, m):
 
 @pytest.mark.parametrize("n", [2, 64, 255, 256, 257])
 @pytest.mark.parametrize("vl,rave", [(3, True), (3, False), (0, True)])
-def test_paths_of_one_tree_are_settled_by_depth(n, vl, rave):
-    """Up to 256 paths from one root are settled by a block a depth without an atomic, and the RAVE blends with them: the
-    statistics, and the next selections, which read the blends, are the checker's.  From two roots, one below the other,
-    a node lies at two depths of the paths, which are settled otherwise."""
-    soa, _ = layered_forest(33, [30, 9, 7, 5], rave=rave)
-    select_both(soa, np.zeros(n, np.int32), 6, vl=vl, rave=rave, steps=3)
+@pytest.mark.parametrize("trees", [1, 2])
+def test_paths_of_one_tree_are_settled_by_depth(n, vl, rave, trees):
+    """With RAVE up to 256 paths from one root are settled by a block a depth without an atomic, and the blends with them;
+    more of them, paths from two roots and paths without RAVE with atomics.  Statistics (sums of 64ths below 2^18, exact in
+    any order), and the next selections, which read the blends, are the checker's; and after these paths of the caller's,
+    where a node lies at several depths."""
+    import torch
     import omoknuni_small_amd as omk
-    soa, _ = layered_forest(34, [12, 9, 7], rave=rave)
+    soa, roots = layered_forest(33, [30, 9, 7, 5], n_trees=trees, rave=rave)
+    soa["W"] = (np.round(soa["W"] * 64.0) / 64.0).astype(np.float32)
+    assert np.abs(soa["W"]).max() + 4 * n < 2 ** 18
+    ref = R.RefTree.from_soa(soa)
+    rp = R.make_params(c_puct=1.4, virtual_loss=vl, use_rave=rave, rave_k=1000.0, max_depth=6)
     f = omk.Forest.from_soa(soa)
-    b = omk.Batch(f, n, 5)
-    b.set_roots(np.where(np.arange(n) % 2 == 0, 0, 1).astype(np.int32))    # node 1 is a child of node 0
-    before = f.download()
-    b.select(omk.SelectParams(c_puct=1.4, virtual_loss=vl, use_rave=rave, rave_k=1000.0))
-    paths, plen, _, _ = b.read()
-    values = (np.random.default_rng(5).integers(-64, 65, n) / 64.0).astype(np.float32)
-    b.set_values(values)
-    b.backup(vl)
-    after = f.download()
-    N, W = before["N"].copy(), before["W"].astype(np.float64)
-    for t in range(n):
-        for d in range(plen[t]):
-            N[paths[t, d]] += 1
-            W[paths[t, d]] += values[t] if (plen[t] - 1 - d) % 2 == 0 else -values[t]
-    assert (after["N"] == N).all()
-    assert np.abs(after["W"] - W).max() <= 1e-3    # at most 257 additions of 1/64ths to sums below 2048: half an ulp, 2^-14, each
+    b = omk.Batch(f, n, 6)
+    troots = roots[np.arange(n) % trees].astype(np.int32)
+    b.set_roots(troots)
+    rng = np.random.default_rng(n)
+
+    def held():
+        got = f.download()
+        assert (got["N"] == ref.N).all() and (got["VL"] == ref.VL).all() and (got["W"] == ref.W).all()
+
+    for step in range(4):
+        rpaths, rlen, _, _ = ref.select_batch(troots, rp, near_ties=False)
+        b.select(omk.SelectParams(c_puct=1.4, virtual_loss=vl, use_rave=rave, rave_k=1000.0))
+        paths, plen, _, _ = b.read()
+        assert (paths == rpaths).all() and (plen == rlen).all(), step
+        values = (rng.integers(-64, 65, n) / 64.0).astype(np.float32)
+        ref.backup_batch(rpaths, rlen, values, vl)
+        b.set_values(values)
+        b.backup(vl)
+        held()
+        if step == 1:
+            rows = np.stack([rng.permutation(12)[:5] for _ in range(n)]).astype(np.int32)  # (the root and some children)
+            lens = rng.integers(1, 6, n).astype(np.int32)
+            rows[np.arange(5)[None, :] >= lens[:, None]] = -1
+            assert n == 2 or any(len(set(np.nonzero(rows == v)[1])) > 1 for v in range(12))
+            ref.backup_batch(rows, lens, values, vl)
+            d = [torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (rows.T, lens, values)]
+            torch.cuda.synchronize()
+            f.backup_paths(d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), n, n, 5, vl)
+            held()
 
 
 def test_boundaries_of_heavy_children_are_worked_out_ahead_of_time():
