@@ -389,7 +389,6 @@ def test_paths_of_one_tree_are_settled_by_depth(n, vl, rave, trees):
     more of them, paths from two roots and paths without RAVE with atomics.  Statistics (sums of 64ths below 2^18, exact in
     any order), and the next selections, which read the blends, are the checker's; and after these paths of the caller's,
     where a node lies at several depths."""
-    import torch
     import omoknuni_small_amd as omk
     soa, roots = layered_forest(33, [30, 9, 7, 5], n_trees=trees, rave=rave)
     soa["W"] = (np.round(soa["W"] * 64.0) / 64.0).astype(np.float32)
@@ -422,10 +421,14 @@ def test_paths_of_one_tree_are_settled_by_depth(n, vl, rave, trees):
             rows[np.arange(5)[None, :] >= lens[:, None]] = -1
             assert n == 2 or any(len(set(np.nonzero(rows == v)[1])) > 1 for v in range(12))
             ref.backup_batch(rows, lens, values, vl)
-            d = [torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (rows.T, lens, values)]
-            torch.cuda.synchronize()
-            f.backup_paths(d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), n, n, 5, vl)
+            arrays = [np.ascontiguousarray(rows.T), lens, values]
+            d = [f.dev_alloc(x.nbytes) for x in arrays]
+            for at, x in zip(d, arrays):
+                f.h2d(at, x)
+            f.backup_paths(*d, n, n, 5, vl)
             held()
+            for at in d:
+                f.dev_free(at)
 
 
 def test_boundaries_of_heavy_children_are_worked_out_ahead_of_time():
