@@ -30,7 +30,6 @@ struct BlockItem {
 };
 
 // What a wavefront settles a node in: the children that matter, one per lane, in child order.
-template <int RMAX>
 struct BlockScratch {
     int child[kWave];  // index in the node
     int n[kWave], vl[kWave], sx[kWave], sy[kWave];
@@ -46,7 +45,7 @@ struct BlockScratch {
 // are listed from kLeastScore on at the lowest, which no lane without a child reaches; what lies below is left to the serial loop.
 constexpr float kNoChild = -3.402823466e38f, kLeastScore = -3.0e38f;
 
-template <int RMAX, bool ROWS>
+template <bool ROWS>
 struct BlockLds {
     int head, tail, open;  // tickets taken, items handed out, visitors that have not reached their leaf
     int ready[kBlockVisitors];  // item i lies in slot i once this is i + 1.  A block hands out at most kBlockVisitors items in
@@ -60,20 +59,8 @@ struct BlockLds {
     int len[ROWS ? kBlockVisitors : 1], leaf[ROWS ? kBlockVisitors : 1], kids[ROWS ? kBlockVisitors : 1],
         visits[ROWS ? kBlockVisitors : 1];
     int path[ROWS ? kBlockVisitors : 1][kBlockDepth + 2];
-    BlockScratch<RMAX> scratch[kBlockWaves];
+    BlockScratch scratch[kBlockWaves];
 };
-
-// (key, position) of the best of per-lane candidates, like wave_best; without the scalar unit until the end.
-__device__ __forceinline__ void wave_best_fast(uint32_t bk, uint32_t bpos, uint32_t &mk, uint32_t &mpos) {
-    const uint32_t top = wave_max_all(bk);
-    uint64_t tie = __ballot(bk == top);
-    mk = (uint32_t)uniform((int)top);
-    if (tie & (tie - 1ull)) {
-        mpos = wave_min_u32(bk == top ? bpos : 0xFFFFFFFFu);
-        return;
-    }
-    mpos = (uint32_t)__builtin_amdgcn_readlane((int)bpos, __ffsll((long long)tie) - 1);
-}
 
 // A contested node: m visitors over the n0 children listed in `s`, one per lane.  order[q] receives the listed child and the
 // number of its visit for every visitor, `visits` the visits of the lane's child.  The score a child shows its j-th visitor of
@@ -91,8 +78,8 @@ __device__ __forceinline__ void wave_best_fast(uint32_t bk, uint32_t bpos, uint3
 // lie at or above a threshold with enough of them, and one more (merge_rest; team_merge).  40 visitors of a Gomoku node, 25
 // passes before: 23 -> 6.5 us; 16 of a Go node, 8 passes: 12 -> 6.
 
-template <int RMAX, bool RAVE>
-__device__ __forceinline__ bool merge_rest(BlockScratch<RMAX> &s, int n0, int m, float ep, uint32_t uvl,
+template <bool RAVE>
+__device__ __forceinline__ bool merge_rest(BlockScratch &s, int n0, int m, float ep, uint32_t uvl,
                                            uint32_t floor_key, int lane, int done, int &visits) {
     constexpr int kSlots = 2 * kWave;
     constexpr int kScaled = 16;  // children up to which a threshold is not looked for where 128 entries are not enough
@@ -105,7 +92,7 @@ __device__ __forceinline__ bool merge_rest(BlockScratch<RMAX> &s, int n0, int m,
         // many as a threshold says.
         const int log_need = need <= 1 ? 0 : 32 - __clz(need - 1), log_room = n0 <= 1 ? 7 : 7 - (32 - __clz(n0 - 1));
         const int log_e = log_need < log_room ? log_need : log_room;
-        const bool all = log_need <= log_room, even = all;
+        const bool all = log_need <= log_room;
         int total = n0 << log_e, c = 1 << log_e, start = lane << log_e;  // slots in all; the lane's child's
         c = c < need ? c : need;
         uint32_t bk = 0u, bl = ~0u;  // the first entry behind which one may be missing
@@ -117,7 +104,7 @@ __device__ __forceinline__ bool merge_rest(BlockScratch<RMAX> &s, int n0, int m,
             if (h == 0) return 63 - __clzll((long long)(m0 & upto));
             return m1 & upto ? 2 * kWave - 1 - __clzll((long long)(m1 & upto)) : 63 - __clzll((long long)m0);
         };
-        if (!even) {
+        if (!all) {
             // ---- how many of every child ----
             slot[lane] = ~0u;
             slot[kWave + lane] = ~0u;
@@ -224,7 +211,7 @@ __device__ __forceinline__ bool merge_rest(BlockScratch<RMAX> &s, int n0, int m,
         // ---- work them out ----
         uint32_t key[2] = {0u, 0u}, low[2] = {~0u, ~0u};
         bool valid[2] = {lane < total, kWave + lane < total};
-        if (even) {
+        if (all) {
 #pragma unroll
             for (int h = 0; h < 2; h++) valid[h] = valid[h] && child[h] < n0 && h * kWave + lane - from[h] < need;
         }
@@ -256,7 +243,7 @@ __device__ __forceinline__ bool merge_rest(BlockScratch<RMAX> &s, int n0, int m,
             bad |= valid[h] && !first && comes_before(key[h], low[h], pk, pl);
             if (!all) {
                 const uint64_t next = h == 0 ? (starts0 >> 1) | (starts1 << 63) : starts1 >> 1;
-                const bool end = even ? e + 1 - from[h] == 1 << log_e : e + 1 == total || ((next >> lane) & 1ull);  // of its child's
+                const bool end = e + 1 == total || ((next >> lane) & 1ull);  // of its child's
                 if (valid[h] && end && e + 1 - from[h] < need && comes_before(key[h], low[h], bk, bl)) {
                     bk = key[h];
                     bl = low[h];
@@ -370,8 +357,8 @@ __device__ __forceinline__ bool merge_rest(BlockScratch<RMAX> &s, int n0, int m,
     return true;
 }
 
-template <int RMAX, bool RAVE>
-__device__ __forceinline__ bool merge_heads(BlockScratch<RMAX> &s, int n0, int m, float ep, uint32_t uvl,
+template <bool RAVE>
+__device__ __forceinline__ bool merge_heads(BlockScratch &s, int n0, int m, float ep, uint32_t uvl,
                                             uint32_t floor_key, int lane, int &visits) {
     visits = 0;
     if (n0 == 0) return false;
@@ -456,7 +443,7 @@ __device__ __forceinline__ bool merge_heads(BlockScratch<RMAX> &s, int n0, int m
         done += total < need ? total : need;
         if (done < m && 4 * total < need) {  // as many of every child is not what it takes
             visits = s.taken[lane];
-            return merge_rest<RMAX, RAVE>(s, n0, m, ep, uvl, floor_key, lane, done, visits);
+            return merge_rest<RAVE>(s, n0, m, ep, uvl, floor_key, lane, done, visits);
         }
     }
     visits = s.taken[lane];
@@ -512,7 +499,7 @@ __device__ __forceinline__ bool pick_few(uint32_t *order, bool mine, int child, 
 template <int RMAX, bool RAVE, bool ROWS>
 __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev f, SelectArgs a, int n_items, int n_singles,
                                                                       LoneOut out) {
-    __shared__ BlockLds<RMAX, ROWS> s;
+    __shared__ BlockLds<ROWS> s;
     const int lane = threadIdx.x & (kWave - 1), wv = uniform((int)threadIdx.x >> 6);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         *a.n_singles = n_singles;
@@ -556,7 +543,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
         }
     }
     __syncthreads();
-    BlockScratch<RMAX> &my = s.scratch[wv];
+    BlockScratch &my = s.scratch[wv];
     const uint32_t uvl = a.vl > 0 ? (uint32_t)a.vl : 0u;
     float c_puct = a.c_puct;
     asm volatile("" : "+v"(c_puct));  // (as above)
@@ -817,7 +804,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                                 wave_sync_memory();
                             }
                         } else if (n0 > 0) {
-                            serial = !merge_heads<RMAX, RAVE>(my, n0, m, ep, uvl, floor_key, lane, visits);
+                            serial = !merge_heads<RAVE>(my, n0, m, ep, uvl, floor_key, lane, visits);
                         }
                         replayed = serial && !together;
                     }

@@ -79,7 +79,8 @@ constexpr int kSortBins = 1 << kSortBits;
 // 194, 176, 195; 4096 Gomoku 181, 207, 199 and 167, 198, 188, Go with RAVE 151, 160, 124 and 142, 164, 129.
 constexpr int kWideTeamMin = 1024;
 static_assert(kWideTeamMin <= kHeavyMin, "what nodes of kHeavyMin visitors need is in that kernel");
-// (Eight wavefronts have 256 registers each: the widest class, of sixteen rounds, would keep 735 of its 512 in memory.)
+// (Eight wavefronts have 256 registers each: the widest class, of sixteen rounds, would spill 735 of them, 848 with RAVE, where
+// it spills 8 and 20 with four wavefronts.)
 template <int RMAX, bool HEAVY>
 constexpr bool kWideTeams = HEAVY && RMAX <= 6;
 template <bool WIDE>
@@ -2522,36 +2523,6 @@ __device__ __forceinline__ void team_merge(const SelectArgs &a, WaveLds<R> &lds,
     }
     if (goff >= 0) wait_stores();  // (the owner's join announces a slice's winners to other blocks)
     __syncthreads();
-}
-
-// A lower end of the key range with at least `least` and at most 64 of the keys that `count` counts at or above it,
-// found by halving; `top`: no key lies above it; 0: there is none (keys tied).
-template <typename Count>
-__device__ __forceinline__ uint32_t halve_to_lanes(const Count &count, uint32_t top, int least) {
-    uint32_t lo = 1u, hi = top + 1u;  // count(lo) > 64, count(hi) < least
-    while (hi - lo > 1u) {
-        const uint32_t mid = lo + ((hi - lo) >> 1);
-        const int n = count(mid);
-        if (n < least) hi = mid;
-        else if (n > kWave) lo = mid;
-        else return mid;
-    }
-    return 0u;
-}
-
-// Of a node's children only those can be chosen by its m visitors whose next entries are among the m first of all:
-// as long as fewer than m visitors have chosen, at least one of m better heads is still there.  For m <= 64 and more
-// children than lanes: a key with at least m and at most 64 heads at or above it.
-template <int R, bool RAVE>
-__device__ __forceinline__ uint32_t first_heads(const Kids<R, RAVE> &k, uint32_t best_key, int m) {
-    auto heads = [&](uint32_t T) {
-        int n = 0;
-#pragma unroll
-        for (int r = 0; r < R; r++) n += __popcll(__ballot(umax32(k.k1[r], k.k2[r]) >= T));
-        return n;
-    };
-    if (heads(1u) <= kWave) return 1u;
-    return halve_to_lanes(heads, wave_max_u32(best_key), m);
 }
 
 // ---- Chains of nodes whose visitors all follow one child ----
