@@ -51,6 +51,14 @@ static bool monotone(const Kid &c, float ep, uint32_t uvl, int j_last) {
                 : keys_provably_monotone<false>(c.n, c.w, c.p, c.vl, c.q2, ep, uvl, j_last);
 }
 
+static float key_score(uint32_t key) {  // what score_key gave it
+    const uint32_t b = key & 0x80000000u ? key & 0x7FFFFFFFu : ~key;
+    float f;
+    memcpy(&f, &b, sizeof(f));
+    return f;
+}
+static long cuts = 0;  // lists of entries that were cut short
+
 struct Played {
     std::vector<Entry> order;
     std::vector<int> taken;  // per child
@@ -71,10 +79,11 @@ static bool merge_rest(const std::vector<Kid> &k, const std::vector<int> &L, int
             c.push_back(n > 0 && n < need ? n + 1 : n);
             total += c.back();
         }
-        if (total > 128) {
+        if (total > 128) {  // in proportion, and one at least
+            const float f = (float)(128 - 16) / (float)total;
             total = 0;
             for (int &n : c) {
-                n = n > 1 ? 1 + (int)((float)(n - 1) * 0.1f) : n;
+                if (n > 1) n = 1 + (int)((float)(n - 1) * (L.size() > 16 ? 0.5f : 1.0f) * f);
                 total += n;
             }
         }
@@ -92,9 +101,34 @@ static bool merge_rest(const std::vector<Kid> &k, const std::vector<int> &L, int
             if (c[q] < need && last.key != 0u && (bar.key == 0u || last.before(bar))) bar = last;
         }
         std::vector<Entry> in;
+        const uint32_t above = std::max(bar.key, floor_key);
         for (const Entry &e : all)
-            if (e.key > floor_key && !bar.before(e)) in.push_back(e);
+            if (e.key > above) in.push_back(e);
+        if ((int)in.size() < need && bar.key > floor_key)  // (those on the bar's own key)
+            for (const Entry &e : all)
+                if (e.key == bar.key && !bar.before(e)) in.push_back(e);
         if (in.empty()) return false;
+        // far more than are needed: those from a key on that few lie above
+        if ((int)in.size() > need + 32) {
+            uint32_t top = 0u, cut = 0u;
+            for (const Entry &e : in) top = std::max(top, e.key);
+            float lo = key_score(above + 1u), hi = key_score(top);
+            for (int it = 0; it < 12; it++) {
+                const float mid = 0.5f * (lo + hi);
+                if (!(mid > lo && mid < hi)) break;
+                int n = 0;
+                for (const Entry &e : in) n += e.key >= score_key(mid);
+                if (n < need) {
+                    hi = mid;
+                } else {
+                    lo = mid;
+                    cut = score_key(mid);
+                    if (n <= need + 8) break;
+                }
+            }
+            in.erase(std::remove_if(in.begin(), in.end(), [&](const Entry &e) { return e.key < cut; }), in.end());
+            cuts++;
+        }
         std::sort(in.begin(), in.end(), [](const Entry &a, const Entry &b) { return a.before(b); });
         for (int r = 0; r < (int)in.size() && r < need; r++) {
             out.order.push_back(in[r]);
@@ -333,6 +367,7 @@ int main(int argc, char **argv) {
         if (m <= 64) hold(by_block(k, m, ep, uvl, lengths, slack, got), got, "block", block_yes, block_no);
         hold(team_merge(k, m, ep, uvl, lengths, got), got, "team", team_yes, team_no);
     }
+    printf("lists cut short: %ld\n", cuts);
     printf("blocks: merged %ld, declined %ld; teams: merged %ld, declined %ld; wrong %ld\n", block_yes, block_no, team_yes, team_no,
            wrong);
     return wrong != 0;

@@ -201,6 +201,8 @@ def test_merge_rules_against_the_serial_loop(tmp_path):
     assert out.returncode == 0, out.stdout[-2000:]
     m = re.search(r"blocks: merged (\d+), declined \d+; teams: merged (\d+), declined \d+; wrong 0", out.stdout)
     assert m and int(m.group(1)) > 30000 and int(m.group(2)) > 30000, out.stdout[-500:]
+    m = re.search(r"lists cut short: (\d+)", out.stdout)
+    assert m and int(m.group(1)) > 30, out.stdout[-500:]
 
 
 def test_bounds_of_scores_hold_the_exact_ones(tmp_path):
