@@ -680,14 +680,17 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                 const uint64_t in_order = __ballot(together || in_order_at_once(tn, tw, tp, tvl, ep, uvl, j_last));
                 const uint32_t lane_top = ordered_bits(c1), top = (uint32_t)uniform((int)wave_max_all(lane_top));
                 const uint64_t tops = __ballot(lane_top == top);
-                if (__builtin_expect_with_probability(__ballot(!(odd == 0.0f)) != 0ull, 0, 0.999)) {
-                    // (not of what stands in an empty slot: in the loop above that would put up to 61 registers into memory)
+                serial = true;
+                bool real = __ballot(!(odd == 0.0f)) == 0ull;
+                if (__builtin_expect_with_probability(!real, 0, 0.999)) {
+                    // (not of what stands in an empty slot.  In the loop above that would put up to 61 registers into memory;
+                    // between it and the reductions just made it would keep them apart: 64 visitors of a Go tree 37 -> 39 us)
                     odd = 0.0f;
 #pragma unroll
                     for (int r = 0; r < RMAX; r++) odd = fmaf(ceil[r], 0.0f, odd);
+                    real = __ballot(!(odd == 0.0f)) == 0ull;
                 }
-                serial = true;
-                if (__builtin_expect_with_probability(__ballot(!(odd == 0.0f)) == 0ull && top > ordered_bits(kLeastScore), 1, 0.999)) {
+                if (__builtin_expect_with_probability(real && top > ordered_bits(kLeastScore), 1, 0.999)) {
                     // ---- does that child win every time?  Its last entry comes before every other child's next one ----
                     const int bl = __ffsll((long long)tops) - 1;
                     const float last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lane_last), bl));
