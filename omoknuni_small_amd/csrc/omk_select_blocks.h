@@ -816,6 +816,7 @@ __global__ __launch_bounds__(kBlockWaves *kWave) void k_select_blocks(ForestDev 
                     // ---- one visitor after the other (no real score, values that are not finite, a child that was
                     // not listed); the children once more, which spares the ways above the registers ----
                     ask();
+                    __builtin_amdgcn_s_waitcnt(0x0F70);  // (as above: else the loop waits in front of its loads, on every way)
                     int cnt[RMAX];
 #pragma unroll
                     for (int r = 0; r < RMAX; r++) {
