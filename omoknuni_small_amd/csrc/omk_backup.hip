@@ -404,7 +404,9 @@ constexpr int kRaveMaxLen = 4097;  // longest path the ABI accepts
 
 // One block per (traversal, depth): the path's actions go to LDS, the node's children are spread over the threads.  What bounds
 // it is a chain of trips to memory (length, node, children's range, their actions); a wavefront alone made the last of them
-// six times for the 362 children of a Go node.  48 paths: 6.2 -> 3.8 us.
+// six times for the 362 children of a Go node.  A call, us, with 64 threads and with 256: Go 48 paths 5.4 and 3.7, 1024 27 and 23,
+// 16384 250 and 213; Gomoku 256 paths 17.6 and 13.2, 16384 512 and 466.  The three wavefronts that a narrow node leaves idle cost
+// 0.5 to 1 % from 1024 paths on (35 children on average, 4096 paths 133 and 134; 9 children 129 and 131) and nothing below.
 constexpr int kRaveThreads = 256;
 __global__ __launch_bounds__(kRaveThreads) void k_rave_backup(ForestMut f, const int32_t *paths, const int32_t *path_len,
                                                     const float *values, int n, int stride) {

@@ -150,10 +150,10 @@ hipError_t launch_select(const ForestDev &f, const SelectArgs &a, int n_items0, 
 
 // The same for a batch whose roots have few visitors each (omk_select_blocks.h): a block a root, without a reset.  The
 // line lies at a visitor per lane and at the children that fit its registers (with 128 for each of 16 wavefronts).  Below
-// it the blocks are the faster ones throughout but for crowds with RAVE that stay together (32 % faster to 11 % slower at 64
-// visitors, where two entries of each of many children settle few of them a pass).  A selection and its reverting, us, of
-// the queue's kernel and of theirs: Gomoku 1 tree x 8 43 and 25, 1 x 64 75 and 55, 64 x 16 66 and 37, 64 x 64 106 and 71,
-// 256 x 24 146 and 31, 4096 x 2 298 and 98; Go re-laid 64 x 16 72 and 42, chess-like 64 x 16 98 and 46, 2048 x 4 206 and 73.
+// it the blocks are the faster ones throughout.  A selection and its reverting, us, of the queue's kernel and of theirs, the
+// median of three seeds: Gomoku 1 tree x 8 59 and 27, 1 x 64 73 and 40, 64 x 16 56 and 24, 64 x 64 73 and 30, 256 x 24 125 and
+// 24, 4096 x 2 291 and 79; Go with RAVE 1 x 8 26 and 11, 1 x 48 42 and 24, 1 x 64 68 and 35, 16 x 64 61 and 32; Go re-laid
+// 64 x 16 55 and 25, chess-like 64 x 16 89 and 46, 2048 x 4 203 and 73.
 constexpr int kBlockMax = 64;       // visitors of one root, at most
 constexpr int kBlockFanout = 384;   // widest node
 inline bool by_blocks(int n_items0, int most_visitors, int max_fanout) {

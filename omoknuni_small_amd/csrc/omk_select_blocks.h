@@ -10,10 +10,12 @@
 // instruction issue of the wavefront that settles the node, 5 cycles an instruction and 8 to 10 where each needs the one
 // before.  So most children are ruled out by bounds of their scores (score_about: two reciprocals where the score takes two
 // IEEE divisions), which settles a node whose visitors stay together, and a lone visitor's, without a division: a level of
-// four rounds 2.5 -> 1.75 us, of which scoring 0.7 -> 0.23 and the test of the best child 0.5 -> 0.15.  Where the bounds leave
-// several children the exact scores of these few decide.  A selection of a tree fresh from an upload: 8 visitors 28 -> 24 us,
-// 64 57 -> 42, 16 in each of 64 Go trees 42 -> 32; of one that thousands of batches have been backed up into, where most
-// nodes are contested, 64 x 16 -4 %, the others as before.
+// four rounds 2.5 -> 1.8 us in the timeline.  Where the bounds leave several children the exact scores of these few decide.
+// A selection and its reverting, us, with scores first and with bounds first, the median of five seeds: of trees fresh from an
+// upload 8 visitors of a Gomoku tree 25 -> 19, 64 49 -> 32, 48 of a Go tree with RAVE 36 -> 22, 64 of a chess-like one 39 -> 31,
+// 64 in each of 16 47 -> 35; of trees that 2000 batches have been backed up into, where most nodes are contested, 26 -> 22,
+// 37 -> 34, 53 -> 44, 34 -> 35, 32 -> 33: nodes of one round have two divisions to lose and contested ones keep them.  (Lone
+// visitors of 200 such chess-like trees 15 -> 16; 8 in one 26 -> 26, 16 in each of 64 31 -> 32.)
 #pragma once
 
 #include "omk_select_kernels.h"

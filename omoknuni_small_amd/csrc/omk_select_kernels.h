@@ -77,6 +77,10 @@ constexpr int kSortBins = 1 << kSortBits;
 // 133, 136 and 133, 130, 134, Go with RAVE 101, 104, 103 and 95, 101, 99, chess-like (with seven) 162, 149, 187 and 169, 155,
 // 190; 1600 Gomoku 150, 145, 161 and 140, 140, 150, Go re-laid 137, 152, 168 and 134, 141, 155, chess-like 203, 175, 196 and
 // 194, 176, 195; 4096 Gomoku 181, 207, 199 and 167, 198, 188, Go with RAVE 151, 160, 124 and 142, 164, 129.
+// The most crowded root decides for the whole batch.  Smaller crowds beside it lose nothing, because the launch has twice the
+// walkers as well (kMaxWalkerBlocks): a root of 1024 and 200 of 65 to 200, with three and seven, Gomoku 195, 206, 197 and 147,
+// 155, 149, Go with RAVE 100, 100, 97 and 91, 91, 89, chess-like 113, 113, 115 and 112, 114, 115; with 40 of these 67, 88, 89 and
+// 65, 82, 81, 76, 71, 68 and 72, 72, 68, 97, 106, 100 and 97, 106, 100; with 1000 of 8 229, 232, 231 and 170, 171, 169.
 constexpr int kWideTeamMin = 1024;
 static_assert(kWideTeamMin <= kHeavyMin, "what nodes of kHeavyMin visitors need is in that kernel");
 // (Eight wavefronts have 256 registers each: the widest class, of sixteen rounds, would spill 735 of them, 848 with RAVE, where
@@ -92,7 +96,11 @@ constexpr int kCountSortLone = 2, kCountSortTeam = 1;
 constexpr int kRunShortcutMin = 128;      // entries from which a run of one child is emitted without sorting
 constexpr int kScatterPart = 256;         // visitors per part of a heavy node's partition, about
 constexpr int kScatterUnroll = 8;         // chunks of 64 visitors whose loads the partition issues together
-constexpr int kMaxWalkerBlocks = 16;         // blocks of walkers of the persistent launch, at most
+// Blocks of walkers of the persistent launch, at most: 64 wavefronts, 128 in the launch with teams of eight.  Idle ones poll and
+// slow the teams: with 64 there too one crowd of 1024 to 16384 takes 2 to 5 us less (1 to 3 %).  But a batch that leaves many
+// visitors alone takes 20 to 60 % longer then (the root of 1024 and 200 smaller ones above: Gomoku 228, 240, 233 us, Go with RAVE
+// 111, 111, 107).
+constexpr int kMaxWalkerBlocks = 16;
 constexpr int kTeamSinglesMaxWaves = 4096;  // wavefronts up to which a batch of lone traversals is walked by blocks (one round of children per wavefront)
 constexpr int kFastSinglesMax = 16384;    // traversals up to which the single-visitor kernel trades bytes for latency
 constexpr int kRunShareMin = 4096;        // a node whose visitors all take one child: visitors from which the scatter
@@ -4653,7 +4661,7 @@ hipError_t launch_select_class(const ForestDev &f, const SelectArgs &a0, int n_i
         const int waves = heavy ? kTeamWaves<kWideTeams<RMAX, true>> : kTeamWaves<false>;
         int walkers = n_traversals / waves;
         if (walkers > capacity / 4) walkers = capacity / 4;
-        if (walkers > kMaxWalkerBlocks) walkers = kMaxWalkerBlocks;  // idle walkers poll: more of them slow the teams
+        if (walkers > kMaxWalkerBlocks) walkers = kMaxWalkerBlocks;
         // (a wavefront per visitor while that is at most kMaxWalkerBlocks: the root of a young tree leaves nearly
         // every visitor of a small batch alone, and 64 of them on 16 walkers took four rounds, 26 us of 54)
         if (walkers < 4) walkers = 4;
