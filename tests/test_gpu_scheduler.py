@@ -381,6 +381,17 @@ def test_crowds_on_both_sides_of_the_wider_teams(fan, rave, m):
     assert st["replayed_nodes"] == 0, st
 
 
+@pytest.mark.parametrize("fan,rave", [(225, False), (362, True)])
+@pytest.mark.parametrize("most", [1023, 1024, 1536])
+def test_smaller_crowds_beside_the_one_that_makes_teams_wide(fan, rave, most):
+    """The most crowded root decides how many wavefronts the teams of the whole batch have: crowds of all sizes and lone
+    visitors beside it."""
+    soa, roots = layered_forest(37, [fan, 20], n_trees=9, rave=rave)
+    troots = np.repeat(roots, [most, 200, 96, 95, 65, 64, 8, 2, 1]).astype(np.int32)
+    st = select_both(soa, np.random.default_rng(most).permutation(troots), 3, rave=rave)
+    assert st["replayed_nodes"] == 0, st
+
+
 @pytest.mark.parametrize("n", [2, 64, 255, 256, 257])
 @pytest.mark.parametrize("vl,rave", [(3, True), (3, False), (0, True)])
 @pytest.mark.parametrize("trees", [1, 2])
