@@ -237,6 +237,18 @@ def test_tickets_are_drawn_between_barriers_of_the_wavefront():
     assert len(re.findall(r"= take_ticket\(", text)) == 4
 
 
+def test_loads_of_a_node_are_waited_for_where_they_are_made():
+    """A wavefront of a block asks for a node's children in two places.  Loads that are not known done where its loop comes
+    round make the compiler wait in front of the next node's, and for the stores of the level before with them: all of
+    them are waited for (vmcnt 0), in both places, before anything but what may overlap with them."""
+    import re
+    with open(os.path.join(ROOT, "omoknuni_small_amd", "csrc", "omk_select_blocks.h")) as f:
+        text = re.sub(r"//[^\n]*", "", f.read())
+    asked = re.findall(r"\n\s*ask\(\);(.*?)__builtin_amdgcn_s_waitcnt\(0x0F70\);", text, re.S)
+    assert len(asked) == 2 and len(re.findall(r"\bask\(\);", text)) == 2
+    assert not any(re.search(r"\bk\.|\bsp\[|\bword\[", between) for between in asked)
+
+
 def test_stores_for_other_blocks_are_waited_for_by_who_made_them():
     """A helper's stores that its owner, or another helper, announces to other blocks with a release of agent scope: that
     release waits for the announcing wavefront's own stores, a release of workgroup scope and a block barrier for none in
